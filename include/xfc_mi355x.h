@@ -114,13 +114,13 @@ int xfc_fwd_grad_coo(const void* X, int64_t ldx, const void* W, int64_t ldw,
 /*
  * xfc_fwd_grad_csr for callers that cannot allocate device memory or hand over a workspace (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the
- * reference.  Same arguments and results as xfc_fwd_grad_csr minus the workspace: the label buckets
- * live in a fixed XFC_STATIC_SCRATCH_BYTES array inside the library's device image (one copy per GPU,
- * held until the process ends), and the call makes no hipMalloc / hipFree.  Problems whose bucket
- * tables do not fit (xfc_fwd_grad_workspace_bytes(L, nnz) > XFC_STATIC_SCRATCH_BYTES, i.e. beyond
- * about 16.7 M labels with 190 k positives) are rejected with XFC_ERR_LIMIT.  All calls on one GPU
- * share that GPU's array: calls that overlap in time on one GPU (two streams, two threads) race;
- * calls in sequence are independent, every table being rebuilt from scratch by each call.
+ * reference.  Same arguments and results as xfc_fwd_grad_csr minus the workspace: the scratch of the
+ * loss is a fixed XFC_STATIC_SCRATCH_BYTES array inside the library's device image (one copy per GPU,
+ * held until the process ends), and the call makes no hipMalloc / hipFree.  Problems whose scratch
+ * does not fit (xfc_fwd_grad_workspace_bytes(L, nnz) > XFC_STATIC_SCRATCH_BYTES, i.e. beyond
+ * about 520 k positives) are rejected with XFC_ERR_LIMIT.  All calls on one GPU
+ * share that GPU's array: calls with a loss that overlap in time on one GPU (two streams, two threads) race;
+ * calls in sequence are independent.
  * Call xfc_init() once per device beforehand (it looks the array's device address up).
  */
 #define XFC_STATIC_SCRATCH_BYTES (2 * 1024 * 1024)

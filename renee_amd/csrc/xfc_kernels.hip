@@ -1,6 +1,6 @@
 // XFC layer step kernels for gfx950 and their C-ABI entry points.
 //
-//   fwd   : G = fp16( sigmoid(X . W^T) - Y )      Y from per-label-tile positive buckets
+//   fwd   : G = fp16( sigmoid(X . W^T) - Y )      Y subtracted pair by pair after the product
 //   dx    : dX = scale * G . W                    split over labels, fp32 partials + reduce
 //   dw    : dW = G^T . X, consumed in the tile by  M = mu*M + dW + wd*W ; W -= lr*M
 // plus the plain six-argument GEMM the reference extension exposes.
@@ -14,6 +14,7 @@
 
 #include "../../include/xfc_mi355x.h"
 #include "pipe_core.hpp"
+#include "wide_core.hpp"
 
 namespace xfc {
 
@@ -37,119 +38,28 @@ __device__ __forceinline__ void xcd_map(int id, int n_inner, int& inner, int& ou
 }
 
 // ---------------------------------------------------------------------------------------------
-// positives: bucket a sparse label list by label tile
-// ---------------------------------------------------------------------------------------------
-// One workgroup.  Input is CSR (rowptr/colidx, pos_x == nullptr) or COO (pos_x/pos_y int64).
-// Output: bucket_ptr[n_tiles+1] and (ent_row, ent_col)[nnz] grouped by col / tile_w.
-// Pairs whose row or column is out of range are dropped.  The per-tile counters live in LDS when
-// they fit (IN_LDS, n_tiles <= BUCKET_LDS_TILES) and in the global scratch array `cursor` otherwise.
-// Both inputs are walked by entry, one coalesced load per thread and pass: a CSR entry finds its row by a
-// binary search of the row pointers, which are staged in LDS when they fit (ROWS_IN_LDS) and searched where they
-// are otherwise.  (One row per thread, each thread reading its row's labels one after the other, costs as many
-// dependent round trips as the longest row has labels: 17 us instead of 11 at 512 rows.)
-constexpr int BUCKET_LDS_TILES = 12288;
-constexpr int BUCKET_DYN_LDS_MAX = 56 * 1024;  // next to the 4 KB of scan scratch, within the default 64 KB
-
-template <bool IN_LDS, bool ROWS_IN_LDS>
-__global__ void __launch_bounds__(1024) bucket_positives_kernel(
-    const int32_t* __restrict__ rowptr, const int32_t* __restrict__ colidx, const int64_t* __restrict__ pos_x,
-    const int64_t* __restrict__ pos_y, int64_t nnz, int B, int64_t L, int tile_w, int n_tiles,
-    int32_t* __restrict__ bucket_ptr, int32_t* __restrict__ cursor_g, int32_t* __restrict__ ent_row,
-    int32_t* __restrict__ ent_col) {
-  __shared__ int32_t wave_tot[16];
-  extern __shared__ int32_t dyn_l[];
-  int32_t* cursor = IN_LDS ? dyn_l : cursor_g;
-  int32_t* rows_l = dyn_l + (IN_LDS ? n_tiles : 0);  // ROWS_IN_LDS: rowptr[0..B]
-  const int32_t* rows = ROWS_IN_LDS ? rows_l : rowptr;
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  for (int i = t; i < n_tiles; i += 1024) cursor[i] = 0;
-  if constexpr (ROWS_IN_LDS)
-    for (int i = t; i <= B; i += 1024) rows_l[i] = rowptr[i];
-  __syncthreads();
-  // pass 0 counts, pass 1 places
-  auto walk = [&](auto visit) {
-    if (pos_x) {
-      for (int64_t p = t; p < nnz; p += 1024) {
-        const int64_t r = pos_x[p], c = pos_y[p];
-        if (r >= 0 && r < B && c >= 0 && c < L) visit((int)r, (int)c);
-      }
-    } else {
-      // whatever the row pointers hold, only colidx[0 .. nnz) is read and every entry is visited at most once
-      const int64_t p0 = rows[0] > 0 ? rows[0] : 0;
-      const int64_t p1 = rows[B] < nnz ? rows[B] : nnz;
-      for (int64_t p = p0 + t; p < p1; p += 1024) {
-        const int64_t c = colidx[p];
-        int lo = 0, hi = B;  // the row b with rowptr[b] <= p < rowptr[b + 1]: first b whose rowptr[b + 1] > p
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (rows[mid + 1] > p) hi = mid; else lo = mid + 1;
-        }
-        if (lo < B && c >= 0 && c < L) visit(lo, (int)c);
-      }
-    }
-  };
-  walk([&](int, int c) { atomicAdd(&cursor[c / tile_w], 1); });
-  __syncthreads();
-  // exclusive scan of the per-tile counts: each thread owns `per` consecutive tiles; lanes scan by shuffles,
-  // the sixteen waves' totals go through LDS
-  const int per = (n_tiles + 1023) / 1024;
-  const int lo = t * per, hi = min(n_tiles, lo + per);
-  int s = 0;
-  for (int i = lo; i < hi; ++i) s += cursor[i];
-  int inc = s;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int v = __shfl_up(inc, off, 64);
-    if (lane >= off) inc += v;
-  }
-  if (lane == 63) wave_tot[wave] = inc;
-  __syncthreads();
-  int before = 0, total = 0;
-#pragma unroll
-  for (int w = 0; w < 16; ++w) {
-    const int v = wave_tot[w];
-    if (w < wave) before += v;
-    total += v;
-  }
-  int run = before + inc - s;
-  for (int i = lo; i < hi; ++i) {
-    const int c = cursor[i];
-    bucket_ptr[i] = run;
-    cursor[i] = run;
-    run += c;
-  }
-  if (t == 1023) bucket_ptr[n_tiles] = total;
-  __syncthreads();
-  walk([&](int r, int c) {
-    const int at = atomicAdd(&cursor[c / tile_w], 1);
-    ent_row[at] = r;
-    ent_col[at] = c;
-  });
-}
-
-// ---------------------------------------------------------------------------------------------
 // forward: out = epilogue(alpha * X . W^T + beta * out)
 // ---------------------------------------------------------------------------------------------
-enum FwdMode { FWD_LINEAR = 0, FWD_SIGMOID = 1, FWD_GRAD = 2, FWD_SIGMOID_PLAIN = 3 };  // PLAIN: alpha 1, beta 0
+enum FwdMode { FWD_LINEAR = 0, FWD_SIGMOID = 1, FWD_SIGMOID_PLAIN = 2 };  // PLAIN: alpha 1, beta 0
 
-// Three row-tile heights: 256 rows for training batches, 128 and 64 for small batches (the reference's
-// B = 32 plumbing case, --accum micro-batches, the last partial batch of an epoch), where a 256-row tile
-// would spend most of its MFMAs on padding.  The label tile is 256 wide in all of them (it is also the
-// width of the positives' buckets).  The smaller tiles leave room for a third ring slot.
+// Batches above 128 rows: 256 labels (the A side, contiguous in the output) x 256 rows, W running ahead.
+using FwdWide = WideCore<256, 256, 2, 2, true, true, AHEAD_A>;
+static_assert(FwdWide::LDS_BYTES <= 160 * 1024, "LDS budget");
+// Batches of up to 128 and 64 rows (the reference's B = 32 plumbing case, --accum micro-batches, the last partial batch
+// of an epoch), where a 256-row tile would spend most of its MFMAs on padding: W streams from HBM, eight waves, three
+// ring slots.  FwdCore is the top-K pass's 256-row tile, whose candidate lists take the LDS of a third slot.
 using FwdCore = PipeCore<256, 256, 64, 2, 4, 2, true, true, false, false, false, 4>;  // one wave per SIMD fetches
 using FwdCore128 = PipeCore<128, 256, 64, 2, 4, 3, true, true, false, false, false, 4>;
 using FwdCore64 = PipeCore<64, 256, 64, 2, 4, 3, true, true, false, false, false, 4>;
-// beside the ring: the tile's positives bitmap, later reused as store staging (8 rows x TN labels per wave)
+// beside the ring: store staging (8 rows x TN labels per wave)
 template <class C>
 struct FwdLds {
   static constexpr int STG_HALVES = 8 * C::TN;
-  static constexpr int BITMAP_BYTES = C::BN * (C::BM / 32) * 4;
-  static constexpr int AUX_BYTES = BITMAP_BYTES > C::NW * STG_HALVES * 2 ? BITMAP_BYTES : C::NW * STG_HALVES * 2;
-  static constexpr int BYTES = C::LDS_BYTES + AUX_BYTES;
+  static constexpr int BYTES = C::LDS_BYTES + C::NW * STG_HALVES * 2;
   static_assert(C::FN % 2 == 0, "staging read-back walks 64-label pieces");
-  static_assert(C::BN == 256 && C::NT == 512, "bucket width and workgroup size are shared by all row-tile heights");
   static_assert(BYTES <= 160 * 1024, "LDS budget");
 };
+static_assert(FwdCore::BN == FwdWide::BM && FwdCore128::BN == FwdWide::BM && FwdCore64::BN == FwdWide::BM, "one label tile width");
 
 struct FwdArgs {
   const half_t* X; int64_t ldx;     // M x K, K-contiguous
@@ -157,26 +67,136 @@ struct FwdArgs {
   half_t* out; int64_t ldo;         // M x n_store, row-major
   int M, N, K, n_store;             // columns N <= c < n_store are written as zero
   float alpha, beta;
-  const int32_t* bucket_ptr; const int32_t* ent_row; const int32_t* ent_col;
-  float* loss_part;                 // FWD_GRAD with LOSS: one partial sum per workgroup
+  float* loss_part;                 // LOSS: one partial sum per workgroup
   int tiles_m, tiles_n, n_ids;      // n_ids = tiles_m * round_up(tiles_n, 8)
 };
 
 // Persistent: workgroup w takes tile ids w, w + gridDim.x, ... (gridDim.x a multiple of 8, so an
 // id keeps its XCD and the row tiles of one label tile run side by side on one L2).
+template <int MODE, bool BETA, bool LOSS = false>
+__global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
+  using C = FwdWide;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
+  half_t* lds = reinterpret_cast<half_t*>(smem_raw);
+  const int G = gridDim.x, w = blockIdx.x;
+  const int n_items = (a.n_ids - w + G - 1) / G;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be
+  const int wm = wave / C::WN, wn = wave % C::WN;
+  float loss_acc = 0.f;  // LOSS: this lane's share of sum softplus(z)
+
+  auto get = [&](int item, C::Operand& oa, C::Operand& ob, int& kb, int& ke) {
+    int mt, nt;
+    xcd_map(item * G + w, a.tiles_m, mt, nt);
+    oa = C::Operand{a.W, a.ldw, nt < a.tiles_n ? nt * C::BM : 0, a.N, a.K};
+    ob = C::Operand{a.X, a.ldx, mt * C::BN, a.M, a.K};
+    kb = 0;
+    ke = a.K;
+  };
+  // A lane owns one batch row and eight consecutive labels of every 32: 16-byte stores straight from the registers,
+  // 64 bytes per row and instruction, the other 64 of the line with the next.  Of a tile's 54,000 cycles this takes
+  // 10,000: the two transcendentals of a sigmoid occupy a SIMD for 32 cycles per 64 elements, which with the conversions
+  // is 9,200 (2,900 without the sigmoid), and the stores hide under them; the wait for the last of them to be written,
+  // in the next tile's first stage, is another 1,900.  Stores of whole lines (8 rows x 128 or 4 x 256 bytes per
+  // instruction) take as long: all CUs together store at 7.3 TB/s into the caches whatever the shape.
+  auto epilogue = [&](int item, float4v (&acc)[C::FM][C::FN]) {
+    int mt, nt;
+    xcd_map(item * G + w, a.tiles_m, mt, nt);
+    if (nt >= a.tiles_n) return;
+    const int row_l = mt * C::BN + wn * C::TN + (lane & 15);
+    const int col_l = nt * C::BM + wm * C::TM + 8 * (lane >> 4);
+    // A tile that crosses the label count is compiled as a path of its own: the common one carries no column checks.
+    auto body = [&](auto edge_tag) {
+      constexpr bool EDGE = decltype(edge_tag)::value;
+#pragma unroll
+      for (int fn = 0; fn < C::FN; ++fn) {
+        const int row = row_l + 16 * fn;
+        half_t* dst = a.out + (int64_t)row * a.ldo + col_l;
+        const bool row_in = row < a.M;
+#pragma unroll
+        for (int p = 0; p < C::FM / 2; ++p) {
+          const int col = col_l + 32 * p;
+          const float4v lo = C::value(acc[2 * p][fn]), hi = C::value(acc[2 * p + 1][fn]);
+          float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          if constexpr (LOSS) {
+            static_assert(MODE == FWD_SIGMOID_PLAIN && !BETA, "the loss is that of the plain logits");
+            // softplus(z) = max(z, 0) + log(1 + e^-|z|) (dl_base.py:578-583); the logarithms of a lane's eight factors in
+            // (1, 2] are taken as one, of their product.  (With one logarithm per element and the sum formed at the end of
+            // the tile the kernel spilled 800 registers: 234 us at 199 x 131,072 x 768, now 90.)
+            float prod = 1.f, lin = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const float t = 1.0f + __builtin_amdgcn_exp2f(fabsf(v[e]) * -1.44269504088896341f);
+              const bool in = !EDGE || col + e < a.N;
+              prod *= in ? t : 1.f;
+              lin += in ? fmaxf(v[e], 0.f) : 0.f;
+            }
+            const float s = lin + 0.69314718056f * __builtin_amdgcn_logf(prod);
+            loss_acc += row_in ? s : 0.f;
+            asm volatile("" : "+v"(loss_acc));  // here, not when the tile is done: that would keep every element until then
+          }
+          if constexpr (BETA) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              v[e] *= a.alpha;
+              if (row_in && col + e < a.N) v[e] += a.beta * (float)dst[32 * p + e];
+            }
+          } else if constexpr (MODE == FWD_SIGMOID) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] *= a.alpha;
+          }
+          if constexpr (MODE != FWD_LINEAR) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = sigmoidf_fast(v[e]);
+          }
+          half8 v8;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v8[e] = !EDGE || col + e < a.N ? (half_t)v[e] : (half_t)0.f;
+          if (row_in) {
+            if (!EDGE || col + 8 <= a.n_store) {
+              // (a non-temporal store of half a line is written back before the other half comes: 1.19 against 1.14 ms)
+              *reinterpret_cast<half8*>(dst + 32 * p) = v8;
+            } else {
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                if (col + e < a.n_store) dst[32 * p + e] = v8[e];
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);  // eight elements in flight are enough; more of them spill
+        }
+      }
+    };
+    if (nt * C::BM + C::BM > a.N) body(std::true_type{});
+    else body(std::false_type{});
+  };
+  C::run(0, n_items, lds, get, epilogue);
+  if constexpr (LOSS) {
+    // deterministic: lanes -> wave (butterfly), waves -> workgroup (LDS, fixed order), one partial per workgroup
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off, 64);
+    float* red = reinterpret_cast<float*>(smem_raw);
+    __syncthreads();
+    if (lane == 0) red[wave] = loss_acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      float t = 0.f;
+      for (int i = 0; i < C::NW; ++i) t += red[i];
+      a.loss_part[w] = t;
+    }
+  }
+}
+
+// The same on the smaller row tiles.
 template <class C, int MODE, bool BETA, bool LOSS = false>
 __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
   constexpr int FWD_STG_HALVES = FwdLds<C>::STG_HALVES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   half_t* lds = reinterpret_cast<half_t*>(smem_raw);
-  // beside the ring: first the tile's positives bitmap, then per-wave store staging
-  uint32_t* bm = reinterpret_cast<uint32_t*>(smem_raw + C::LDS_BYTES);
   const int G = gridDim.x, w = blockIdx.x;
   const int n_items = (a.n_ids - w + G - 1) / G;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be
   const int wm = wave / C::WN, wn = wave % C::WN;
-  half_t* stg = reinterpret_cast<half_t*>(bm) + wave * FWD_STG_HALVES;  // 8 rows x TN labels
-  float loss_acc = 0.f;  // LOSS: this lane's share of sum softplus(z) - sum z[positives]
+  half_t* stg = reinterpret_cast<half_t*>(smem_raw + C::LDS_BYTES) + wave * FWD_STG_HALVES;  // 8 rows x TN labels
+  float loss_acc = 0.f;  // LOSS: this lane's share of sum softplus(z)
 
   auto get = [&](int item, typename C::Operand& oa, typename C::Operand& ob, int& kb, int& ke) {
     int mt, nt;
@@ -191,71 +211,33 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
     xcd_map(item * G + w, a.tiles_m, mt, nt);
     if (nt >= a.tiles_n) return;
     const int m0 = mt * C::BM, n0 = nt * C::BN;
-    // positives of this tile -> bitmap [label][row word] -> one word per 32x32 block and lane
-    uint32_t words[C::FM][C::FN];
-#pragma unroll
-    for (int fm = 0; fm < C::FM; ++fm)
-#pragma unroll
-      for (int fn = 0; fn < C::FN; ++fn) words[fm][fn] = 0u;
-    bool has_pos = false;
-    if constexpr (MODE == FWD_GRAD) {
-      // read through the scalar path (the tile id is uniform and the table is read-only here): a vector
-      // load would make the compiler wait for every outstanding vector-memory operation before the first
-      // use, which includes the next tile's operand fetches that the main loop has just issued
-      typedef const int32_t __attribute__((address_space(4))) * const_i32_ptr;
-      const const_i32_ptr bp = (const_i32_ptr)(uintptr_t)a.bucket_ptr;
-      const int s = bp[nt], e = bp[nt + 1];
-      has_pos = e > s;
-      if (has_pos) {
-        __syncthreads();  // every wave is done staging the previous tile
-        for (int i = threadIdx.x; i < C::BN * (C::BM / 32); i += C::NT) bm[i] = 0u;
-        __syncthreads();
-        for (int p = s + threadIdx.x; p < e; p += C::NT) {
-          const int r = a.ent_row[p] - m0, c = a.ent_col[p] - n0;
-          if (r >= 0 && r < C::BM) atomicOr(&bm[c * (C::BM / 32) + (r >> 5)], 1u << (r & 31));
-        }
-        __syncthreads();
-#pragma unroll
-        for (int fm = 0; fm < C::FM; ++fm)
-#pragma unroll
-          for (int fn = 0; fn < C::FN; ++fn)
-            words[fm][fn] = bm[(wn * C::TN + fn * 32 + (lane & 31)) * (C::BM / 32) + ((wm * C::TM + fm * 32) >> 5)];
-        __syncthreads();  // bitmap consumed: the area is staging again
-      }
-    }
     const int h = lane >> 5;
     constexpr int CHS = C::TN / 8;  // 16-byte chunks per staged row
-    // The per-element work below is the vector ALU cost of the whole tile (the SIMD cannot overlap it
-    // with MFMAs), so the rare cases -- a tile holding positives, a tile crossing the label count -- are
-    // compiled as separate paths and the common one carries neither.
+    // A tile that crosses the label count is compiled as a path of its own: the common one carries no column checks.
     int64_t lane_off[C::FN / 2];  // where this lane's 16 bytes of a staged strip go, relative to the strip
 #pragma unroll
     for (int p = 0; p < C::FN / 2; ++p) lane_off[p] = (int64_t)((lane + 64 * p) / CHS) * a.ldo + ((lane + 64 * p) % CHS) * 8;
-    auto body = [&](auto pos_tag, auto edge_tag) {
-      constexpr bool POS = decltype(pos_tag)::value, EDGE = decltype(edge_tag)::value;
-      float tile_loss = 0.f;
+    auto body = [&](auto edge_tag) {
+      constexpr bool EDGE = decltype(edge_tag)::value;
       if constexpr (LOSS) {
-        static_assert(MODE == FWD_GRAD && !BETA, "the loss is that of the plain logits");
-        // The loss terms in a pass of their own over the accumulators, one block at a time: interleaved
-        // with the sigmoid and the staging below, the scheduler keeps dozens of elements in flight to
-        // hide the transcendentals' latency and spills hundreds of registers.
-        // softplus(z) = max(z,0) + log(1 + e^-|z|), minus z where the label is positive (dl_base.py:578-583)
+        static_assert(MODE == FWD_SIGMOID_PLAIN && !BETA, "the loss is that of the plain logits");
+        // The loss terms in a pass of their own over the accumulators, one block at a time (see fwd_wide_kernel)
 #pragma unroll
         for (int fm = 0; fm < C::FM; ++fm)
 #pragma unroll
           for (int fn = 0; fn < C::FN; ++fn) {
             const int ecol = n0 + wn * C::TN + fn * 32 + (lane & 31);
+            float prod = 1.f, lin = 0.f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
               const float v = acc[fm][fn][r];
-              float t = fmaxf(v, 0.f) + 0.69314718f * __log2f(1.0f + __expf(-fabsf(v)));
-              if constexpr (POS) t -= v * (float)((words[fm][fn] >> c_row(r, lane)) & 1u);
-              if constexpr (EDGE) {
-                const int erow = m0 + wm * C::TM + fm * 32 + c_row(r, lane);
-                t = (erow < a.M && ecol < a.N) ? t : 0.f;
-              }
-              tile_loss += t;
+              const float t = 1.0f + __builtin_amdgcn_exp2f(fabsf(v) * -1.44269504088896341f);
+              const bool in = !EDGE || (m0 + wm * C::TM + fm * 32 + c_row(r, lane) < a.M && ecol < a.N);
+              prod *= in ? t : 1.f;
+              lin += in ? fmaxf(v, 0.f) : 0.f;
             }
+            loss_acc += lin + 0.69314718056f * __builtin_amdgcn_logf(prod);
+            asm volatile("" : "+v"(loss_acc));
             __builtin_amdgcn_sched_barrier(0);
           }
       }
@@ -278,7 +260,6 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
                 v *= a.alpha;
               }
               if constexpr (MODE != FWD_LINEAR) v = sigmoidf_fast(v);
-              if constexpr (POS) v -= (float)((words[fm][fn] >> c_row(r, lane)) & 1u);
               if constexpr (EDGE) { if (ecol >= a.N) v = 0.f; }
               stg[(4 * h + rr) * C::TN + fn * 32 + (lane & 31)] = (half_t)v;
             }
@@ -307,20 +288,16 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
       }
-      if constexpr (LOSS) loss_acc += tile_loss;
     };
-    using T = std::true_type;
-    using F = std::false_type;
-    const bool edge = n0 + C::BN > a.N || (LOSS && m0 + C::BM > a.M);
-    if (edge) { if (has_pos) body(T{}, T{}); else body(F{}, T{}); }
-    else { if (has_pos) body(T{}, F{}); else body(F{}, F{}); }
+    if (n0 + C::BN > a.N || (LOSS && m0 + C::BM > a.M)) body(std::true_type{});
+    else body(std::false_type{});
   };
   C::run(0, n_items, lds, get, epilogue);
   if constexpr (LOSS) {
     // deterministic: lanes -> wave (butterfly), waves -> workgroup (LDS, fixed order), one partial per workgroup
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off, 64);
-    float* red = reinterpret_cast<float*>(bm);
+    float* red = reinterpret_cast<float*>(smem_raw);
     __syncthreads();
     if (lane == 0) red[wave] = loss_acc;
     __syncthreads();
@@ -332,13 +309,95 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
   }
 }
 
-// Sum of the per-workgroup loss partials, in double, in index order.
-__global__ void __launch_bounds__(64) loss_reduce_kernel(const float* __restrict__ part, int n, float* __restrict__ out) {
+// ---------------------------------------------------------------------------------------------
+// positives: G -= 1 at the (row, label) pairs of a sparse label list, after the forward pass
+// ---------------------------------------------------------------------------------------------
+// One wave per pair.  The pair's logit is computed again, in fp32 from the fp16 operands (two rows of d, from the L2 or
+// HBM), because G holds sigmoid(z) already rounded to fp16 and sigmoid(z) - 1 has to be rounded once, as a whole.  Pairs
+// are independent: no pass over the list that sorts them by tile, no list look-up in the forward epilogue, and a pair
+// listed twice writes the same value twice.  Input is CSR (rowptr/colidx, pos_x == nullptr; a pair finds its row by a
+// 64-way search of the row pointers, two rounds of loads up to 4096 rows) or COO (pos_x/pos_y int64).  Pairs whose row
+// or column is out of range are dropped.  (The pass that bucketed the list by label tile ran in one workgroup in front
+// of the forward pass: 11.6 us at 2729 pairs, 23 us at 8357; this one takes 5.9 and 7.3.)
+// LOSS: loss_pos[p] = z of the pair, or 0 if it was dropped or another copy of it was first.  The copies are told apart
+// by G's sign bit, which sigmoid leaves clear and a visited positive sets (a zero difference is stored as -0).
+template <bool LOSS>
+__global__ void __launch_bounds__(256) positives_kernel(const half_t* __restrict__ X, int64_t ldx, const half_t* __restrict__ W,
+                                                        int64_t ldw, const int32_t* __restrict__ rowptr,
+                                                        const int32_t* __restrict__ colidx, const int64_t* __restrict__ pos_x,
+                                                        const int64_t* __restrict__ pos_y, int64_t nnz, int B, int64_t L, int d,
+                                                        half_t* G, int64_t ldg, float* __restrict__ loss_pos) {
+  const int lane = threadIdx.x & 63;
+  const int64_t wave = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int64_t p = wave; p < nnz; p += (int64_t)gridDim.x * 4) {
+    int64_t r = -1, c = -1;
+    if (pos_x) {
+      r = pos_x[p];
+      c = pos_y[p];
+    } else if (p >= rowptr[0] && p < rowptr[B]) {  // whatever the row pointers hold, an entry is read at most once
+      c = colidx[p];
+      int lo = 0, n = B;  // the row is the first b in [lo, lo + n) with rowptr[b + 1] > p
+      while (n > 1) {
+        const int step = (n + 63) >> 6, at = lo + min((lane + 1) * step, n);
+        const unsigned long long above = __ballot(rowptr[at] > p);
+        const int s = above ? __builtin_ctzll(above) : 63;
+        lo += min(s * step, n - 1);
+        n = min(step, B - lo);
+        if (step == 1) break;
+      }
+      r = lo;
+    }
+    const bool in = r >= 0 && r < B && c >= 0 && c < L;
+    float z = 0.f;
+    if (in) {
+      const half_t* x = X + r * ldx;
+      const half_t* w = W + c * ldw;
+      for (int k = lane * 8; k < d; k += 512) {
+        const half8 xv = *reinterpret_cast<const half8*>(x + k), wv = *reinterpret_cast<const half8*>(w + k);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) z = fmaf((float)xv[e], (float)wv[e], z);
+      }
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) z += __shfl_xor(z, off, 64);
+      if (lane == 0) {
+        half_t* g = G + r * ldg + c;
+        const half_t v = (half_t)(sigmoidf_fast(z) - 1.0f);
+        if constexpr (!LOSS) {
+          *g = v;
+        } else {
+          const uint32_t bits = __builtin_bit_cast(uint16_t, v) | 0x8000u;
+          const bool high = reinterpret_cast<uintptr_t>(g) & 2;
+          uint32_t* word = reinterpret_cast<uint32_t*>(reinterpret_cast<uintptr_t>(g) & ~(uintptr_t)3);
+          uint32_t old = *word;
+          for (;;) {
+            if (old & (high ? 0x80000000u : 0x8000u)) { z = 0.f; break; }  // another copy was first
+            const uint32_t now = high ? (old & 0xffffu) | (bits << 16) : (old & 0xffff0000u) | bits;
+            const uint32_t seen = atomicCAS(word, old, now);
+            if (seen == old) break;
+            old = seen;
+          }
+        }
+      }
+    }
+    if constexpr (LOSS) { if (lane == 0) loss_pos[p] = z; }
+  }
+}
+
+// Sum of the per-workgroup loss partials less the positives' logits, in double, in index order.
+__global__ void __launch_bounds__(1024) loss_reduce_kernel(const float* __restrict__ part, int n, const float* __restrict__ pos,
+                                                           int64_t n_pos, float* __restrict__ out) {
+  __shared__ double wave_sum[16];
   double t = 0.0;
-  for (int i = threadIdx.x; i < n; i += 64) t += (double)part[i];
+  for (int i = threadIdx.x; i < n; i += 1024) t += (double)part[i];
+  for (int64_t i = threadIdx.x; i < n_pos; i += 1024) t -= (double)pos[i];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
-  if (threadIdx.x == 0) *out = (float)t;
+  if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = t;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) t += wave_sum[w];
+    *out = (float)t;
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -835,9 +894,10 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const half_t* 
 // ---------------------------------------------------------------------------------------------
 // dX = alpha * G . W (+ beta * dX): split over the label axis, fp32 partials, then a reduce
 // ---------------------------------------------------------------------------------------------
-using DxCore = PipeCore<256, 256, 64, 2, 4, 2, true, false, true, false, false, 4>;  // accumulators in AGPRs; one wave per SIMD fetches
-using DxCore128 = PipeCore<128, 256, 64, 2, 4, 3, true, false, true, false, false, 4>;  // small batches, as in the forward pass
-using DxCore64 = PipeCore<64, 256, 64, 2, 4, 3, true, false, true, false, false, 4>;
+// Batches above 128 rows: 256 dims (the A side, contiguous in dX) x 256 rows x 64 labels per stage.  W runs ahead.
+using DxWide = WideCore<256, 256, 2, 2, false, true, AHEAD_A>;
+using DxCore = PipeCore<128, 256, 64, 2, 4, 3, true, false, true, false, false, 4>;   // up to 128 rows; accumulators in AGPRs
+using DxCore64 = PipeCore<64, 256, 64, 2, 4, 3, true, false, true, false, false, 4>;  // up to 64
 
 struct DxArgs {
   const half_t* G; int64_t ldg;   // M x K, K-contiguous (K = labels)
@@ -848,6 +908,50 @@ struct DxArgs {
 };
 
 // One workgroup per (output tile, slice of the label axis); the tiles of one slice get ids on one XCD.
+__global__ void __launch_bounds__(DxWide::NT) dx_wide_kernel(DxArgs a) {
+  using C = DxWide;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
+  half_t* lds = reinterpret_cast<half_t*>(smem_raw);
+  int tile, split;
+  xcd_map(blockIdx.x, a.tiles_m * a.tiles_n, tile, split);
+  const int mt = tile % a.tiles_m, nt = tile / a.tiles_m;
+  const int m0 = mt * C::BN, n0 = nt * C::BM;
+  const int64_t kb64 = (int64_t)split * a.k_per_split;
+  const int k_begin = (int)(kb64 < a.K ? kb64 : a.K);
+  const int k_end = (int)(kb64 + a.k_per_split < a.K ? kb64 + a.k_per_split : a.K);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be
+  const int wm = wave / C::WN, wn = wave % C::WN;
+  float* part = a.part + (int64_t)split * a.M * a.N;
+  auto store = [&](float4v (&acc)[C::FM][C::FN]) {
+#pragma unroll
+    for (int fn = 0; fn < C::FN; ++fn) {
+      const int row = m0 + wn * C::TN + fn * 16 + (lane & 15);
+      if (row < a.M) {
+#pragma unroll
+        for (int fm = 0; fm < C::FM; ++fm) {
+          const int col = n0 + wm * C::TM + fm * 16 + 4 * (lane >> 4);
+          if (col < a.N) *reinterpret_cast<float4v*>(part + (int64_t)row * a.N + col) = acc[fm][fn];
+        }
+      }
+    }
+  };
+  if (k_end <= k_begin) {  // a slice past the end of the label axis contributes zeros
+    float4v acc[C::FM][C::FN];
+    C::zero(acc);
+    store(acc);
+    return;
+  }
+  auto get = [&](int, C::Operand& oa, C::Operand& ob, int& kb, int& ke) {
+    oa = C::Operand{a.W, a.ldw, n0, a.N, a.K};
+    ob = C::Operand{a.G, a.ldg, m0, a.M, a.K};
+    kb = k_begin;
+    ke = k_end;
+  };
+  auto epilogue = [&](int, float4v (&acc)[C::FM][C::FN]) { store(acc); };
+  C::run(0, 1, lds, get, epilogue);
+}
+
+// The same on the smaller row tiles.
 template <class C>
 __global__ void __launch_bounds__(C::NT) dx_kernel(DxArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
@@ -1331,52 +1435,34 @@ void* static_scratch_ptr() {
   return p;
 }
 
-constexpr size_t LOSS_PART_BYTES = 4096;  // one float per forward workgroup (at most 1024)
-struct BucketWs {
-  int32_t *bucket_ptr, *cursor, *ent_row, *ent_col;
-  float* loss_part;
-};
+// Scratch of the forward pass with the loss: one float per forward workgroup (at most 1024) and one per label pair.
+constexpr size_t LOSS_PART_BYTES = 4096;
+size_t fwd_ws_bytes(int64_t nnz) { return LOSS_PART_BYTES + (size_t)round_up((nnz > 0 ? nnz : 1) * 4, 256); }
 
-size_t bucket_ws_bytes(int64_t L, int64_t nnz) {
-  const int64_t n_tiles = round_up(ceil_div(L, FwdCore::BN), 8);
-  return (size_t)round_up((n_tiles + 1) * 4, 256) + (size_t)round_up(n_tiles * 4, 256) +
-         2 * (size_t)round_up((nnz > 0 ? nnz : 1) * 4, 256) + LOSS_PART_BYTES;
-}
-
-BucketWs carve_bucket_ws(void* ws, int64_t L, int64_t nnz) {
-  const int64_t n_tiles = round_up(ceil_div(L, FwdCore::BN), 8);
-  unsigned char* p = reinterpret_cast<unsigned char*>(ws);
-  BucketWs b;
-  b.bucket_ptr = reinterpret_cast<int32_t*>(p); p += round_up((n_tiles + 1) * 4, 256);
-  b.cursor = reinterpret_cast<int32_t*>(p); p += round_up(n_tiles * 4, 256);
-  b.ent_row = reinterpret_cast<int32_t*>(p); p += round_up((nnz > 0 ? nnz : 1) * 4, 256);
-  b.ent_col = reinterpret_cast<int32_t*>(p); p += round_up((nnz > 0 ? nnz : 1) * 4, 256);
-  b.loss_part = reinterpret_cast<float*>(p);
-  return b;
-}
-
-// Row-tile height for a batch of M rows (see FwdCore / FwdCore128 / FwdCore64).
+// Row-tile height for a batch of M rows (see FwdWide / FwdCore128 / FwdCore64).
 inline int row_tile(int64_t M) { return M <= 64 ? 64 : M <= 128 ? 128 : 256; }
 
+// Workgroups of the forward pass: one resident per CU (the number of tile ids is a multiple of 8).
+inline int64_t fwd_grid(int64_t ids) {
+  const int64_t grid = round_up(num_cus(), 8);
+  return grid < ids ? grid : ids;
+}
+
+int launch_fwd_wide(int mode, const FwdArgs& a, dim3 g, hipStream_t st) {
+  constexpr int LDS = FwdWide::LDS_BYTES;
+  const dim3 b(FwdWide::NT);
+  if (a.loss_part) return launch_k<fwd_wide_kernel<FWD_SIGMOID_PLAIN, false, true>>(g, b, LDS, st, a);
+  if (mode == FWD_SIGMOID && a.beta != 0.f) return launch_k<fwd_wide_kernel<FWD_SIGMOID, true>>(g, b, LDS, st, a);
+  if (mode == FWD_SIGMOID && a.alpha == 1.0f) return launch_k<fwd_wide_kernel<FWD_SIGMOID_PLAIN, false>>(g, b, LDS, st, a);
+  if (mode == FWD_SIGMOID) return launch_k<fwd_wide_kernel<FWD_SIGMOID, false>>(g, b, LDS, st, a);
+  return launch_k<fwd_wide_kernel<FWD_LINEAR, false>>(g, b, LDS, st, a);
+}
+
 template <class C>
-int launch_fwd_c(int mode, FwdArgs a, hipStream_t st, float* loss_part, float* loss_out) {
+int launch_fwd_c(int mode, const FwdArgs& a, dim3 g, hipStream_t st) {
   constexpr int LDS = FwdLds<C>::BYTES;
-  a.tiles_m = ceil_div(a.M, C::BM);
-  a.tiles_n = ceil_div(a.n_store, C::BN);
-  const int64_t ids = (int64_t)a.tiles_m * round_up(a.tiles_n, 8);
-  if (ids <= 0) return XFC_OK;
-  if (ids > 0x7fffffff) return XFC_ERR_INVALID;
-  a.n_ids = (int)ids;
-  int64_t grid = (int64_t)round_up(num_cus(), 8);  // one resident workgroup per CU
-  if (grid > ids) grid = ids;                    // ids is a multiple of 8
-  dim3 g((unsigned)grid), b(C::NT);
-  if (mode == FWD_GRAD && loss_part) {
-    int rc = launch_k<fwd_kernel<C, FWD_GRAD, false, true>>(g, b, LDS, st, a);
-    if (rc) return rc;
-    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(64), 0, st, loss_part, (int)grid, loss_out);
-    return check_launch();
-  }
-  if (mode == FWD_GRAD) return launch_k<fwd_kernel<C, FWD_GRAD, false>>(g, b, LDS, st, a);
+  const dim3 b(C::NT);
+  if (a.loss_part) return launch_k<fwd_kernel<C, FWD_SIGMOID_PLAIN, false, true>>(g, b, LDS, st, a);
   if (mode == FWD_SIGMOID && a.beta != 0.f) return launch_k<fwd_kernel<C, FWD_SIGMOID, true>>(g, b, LDS, st, a);
   if (mode == FWD_SIGMOID && a.alpha == 1.0f) return launch_k<fwd_kernel<C, FWD_SIGMOID_PLAIN, false>>(g, b, LDS, st, a);
   if (mode == FWD_SIGMOID) return launch_k<fwd_kernel<C, FWD_SIGMOID, false>>(g, b, LDS, st, a);
@@ -1384,20 +1470,22 @@ int launch_fwd_c(int mode, FwdArgs a, hipStream_t st, float* loss_part, float* l
 }
 
 int launch_fwd(int mode, const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, half_t* out, int64_t ldo, int M,
-               int N, int K, int n_store, float alpha, float beta, const BucketWs* bk, hipStream_t st,
-               float* loss_part = nullptr, float* loss_out = nullptr) {
+               int N, int K, int n_store, float alpha, float beta, hipStream_t st, float* loss_part = nullptr) {
   FwdArgs a;
   a.X = X; a.ldx = ldx; a.W = W; a.ldw = ldw; a.out = out; a.ldo = ldo;
   a.M = M; a.N = N; a.K = K; a.n_store = n_store; a.alpha = alpha; a.beta = beta;
-  a.bucket_ptr = bk ? bk->bucket_ptr : nullptr;
-  a.ent_row = bk ? bk->ent_row : nullptr;
-  a.ent_col = bk ? bk->ent_col : nullptr;
   a.loss_part = loss_part;
-  a.tiles_m = a.tiles_n = a.n_ids = 0;
+  a.tiles_m = ceil_div(M, row_tile(M));
+  a.tiles_n = ceil_div(n_store, FwdWide::BM);
+  const int64_t ids = (int64_t)a.tiles_m * round_up(a.tiles_n, 8);
+  if (ids <= 0) return XFC_OK;
+  if (ids > 0x7fffffff) return XFC_ERR_INVALID;
+  a.n_ids = (int)ids;
+  const dim3 g((unsigned)fwd_grid(ids));
   switch (row_tile(M)) {
-    case 64: return launch_fwd_c<FwdCore64>(mode, a, st, loss_part, loss_out);
-    case 128: return launch_fwd_c<FwdCore128>(mode, a, st, loss_part, loss_out);
-    default: return launch_fwd_c<FwdCore>(mode, a, st, loss_part, loss_out);
+    case 64: return launch_fwd_c<FwdCore64>(mode, a, g, st);
+    case 128: return launch_fwd_c<FwdCore128>(mode, a, g, st);
+    default: return launch_fwd_wide(mode, a, g, st);
   }
 }
 
@@ -1413,11 +1501,11 @@ void dx_plan(int M, int N, int K, int& tiles_m, int& tiles_n, int& splits, int& 
              size_t ws_limit = ~(size_t)0) {
   const int bm = row_tile(M);
   tiles_m = ceil_div(M, bm);
-  tiles_n = ceil_div(N, DxCore::BN);
+  tiles_n = ceil_div(N, DxWide::BM);
   const int64_t tiles = (int64_t)tiles_m * tiles_n > 0 ? (int64_t)tiles_m * tiles_n : 1;
   const int cus = num_cus();
-  const double nk = (double)ceil_div(K, DxCore::BK);
-  const int max_s = (int)round_up(ceil_div(K, DxCore::BK), 8);
+  const double nk = (double)ceil_div(K, DxWide::BK);
+  const int max_s = (int)round_up(ceil_div(K, DxWide::BK), 8);
   const double STAGE_US = 2.4 * (bm + 256) / 512.0;
   constexpr double FIXED_STAGES = 6.0, PART_BYTES_PER_US = 3.0e6;
   int best = 8;
@@ -1428,7 +1516,7 @@ void dx_plan(int M, int N, int K, int& tiles_m, int& tiles_n, int& splits, int& 
     const double cost = rounds * (nk / s + FIXED_STAGES) * STAGE_US + 2.0 * s * (double)M * N * 4.0 / PART_BYTES_PER_US;
     if (s == 8 || cost < best_cost) { best = s; best_cost = cost; }
   }
-  k_per_split = (int)round_up(ceil_div(K, best), DxCore::BK);
+  k_per_split = (int)round_up(ceil_div(K, best), DxWide::BK);
   splits = best;
 }
 
@@ -1442,12 +1530,12 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
   a.M = M; a.N = N; a.K = K;
   const int64_t grid = (int64_t)a.tiles_m * a.tiles_n * a.splits;
   if (grid <= 0 || M <= 0 || N <= 0) return XFC_OK;
-  const dim3 g((unsigned)grid), b(DxCore::NT);
+  const dim3 g((unsigned)grid);
   int rc;
   switch (row_tile(M)) {
-    case 64: rc = launch_k<dx_kernel<DxCore64>>(g, b, DxCore64::LDS_BYTES, st, a); break;
-    case 128: rc = launch_k<dx_kernel<DxCore128>>(g, b, DxCore128::LDS_BYTES, st, a); break;
-    default: rc = launch_k<dx_kernel<DxCore>>(g, b, DxCore::LDS_BYTES, st, a); break;
+    case 64: rc = launch_k<dx_kernel<DxCore64>>(g, dim3(DxCore64::NT), DxCore64::LDS_BYTES, st, a); break;
+    case 128: rc = launch_k<dx_kernel<DxCore>>(g, dim3(DxCore::NT), DxCore::LDS_BYTES, st, a); break;
+    default: rc = launch_k<dx_wide_kernel>(g, dim3(DxWide::NT), DxWide::LDS_BYTES, st, a); break;
   }
   if (rc) return rc;
   const int64_t nq = (int64_t)M * (N / 4);
@@ -1525,12 +1613,18 @@ int xfc_abi_version(void) { return XFC_ABI_VERSION; }
 int xfc_init(void) {
   hipError_t e = hipSuccess;
   auto keep = [&](hipError_t r) { if (e == hipSuccess) e = r; };
-  auto fwd_limits = [&](auto core_tag, auto dx_tag) {
+  keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID_PLAIN, false, true>>(FwdWide::LDS_BYTES));
+  keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID, true>>(FwdWide::LDS_BYTES));
+  keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID, false>>(FwdWide::LDS_BYTES));
+  keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID_PLAIN, false>>(FwdWide::LDS_BYTES));
+  keep(raise_lds_limit<fwd_wide_kernel<FWD_LINEAR, false>>(FwdWide::LDS_BYTES));
+  keep(raise_lds_limit<topk_kernel<FwdCore>>(TopkLds<FwdCore>::BYTES));
+  keep(raise_lds_limit<dx_wide_kernel>(DxWide::LDS_BYTES));
+  auto small_limits = [&](auto core_tag, auto dx_tag) {
     using C = typename decltype(core_tag)::type;
     using D = typename decltype(dx_tag)::type;
     constexpr int LDS = FwdLds<C>::BYTES;
-    keep(raise_lds_limit<fwd_kernel<C, FWD_GRAD, false, true>>(LDS));
-    keep(raise_lds_limit<fwd_kernel<C, FWD_GRAD, false>>(LDS));
+    keep(raise_lds_limit<fwd_kernel<C, FWD_SIGMOID_PLAIN, false, true>>(LDS));
     keep(raise_lds_limit<fwd_kernel<C, FWD_SIGMOID, true>>(LDS));
     keep(raise_lds_limit<fwd_kernel<C, FWD_SIGMOID, false>>(LDS));
     keep(raise_lds_limit<fwd_kernel<C, FWD_SIGMOID_PLAIN, false>>(LDS));
@@ -1538,9 +1632,8 @@ int xfc_init(void) {
     keep(raise_lds_limit<topk_kernel<C>>(TopkLds<C>::BYTES));
     keep(raise_lds_limit<dx_kernel<D>>(D::LDS_BYTES));
   };
-  fwd_limits(std::type_identity<FwdCore>{}, std::type_identity<DxCore>{});
-  fwd_limits(std::type_identity<FwdCore128>{}, std::type_identity<DxCore128>{});
-  fwd_limits(std::type_identity<FwdCore64>{}, std::type_identity<DxCore64>{});
+  small_limits(std::type_identity<FwdCore128>{}, std::type_identity<DxCore>{});
+  small_limits(std::type_identity<FwdCore64>{}, std::type_identity<DxCore64>{});
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_SMALL>>((int)sizeof(SelLds<SEL_CAP_SMALL>)));
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_LARGE>>((int)sizeof(SelLds<SEL_CAP_LARGE>)));
   keep(raise_lds_limit<dw_kernel<DW_UPDATE>>(DW_LDS_BYTES));
@@ -1580,7 +1673,7 @@ int xfc_gemm(const void* in1, int64_t in1_rows, int64_t in1_cols, int64_t in1_s0
                       K % 8 == 0 && aligned16(in1) && aligned16(in2) && K > 0;
     if (fast)
       return launch_fwd(FWD_SIGMOID, (const half_t*)in1, in1_s0, (const half_t*)in2, in2_s1, (half_t*)out, out_s0,
-                        (int)M, (int)N, (int)K, (int)N, alpha, beta, nullptr, st);
+                        (int)M, (int)N, (int)K, (int)N, alpha, beta, st);
     return launch_generic(in1, in1_s0, in1_s1, in2, in2_s0, in2_s1, out, out_s0, out_s1, (int)M, (int)N, (int)K, alpha,
                           beta, 1, 1, st);
   }
@@ -1621,12 +1714,12 @@ int xfc_logits(const void* X, int64_t ldx, const void* W, int64_t ldw, void* out
     return XFC_ERR_ALIGN;
   if (ldo < L) return XFC_ERR_SHAPE;
   return launch_fwd(FWD_LINEAR, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)out, ldo, (int)B, (int)L, (int)d,
-                    (int)L, 1.0f, 0.0f, nullptr, reinterpret_cast<hipStream_t>(stream));
+                    (int)L, 1.0f, 0.0f, reinterpret_cast<hipStream_t>(stream));
 }
 
 size_t xfc_fwd_grad_workspace_bytes(int64_t L, int64_t nnz) {
   if (!dims_ok(L) || nnz < 0) return 0;
-  return bucket_ws_bytes(L, nnz);
+  return fwd_ws_bytes(nnz);
 }
 
 static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw, const int32_t* rowptr,
@@ -1640,30 +1733,32 @@ static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw,
   if (ldx % 8 || ldw % 8 || ldg % 8 || d % 8 || !aligned16(X) || !aligned16(W) || !aligned16(G))
     return XFC_ERR_ALIGN;
   if (ldg < L) return XFC_ERR_SHAPE;
-  if (!ws || ws_bytes < bucket_ws_bytes(L, nnz)) return XFC_ERR_WORKSPACE;
-  BucketWs bk = carve_bucket_ws(ws, L, nnz);
-  const int n_tiles = (int)round_up(ceil_div(L, FwdCore::BN), 8);
-  const bool coo = pos_x != nullptr;
-  const bool in_lds = n_tiles <= BUCKET_LDS_TILES;
-  const size_t dyn_tiles = in_lds ? (size_t)n_tiles * 4 : 0;
-  const bool rows_in_lds = !coo && dyn_tiles + ((size_t)B + 1) * 4 <= (size_t)BUCKET_DYN_LDS_MAX;
-  const size_t dyn = dyn_tiles + (rows_in_lds ? ((size_t)B + 1) * 4 : 0);
-  auto launch_bucket = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), dyn, st, coo ? nullptr : rowptr, coo ? nullptr : colidx,
-                       coo ? pos_x : nullptr, coo ? pos_y : nullptr, nnz, (int)B, L, FwdCore::BN, n_tiles, bk.bucket_ptr,
-                       bk.cursor, bk.ent_row, bk.ent_col);
-  };
-  if (in_lds && rows_in_lds) launch_bucket(bucket_positives_kernel<true, true>);
-  else if (in_lds) launch_bucket(bucket_positives_kernel<true, false>);
-  else if (rows_in_lds) launch_bucket(bucket_positives_kernel<false, true>);
-  else launch_bucket(bucket_positives_kernel<false, false>);
-  int rc = check_launch();
-  if (rc) return rc;
+  if (!ws || ws_bytes < fwd_ws_bytes(nnz)) return XFC_ERR_WORKSPACE;
+  float* loss_part = loss ? reinterpret_cast<float*>(ws) : nullptr;
+  float* loss_pos = loss ? loss_part + LOSS_PART_BYTES / 4 : nullptr;
   // label columns L .. round_up(L, 8) are written as zero so that G can be read in 16-byte
   // pieces along the label axis by the dX and dW kernels (ldg is a multiple of 8, so they exist)
   const int64_t n_store = round_up(L, 8);
-  return launch_fwd(FWD_GRAD, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)G, ldg, (int)B, (int)L, (int)d,
-                    (int)n_store, 1.0f, 0.0f, &bk, st, loss ? bk.loss_part : nullptr, loss);
+  int rc = launch_fwd(FWD_SIGMOID, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)G, ldg, (int)B, (int)L, (int)d,
+                      (int)n_store, 1.0f, 0.0f, st, loss_part);
+  if (rc) return rc;
+  if (nnz > 0) {
+    const int64_t blocks = ceil_div(nnz, 4) < 16384 ? ceil_div(nnz, 4) : 16384;
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, (const half_t*)X, ldx, (const half_t*)W, ldw,
+                         rowptr, colidx, pos_x, pos_y, nnz, (int)B, L, (int)d, (half_t*)G, ldg, loss_pos);
+    };
+    if (loss) launch(positives_kernel<true>);
+    else launch(positives_kernel<false>);
+    if ((rc = check_launch())) return rc;
+  }
+  if (loss) {
+    const int64_t ids = (int64_t)ceil_div(B, row_tile(B)) * round_up(ceil_div(n_store, FwdWide::BM), 8);
+    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(1024), 0, st, (const float*)loss_part, (int)fwd_grid(ids),
+                       (const float*)loss_pos, nnz, loss);
+    return check_launch();
+  }
+  return XFC_OK;
 }
 
 int xfc_fwd_grad_csr(const void* X, int64_t ldx, const void* W, int64_t ldw, const int32_t* rowptr,
@@ -1679,16 +1774,16 @@ int xfc_fwd_grad_csr_static(const void* X, int64_t ldx, const void* W, int64_t l
                             float* loss, void* stream) {
   if (B > 0 && !rowptr) return XFC_ERR_INVALID;
   if (!dims_ok(L) || nnz < 0) return XFC_ERR_INVALID;
-  if (bucket_ws_bytes(L, nnz) > (size_t)XFC_STATIC_SCRATCH_BYTES) {
+  if (fwd_ws_bytes(nnz) > (size_t)XFC_STATIC_SCRATCH_BYTES) {
     fprintf(stderr, "xfc_fwd_grad_csr_static: L = %lld labels with %lld positives need %zu bytes of scratch, the static "
                     "buffer holds %d; use xfc_fwd_grad_csr with a caller workspace\n",
-            (long long)L, (long long)nnz, bucket_ws_bytes(L, nnz), XFC_STATIC_SCRATCH_BYTES);
+            (long long)L, (long long)nnz, fwd_ws_bytes(nnz), XFC_STATIC_SCRATCH_BYTES);
     return XFC_ERR_LIMIT;
   }
   void* scratch = static_scratch_ptr();
   if (scratch == nullptr) return XFC_ERR_HIP;
-  // every table in the scratch is rebuilt from its first entry by the bucket pass, so nothing of the
-  // previous call's contents survives into this one
+  // what the loss reduction reads is written by this call first, so nothing of the previous call's contents
+  // survives into this one
   return fwd_grad_impl(X, ldx, W, ldw, rowptr, colidx, nullptr, nullptr, nnz, G, ldg, B, L, d, loss, scratch,
                        (size_t)XFC_STATIC_SCRATCH_BYTES, reinterpret_cast<hipStream_t>(stream));
 }
@@ -1697,10 +1792,8 @@ int xfc_fwd_grad_coo(const void* X, int64_t ldx, const void* W, int64_t ldw, con
                      int64_t nnz, void* G, int64_t ldg, int64_t B, int64_t L, int64_t d, float* loss, void* workspace,
                      size_t workspace_bytes, void* stream) {
   if (nnz > 0 && !(pos_x && pos_y)) return XFC_ERR_INVALID;
-  // an empty list still goes through the bucket pass (it zeroes the bucket table)
-  static const int64_t dummy = 0;
-  return fwd_grad_impl(X, ldx, W, ldw, nullptr, nullptr, pos_x ? pos_x : &dummy, pos_y ? pos_y : &dummy, nnz, G, ldg, B,
-                       L, d, loss, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+  return fwd_grad_impl(X, ldx, W, ldw, nullptr, nullptr, pos_x, pos_y, nnz, G, ldg, B, L, d, loss, workspace, workspace_bytes,
+                       reinterpret_cast<hipStream_t>(stream));
 }
 
 size_t xfc_dx_workspace_bytes(int64_t B, int64_t L, int64_t d) { return xfc_gemm_workspace_bytes(B, d, L); }
@@ -1891,7 +1984,7 @@ int xfc_topk(const void* X, int64_t ldx, const void* W, int64_t ldw, int64_t B, 
     for (int64_t r0 = 0; r0 < B; r0 += block) {
       const int64_t rows = B - r0 < block ? B - r0 : block;
       int rc = launch_fwd(FWD_LINEAR, (const half_t*)X + r0 * ldx, ldx, (const half_t*)W, ldw, (half_t*)workspace, ldl,
-                          (int)rows, (int)L, (int)d, (int)L, 1.0f, 0.0f, nullptr, st);
+                          (int)rows, (int)L, (int)d, (int)L, 1.0f, 0.0f, st);
       if (rc) return rc;
       // sample every stride-th 16 KB block first when that still holds 16 K elements and points at about a
       // thousand candidates at most (half the sort buffer)
@@ -1925,7 +2018,7 @@ int xfc_topk(const void* X, int64_t ldx, const void* W, int64_t ldw, int64_t B, 
     int64_t* sample_i = reinterpret_cast<int64_t*>(sample + (size_t)B * TOPK_SAMPLE);
     float* sample_v = reinterpret_cast<float*>(sample_i + (size_t)B * K);
     int rc0 = launch_fwd(FWD_LINEAR, (const half_t*)X, ldx, (const half_t*)W, ldw, sample, TOPK_SAMPLE, (int)B, TOPK_SAMPLE,
-                         (int)d, TOPK_SAMPLE, 1.0f, 0.0f, nullptr, st);
+                         (int)d, TOPK_SAMPLE, 1.0f, 0.0f, st);
     if (rc0) return rc0;
     const SelArgs sa = {(const half_t*)sample, (int64_t)TOPK_SAMPLE, TOPK_SAMPLE, (int64_t)TOPK_SAMPLE, K, 1, sample_v, sample_i};
     if ((rc0 = launch_select<SEL_CAP_SMALL>((int)B, sa, st))) return rc0;
