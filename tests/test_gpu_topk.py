@@ -291,3 +291,30 @@ def test_topk_select_large_k_with_heavy_ties(dev):
     W[:, 0] = torch.randint(0, 3, (L,), generator=g).float() * 0.25     # three distinct scores, ~20,000 copies each
     _check_select(dev, X.half(), W.half(), 6000, vs_oracle=False)
     _check_select(dev, X.half(), W.half(), 1500, vs_oracle=False)
+
+
+# the 64-row tile takes a label group's first tile 32 columns at a time; whole-number scores make long runs of ties.  One
+# partial tile, one and two tiles to a group, rows past the batch, every K of the pass's range
+@pytest.mark.parametrize("B,L,K", [(1, 8, 8), (16, 33, 1), (64, 256, 5), (65, 257, 8), (33, 65537, 8), (64, 70001, 3),
+                                   (16, 131072, 5), (3, 540001, 5), (130, 540001, 8)])
+def test_topk_small_batches_with_ties(dev, B, L, K):
+    g = torch.Generator().manual_seed(B + L)
+    X = torch.randint(-2, 3, (B, 64), generator=g).half()
+    W = torch.randint(-2, 3, (L, 64), generator=g).half()
+    lay = XFCLayer(L, 64, B, dev, weight=W)
+    print(f"top-{K}: B={B} L={L}", flush=True)
+    for _ in range(2):
+        v, i = lay.topk(X.to(dev), K)
+        z = X.float() @ W.float().t()   # whole numbers: exact in fp32
+        order = (z.double() * 2.0 ** 21 - torch.arange(L, dtype=torch.float64)).topk(K, dim=1).indices
+        assert torch.equal(i.cpu(), order) and torch.equal(v.cpu(), z.gather(1, order))
+
+
+def test_topk_small_batch_lists_scores_of_minus_infinity(dev):
+    """Labels whose score is -inf are listed last, in label order, when a tile holds fewer finite ones than K."""
+    W = torch.full((8, 8), -float("inf"), dtype=torch.float16)
+    W[3], W[6] = 1.0, 2.0
+    lay = XFCLayer(8, 8, 2, dev, weight=W)
+    v, i = lay.topk(torch.ones(2, 8, dtype=torch.float16, device=dev), 8)
+    assert i.cpu().tolist() == [[6, 3, 0, 1, 2, 4, 5, 7]] * 2
+    assert v.cpu()[:, :2].tolist() == [[16.0, 8.0]] * 2 and bool(torch.isneginf(v[:, 2:]).all())
