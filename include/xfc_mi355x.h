@@ -193,10 +193,20 @@ int xfc_sgd_momentum_master(float* W32, float* M32, void* W16, const float* grad
  * xfc_fwd_grad_csr, xfc_dx (with W before the update), xfc_dw_update.
  * G is caller-provided scratch of B x ldg halves, ldg >= round_up(L,8)
  * (the reference's preallocated `outsoft`, dl_base.py:176).
+ * Batches of up to 64 rows (32 at d = 1024) with d one of 128, 256, 384, 512, 768, 1024 and at most 2048
+ * label pairs run in one pass over the labels when the workspace has xfc_step_workspace_bytes(); with less,
+ * down to the need of xfc_fwd_grad_* + xfc_dx, they run as the three passes.
  */
 size_t xfc_step_workspace_bytes(int64_t B, int64_t L, int64_t d, int64_t nnz);
 int xfc_step_csr(const void* X, int64_t ldx, void* W, int64_t ldw, void* M, int64_t ldm,
                  const int32_t* rowptr, const int32_t* colidx, int64_t nnz,
+                 void* G, int64_t ldg, float* dX, int64_t lddx,
+                 int64_t B, int64_t L, int64_t d,
+                 float lr, float momentum, float weight_decay, float scale,
+                 void* workspace, size_t workspace_bytes, void* stream);
+/* The same from a row-sorted COO label list (see xfc_fwd_grad_coo). */
+int xfc_step_coo(const void* X, int64_t ldx, void* W, int64_t ldw, void* M, int64_t ldm,
+                 const int64_t* pos_x, const int64_t* pos_y, int64_t nnz,
                  void* G, int64_t ldg, float* dX, int64_t lddx,
                  int64_t B, int64_t L, int64_t d,
                  float lr, float momentum, float weight_decay, float scale,

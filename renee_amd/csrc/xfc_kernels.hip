@@ -14,6 +14,7 @@
 
 #include "../../include/xfc_mi355x.h"
 #include "pipe_core.hpp"
+#include "small_step.hpp"
 #include "wide_core.hpp"
 
 namespace xfc {
@@ -21,13 +22,6 @@ namespace xfc {
 // ---------------------------------------------------------------------------------------------
 // helpers
 // ---------------------------------------------------------------------------------------------
-// 1 / (1 + 2^(-z log2 e)) with the bare v_exp_f32 / v_rcp_f32: the exponential may flush to zero or
-// overflow to infinity at the ends, where the quotient is 1 or 0 either way, so the range fix-up that
-// __expf carries (a compare and a select per element) buys nothing here.
-__device__ __forceinline__ float sigmoidf_fast(float z) {
-  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.44269504088896341f));
-}
-
 // Workgroup ids are dealt round-robin to the 8 XCDs, each with its own L2.  Tiles that
 // share an operand slice are given ids that land on one XCD next to each other:
 // id -> (inner, outer) with `inner` (size n_inner) varying fastest among ids of one XCD.
@@ -1626,6 +1620,17 @@ void dx_plan(int M, int N, int K, int& tiles_m, int& tiles_n, int& splits, int& 
   splits = best;
 }
 
+void launch_dx_reduce(const float* part, float* out, int64_t ldo, int M, int N, int splits, float alpha, float beta,
+                      hipStream_t st) {
+  // threads to a piece: as many as keep the slices of a small output in flight at once; a large one fills the chip with 8
+  const int64_t blocks = ceil_div((int64_t)M * (N / 4), 32);
+  auto reduce = [&](auto kernel, int sg) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(32 * sg), 0, st, part, out, ldo, M, N, splits, alpha, beta);
+  };
+  if (blocks < 1024) reduce(dx_reduce_kernel<32>, 32);
+  else reduce(dx_reduce_kernel<8>, 8);
+}
+
 int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float* out, int64_t ldo, int M, int N, int K,
               float alpha, float beta, void* ws, size_t ws_bytes, hipStream_t st) {
   DxArgs a;
@@ -1644,13 +1649,7 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
     default: rc = launch_k<dx_wide_kernel>(g, dim3(DxWide::NT), DxWide::LDS_BYTES, st, a); break;
   }
   if (rc) return rc;
-  // threads to a piece: as many as keep the slices of a small output in flight at once; a large one fills the chip with 8
-  const int64_t blocks = ceil_div((int64_t)M * (N / 4), 32);
-  auto reduce = [&](auto kernel, int sg) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(32 * sg), 0, st, a.part, out, ldo, M, N, a.splits, alpha, beta);
-  };
-  if (blocks < 1024) reduce(dx_reduce_kernel<32>, 32);
-  else reduce(dx_reduce_kernel<8>, 8);
+  launch_dx_reduce(a.part, out, ldo, M, N, a.splits, alpha, beta, st);
   return check_launch();
 }
 
@@ -1667,6 +1666,43 @@ int launch_dw(int mode, DwArgs a, hipStream_t st) {
   if (mode == DW_UPDATE) return launch_k<dw_kernel<DW_UPDATE>>(g, b, DW_LDS_BYTES, st, a);
   if (mode == DW_UPDATE_MASTER) return launch_k<dw_kernel<DW_UPDATE_MASTER>>(g, b, DW_LDS_BYTES, st, a);
   return launch_k<dw_kernel<DW_OUT>>(g, b, DW_LDS_BYTES, st, a);
+}
+
+// The one-pass step of small batches (small_step.hpp).  Fn::operator()<S>() is called with the kernel for d dims and B
+// rows; false if there is none: other widths do not divide among the waves in 32s, and 64 rows of 1024 dims with the
+// waves' regions exceed the LDS.  Wherever there is one it is the faster: 1.24 to 4.1 times over 8 to 64 rows and 4,097 to
+// 400,001 labels, least at 64 x 400,001 x 768 (768 -> 618 us).  384 dims and 64 rows take 12 waves of one block of dims:
+// with 4 waves of three, 41 spills, 456 us at 64 x 400,001 instead of 307.
+template <class Fn>
+bool small_step_for(int64_t B, int64_t d, Fn&& fn) {
+  if (B < 1 || B > SMALL_MAX_ROWS) return false;
+  auto rows = [&](auto narrow, auto wide) {
+    if (B <= 32) fn(narrow);
+    else fn(wide);
+    return true;
+  };
+  switch (d) {
+    case 128: return rows(SmallStep<4, 1, 2>{}, SmallStep<4, 1, 4>{});
+    case 256: return rows(SmallStep<8, 1, 2>{}, SmallStep<8, 1, 4>{});
+    case 384: return rows(SmallStep<4, 3, 2>{}, SmallStep<12, 1, 4>{});
+    case 512: return rows(SmallStep<8, 2, 2>{}, SmallStep<8, 2, 4>{});
+    case 768: return rows(SmallStep<8, 3, 2>{}, SmallStep<8, 3, 4>{});
+    case 1024: if (B <= 32) { fn(SmallStep<8, 4, 2>{}); return true; } return false;
+    default: return false;
+  }
+}
+inline int small_step_tiles(int64_t L) { return ceil_div(round_up(L, 8), 32); }
+// Workgroups, each with a partial dX of its own: as many as run at once.
+template <class S>
+int small_step_grid(int64_t L) {
+  const int most = S::PER_CU * num_cus(), tiles = small_step_tiles(L);
+  return tiles < most ? tiles : most;
+}
+// Bytes of the partial sums, 0 if there is no such kernel.
+size_t small_step_ws_bytes(int64_t B, int64_t L, int64_t d) {
+  size_t need = 0;
+  if (L > 0) small_step_for(B, d, [&](auto s) { need = (size_t)small_step_grid<decltype(s)>(L) * B * d * 4; });
+  return need;
 }
 
 int launch_generic(const void* in1, int64_t as0, int64_t as1, const void* in2, int64_t bs0, int64_t bs1, void* out,
@@ -1744,6 +1780,9 @@ int xfc_init(void) {
   };
   small_limits(std::type_identity<FwdCore128>{}, std::type_identity<DxCore>{});
   small_limits(std::type_identity<FwdCore64>{}, std::type_identity<DxCore64>{});
+  for (int64_t rows : {32, 64})
+    for (int64_t d : {128, 256, 384, 512, 768, 1024})
+      small_step_for(rows, d, [&](auto s) { keep(raise_lds_limit<small_step_kernel<decltype(s)>>(decltype(s)::LDS_BYTES)); });
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_SMALL>>((int)sizeof(SelLds<SEL_CAP_SMALL>)));
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_LARGE>>((int)sizeof(SelLds<SEL_CAP_LARGE>)));
   keep(raise_lds_limit<dw_kernel<DW_UPDATE>>(DW_LDS_BYTES));
@@ -2000,22 +2039,80 @@ int xfc_sgd_momentum(void* W, void* Mo, const float* grad, int64_t count, float 
 }
 
 size_t xfc_step_workspace_bytes(int64_t B, int64_t L, int64_t d, int64_t nnz) {
-  return (size_t)round_up(xfc_fwd_grad_workspace_bytes(L, nnz), 256) + xfc_dx_workspace_bytes(B, L, d);
+  const size_t dx = xfc_dx_workspace_bytes(B, L, d), small = dims_ok(B) && dims_ok(L) && dims_ok(d) ? small_step_ws_bytes(B, L, d) : 0;
+  return (size_t)round_up(xfc_fwd_grad_workspace_bytes(L, nnz), 256) + (dx > small ? dx : small);
+}
+
+// The step in one pass, if the call is one that small_step_kernel takes: its sizes, every operand present and aligned as
+// the three passes require (which report what is not), no more label pairs than the workgroups' threads hold, and a
+// workspace for the partial sums of all workgroups.  XFC_OK with *taken false otherwise.
+static int small_step(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo, int64_t ldm, const int32_t* rowptr,
+                      const int32_t* colidx, const int64_t* pos_x, const int64_t* pos_y, int64_t nnz, void* G, int64_t ldg,
+                      float* dX, int64_t lddx, int64_t B, int64_t L, int64_t d, float lr, float momentum,
+                      float weight_decay, float scale, void* ws, size_t ws_bytes, hipStream_t st, bool* taken) {
+  *taken = false;
+  if (B < 1 || B > SMALL_MAX_ROWS || !dims_ok(L) || L < 1 || !dims_ok(d) || nnz < 0 || nnz > SMALL_MAX_PAIRS) return XFC_OK;
+  if (!X || !W || !Mo || !G || !dX || (nnz > 0 && !((rowptr && colidx) || (pos_x && pos_y)))) return XFC_OK;
+  if (ldx % 8 || ldw % 8 || ldm % 8 || ldg % 8 || ldg < round_up(L, 8) || !aligned16(X) || !aligned16(W) || !aligned16(Mo) ||
+      !aligned16(G) || !aligned16(ws))
+    return XFC_OK;
+  const size_t need = small_step_ws_bytes(B, L, d);
+  if (need == 0 || ws_bytes < need) return XFC_OK;
+  SmallArgs a;
+  a.X = (const half_t*)X; a.ldx = ldx; a.W = (half_t*)W; a.ldw = ldw; a.Mo = (half_t*)Mo; a.ldm = ldm;
+  a.G = (half_t*)G; a.ldg = ldg;
+  a.rowptr = rowptr; a.colidx = colidx; a.pos_x = pos_x; a.pos_y = pos_y;
+  a.nnz = (int)nnz; a.B = (int)B; a.L = (int)L; a.n_store = (int)round_up(L, 8); a.tiles = small_step_tiles(L);
+  a.lr = lr; a.mu = momentum; a.wd = weight_decay; a.part = reinterpret_cast<float*>(ws);
+  int rc = XFC_OK;
+  small_step_for(B, d, [&](auto s) {
+    using S = decltype(s);
+    const int grid = small_step_grid<S>(L);
+    rc = launch_k<small_step_kernel<S>>(dim3((unsigned)grid), dim3(S::NT), S::LDS_BYTES, st, a);
+    if (rc) return;
+    launch_dx_reduce(a.part, dX, lddx, (int)B, (int)d, grid, scale, 0.0f, st);
+    rc = check_launch();
+  });
+  *taken = true;
+  return rc;
+}
+
+static int step_impl(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo, int64_t ldm, const int32_t* rowptr,
+                     const int32_t* colidx, const int64_t* pos_x, const int64_t* pos_y, int64_t nnz, void* G, int64_t ldg,
+                     float* dX, int64_t lddx, int64_t B, int64_t L, int64_t d, float lr, float momentum,
+                     float weight_decay, float scale, void* workspace, size_t workspace_bytes, void* stream) {
+  const size_t off = (size_t)round_up(xfc_fwd_grad_workspace_bytes(L, nnz), 256);
+  if (!workspace || workspace_bytes < off) return XFC_ERR_WORKSPACE;  // xfc_dx checks its own share
+  if (ldg < round_up(L, 8)) return XFC_ERR_SHAPE;
+  unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  bool taken;
+  int rc = small_step(X, ldx, W, ldw, Mo, ldm, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, dX, lddx, B, L, d, lr, momentum,
+                      weight_decay, scale, ws + off, workspace_bytes - off, st, &taken);
+  if (taken) return rc;
+  rc = fwd_grad_impl(X, ldx, W, ldw, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, B, L, d, nullptr, ws, off, st);
+  if (rc) return rc;
+  rc = xfc_dx(G, ldg, W, ldw, dX, lddx, B, L, d, scale, ws + off, workspace_bytes - off, stream);
+  if (rc) return rc;
+  return xfc_dw_update(G, ldg, X, ldx, W, ldw, Mo, ldm, B, L, d, lr, momentum, weight_decay, nullptr, 0, stream);
 }
 
 int xfc_step_csr(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo, int64_t ldm, const int32_t* rowptr,
                  const int32_t* colidx, int64_t nnz, void* G, int64_t ldg, float* dX, int64_t lddx, int64_t B,
                  int64_t L, int64_t d, float lr, float momentum, float weight_decay, float scale, void* workspace,
                  size_t workspace_bytes, void* stream) {
-  const size_t off = (size_t)round_up(xfc_fwd_grad_workspace_bytes(L, nnz), 256);
-  if (!workspace || workspace_bytes < off) return XFC_ERR_WORKSPACE;  // xfc_dx checks its own share
-  if (ldg < round_up(L, 8)) return XFC_ERR_SHAPE;
-  unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
-  int rc = xfc_fwd_grad_csr(X, ldx, W, ldw, rowptr, colidx, G, ldg, B, L, d, nnz, nullptr, ws, off, stream);
-  if (rc) return rc;
-  rc = xfc_dx(G, ldg, W, ldw, dX, lddx, B, L, d, scale, ws + off, workspace_bytes - off, stream);
-  if (rc) return rc;
-  return xfc_dw_update(G, ldg, X, ldx, W, ldw, Mo, ldm, B, L, d, lr, momentum, weight_decay, nullptr, 0, stream);
+  if (B > 0 && !rowptr) return XFC_ERR_INVALID;
+  return step_impl(X, ldx, W, ldw, Mo, ldm, rowptr, colidx, nullptr, nullptr, nnz, G, ldg, dX, lddx, B, L, d, lr, momentum,
+                   weight_decay, scale, workspace, workspace_bytes, stream);
+}
+
+int xfc_step_coo(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo, int64_t ldm, const int64_t* pos_x,
+                 const int64_t* pos_y, int64_t nnz, void* G, int64_t ldg, float* dX, int64_t lddx, int64_t B, int64_t L,
+                 int64_t d, float lr, float momentum, float weight_decay, float scale, void* workspace,
+                 size_t workspace_bytes, void* stream) {
+  if (nnz > 0 && !(pos_x && pos_y)) return XFC_ERR_INVALID;
+  return step_impl(X, ldx, W, ldw, Mo, ldm, nullptr, nullptr, pos_x, pos_y, nnz, G, ldg, dX, lddx, B, L, d, lr, momentum,
+                   weight_decay, scale, workspace, workspace_bytes, stream);
 }
 
 constexpr int TOPK_SAMPLE = 2048;
@@ -2067,8 +2164,9 @@ size_t xfc_layer_workspace_bytes(int64_t max_batch, int64_t L, int64_t d, int64_
   size_t dx = 0, topk = 0;
   const int64_t k8 = L < TOPK_MAX ? L : TOPK_MAX;
   for (int64_t b = 1; b <= max_batch; ++b) {
-    const size_t a = xfc_dx_workspace_bytes(b, L, d);
+    const size_t a = xfc_dx_workspace_bytes(b, L, d), small = small_step_ws_bytes(b, L, d);
     if (a > dx) dx = a;
+    if (small > dx) dx = small;
     const size_t t = k8 > 0 ? xfc_topk_workspace_bytes(b, L, k8) : 0;
     if (t > topk) topk = t;
   }

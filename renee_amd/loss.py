@@ -73,9 +73,14 @@ class BCELossMultiNode:
         sample = self.compute_loss and self.count % self.loss_sample_freq == 0
         # sigmoid(embed . W^T) - Y into `out` in one pass (use_custom or not: logits that xfc_forward may
         # have left in `out` are recomputed, not read), with the summed loss on the sampled steps (:578-583)
-        lay.fwd_grad(embed_out, pos_x, pos_y, loss_out=self.loss if sample else None, out=out)
+        whole = self.accum == 1 and not sample and not lay.master_weights
+        if not whole:
+            lay.fwd_grad(embed_out, pos_x, pos_y, loss_out=self.loss if sample else None, out=out)
         if lay.xfc_weight_grad is None and self.scaler is not None:   # first micro-batch of a step (:598-600)
             self.scale_bwd = float(self.scaler.get_scale())
+        if whole:                                                     # one call: small batches take a single pass
+            lay._step_coo(embed_out, pos_x, pos_y, grad_input, self.scale_bwd, self.lr, out)
+            return self.loss
         bsz = embed_out.shape[0]
         lay.dx(bsz, grad_input, self.scale_bwd, out=out)              # :602-608
         if self.accum == 1:

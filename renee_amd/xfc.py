@@ -255,6 +255,14 @@ class XFCLayer:
                  "and at least numy rounded up to 8")
         return out
 
+    def _grad_input(self, bsz: int, grad_input: torch.Tensor | None) -> torch.Tensor:
+        if grad_input is None:
+            return self.grad_input[0:bsz]
+        _require(grad_input.dtype == torch.float32 and grad_input.stride(1) == 1 and
+                 tuple(grad_input.shape) == (bsz, self.dims) and grad_input.device == self.device,
+                 "grad_input must be float32 (batch, dims) on the layer's device")
+        return grad_input
+
     def _index(self, t: torch.Tensor, dtype: torch.dtype, what: str) -> torch.Tensor:
         """An index tensor as the kernels read it: 1-D, contiguous, of `dtype`, on this layer's GPU.
         The dtype is checked, never converted (a silent int64 -> int32 pass would hide a caller's
@@ -362,11 +370,7 @@ class XFCLayer:
     def dx(self, bsz: int, grad_input: torch.Tensor | None = None, scale: float = 1.0,
            out: torch.Tensor | None = None) -> torch.Tensor:
         """grad_input = scale * G . W with W before the update (dl_base.py:602-608)."""
-        if grad_input is None:
-            grad_input = self.grad_input[0:bsz]
-        _require(grad_input.dtype == torch.float32 and grad_input.stride(1) == 1 and
-                 tuple(grad_input.shape) == (bsz, self.dims) and grad_input.device == self.device,
-                 "grad_input must be float32 (batch, dims) on the layer's device")
+        grad_input = self._grad_input(bsz, grad_input)
         L = lib()
         G = self._g_view(bsz, out)
         ws = self._ws
@@ -488,12 +492,38 @@ class XFCLayer:
         into the dW pass; with accumulate=True dW is added to the fp32 grad and
         optimizer_step() finishes the step."""
         bsz = embed_out.shape[0]
-        self.fwd_grad(embed_out, pos_x, pos_y)
-        gi = self.dx(bsz, grad_input, scale)
-        if accumulate:
-            self.dw_accumulate(embed_out)
-        else:
-            self.dw_update(embed_out, lr=lr)
+        if accumulate or self.master_weights:
+            self.fwd_grad(embed_out, pos_x, pos_y)
+            gi = self.dx(bsz, grad_input, scale)
+            if accumulate:
+                self.dw_accumulate(embed_out)
+            else:
+                self.dw_update(embed_out, lr=lr)
+            return gi
+        return self._step_coo(embed_out, pos_x, pos_y, grad_input, scale, lr)
+
+    def _step_coo(self, embed_out, pos_x, pos_y, grad_input=None, scale: float = 1.0, lr: float | None = None,
+                  out: torch.Tensor | None = None) -> torch.Tensor:
+        """The whole step through the single C entry point xfc_step_coo (no fp32 master weights)."""
+        x = self._x16(embed_out)
+        bsz = x.shape[0]
+        G = self._g_view(bsz, out)
+        nnz = 0 if pos_x is None else int(pos_x.numel())
+        if nnz:
+            pos_x = self._index(pos_x, torch.int64, "pos_x")
+            pos_y = self._index(pos_y, torch.int64, "pos_y")
+            _require(pos_x.numel() == pos_y.numel(), "pos_x / pos_y length")
+        self._check_nnz(nnz)
+        gi = self._grad_input(bsz, grad_input)
+        ws = self._ws
+        with torch.cuda.device(self.device):
+            rc = lib().xfc_step_coo(x.data_ptr(), x.stride(0), self.xfc_weight.data_ptr(), self.dims,
+                                    self.momentum_buffer.data_ptr(), self.dims, pos_x.data_ptr() if nnz else None,
+                                    pos_y.data_ptr() if nnz else None, nnz, G.data_ptr(), G.stride(0), gi.data_ptr(),
+                                    gi.stride(0), bsz, self.numy, self.dims, self.lr if lr is None else float(lr),
+                                    self.momentum, self.weight_decay, float(scale), ws.data_ptr(), ws.numel(), _stream(x))
+        check(rc, "xfc_step_coo")
+        self._g_live = self._g_live and out is not None
         return gi
 
     def step_csr(self, embed, rowptr, colidx, scale: float = 1.0, lr: float | None = None) -> torch.Tensor:
