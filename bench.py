@@ -337,7 +337,7 @@ def summarise(r, cfg=None):
     s = {"workload": f"batch {B}, d={d}, L={L}, {r['nnz']} positives (Zipf s={r['zipf']})",
          "ms_per_step": ms, "samples_per_s": B / (ms * 1e-3), "step_tflops": tf,
          "mfma_peak_frac": tf / MFMA_F16_PEAK_TFLOPS,
-         "kernels_ms": {"fwd_grad(+bucket)": r["k_ms"][0], "dx(+reduce)": r["k_ms"][1], "dw_update": r["k_ms"][2]},
+         "kernels_ms": {"fwd_grad(+positives)": r["k_ms"][0], "dx(+reduce)": r["k_ms"][1], "dw_update": r["k_ms"][2]},
          "w_update_gbs": 8.0 * L * d / (r["k_ms"][2] * 1e-3) / 1e9,
          "w_update_hbm_frac": 8.0 * L * d / (r["k_ms"][2] * 1e-3) / 1e9 / HBM_PEAK_GBS}
     if cfg in DW_UPDATE_TRAFFIC_BYTES:
@@ -417,10 +417,10 @@ def main() -> int:
                      "copy_kernel_gbs_same_run": r.get("copy_gbs")},
         # the two MFMA-bound kernels of the step, each against the dense fp16 matrix peak on 2*B*L*d flop
         "rooflines": [
-            {"kernel": "fwd_kernel<FWD_GRAD> (logits GEMM + sigmoid - target epilogue, incl. the bucket pass)",
+            {"kernel": "fwd_wide_kernel (logits GEMM + sigmoid epilogue, incl. positives_kernel)",
              "bound": "mfma", "achieved": gemm_flop / k_ms[0] / 1e9, "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
              "frac": gemm_flop / k_ms[0] / 1e9 / MFMA_F16_PEAK_TFLOPS},
-            {"kernel": "dx_kernel (G . W over label slices, incl. the reduce of the partial sums)",
+            {"kernel": "dx_wide_kernel (G . W over label slices, incl. the reduce of the partial sums)",
              "bound": "mfma", "achieved": gemm_flop / k_ms[1] / 1e9, "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
              "frac": gemm_flop / k_ms[1] / 1e9 / MFMA_F16_PEAK_TFLOPS}],
     }
