@@ -248,7 +248,9 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
           for (int r = 0; r < 4; ++r) {
             float v = sigmoidf_fast(t[r]);
             if ((bits >> r) & 1u) v -= 1.0f;
-            gs[(row + r) * 32 + label] = in ? (half_t)v : (half_t)0.f;
+            // rows past the batch as zeros too: z there is 0 . W, which is no number if a weight is not finite, and in
+            // dW the zeros of X do not take that away
+            gs[(row + r) * 32 + label] = in && row + r < a.B ? (half_t)v : (half_t)0.f;
           }
         }
       }

@@ -96,8 +96,10 @@ def test_one_pass_label_lists(dev):
         assert (lay.outsoft[:B, :L].double().cpu() - want).abs().max() <= 2.0 ** -11 + 1e-5
 
 
-def test_one_pass_infinite_weight_stays_in_its_label_and_dim(dev):
-    B, L, d = 20, 300, 128
+# rows past the batch in the first or the second 16 of a pair, both row tiles
+@pytest.mark.parametrize("B,d", [(20, 128), (50, 768), (9, 1024)])
+def test_one_pass_infinite_weight_stays_in_its_label_and_dim(dev, B, d):
+    L = 300
     X, W = synth.make_X(B, d, 9).half().to(dev), synth.make_W(L, d, 9).half()
     W[70, 5] = float("inf")
     lay = XFCLayer(L, d, B, dev, weight=W)
@@ -106,3 +108,11 @@ def test_one_pass_infinite_weight_stays_in_its_label_and_dim(dev):
     assert bool(torch.isfinite(dX[:, cols]).all()) and not bool(torch.isfinite(dX[:, 5]).all())
     rows = torch.arange(L) != 70
     assert bool(torch.isfinite(lay.xfc_weight[rows]).all()) and bool(torch.isfinite(lay.outsoft[:B, :L]).all())
+    # the other dims of that label are updated as those of any other, in fp32 and rounded once
+    Gd = lay.outsoft[:B, :L].double().cpu()
+    m = Gd.t() @ X.double().cpu()
+    w = W.double() - 0.05 * m
+    for got, want in ((lay.momentum_buffer, m), (lay.xfc_weight, w)):
+        got = got.double().cpu()
+        assert bool(torch.isfinite(got[70, cols]).all())
+        assert ((got - want).abs() <= 2.0 ** -11 * want.abs() + 1e-5)[:, cols].all()
