@@ -156,6 +156,9 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
   }
   for (int w = tid; w < 2 * S::MASK_WORDS; w += S::NT) mask[w] = 0u;
 
+  // Rows past the batch: zeros for dW, so that they add nothing; the last row again for z.  Zeros there too would make z of
+  // a label with an infinite weight no number, hence G, and dW in all dims of that label (0 . NaN); this way G holds
+  // nothing there that it does not hold for a row of the batch.
   half8 xt[P][SB][2];  // A side of dW: dim 8 (i / 4) + 4 b + i % 4, rows 8 g ..+7
 #pragma unroll
   for (int p = 0; p < P; ++p)
@@ -165,9 +168,9 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
       for (int b = 0; b < 2; ++b) {
         const int rel = 8 * (i >> 2) + 4 * b + (i & 3), row = 32 * p + rel;
         half8 v = xv[p][s][b];
+        *reinterpret_cast<half8*>(xf + ((p * 2 + b) * SB + s) * 512) = v;
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = row < a.B ? v[e] : (half_t)0.f;
-        *reinterpret_cast<half8*>(xf + ((p * 2 + b) * SB + s) * 512) = v;
         *reinterpret_cast<half8*>(stage + rel * 32 + 8 * g) = v;
       }
       S::lds_done();
@@ -248,9 +251,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
           for (int r = 0; r < 4; ++r) {
             float v = sigmoidf_fast(t[r]);
             if ((bits >> r) & 1u) v -= 1.0f;
-            // rows past the batch as zeros too: z there is 0 . W, which is no number if a weight is not finite, and in
-            // dW the zeros of X do not take that away
-            gs[(row + r) * 32 + label] = in && row + r < a.B ? (half_t)v : (half_t)0.f;
+            gs[(row + r) * 32 + label] = in ? (half_t)v : (half_t)0.f;
           }
         }
       }
