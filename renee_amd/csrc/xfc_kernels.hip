@@ -61,7 +61,7 @@ struct FwdArgs {
   half_t* out; int64_t ldo;         // M x n_store, row-major
   int M, N, K, n_store;             // columns N <= c < n_store are written as zero
   float alpha, beta;
-  float* loss_part;                 // LOSS: one partial sum per workgroup
+  double* loss_part;                // LOSS: one partial sum per workgroup
   int tiles_m, tiles_n, n_ids;      // n_ids = tiles_m * round_up(tiles_n, 8)
 };
 
@@ -76,7 +76,7 @@ __global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
   const int n_items = (a.n_ids - w + G - 1) / G;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be
   const int wm = wave / C::WN, wn = wave % C::WN;
-  float loss_acc = 0.f;  // LOSS: this lane's share of sum softplus(z)
+  double loss_acc = 0.0;  // LOSS: this lane's share of sum softplus(z)
 
   auto get = [&](int item, C::Operand& oa, C::Operand& ob, int& kb, int& ke) {
     int mt, nt;
@@ -115,17 +115,20 @@ __global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
             static_assert(MODE == FWD_SIGMOID_PLAIN && !BETA, "the loss is that of the plain logits");
             // softplus(z) = max(z, 0) + log(1 + e^-|z|) (dl_base.py:578-583); the logarithms of a lane's eight factors in
             // (1, 2] are taken as one, of their product.  (With one logarithm per element and the sum formed at the end of
-            // the tile the kernel spilled 800 registers: 234 us at 199 x 131,072 x 768, now 90.)
-            float prod = 1.f, lin = 0.f;
+            // the tile the kernel spilled 800 registers: 234 us at 199 x 131,072 x 768, now 84.)
+            // The parts are summed apart and in double: of a positive that has been learnt, max(z, 0) goes again with
+            // positives_kernel's z and the logarithm is what remains, 4.5e-5 beside 10.
+            float prod = 1.f, lin[2] = {0.f, 0.f};
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
               const float t = 1.0f + __builtin_amdgcn_exp2f(fabsf(v[e]) * -1.44269504088896341f);
               const bool in = !EDGE || col + e < a.N;
               prod *= in ? t : 1.f;
-              lin += in ? fmaxf(v[e], 0.f) : 0.f;
+              lin[e >> 2] += in ? fmaxf(v[e], 0.f) : 0.f;
             }
-            const float s = lin + 0.69314718056f * __builtin_amdgcn_logf(prod);
-            loss_acc += row_in ? s : 0.f;
+            loss_acc += (double)(row_in ? lin[0] : 0.f);
+            loss_acc += (double)(row_in ? lin[1] : 0.f);
+            loss_acc += (double)(row_in ? 0.69314718056f * __builtin_amdgcn_logf(prod) : 0.f);
             asm volatile("" : "+v"(loss_acc));  // here, not when the tile is done: that would keep every element until then
           }
           if constexpr (BETA) {
@@ -167,12 +170,12 @@ __global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
     // deterministic: lanes -> wave (butterfly), waves -> workgroup (LDS, fixed order), one partial per workgroup
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off, 64);
-    float* red = reinterpret_cast<float*>(smem_raw);
+    double* red = reinterpret_cast<double*>(smem_raw);
     __syncthreads();
     if (lane == 0) red[wave] = loss_acc;
     __syncthreads();
     if (threadIdx.x == 0) {
-      float t = 0.f;
+      double t = 0.0;
       for (int i = 0; i < C::NW; ++i) t += red[i];
       a.loss_part[w] = t;
     }
@@ -190,7 +193,7 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be
   const int wm = wave / C::WN, wn = wave % C::WN;
   half_t* stg = reinterpret_cast<half_t*>(smem_raw + C::LDS_BYTES) + wave * FWD_STG_HALVES;  // 8 rows x TN labels
-  float loss_acc = 0.f;  // LOSS: this lane's share of sum softplus(z)
+  double loss_acc = 0.0;  // LOSS: this lane's share of sum softplus(z)
 
   auto get = [&](int item, typename C::Operand& oa, typename C::Operand& ob, int& kb, int& ke) {
     int mt, nt;
@@ -229,8 +232,12 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
               const bool in = !EDGE || (m0 + wm * C::TM + fm * 32 + c_row(r, lane) < a.M && ecol < a.N);
               prod *= in ? t : 1.f;
               lin += in ? fmaxf(v, 0.f) : 0.f;
+              if ((r & 3) == 3) {
+                loss_acc += (double)lin;
+                lin = 0.f;
+              }
             }
-            loss_acc += lin + 0.69314718056f * __builtin_amdgcn_logf(prod);
+            loss_acc += (double)(0.69314718056f * __builtin_amdgcn_logf(prod));
             asm volatile("" : "+v"(loss_acc));
             __builtin_amdgcn_sched_barrier(0);
           }
@@ -291,12 +298,12 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
     // deterministic: lanes -> wave (butterfly), waves -> workgroup (LDS, fixed order), one partial per workgroup
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) loss_acc += __shfl_xor(loss_acc, off, 64);
-    float* red = reinterpret_cast<float*>(smem_raw);
+    double* red = reinterpret_cast<double*>(smem_raw);
     __syncthreads();
     if (lane == 0) red[wave] = loss_acc;
     __syncthreads();
     if (threadIdx.x == 0) {
-      float t = 0.f;
+      double t = 0.0;
       for (int i = 0; i < C::NW; ++i) t += red[i];
       a.loss_part[w] = t;
     }
@@ -314,8 +321,12 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
 // or column is out of range are dropped.  (The pass that bucketed the list by label tile ran in one workgroup in front
 // of the forward pass: 11.6 us at 2729 pairs, 23 us at 8357; this one takes 5.9 and 7.3.)
 // LOSS: loss_pos[p] = z of the pair, or 0 if it was dropped or another copy of it was first.  The copies are told apart
-// by G's sign bit, which sigmoid leaves clear and a visited positive sets (a zero difference is stored as -0).
-template <bool LOSS>
+// by G's sign bit, which sigmoid leaves clear and a visited positive sets (a zero difference is stored as -0).  This z is
+// the forward pass's to the last bit, made by the same MFMAs in the same order: it cancels the max(z, 0) that the pass
+// added, and a difference of 1e-6 between two sums of the same products is not small beside what is left, 4.5e-5 at z = 10.
+enum PosMode { POS_G = 0, POS_LOSS_WIDE = 1, POS_LOSS = 2 };  // the loss with the z of fwd_wide_kernel or of fwd_kernel
+
+template <int MODE>
 __global__ void __launch_bounds__(256) positives_kernel(const half_t* __restrict__ X, int64_t ldx, const half_t* __restrict__ W,
                                                         int64_t ldw, const int32_t* __restrict__ rowptr,
                                                         const int32_t* __restrict__ colidx, const int64_t* __restrict__ pos_x,
@@ -323,6 +334,9 @@ __global__ void __launch_bounds__(256) positives_kernel(const half_t* __restrict
                                                         half_t* G, int64_t ldg, float* __restrict__ loss_pos) {
   const int lane = threadIdx.x & 63;
   const int64_t wave = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int KQ = MODE == POS_LOSS_WIDE ? 4 : 2;  // pieces of 8 k per MFMA
+  [[maybe_unused]] __shared__ half8 xw_all[MODE == POS_G ? 1 : 4][2][64];
+  [[maybe_unused]] half8 (&xw)[2][64] = xw_all[MODE == POS_G ? 0 : threadIdx.x >> 6];
   for (int64_t p = wave; p < nnz; p += (int64_t)gridDim.x * 4) {
     int64_t r = -1, c = -1;
     if (pos_x) {
@@ -343,20 +357,43 @@ __global__ void __launch_bounds__(256) positives_kernel(const half_t* __restrict
     }
     const bool in = r >= 0 && r < B && c >= 0 && c < L;
     float z = 0.f;
+    [[maybe_unused]] std::conditional_t<MODE == POS_LOSS_WIDE, float4v, float16v> zc = {};
     if (in) {
       const half_t* x = X + r * ldx;
       const half_t* w = W + c * ldw;
-      for (int k = lane * 8; k < d; k += 512) {
-        const half8 xv = *reinterpret_cast<const half8*>(x + k), wv = *reinterpret_cast<const half8*>(w + k);
+      for (int k0 = 0; k0 < d; k0 += 512) {
+        const int k = k0 + lane * 8;
+        half8 xv = {}, wv = {};
+        if (k < d) {
+          xv = *reinterpret_cast<const half8*>(x + k);
+          wv = *reinterpret_cast<const half8*>(w + k);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) z = fmaf((float)xv[e], (float)wv[e], z);
+          for (int e = 0; e < 8; ++e) z = fmaf((float)xv[e], (float)wv[e], z);
+        }
+        if constexpr (MODE != POS_G) {
+          // from "a lane has its eight k" to "a lane has those of its fragment" (zeros past d add nothing)
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          xw[0][lane] = xv;
+          xw[1][lane] = wv;
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+          for (int q = 0; q < 64; q += KQ) {
+            const half8 xf = xw[0][q + lane * KQ / 64], wf = xw[1][q + lane * KQ / 64];
+            if constexpr (MODE == POS_LOSS_WIDE) zc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf, xf, zc, 0, 0, 0);
+            else zc = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf, wf, zc, 0, 0, 0);
+          }
+          __builtin_amdgcn_wave_barrier();
+        }
       }
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) z += __shfl_xor(z, off, 64);
+      const half_t v = (half_t)(sigmoidf_fast(z) - 1.0f);
+      if constexpr (MODE != POS_G) z = zc[0];  // every element of the block is the pair's z
       if (lane == 0) {
         half_t* g = G + r * ldg + c;
-        const half_t v = (half_t)(sigmoidf_fast(z) - 1.0f);
-        if constexpr (!LOSS) {
+        if constexpr (MODE == POS_G) {
           *g = v;
         } else {
           const uint32_t bits = __builtin_bit_cast(uint16_t, v) | 0x8000u;
@@ -373,16 +410,16 @@ __global__ void __launch_bounds__(256) positives_kernel(const half_t* __restrict
         }
       }
     }
-    if constexpr (LOSS) { if (lane == 0) loss_pos[p] = z; }
+    if constexpr (MODE != POS_G) { if (lane == 0) loss_pos[p] = z; }
   }
 }
 
 // Sum of the per-workgroup loss partials less the positives' logits, in double, in index order.
-__global__ void __launch_bounds__(1024) loss_reduce_kernel(const float* __restrict__ part, int n, const float* __restrict__ pos,
+__global__ void __launch_bounds__(1024) loss_reduce_kernel(const double* __restrict__ part, int n, const float* __restrict__ pos,
                                                            int64_t n_pos, float* __restrict__ out) {
   __shared__ double wave_sum[16];
   double t = 0.0;
-  for (int i = threadIdx.x; i < n; i += 1024) t += (double)part[i];
+  for (int i = threadIdx.x; i < n; i += 1024) t += part[i];
   for (int64_t i = threadIdx.x; i < n_pos; i += 1024) t -= (double)pos[i];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
@@ -1535,8 +1572,9 @@ void* static_scratch_ptr() {
   return p;
 }
 
-// Scratch of the forward pass with the loss: one float per forward workgroup (at most 1024) and one per label pair.
+// Scratch of the forward pass with the loss: a double per forward workgroup and a float per label pair.
 constexpr size_t LOSS_PART_BYTES = 4096;
+constexpr int MAX_FWD_GRID = LOSS_PART_BYTES / sizeof(double) - 8;  // 504, with room to align; a multiple of 8
 size_t fwd_ws_bytes(int64_t nnz) { return LOSS_PART_BYTES + (size_t)round_up((nnz > 0 ? nnz : 1) * 4, 256); }
 
 // Row-tile height for a batch of M rows (see FwdWide / FwdCore128 / FwdCore64).
@@ -1544,7 +1582,7 @@ inline int row_tile(int64_t M) { return M <= 64 ? 64 : M <= 128 ? 128 : 256; }
 
 // Workgroups of the forward pass: one resident per CU (the number of tile ids is a multiple of 8).
 inline int64_t fwd_grid(int64_t ids) {
-  const int64_t grid = round_up(num_cus(), 8);
+  const int64_t grid = round_up(num_cus(), 8) < MAX_FWD_GRID ? round_up(num_cus(), 8) : MAX_FWD_GRID;
   return grid < ids ? grid : ids;
 }
 
@@ -1570,7 +1608,7 @@ int launch_fwd_c(int mode, const FwdArgs& a, dim3 g, hipStream_t st) {
 }
 
 int launch_fwd(int mode, const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, half_t* out, int64_t ldo, int M,
-               int N, int K, int n_store, float alpha, float beta, hipStream_t st, float* loss_part = nullptr) {
+               int N, int K, int n_store, float alpha, float beta, hipStream_t st, double* loss_part = nullptr) {
   FwdArgs a;
   a.X = X; a.ldx = ldx; a.W = W; a.ldw = ldw; a.out = out; a.ldo = ldo;
   a.M = M; a.N = N; a.K = K; a.n_store = n_store; a.alpha = alpha; a.beta = beta;
@@ -1883,8 +1921,8 @@ static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw,
     return XFC_ERR_ALIGN;
   if (ldg < L) return XFC_ERR_SHAPE;
   if (!ws || ws_bytes < fwd_ws_bytes(nnz)) return XFC_ERR_WORKSPACE;
-  float* loss_part = loss ? reinterpret_cast<float*>(ws) : nullptr;
-  float* loss_pos = loss ? loss_part + LOSS_PART_BYTES / 4 : nullptr;
+  double* loss_part = loss ? reinterpret_cast<double*>((reinterpret_cast<uintptr_t>(ws) + 7) & ~(uintptr_t)7) : nullptr;
+  float* loss_pos = loss ? reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(ws) + LOSS_PART_BYTES) : nullptr;
   // label columns L .. round_up(L, 8) are written as zero so that G can be read in 16-byte
   // pieces along the label axis by the dX and dW kernels (ldg is a multiple of 8, so they exist)
   const int64_t n_store = round_up(L, 8);
@@ -1897,13 +1935,14 @@ static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw,
       hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, (const half_t*)X, ldx, (const half_t*)W, ldw,
                          rowptr, colidx, pos_x, pos_y, nnz, (int)B, L, (int)d, (half_t*)G, ldg, loss_pos);
     };
-    if (loss) launch(positives_kernel<true>);
-    else launch(positives_kernel<false>);
+    if (!loss) launch(positives_kernel<POS_G>);
+    else if (row_tile(B) == FwdWide::BN) launch(positives_kernel<POS_LOSS_WIDE>);
+    else launch(positives_kernel<POS_LOSS>);
     if ((rc = check_launch())) return rc;
   }
   if (loss) {
     const int64_t ids = (int64_t)ceil_div(B, row_tile(B)) * round_up(ceil_div(n_store, FwdWide::BM), 8);
-    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(1024), 0, st, (const float*)loss_part, (int)fwd_grid(ids),
+    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(1024), 0, st, (const double*)loss_part, (int)fwd_grid(ids),
                        (const float*)loss_pos, nnz, loss);
     return check_launch();
   }
