@@ -47,55 +47,48 @@ __device__ __forceinline__ void wide_load16(int64_t ubase, uint32_t voff, uint32
 // Swizzles: the 16 lanes (b128) or 32 lanes (b64) the LDS serves at a time must spread over all 64 banks.
 // KC, 128-byte rows: the 16 rows of a fragment cover the 256 bytes of a bank line.
 __device__ __forceinline__ int wide_kc_swz(int row) { return (row >> 1) & 7; }
-// MC: half a wave reads 32 bytes of each of the k-rows {0..3, 8..11} (mod 16) of one column block; a k-row is
-// 2R bytes, so with R a multiple of 128 all eight rows start at the same bank and need eight different 32-byte
-// segments, and otherwise (2R = 128 mod 256) odd and even rows already differ and four segments are enough,
-// which also keeps the XOR inside the 8-chunk groups that such an R is made of.
-template <int R>
-__device__ __forceinline__ int wide_mc_swz(int k) {
-  if constexpr (R % 128 == 0) return ((k & 3) << 1) | (((k >> 3) & 1) << 3);
-  else return (((k >> 1) & 1) << 1) | (((k >> 3) & 1) << 2);
-}
+// MC: half a wave reads 32 bytes of each of the k-rows {0..3, 8..11} (mod 16) of one column block; a k-row is 2R
+// bytes with R a multiple of 128, so all eight rows start at the same bank and need eight different 32-byte segments.
+__device__ __forceinline__ int wide_mc_swz(int k) { return ((k & 3) << 1) | (((k >> 3) & 1) << 3); }
 
-// Which operand's ring has three slots instead of two and is fetched half a stage earlier.
-enum Ahead { AHEAD_A, AHEAD_B };
-
-template <int BM_, int BN_, int WM_, int WN_, bool A_KC_, bool B_KC_, Ahead AHEAD_>
+// The A side comes from HBM: its ring has three slots, and it is fetched half a stage earlier than the B side, whose
+// ring has two.  The B side is K-contiguous.
+template <int BM_, int BN_, int WM_, int WN_, bool A_KC_>
 struct WideCore {
   static constexpr int BM = BM_, BN = BN_, BK = 64, WM = WM_, WN = WN_;
-  static constexpr bool A_KC = A_KC_, B_KC = B_KC_;
+  static constexpr bool A_KC = A_KC_;
   static constexpr int NW = WM * WN, NT = 64 * NW;
   static constexpr int TM = BM / WM, TN = BN / WN;   // a wave's tile
   static constexpr int FM = TM / 16, FN = TN / 16;   // in 16 x 16 blocks
   static constexpr int A_HALVES = BM * BK, B_HALVES = BN * BK;
-  static constexpr int A_SLOTS = AHEAD_ == AHEAD_A ? 3 : 2, B_SLOTS = AHEAD_ == AHEAD_B ? 3 : 2;
+  static constexpr int A_SLOTS = 3, B_SLOTS = 2;
   static constexpr int LDS_BYTES = (A_SLOTS * A_HALVES + B_SLOTS * B_HALVES) * 2;
   static constexpr int A_CH = BM * BK / 8 / NT, B_CH = BN * BK / 8 / NT;  // fetch instructions per wave and stage
-  static constexpr int AHEAD_CH = AHEAD_ == AHEAD_A ? A_CH : B_CH, LATE_CH = A_CH + B_CH - AHEAD_CH;
   static constexpr int NM = FM * FN;                   // MFMAs of a sub-step of 32 k
-  static constexpr int A_RD = A_KC ? FM : 2 * FM, B_RD = B_KC ? FN : 2 * FN, NR = A_RD + B_RD;  // its fragment reads
+  static constexpr int A_RD = A_KC ? FM : 2 * FM, B_RD = FN, NR = A_RD + B_RD;  // its fragment reads
   // A sub-step's reads go into the first half of the previous sub-step's MFMAs, so that the last has landed before it is
-  // wanted.  The fetches that have less time to land (the late operand's) go into the first half of the second sub-step,
+  // wanted.  The fetches that have less time to land (the B side's) go into the first half of the second sub-step,
   // the others are spread over the first.  A fetch's address is advanced two MFMAs after the next fetch.
   static constexpr int READ_EVERY = NM / (2 * NR) > 0 ? NM / (2 * NR) : 1;
-  static constexpr int LATE_EVERY = NM / (2 * LATE_CH), AHEAD_EVERY = NM / (AHEAD_CH + 1);
+  static constexpr int B_EVERY = NM / (2 * B_CH), A_EVERY = NM / (A_CH + 1);
   static_assert(BM % (32 * WM) == 0 && BN % (16 * WN) == 0, "wave tile: pairs of 16-row blocks by 16-column blocks");
   static_assert((BM * BK / 8) % NT == 0 && (BN * BK / 8) % NT == 0, "chunk split");
-  static_assert((BM % 64) == 0 && (BN % 64) == 0, "swizzle");
+  static_assert(A_KC ? BM % 64 == 0 : BM % 128 == 0 && 512 % BM == 0, "swizzle; a fetch instruction covers whole k-rows");
+  static_assert(BN % 64 == 0, "swizzle");
   static_assert((NR - 1) * READ_EVERY < NM, "the reads fit their sub-step");
-  static_assert(LATE_EVERY > 1 && AHEAD_EVERY > 1 && LATE_CH * LATE_EVERY + 1 < NM && AHEAD_CH * AHEAD_EVERY + 1 < NM, "so do the fetches");
+  static_assert(B_EVERY > 1 && A_EVERY > 1 && B_CH * B_EVERY + 1 < NM && A_CH * A_EVERY + 1 < NM, "so do the fetches");
   static_assert(NW % 2 == 0, "the KC swizzle assumes that a fetch instruction's rows are 8 times an even step apart");
 
-  // One operand's tile: base pointer, leading dimension (halves), first row (KC) or column (MC) of the
-  // tile, the limit of that index and the limit of the contraction index.  Requirements: r0 < rmax; ld is
-  // a multiple of 8 and ld * 2 * 32 < 2^32 (an MC side whose width is not a power of two: ld * 2 * 64 < 2^32); for MC
-  // operands rmax is a multiple of 8.  Rows (columns) at or past rmax are fetched from the last valid row (column chunk)
-  // instead: they only ever feed outputs the caller discards.  Contraction indices at or past kmax are fetched
+  // One operand's tile: base pointer, leading dimension (halves), first row (KC) or column (MC) of the tile and the limit
+  // of that index.  Requirements: r0 < rmax; ld is a multiple of 8 and ld * 2 * 32 < 2^32; for MC operands rmax is a
+  // multiple of 8.  Rows (columns) at or past rmax are fetched from the last valid row (column chunk) instead: they only
+  // ever feed outputs the caller discards.  The limit of the contraction index is the item's k_end, up to which (KC: up to
+  // the next multiple of 8) both operands must be readable: nothing past it is read, and what a stage holds past it counts
   // as zeros.
   struct Operand {
     const half_t* p;
     int64_t ld;
-    int r0, rmax, kmax;
+    int r0, rmax;
   };
 
   // Addresses of the CH 16-byte pieces a thread fetches for one operand each stage.  Every fetch is
@@ -104,8 +97,7 @@ struct WideCore {
   template <bool KC, int R, int CH, bool PERM>
   struct Loader {
     static constexpr int CPI = KC ? BK / 8 : R / 8;  // 16-byte chunks per tile row (KC) or per k-row (MC)
-    static constexpr bool WHOLE = 64 % CPI == 0;     // an instruction covers whole rows
-    static constexpr int RPI = WHOLE ? 64 / CPI : 0;
+    static constexpr int RPI = 64 / CPI;             // rows per instruction
     int64_t at[CH];      // uniform address of each instruction's first row at its next stage's first k
     int64_t kstep;       // uniform
     uint32_t voff[CH];   // per-thread byte offset from there
@@ -134,14 +126,14 @@ struct WideCore {
 #pragma unroll
         for (int i = 0; i < CH; ++i) {
           const int q = (i * NW + wave) * 64 + lane, k = q / CPI, pc = q % CPI;
-          const int c = (pc ^ wide_mc_swz<R>(k)) * 8;
-          const int k0 = WHOLE ? (i * NW + wave) * RPI : 0;
+          const int c = (pc ^ wide_mc_swz(k)) * 8;
+          const int k0 = (i * NW + wave) * RPI;
           at[i] = uniform64(reinterpret_cast<int64_t>(base + (int64_t)k0 * o.ld));
           voff[i] = (uint32_t)(k - k0) * (uint32_t)(o.ld * 2) + (uint32_t)(c < last ? c : last) * 2u;
         }
       }
     }
-    // For the stage that crosses kmax (n < BK of its k are left), the last of an item: lanes whose piece lies past the
+    // For the stage that crosses k_end (n < BK of its k are left), the last of an item: lanes whose piece lies past the
     // end fetch an earlier k, which is inside the operand; clear_tail() replaces what they brought.
     __device__ __forceinline__ void retarget(int n, int64_t ld, int wave, int lane) {
 #pragma unroll
@@ -150,7 +142,7 @@ struct WideCore {
         if constexpr (KC) {
           voff[i] -= k >= n ? (uint32_t)k * 2u : 0u;
         } else {
-          const int k0 = WHOLE ? (i * NW + wave) * RPI : 0;  // the instruction's first k-row
+          const int k0 = (i * NW + wave) * RPI;  // the instruction's first k-row
           voff[i] -= k >= n ? (uint32_t)(k - k0) * (uint32_t)(ld * 2) : 0u;
           at[i] -= k0 < n ? 0 : uniform64((int64_t)k0 * ld * 2);
         }
@@ -172,7 +164,7 @@ struct WideCore {
   template <bool IS_A>
   struct Cursor {
     static constexpr int SLOTS = IS_A ? A_SLOTS : B_SLOTS, BYTES = (IS_A ? A_HALVES : B_HALVES) * 2, CH = IS_A ? A_CH : B_CH;
-    using Load = std::conditional_t<IS_A, Loader<A_KC, BM, A_CH, A_KC>, Loader<B_KC, BN, B_CH, false>>;
+    using Load = std::conditional_t<IS_A, Loader<A_KC, BM, A_CH, A_KC>, Loader<true, BN, B_CH, false>>;
     Load load;
     uint32_t ring, dst;  // LDS address of this wave's first piece in slot 0 and in the stage's slot
     int item, k_left;    // k of the item from this stage on
@@ -225,7 +217,7 @@ struct WideCore {
     } else {
       const int g = lane >> 4, t = lane & 15;
       const int k = kk * 32 + 8 * g + 4 * half + (t >> 2), c = r0 + 4 * (t & 3);
-      const int off = k * R + ((((c >> 3) ^ wide_mc_swz<R>(k)) << 3) | (c & 7));
+      const int off = k * R + ((((c >> 3) ^ wide_mc_swz(k)) << 3) | (c & 7));
       const fp16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4f16((XFC_LDS fp16x4_t*)(lds + off));
 #pragma unroll
       for (int e = 0; e < 4; ++e) f[4 * half + e] = (half_t)v[e];
@@ -234,12 +226,11 @@ struct WideCore {
   // The j-th read of a sub-step's fragments, in the order in which its MFMAs want them: a[0], all of b, the rest of a.
   __device__ __forceinline__ static void read_one(int j, const half_t* sa, const half_t* sb, int kk, int wm, int wn, int lane,
                                                   Frags& f) {
-    constexpr int SA = A_KC ? 1 : 2, SB = B_KC ? 1 : 2;
+    constexpr int SA = A_KC ? 1 : 2;
     if (j < SA) {
       read_piece<A_KC, BM>(sa, wm * TM, kk, j, lane, f.a[0]);
     } else if (j < SA + B_RD) {
-      const int q = j - SA;
-      read_piece<B_KC, BN>(sb, wn * TN + (q / SB) * 16, kk, q % SB, lane, f.b[q / SB]);
+      read_piece<true, BN>(sb, wn * TN + (j - SA) * 16, kk, 0, lane, f.b[j - SA]);
     } else {
       const int q = j - B_RD;
       read_piece<A_KC, BM>(sa, wm * TM + (q / SA) * 16, kk, q % SA, lane, f.a[q / SA]);
@@ -292,10 +283,10 @@ struct WideCore {
   //                                      outside the ring's LDS_BYTES
   // All threads of the workgroup call this together.
   //
-  // Schedule per stage c: under the MFMAs of its first sub-step the fragments of the second are read and the operand that
-  // runs ahead fetches its part of stage c+2, into the slot that stage c-1 left.  Between the sub-steps the wave waits for
+  // Schedule per stage c: under the MFMAs of its first sub-step the fragments of the second are read and the A side
+  // fetches its part of stage c+2, into the slot that stage c-1 left.  Between the sub-steps the wave waits for
   // its part of stage c+1 to have landed (all but the fetches just issued) and joins the barrier; past it, every wave has
-  // finished reading stage c, so under the MFMAs of the second sub-step the other operand's slot is refilled, with its part
+  // finished reading stage c, so under the MFMAs of the second sub-step the B side's slot is refilled, with its part
   // of stage c+2, and the first fragments of stage c+1 are read.
   template <class GetItem, class Epilogue>
   __device__ __forceinline__ static void run(int item_begin, int item_end, half_t* lds, GetItem get, Epilogue epilogue) {
@@ -348,18 +339,14 @@ struct WideCore {
     for (int j = 0; j < NR; ++j) read_one(j, sa, sb, 0, wm, wn, lane, f0);
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     bool drain_all = false;
-    auto ahead_piece = [&](int j) { if constexpr (AHEAD_ == AHEAD_A) ca.piece(j); else cb.piece(j); };
-    auto ahead_bump = [&](int j) { if constexpr (AHEAD_ == AHEAD_A) ca.bump(j); else cb.bump(j); };
-    auto late_piece = [&](int j) { if constexpr (AHEAD_ == AHEAD_A) cb.piece(j); else ca.piece(j); };
-    auto late_bump = [&](int j) { if constexpr (AHEAD_ == AHEAD_A) cb.bump(j); else ca.bump(j); };
     // The order below is the schedule: nothing may move across a sched_barrier.
     auto sub_step0 = [&](auto first_tag) {
 #pragma unroll
       for (int n = 0; n < NM; ++n) {
         mfma<decltype(first_tag)::value>(n, f0, acc);
         if (n % READ_EVERY == 0 && n / READ_EVERY < NR) read_one(n / READ_EVERY, sa, sb, 1, wm, wn, lane, f1);
-        if (n % AHEAD_EVERY == AHEAD_EVERY - 1 && n / AHEAD_EVERY < AHEAD_CH) ahead_piece(n / AHEAD_EVERY);
-        if (n % AHEAD_EVERY == 1 && n > AHEAD_EVERY && n / AHEAD_EVERY - 1 < AHEAD_CH) ahead_bump(n / AHEAD_EVERY - 1);
+        if (n % A_EVERY == A_EVERY - 1 && n / A_EVERY < A_CH) ca.piece(n / A_EVERY);
+        if (n % A_EVERY == 1 && n > A_EVERY && n / A_EVERY - 1 < A_CH) ca.bump(n / A_EVERY - 1);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -368,8 +355,8 @@ struct WideCore {
       for (int n = 0; n < NM; ++n) {
         mfma<false>(n, f1, acc);
         if (n % READ_EVERY == 0 && n / READ_EVERY < NR) read_one(n / READ_EVERY, sa, sb, 0, wm, wn, lane, f0);
-        if (n % LATE_EVERY == LATE_EVERY - 1 && n / LATE_EVERY < LATE_CH) late_piece(n / LATE_EVERY);
-        if (n % LATE_EVERY == 1 && n > LATE_EVERY && n / LATE_EVERY - 1 < LATE_CH) late_bump(n / LATE_EVERY - 1);
+        if (n % B_EVERY == B_EVERY - 1 && n / B_EVERY < B_CH) cb.piece(n / B_EVERY);
+        if (n % B_EVERY == 1 && n > B_EVERY && n / B_EVERY - 1 < B_CH) cb.bump(n / B_EVERY - 1);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -378,8 +365,7 @@ struct WideCore {
       for (int kt = 0; kt < nk; ++kt) {
         if (kt == 0) sub_step0(std::true_type{});
         else sub_step0(std::false_type{});
-        if constexpr (AHEAD_ == AHEAD_A) ca.advance(get, item_end, wave, lane);
-        else cb.advance(get, item_end, wave, lane);
+        ca.advance(get, item_end, wave, lane);
         sa = sa == a_ring + (A_SLOTS - 1) * A_HALVES ? a_ring : sa + A_HALVES;
         sb = sb == b_ring + (B_SLOTS - 1) * B_HALVES ? b_ring : sb + B_HALVES;
         k_left -= BK;
@@ -392,10 +378,9 @@ struct WideCore {
         // order with them, so the first wait after one drains everything.
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), in a form the compiler's own wait bookkeeping sees
         if (drain_all) { wait_lds_vmcnt_barrier<0>(); drain_all = false; }
-        else wait_lds_vmcnt_barrier<AHEAD_CH>();
+        else wait_lds_vmcnt_barrier<A_CH>();
         sub_step1();
-        if constexpr (AHEAD_ == AHEAD_A) cb.advance(get, item_end, wave, lane);
-        else ca.advance(get, item_end, wave, lane);
+        cb.advance(get, item_end, wave, lane);
         // No LDS read stays pending across the loop edge (the reads above finished long before the
         // MFMAs were all issued): the compiler then knows the next stage's first MFMAs need no wait.
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)

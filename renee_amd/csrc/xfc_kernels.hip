@@ -37,7 +37,7 @@ __device__ __forceinline__ void xcd_map(int id, int n_inner, int& inner, int& ou
 enum FwdMode { FWD_LINEAR = 0, FWD_SIGMOID = 1, FWD_SIGMOID_PLAIN = 2 };  // PLAIN: alpha 1, beta 0
 
 // Batches above 128 rows: 256 labels (the A side, contiguous in the output) x 256 rows, W running ahead.
-using FwdWide = WideCore<256, 256, 2, 2, true, true, AHEAD_A>;
+using FwdWide = WideCore<256, 256, 2, 2, true>;
 static_assert(FwdWide::LDS_BYTES <= 160 * 1024, "LDS budget");
 // Batches of up to 128 and 64 rows (the reference's B = 32 plumbing case, --accum micro-batches, the last partial batch
 // of an epoch), where a 256-row tile would spend most of its MFMAs on padding: W streams from HBM, eight waves, three
@@ -81,8 +81,8 @@ __global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
   auto get = [&](int item, C::Operand& oa, C::Operand& ob, int& kb, int& ke) {
     int mt, nt;
     xcd_map(item * G + w, a.tiles_m, mt, nt);
-    oa = C::Operand{a.W, a.ldw, nt < a.tiles_n ? nt * C::BM : 0, a.N, a.K};
-    ob = C::Operand{a.X, a.ldx, mt * C::BN, a.M, a.K};
+    oa = C::Operand{a.W, a.ldw, nt < a.tiles_n ? nt * C::BM : 0, a.N};
+    ob = C::Operand{a.X, a.ldx, mt * C::BN, a.M};
     kb = 0;
     ke = a.K;
   };
@@ -1017,7 +1017,7 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const half_t* 
 // dX = alpha * G . W (+ beta * dX): split over the label axis, fp32 partials, then a reduce
 // ---------------------------------------------------------------------------------------------
 // Batches above 128 rows: 256 dims (the A side, contiguous in dX) x 256 rows x 64 labels per stage.  W runs ahead.
-using DxWide = WideCore<256, 256, 2, 2, false, true, AHEAD_A>;
+using DxWide = WideCore<256, 256, 2, 2, false>;
 using DxCore = PipeCore<128, 256, 64, 2, 4, 3, true, false, true, false, false, 4>;   // up to 128 rows; accumulators in AGPRs
 using DxCore64 = PipeCore<64, 256, 64, 2, 4, 3, true, false, true, false, false, 4>;  // up to 64
 
@@ -1064,8 +1064,8 @@ __global__ void __launch_bounds__(DxWide::NT) dx_wide_kernel(DxArgs a) {
     return;
   }
   auto get = [&](int, C::Operand& oa, C::Operand& ob, int& kb, int& ke) {
-    oa = C::Operand{a.W, a.ldw, n0, a.N, a.K};
-    ob = C::Operand{a.G, a.ldg, m0, a.M, a.K};
+    oa = C::Operand{a.W, a.ldw, n0, a.N};
+    ob = C::Operand{a.G, a.ldg, m0, a.M};
     kb = k_begin;
     ke = k_end;
   };
