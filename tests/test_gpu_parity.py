@@ -498,10 +498,9 @@ def test_batches_above_1024(dev, B, L, d):
 
 
 @pytest.mark.parametrize("B,L,d,csr", [(16, 3_200_000, 8, False), (16, 3_200_000, 8, True), (15000, 520, 8, True)])
-def test_bucket_pass_variants(dev, B, L, d, csr):
-    """The pass that groups the positives by label tile keeps its per-tile counters in LDS up to 12,288 label tiles
-    and in global memory above (3.2 M labels: 12,500 tiles), and walks a CSR list by entry with the row pointers in
-    LDS while they fit next to the counters (15,000 rows do not: one row per thread then)."""
+def test_positives_pass_at_the_ends_of_its_range(dev, B, L, d, csr):
+    """3.2 M labels (a row of G is 6.4 MB) and a CSR list over 15,000 rows, whose row is found in
+    three rounds of the search."""
     X, W, P = _problem(B, L, d, kmax=6, kmean=3.0, seed=77)
     px, py = P.coo()
     _check_step(dev, X, W, px, py, csr=(torch.from_numpy(P.rowptr), torch.from_numpy(P.colidx)) if csr else None)

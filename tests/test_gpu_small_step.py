@@ -74,10 +74,12 @@ def test_one_pass_matches_three(dev, B, L, d, coo):
     assert ((Wn.double().cpu() - w).abs() <= 2.0 ** -11 * w.abs() + 1e-5).all()
 
 
-def test_one_pass_label_lists(dev):
+# a thread holds 4, 8, 4 and 3 pairs (three times 768 threads overhang the 2048)
+@pytest.mark.parametrize("B,d", [(32, 256), (32, 128), (50, 512), (50, 384)])
+def test_one_pass_label_lists(dev, B, d):
     """Pairs out of range are dropped, one listed twice counts once, and lists longer than the workgroups hold (2048) or
     empty give the same step."""
-    B, L, d = 32, 5000, 256
+    L = 5000
     X, W = synth.make_X(B, d, 8).half().to(dev), synth.make_W(L, d, 8).half()
     g = torch.Generator().manual_seed(1)
     for n, extra in ((0, 0), (3, 3), (2048, 0), (2049, 0)):

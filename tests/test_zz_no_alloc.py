@@ -1,4 +1,4 @@
-"""xfc_fwd_grad_csr_static (the entry point that allocates nothing: its label buckets live in a fixed
+"""xfc_fwd_grad_csr_static (the entry point that allocates nothing: the scratch of its loss is a fixed
 array inside the library's device image) against xfc_fwd_grad_csr with a caller workspace, through
 the C ABI: bit-identical G and loss, on two calls in a row, the second with a smaller input, so that
 whatever the first call left in the shared array must not leak into the second."""
@@ -54,7 +54,8 @@ def test_static_entry_point_rejects_what_does_not_fit(dev):
     h = lib()
     t = torch.zeros(64, dtype=torch.float16, device=dev)
     i32 = torch.zeros(9, dtype=torch.int32, device=dev)
-    # 4 M positives need 32 MB of bucket entries: beyond the fixed array, refused before any launch
+    # 4 M positives need 16 MB, four bytes each: beyond the fixed array (whether a loss is asked for or not), refused
+    # before any launch
     rc = h.xfc_fwd_grad_csr_static(t.data_ptr(), 8, t.data_ptr(), 8, i32.data_ptr(), i32.data_ptr(), t.data_ptr(), 8,
                                    8, 8, 8, 4_000_000, None, torch.cuda.current_stream().cuda_stream)
     assert rc == 7 and b"capacity" in h.xfc_strerror(rc)
