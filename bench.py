@@ -40,9 +40,9 @@ HBM_PEAK_GBS = 8000.0           # MI355X HBM3E, AMD's published figure
 # copy in the same run) + WRITE_SIZE (KiB, x1.000); see profiles/xfc_step_cfg2_hbm_traffic_pmc.md.
 DW_UPDATE_TRAFFIC_BYTES = {2: (2.000 * 2815091.2 + 1.000 * 3932160.0) * 1024.0,
                            # the other configurations: profiles/xfc_step_other_configs_hbm_traffic_pmc.md
-                           1: (2.000 * 285086.0 + 1.000 * 393216.0) * 1024.0,
-                           3: (2.000 * 8560528.2 + 1.000 * 8436843.0) * 1024.0,
-                           4: (2.000 * 49418471.8 + 1.000 * 50331648.0) * 1024.0}
+                           1: (2.000 * 285002.6 + 1.000 * 393216.0) * 1024.0,
+                           3: (2.000 * 8609197.2 + 1.000 * 8436843.0) * 1024.0,
+                           4: (2.000 * 49335013.9 + 1.000 * 50331648.0) * 1024.0}
 
 
 def _oracle_steps(B, L, d, c, seed, n_max, budget_s, warm):

@@ -3,7 +3,7 @@
 //
 // What bounds it.  The step's products are small (16 to 64 rows against each weight), its traffic is not: 8 bytes per
 // weight.  As three products the weights came from memory twice more, and each launch filled and drained the chip anew.
-// Whole steps, three passes -> one: 32 rows x 131,072 labels x 768 dims 245 -> 193 us (this kernel 154 to 173: 4.7 to 5.2 TB/s of
+// Whole steps, three passes -> one: 32 rows x 131,072 labels x 768 dims 245 -> 193 us (this kernel 172 to 188: 4.3 to 4.7 TB/s of
 // those 8 bytes); 64 x 4,097 x 768 41 -> 30 us; 32 x 400,001 x 768 753 -> 540 us; 8 x 40,001 x 128 96 -> 23 us; 64 x
 // 400,001 x 384 471 -> 307 us.  What is left: the weights' and the momentum's loads come in pieces of 64 bytes, and a
 // small label count is one tile to a workgroup, a chain of loads, z, the two barriers and the update (17 to 27 us).
@@ -57,9 +57,10 @@ struct SmallStep {
   // Workgroups per CU: as many as the registers (256 a wave, 128 with one block of dims and 32 rows, 168 with 12 waves) and the LDS allow.
   static constexpr int WAVES_PER_EU = NW == 12 ? 3 : SB == 1 && RB == 2 ? 4 : 2;
   // With 32 rows the next tile's weights and momentum are both fetched while a tile is worked on.  With more rows, or 128
-  // dims a wave, the registers do not hold them beside the sums (40 to 60 spills, 749 us instead of 618 at 64 rows x
+  // dims a wave, the registers do not hold them beside the sums (40 to 60 spilled, 749 us instead of 618 at 64 rows x
   // 400,001 labels x 768): there the momentum's loads wait until z has left its registers, and the weights move to the LDS
-  // after that and the next tile's are fetched in their place.
+  // after that and the next tile's are fetched in their place.  Spills that are left: 22 registers at 64 rows x 768, 5 at
+  // 32 x 128, 1 at 32 x 384.
   static constexpr bool AHEAD = RB == 2 && SB <= 3;
   static constexpr int BY_REGS = 4 * WAVES_PER_EU / NW, BY_LDS = 160 * 1024 / LDS_BYTES;
   static constexpr int PER_CU = BY_REGS < BY_LDS ? BY_REGS : BY_LDS;

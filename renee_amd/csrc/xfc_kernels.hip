@@ -1629,9 +1629,13 @@ int launch_fwd(int mode, const half_t* X, int64_t ldx, const half_t* W, int64_t 
 
 // Split count for dX: a multiple of 8 slices of the label axis (workgroup ids are dealt round-robin over
 // the 8 XCDs, so the tiles of one slice then meet in one L2), each slice a multiple of the k-step.  The
-// count minimises a cost model fitted to measurements: workgroups run in rounds of one per CU, every
-// workgroup pays a fixed prologue + partial-tile store, and the partial sums are written and read once.
-// A stage of a smaller row tile takes proportionally less time.
+// count minimises a cost model: workgroups run in rounds of one per CU, every workgroup pays a fixed prologue +
+// partial-tile store, and the partial sums are written and read once.  A stage of a smaller row tile takes
+// proportionally less time.  The model's constants were fitted to an eight-wave loop (2.4 us a stage; dx_wide_kernel takes
+// 1.6) and a slower reduction; what decides is the number of rounds, which they do not touch.  Timed over 8 to 256 slices
+// at 199, 256, 512 and 1024 rows x 131,072, 320,001 (384 dims), 655,363, 1,310,720 and 2,812,281 labels, the chosen count
+// is within 1.6 % of the best one everywhere but at 199 x 131,072, where 64 slices take 67 us and the chosen 80 take 71
+// to 74.
 // With ws_limit the choice is restricted to slice counts whose partial sums fit that many bytes (8 slices, the
 // minimum, is always a candidate: the caller checks the final need).  The unrestricted need is not monotone in M
 // (a smaller batch may pick more slices), so a workspace sized for one batch serves smaller ones through this limit.
@@ -1707,8 +1711,9 @@ int launch_dw(int mode, DwArgs a, hipStream_t st) {
 }
 
 // The one-pass step of small batches (small_step.hpp).  Fn::operator()<S>() is called with the kernel for d dims and B
-// rows; false if there is none: other widths do not divide among the waves in 32s, and 64 rows of 1024 dims with the
-// waves' regions exceed the LDS.  Wherever there is one it is the faster: 1.24 to 4.1 times over 8 to 64 rows and 4,097 to
+// rows; false if there is none: these six widths are the ones that are built (each is two kernels; 64, 192, 320, 640 and
+// others would divide among waves in 32s too, and run as three passes), and 64 rows of 1024 dims with the waves' regions
+// exceed the LDS.  Wherever there is one it is the faster: 1.24 to 4.1 times over 8 to 64 rows and 4,097 to
 // 400,001 labels, least at 64 x 400,001 x 768 (768 -> 618 us).  384 dims and 64 rows take 12 waves of one block of dims:
 // with 4 waves of three, 41 spills, 456 us at 64 x 400,001 instead of 307.
 template <class Fn>
