@@ -339,14 +339,19 @@ struct WideCore {
     for (int j = 0; j < NR; ++j) read_one(j, sa, sb, 0, wm, wn, lane, f0);
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
     bool drain_all = false;
+    // (lambdas, not calls: written out, the compiler deals the forward kernel's scalar registers in another order)
+    auto a_piece = [&](int j) { ca.piece(j); };
+    auto a_bump = [&](int j) { ca.bump(j); };
+    auto b_piece = [&](int j) { cb.piece(j); };
+    auto b_bump = [&](int j) { cb.bump(j); };
     // The order below is the schedule: nothing may move across a sched_barrier.
     auto sub_step0 = [&](auto first_tag) {
 #pragma unroll
       for (int n = 0; n < NM; ++n) {
         mfma<decltype(first_tag)::value>(n, f0, acc);
         if (n % READ_EVERY == 0 && n / READ_EVERY < NR) read_one(n / READ_EVERY, sa, sb, 1, wm, wn, lane, f1);
-        if (n % A_EVERY == A_EVERY - 1 && n / A_EVERY < A_CH) ca.piece(n / A_EVERY);
-        if (n % A_EVERY == 1 && n > A_EVERY && n / A_EVERY - 1 < A_CH) ca.bump(n / A_EVERY - 1);
+        if (n % A_EVERY == A_EVERY - 1 && n / A_EVERY < A_CH) a_piece(n / A_EVERY);
+        if (n % A_EVERY == 1 && n > A_EVERY && n / A_EVERY - 1 < A_CH) a_bump(n / A_EVERY - 1);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -355,8 +360,8 @@ struct WideCore {
       for (int n = 0; n < NM; ++n) {
         mfma<false>(n, f1, acc);
         if (n % READ_EVERY == 0 && n / READ_EVERY < NR) read_one(n / READ_EVERY, sa, sb, 0, wm, wn, lane, f0);
-        if (n % B_EVERY == B_EVERY - 1 && n / B_EVERY < B_CH) cb.piece(n / B_EVERY);
-        if (n % B_EVERY == 1 && n > B_EVERY && n / B_EVERY - 1 < B_CH) cb.bump(n / B_EVERY - 1);
+        if (n % B_EVERY == B_EVERY - 1 && n / B_EVERY < B_CH) b_piece(n / B_EVERY);
+        if (n % B_EVERY == 1 && n > B_EVERY && n / B_EVERY - 1 < B_CH) b_bump(n / B_EVERY - 1);
         __builtin_amdgcn_sched_barrier(0);
       }
     };

@@ -319,7 +319,7 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
 // listed twice writes the same value twice.  Input is CSR (rowptr/colidx, pos_x == nullptr; a pair finds its row by a
 // 64-way search of the row pointers, two rounds of loads up to 4096 rows) or COO (pos_x/pos_y int64).  Pairs whose row
 // or column is out of range are dropped.  (The pass that bucketed the list by label tile ran in one workgroup in front
-// of the forward pass: 11.6 us at 2729 pairs, 23 us at 8357; this one takes 5.9 and 7.3.)
+// of the forward pass: 11.6 us at 2729 pairs, 23 us at 8357; this one takes 5.9 and 7.3, with the loss 8.0 at 2729.)
 // LOSS: loss_pos[p] = z of the pair, or 0 if it was dropped or another copy of it was first.  The copies are told apart
 // by G's sign bit, which sigmoid leaves clear and a visited positive sets (a zero difference is stored as -0).  This z is
 // the forward pass's to the last bit, made by the same MFMAs in the same order: it cancels the max(z, 0) that the pass
