@@ -219,8 +219,9 @@ int xfc_step_coo(const void* X, int64_t ldx, void* W, int64_t ldw, void* M, int6
  * Replaces FullPredictor's scoring loop, dl_base.py:736-756 (xfc_forward into outsoft,
  * then torch.max K times with the winners overwritten, or torch.topk for K > 5) and the
  * pad clamp at dl_base.py:782: indices >= numy are returned as numy-1.  1 <= K <= 8192, K <= L.
- *   K <= 8 (the reference's per-epoch K = 5): one fused pass, the logits are never
- *     written; values are the fp32 accumulators (the reference returns fp16-rounded logits).
+ *   K <= 8 (the reference's per-epoch K = 5): the logits are never written, only the largest of every
+ *     block of 16 or 32 labels; the best blocks' scores are then formed again.  Values are the fp32
+ *     accumulators (the reference returns fp16-rounded logits).
  *   8 < K <= 8192 (the reference's final evaluation, K = 100, dl_base.py:817-818; torch.topk at
  *     dl_base.py:756 takes any K; above 1024 the selection sorts in a 128 KB LDS buffer, one row per CU): the fp16
  *     logits of a block of rows go to the workspace and an exact selection kernel picks each
@@ -228,12 +229,12 @@ int xfc_step_coo(const void* X, int64_t ldx, void* W, int64_t ldw, void* M, int6
  *     fp16 values.  xfc_topk_workspace_bytes() asks for all B rows at once (B*round_up(L,8)*2
  *     bytes); any 16-byte aligned workspace that holds min(B, 256) rows is accepted and the
  *     rows are then processed in blocks of a multiple of 256.
- * Scores are expected to be finite: NaN and -inf are never selected by the K <= 8 pass, and a row with
- * fewer than K selectable scores reports (-inf, numy-1) in the remaining places.
+ * K <= 8: a score that is NaN is never selected, and a row with fewer than K other scores reports
+ * (-inf, numy-1) in the remaining places.
  * Workspace: 16-byte aligned (for every K), xfc_topk_workspace_bytes(B, L, K) bytes.  For K <= 8 that is
- * the need of the fastest plan (label groups x B x K x 8 bytes and small extras) and is NOT monotone in B (a
- * smaller batch has fewer row tiles and so more label groups); a smaller workspace is accepted down to the
- * need of 8 label groups.  Use xfc_layer_workspace_bytes() for a buffer that serves every batch size.
+ * B x L x 4 / 16 (up to 32 rows) or / 32 bytes, and NOT monotone in B; a smaller workspace is accepted down to
+ * 64*B*K + 4*round_up(B,4) bytes, and the labels then go in ranges (more launches, the same result).  Use
+ * xfc_layer_workspace_bytes() for a buffer that serves every batch size.
  */
 size_t xfc_topk_workspace_bytes(int64_t B, int64_t L, int64_t K);
 int xfc_topk(const void* X, int64_t ldx, const void* W, int64_t ldw,

@@ -15,6 +15,7 @@
 #include "../../include/xfc_mi355x.h"
 #include "pipe_core.hpp"
 #include "small_step.hpp"
+#include "topk.hpp"
 #include "wide_core.hpp"
 
 namespace xfc {
@@ -41,9 +42,8 @@ using FwdWide = WideCore<256, 256, 2, 2, true>;
 static_assert(FwdWide::LDS_BYTES <= 160 * 1024, "LDS budget");
 // Batches of up to 128 and 64 rows (the reference's B = 32 plumbing case, --accum micro-batches, the last partial batch
 // of an epoch), where a 256-row tile would spend most of its MFMAs on padding: W streams from HBM, eight waves, three
-// ring slots.  FwdCore is the top-K pass's 256-row tile, whose candidate lists take the LDS of a third slot.
-using FwdCore = PipeCore<256, 256, 64, 2, 4, 2, true, true, false, false, false, 4>;  // one wave per SIMD fetches
-using FwdCore128 = PipeCore<128, 256, 64, 2, 4, 3, true, true, false, false, false, 4>;
+// ring slots.
+using FwdCore = PipeCore<128, 256, 64, 2, 4, 3, true, true, false, false, false, 4>;  // one wave per SIMD fetches
 using FwdCore64 = PipeCore<64, 256, 64, 2, 4, 3, true, true, false, false, false, 4>;
 // beside the ring: store staging (8 rows x TN labels per wave)
 template <class C>
@@ -53,7 +53,7 @@ struct FwdLds {
   static_assert(C::FN % 2 == 0, "staging read-back walks 64-label pieces");
   static_assert(BYTES <= 160 * 1024, "LDS budget");
 };
-static_assert(FwdCore::BN == FwdWide::BM && FwdCore128::BN == FwdWide::BM && FwdCore64::BN == FwdWide::BM, "one label tile width");
+static_assert(FwdCore::BN == FwdWide::BM && FwdCore64::BN == FwdWide::BM, "one label tile width");
 
 struct FwdArgs {
   const half_t* X; int64_t ldx;     // M x K, K-contiguous
@@ -428,343 +428,6 @@ __global__ void __launch_bounds__(1024) loss_reduce_kernel(const double* __restr
   if (threadIdx.x == 0) {
     for (int w = 1; w < 16; ++w) t += wave_sum[w];
     *out = (float)t;
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// top-K labels per row of X . W^T, never writing the logits (K <= 8)
-// ---------------------------------------------------------------------------------------------
-// Each workgroup owns 256 query rows and walks every n_groups-th label tile with the forward main loop.
-// Per row it keeps the K best (score, label) pairs seen so far, ordered by score descending and label
-// ascending (the order iterated torch.max produces: first maximum wins ties).  A finished tile is first
-// filtered against each row's current K-th score; survivors (few once the lists have warmed up) go to
-// a small per-row buffer that the row's owner thread merges.  If any row overflows its buffer, the tile
-// is taken again exactly, a few columns at a time.  A second kernel merges the groups' lists.
-// The workgroups that share a row tile also share what they have learnt: each publishes its rows' K-th
-// scores to `bound` (atomic max) and filters against the largest published one as well.  Any published
-// value is the K-th score of K real labels, so nothing below it can be in the row's final list; ties with
-// it pass (a tying label of lower id may still rank above).  This only makes the filter tighter sooner:
-// the lists, and so the results, do not depend on when a bound becomes visible.
-constexpr int TOPK_MAX = 8;
-// Filtered candidates a row can take per tile on the fast path.  What the LDS leaves room for is 6; the 64-row tile has
-// room for 32, a whole 32-column block, which turns the exact retake of a tile from 32 staged pieces of 8 columns into 8
-// blocks of which only the candidates are looked at.  With small batches the label groups are one or two tiles long, so
-// the first tile of each, which starts from no bound, is much of the work: 16 rows x 131,072 labels x 768, K = 5: the
-// pass took 171 us with the staged retake on the 64-row tile, now 99.
-template <class C>
-constexpr int TOPK_CAP = C::BM == 64 ? 32 : 6;
-template <class C>
-struct TopkLds {
-  float list_v[C::BM][TOPK_MAX];
-  int32_t list_i[C::BM][TOPK_MAX];
-  float tau[C::BM];
-  int32_t cnt[C::BM];
-  static constexpr int CAP = TOPK_CAP<C>;
-  float buf_v[C::BM][CAP];  // candidates; CAP < 32, slow path: 8 staged columns (with buf_i)
-  int32_t buf_i[C::BM][CAP];
-  int32_t overflow;
-  static constexpr int BYTES = C::LDS_BYTES + (int)(sizeof(float) * C::BM * (2 * TOPK_MAX + 2 + 2 * TOPK_CAP<C>) + 16);
-};
-static_assert(TopkLds<FwdCore>::BYTES <= 160 * 1024 && TopkLds<FwdCore128>::BYTES <= 160 * 1024 &&
-              TopkLds<FwdCore64>::BYTES <= 160 * 1024, "top-K LDS budget");
-static_assert(2 * TOPK_CAP<FwdCore> >= 8, "the exact rescan stages 8 columns in the candidate buffers");
-
-struct TopkArgs {
-  const half_t* X; int64_t ldx;
-  const half_t* W; int64_t ldw;
-  int M, N, K;          // rows, labels, feature dims
-  int topk;
-  float* cand_v; int32_t* cand_i;  // [n_groups][M][topk]
-  uint32_t* bound;                 // [M] shared lower bounds of the rows' final K-th scores (ordered keys, 0 = none yet)
-  int tiles_m, tiles_n, n_groups;
-};
-
-// Floats as unsigned keys in the same order (for atomicMax), and back.
-__device__ __forceinline__ uint32_t topk_key(float f) {
-  const uint32_t b = __float_as_uint(f);
-  return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-__device__ __forceinline__ float topk_unkey(uint32_t k) {
-  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
-}
-// A value strictly below x (x finite or +inf) and as close to it as a normal number allows: "v > below(x)"
-// admits every v >= x.  Tiny magnitudes step to a fixed small negative so that no denormal is ever compared.
-__device__ __forceinline__ float topk_below(float x) {
-  if (fabsf(x) < 1e-30f) return -1e-30f;
-  const uint32_t b = __float_as_uint(x);
-  return __uint_as_float(x > 0.f ? b - 1u : b + 1u);
-}
-
-__device__ __forceinline__ bool topk_better(float av, int ai, float bv, int bi) {
-  return av > bv || (av == bv && ai < bi);
-}
-__device__ __forceinline__ void topk_insert(float* lv, int32_t* li, int K, float v, int i) {
-  if (!topk_better(v, i, lv[K - 1], li[K - 1])) return;
-  int p = K - 1;
-  while (p > 0 && topk_better(v, i, lv[p - 1], li[p - 1])) {
-    lv[p] = lv[p - 1];
-    li[p] = li[p - 1];
-    --p;
-  }
-  lv[p] = v;
-  li[p] = i;
-}
-
-// The same on a list of TOPK_MAX held in registers.
-__device__ __forceinline__ void topk_insert_regs(float (&lv)[TOPK_MAX], int32_t (&li)[TOPK_MAX], float v, int i) {
-#pragma unroll
-  for (int j = TOPK_MAX - 1; j >= 0; --j) {
-    const bool here = topk_better(v, i, lv[j], li[j]);
-    const bool above = j > 0 && topk_better(v, i, lv[j > 0 ? j - 1 : 0], li[j > 0 ? j - 1 : 0]);
-    const float sv = above ? lv[j > 0 ? j - 1 : 0] : v;
-    const int32_t si = above ? li[j > 0 ? j - 1 : 0] : i;
-    lv[j] = here ? sv : lv[j];
-    li[j] = here ? si : li[j];
-  }
-}
-
-// Inlined on purpose: a function that is called waits for every outstanding memory operation on entry
-// (the calling convention cannot know what is in flight), which here is the next tile's prefetch.
-template <class S_t>
-__device__ __forceinline__ void topk_push(S_t& S, int row, float v, int col) {
-  const int slot = atomicAdd(&S.cnt[row], 1);
-  if (slot < S_t::CAP) { S.buf_v[row][slot] = v; S.buf_i[row][slot] = col; }
-  else S.overflow = 1;
-}
-
-template <class C>
-__global__ void __launch_bounds__(C::NT) topk_kernel(TopkArgs a) {
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
-  half_t* lds = reinterpret_cast<half_t*>(smem_raw);
-  TopkLds<C>& S = *reinterpret_cast<TopkLds<C>*>(smem_raw + C::LDS_BYTES);
-  // ids are dealt round-robin to XCDs: the row tiles of one label group sit side by side on one XCD
-  int mt, grp;
-  xcd_map(blockIdx.x, a.tiles_m, mt, grp);
-  const int n_items = grp < a.tiles_n ? (a.tiles_n - grp + a.n_groups - 1) / a.n_groups : 0;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be
-  const int wm = wave / C::WN, wn = wave % C::WN;
-  const int m0 = mt * C::BM;
-  const int K = a.topk;
-  const float NEG_INF = -__builtin_huge_valf();
-  auto bound_of = [&](uint32_t key) { return key > topk_key(NEG_INF) ? topk_below(topk_unkey(key)) : NEG_INF; };
-  if (threadIdx.x == 0) S.overflow = 0;
-  __syncthreads();
-  for (int t = threadIdx.x; t < C::BM; t += C::NT) {
-    for (int j = 0; j < TOPK_MAX; ++j) { S.list_v[t][j] = NEG_INF; S.list_i[t][j] = 0x7fffffff; }
-    // the first tile is filtered against a seeded bound, if there is one (1024 rows x 2,812,281 labels: 4.54 -> 4.32 ms
-    // against a first tile that starts from nothing and is taken twice); rows past the batch never take anything
-    float tau = -NEG_INF;
-    if (m0 + t < a.M) tau = bound_of(__hip_atomic_load(a.bound + m0 + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    S.tau[t] = tau;
-    S.cnt[t] = 0;
-    // without one the first tile is taken the exact way at once, which also admits scores of -inf
-    if (TopkLds<C>::CAP >= 32 && tau == NEG_INF) S.overflow = 1;
-  }
-  __syncthreads();
-
-  auto get = [&](int item, typename C::Operand& oa, typename C::Operand& ob, int& kb, int& ke) {
-    const int nt = grp + item * a.n_groups;
-    oa = typename C::Operand{a.X, a.ldx, m0, a.M, a.K};
-    ob = typename C::Operand{a.W, a.ldw, nt * C::BN, a.N, a.K};
-    kb = 0;
-    ke = a.K;
-  };
-  auto epilogue = [&](int item, float16v (&acc)[C::FM][C::FN]) {
-    const int nt = grp + item * a.n_groups;
-    const int n0 = nt * C::BN;
-    const bool ragged = n0 + C::BN > a.N;
-    const int h = lane >> 5;
-    // the row owners ask for the shared bound now and use it after the filter
-    const bool owner = threadIdx.x < C::BM && m0 + (int)threadIdx.x < a.M;
-    uint32_t shared_key = 0u;
-    if (owner) shared_key = __hip_atomic_load(a.bound + m0 + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // what the filter compares with from the next tile on: the list's K-th score, or just below the shared bound
-    auto settle = [&](int t, bool changed) {
-      const float mine = S.list_v[t][K - 1];
-      if (changed && owner && mine > NEG_INF)
-        __hip_atomic_fetch_max(a.bound + m0 + t, topk_key(mine), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      S.tau[t] = owner ? fmaxf(mine, bound_of(shared_key)) : -NEG_INF;
-      S.cnt[t] = 0;
-    };
-    // filter against each row's K-th best so far (a flag that is set already is the first tile's: wave-uniform, all agree)
-    if (TopkLds<C>::CAP < 32 || S.overflow == 0)
-#pragma unroll
-    for (int fm = 0; fm < C::FM; ++fm) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int row0 = wm * C::TM + fm * 32 + 8 * q + 4 * h;
-        const float4v tau4 = *reinterpret_cast<const float4v*>(&S.tau[row0]);
-        // one branch per strip of 4 rows x TN labels: the compares are combined as lane masks, and only a
-        // strip in which some lane holds a survivor walks its elements (rare once the lists have warmed up)
-        bool any = false;
-#pragma unroll
-        for (int fn = 0; fn < C::FN; ++fn)
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) any |= acc[fm][fn][4 * q + rr] > tau4[rr];
-        if (__builtin_amdgcn_ballot_w64(any) != 0) {
-          // opaque on purpose: the compiler otherwise computes the list addresses of all 128 elements when
-          // the kernel starts, spills them, and reloads them here behind a wait for every outstanding fetch
-          int r0 = row0;
-          asm volatile("" : "+v"(r0));
-#pragma unroll
-          for (int fn = 0; fn < C::FN; ++fn) {
-            const int col = n0 + wn * C::TN + fn * 32 + (lane & 31);
-            const bool col_ok = !ragged || col < a.N;
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-              const float v = acc[fm][fn][4 * q + rr];
-              if (v > tau4[rr] && col_ok) topk_push(S, r0 + rr, v, col);
-            }
-          }
-        }
-        asm volatile("" ::: "memory");  // keep the threshold reads of later strips from being hoisted up here
-      }
-    }
-    __syncthreads();
-    const bool overflow = S.overflow != 0;
-    if (!overflow) {
-      if (threadIdx.x < C::BM) {
-        const int t = threadIdx.x;
-        const int n = S.cnt[t];
-        for (int i = 0; i < n; ++i) topk_insert(S.list_v[t], S.list_i[t], K, S.buf_v[t][i], S.buf_i[t][i]);
-        settle(t, n != 0);
-      }
-    } else if constexpr (TopkLds<C>::CAP >= 32) {
-      // exact retake, a block of 32 columns at a time: no row can have more candidates than its buffer holds, and from
-      // the second block on only those that pass the bound the earlier blocks have raised.  ("At least the bound" here:
-      // a list that is not full takes scores of -inf too.)
-      const int t = threadIdx.x;
-      float lv[TOPK_MAX];
-      int32_t li[TOPK_MAX];
-      __syncthreads();
-      if (t < C::BM) {
-#pragma unroll
-        for (int j = 0; j < TOPK_MAX; ++j) { lv[j] = S.list_v[t][j]; li[j] = S.list_i[t][j]; }
-        S.cnt[t] = 0;
-      }
-      if (t == 0) S.overflow = 0;
-      __syncthreads();
-#pragma unroll
-      for (int sfn = 0; sfn < C::FN; ++sfn) {
-        for (int swn = 0; swn < C::WN; ++swn) {
-          if (wn == swn) {
-            const int col = n0 + swn * C::TN + sfn * 32 + (lane & 31);
-            if (col < a.N) {
-#pragma unroll
-              for (int fm = 0; fm < C::FM; ++fm)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                  const int row = wm * C::TM + fm * 32 + c_row(r, lane);
-                  const float v = acc[fm][sfn][r];
-                  if (v >= S.tau[row]) topk_push(S, row, v, col);
-                }
-            }
-          }
-          __syncthreads();
-          if (t < C::BM) {
-            const int n = S.cnt[t];
-            for (int i = 0; i < n; ++i) topk_insert_regs(lv, li, S.buf_v[t][i], S.buf_i[t][i]);
-            float kth = lv[0];
-#pragma unroll
-            for (int j = 1; j < TOPK_MAX; ++j) kth = j < K ? lv[j] : kth;
-            S.tau[t] = fmaxf(S.tau[t], kth);
-            S.cnt[t] = 0;
-          }
-          __syncthreads();
-        }
-      }
-      if (t < C::BM) {
-#pragma unroll
-        for (int j = 0; j < TOPK_MAX; ++j) { S.list_v[t][j] = lv[j]; S.list_i[t][j] = li[j]; }
-        settle(t, true);
-      }
-    } else {
-      // exact rescan: stage 8 columns of all 256 rows at a time, each row's owner inserts them
-      float* stage = &S.buf_v[0][0];  // 256 x 8 floats: buf_v and buf_i are adjacent
-      __syncthreads();
-#pragma unroll
-      for (int swn = 0; swn < C::WN; ++swn) {
-#pragma unroll
-        for (int sfn = 0; sfn < C::FN; ++sfn) {
-          for (int sg = 0; sg < 4; ++sg) {
-            if (wn == swn && ((lane & 31) >> 3) == sg) {
-#pragma unroll
-              for (int fm = 0; fm < C::FM; ++fm)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                  stage[(wm * C::TM + fm * 32 + c_row(r, lane)) * 8 + (lane & 7)] = acc[fm][sfn][r];
-            }
-            __syncthreads();
-            if (threadIdx.x < C::BM) {
-              const int t = threadIdx.x;
-              const int cbase = n0 + swn * C::TN + sfn * 32 + sg * 8;
-              for (int e = 0; e < 8; ++e)
-                if (cbase + e < a.N) topk_insert(S.list_v[t], S.list_i[t], K, stage[t * 8 + e], cbase + e);
-            }
-            __syncthreads();
-          }
-        }
-      }
-      if (threadIdx.x < C::BM) settle(threadIdx.x, true);
-      if (threadIdx.x == 0) S.overflow = 0;
-    }
-    __syncthreads();
-  };
-  C::run(0, n_items, lds, get, epilogue);
-  __syncthreads();
-  if (threadIdx.x < C::BM && m0 + threadIdx.x < a.M && grp < a.n_groups) {
-    const int64_t o = ((int64_t)grp * a.M + m0 + threadIdx.x) * K;
-    for (int j = 0; j < K; ++j) { a.cand_v[o + j] = S.list_v[threadIdx.x][j]; a.cand_i[o + j] = S.list_i[threadIdx.x][j]; }
-  }
-}
-
-// One workgroup per row, one thread per group (and every 256th): K rounds of "best head of the groups' lists", which are
-// in order.  Bound by latency: the candidates are read once, up front.  (One wave per row that read all candidates anew in
-// each round took 33 us for 256 groups, K = 5; this one 6.7.)
-__global__ void __launch_bounds__(256) topk_merge_kernel(const float* __restrict__ cand_v, const int32_t* __restrict__ cand_i,
-                                                         int M, int n_groups, int K, int64_t numy,
-                                                         float* __restrict__ out_v, int64_t* __restrict__ out_i) {
-  __shared__ unsigned long long wave_best[2][4];
-  const int row = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // this thread's best TOPK_MAX, in order; entries past K are those of a list that is not full, and lose to all others
-  float lv[TOPK_MAX];
-  int32_t li[TOPK_MAX];
-#pragma unroll
-  for (int j = 0; j < TOPK_MAX; ++j) { lv[j] = -__builtin_huge_valf(); li[j] = 0x7fffffff; }
-  for (int g = threadIdx.x; g < n_groups; g += 256) {
-    const int64_t o = ((int64_t)g * M + row) * K;
-    if (g == (int)threadIdx.x) {
-#pragma unroll
-      for (int j = 0; j < TOPK_MAX; ++j)
-        if (j < K) { lv[j] = cand_v[o + j]; li[j] = cand_i[o + j]; }
-    } else {
-      for (int j = 0; j < K; ++j) topk_insert_regs(lv, li, cand_v[o + j], cand_i[o + j]);
-    }
-  }
-  for (int r = 0; r < K; ++r) {
-    // score descending, then label ascending, as one number; a score of -0 ranks with +0
-    const unsigned long long mine = ((unsigned long long)topk_key(lv[0] == 0.f ? 0.f : lv[0]) << 32) | (uint32_t)~li[0];
-    unsigned long long best = mine;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const unsigned long long other = __shfl_xor(best, off, 64);
-      best = other > best ? other : best;
-    }
-    if (lane == 0) wave_best[r & 1][wave] = best;
-    __syncthreads();  // one per round: the next round writes the other half, and the one after it waits for this read
-    best = wave_best[r & 1][0];
-#pragma unroll
-    for (int w = 1; w < 4; ++w) best = wave_best[r & 1][w] > best ? wave_best[r & 1][w] : best;
-    if (mine == best) {  // one thread, or all that hold nothing more
-      out_v[(int64_t)row * K + r] = lv[0];
-      int64_t idx = li[0];
-      if (idx >= numy) idx = numy - 1;  // padded labels are clamped, as the reference does
-      out_i[(int64_t)row * K + r] = idx;
-#pragma unroll
-      for (int j = 0; j + 1 < TOPK_MAX; ++j) { lv[j] = lv[j + 1]; li[j] = li[j + 1]; }
-      lv[TOPK_MAX - 1] = -__builtin_huge_valf();
-      li[TOPK_MAX - 1] = 0x7fffffff;
-    }
   }
 }
 
@@ -1415,23 +1078,6 @@ __global__ void __launch_bounds__(256) generic_gemm_kernel(const half_t* __restr
 }
 
 // Plain copy, 16 bytes per thread step: the known-size kernel that HBM traffic counters are scaled by.
-__global__ void __launch_bounds__(256) fill_u32_kernel(uint32_t* __restrict__ dst, uint32_t value, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) dst[i] = value;
-}
-
-// bound[r] = key of a value safely below the K-th largest of row r's sample scores.  The sample scores
-// are fp16 roundings (half an ulp from the fp32 score at most), so one part in 1024 plus the smallest fp16
-// step below the K-th rounded score is below the K-th fp32 score of the sample, hence of the whole row.
-__global__ void __launch_bounds__(256) topk_seed_kernel(const float* __restrict__ sample_v, int K, uint32_t* __restrict__ bound,
-                                                        int64_t n) {
-  const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (r >= n) return;
-  const float x = sample_v[r * K + K - 1];
-  const float lo = x - (fabsf(x) * 0.0009765625f + 1.2e-7f);
-  bound[r] = (lo == lo && lo > -__builtin_huge_valf()) ? topk_key(lo) : 0u;  // NaN or -inf: no bound
-}
-
 __global__ void __launch_bounds__(256) copy_kernel(const uint4v* __restrict__ src, uint4v* __restrict__ dst, int64_t n16) {
   const int64_t stride = (int64_t)gridDim.x * 256;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += stride) dst[i] = src[i];
@@ -1519,6 +1165,8 @@ int current_device() {
   return dev;
 }
 
+constexpr int FULL_LDS = 160 * 1024;
+
 // Dynamic LDS above the default limit needs the attribute once per kernel and device.
 template <auto Kernel>
 hipError_t raise_lds_limit(int lds) {
@@ -1577,7 +1225,7 @@ constexpr size_t LOSS_PART_BYTES = 4096;
 constexpr int MAX_FWD_GRID = LOSS_PART_BYTES / sizeof(double) - 8;  // 504, with room to align; a multiple of 8
 size_t fwd_ws_bytes(int64_t nnz) { return LOSS_PART_BYTES + (size_t)round_up((nnz > 0 ? nnz : 1) * 4, 256); }
 
-// Row-tile height for a batch of M rows (see FwdWide / FwdCore128 / FwdCore64).
+// Row-tile height for a batch of M rows (see FwdWide / FwdCore / FwdCore64).
 inline int row_tile(int64_t M) { return M <= 64 ? 64 : M <= 128 ? 128 : 256; }
 
 // Workgroups of the forward pass: one resident per CU (the number of tile ids is a multiple of 8).
@@ -1622,7 +1270,7 @@ int launch_fwd(int mode, const half_t* X, int64_t ldx, const half_t* W, int64_t 
   const dim3 g((unsigned)fwd_grid(ids));
   switch (row_tile(M)) {
     case 64: return launch_fwd_c<FwdCore64>(mode, a, g, st);
-    case 128: return launch_fwd_c<FwdCore128>(mode, a, g, st);
+    case 128: return launch_fwd_c<FwdCore>(mode, a, g, st);
     default: return launch_fwd_wide(mode, a, g, st);
   }
 }
@@ -1760,6 +1408,25 @@ int launch_generic(const void* in1, int64_t as0, int64_t as1, const void* in2, i
   return check_launch();
 }
 
+template <int RB>
+int launch_score_small(ScoreArgs a, hipStream_t st) {
+  constexpr int NW = SCORE_SMALL_WAVES;
+  const int64_t most = (int64_t)2 * num_cus(), units = ceil_div(a.N, SCORE_SMALL_BLOCK), waves = most * NW;
+  // Units in a row for a wave: a row's maxima are then stored 8 or 16 bytes at a time (32 rows x 700,001 labels x 768: 217 -> 208
+  // us), as long as that leaves the longest wave's work what it is, or with 32 rows to store for a tenth more.
+  a.run = 1;
+  for (int run : {2, 4})
+    if (10 * run * ceil_div(units, run * waves) <= (RB == 1 ? 10 : 11) * ceil_div(units, waves)) a.run = run;
+  const int64_t want = ceil_div(units, a.run * NW);
+  // (the limit is raised once, for any width)
+  const hipError_t e = raise_lds_limit<score_small_kernel<RB>>(FULL_LDS);
+  if (e != hipSuccess) {
+    fprintf(stderr, "xfc: cannot raise the dynamic LDS limit to %d bytes: %s\n", FULL_LDS, hipGetErrorString(e));
+    return XFC_ERR_HIP;
+  }
+  return launch_k<score_small_kernel<RB>>(dim3((unsigned)(want < most ? want : most)), dim3(64 * NW), score_small_lds<RB>(a.K), st, a);
+}
+
 struct SelArgs {
   const half_t* logits; int64_t ldl; int L; int64_t numy; int K; int stride; float* out_v; int64_t* out_i;
 };
@@ -1807,7 +1474,8 @@ int xfc_init(void) {
   keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID, false>>(FwdWide::LDS_BYTES));
   keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID_PLAIN, false>>(FwdWide::LDS_BYTES));
   keep(raise_lds_limit<fwd_wide_kernel<FWD_LINEAR, false>>(FwdWide::LDS_BYTES));
-  keep(raise_lds_limit<topk_kernel<FwdCore>>(TopkLds<FwdCore>::BYTES));
+  keep(raise_lds_limit<score_wide_kernel<ScoreWide>>(ScoreWide::LDS_BYTES));
+  keep(raise_lds_limit<score_wide_kernel<ScoreWide128>>(ScoreWide128::LDS_BYTES));
   keep(raise_lds_limit<dx_wide_kernel>(DxWide::LDS_BYTES));
   auto small_limits = [&](auto core_tag, auto dx_tag) {
     using C = typename decltype(core_tag)::type;
@@ -1818,14 +1486,15 @@ int xfc_init(void) {
     keep(raise_lds_limit<fwd_kernel<C, FWD_SIGMOID, false>>(LDS));
     keep(raise_lds_limit<fwd_kernel<C, FWD_SIGMOID_PLAIN, false>>(LDS));
     keep(raise_lds_limit<fwd_kernel<C, FWD_LINEAR, false>>(LDS));
-    keep(raise_lds_limit<topk_kernel<C>>(TopkLds<C>::BYTES));
     keep(raise_lds_limit<dx_kernel<D>>(D::LDS_BYTES));
   };
-  small_limits(std::type_identity<FwdCore128>{}, std::type_identity<DxCore>{});
+  small_limits(std::type_identity<FwdCore>{}, std::type_identity<DxCore>{});
   small_limits(std::type_identity<FwdCore64>{}, std::type_identity<DxCore64>{});
   for (int64_t rows : {32, 64})
     for (int64_t d : {128, 256, 384, 512, 768, 1024})
       small_step_for(rows, d, [&](auto s) { keep(raise_lds_limit<small_step_kernel<decltype(s)>>(decltype(s)::LDS_BYTES)); });
+  keep(raise_lds_limit<score_small_kernel<1>>(FULL_LDS));
+  keep(raise_lds_limit<score_small_kernel<2>>(FULL_LDS));
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_SMALL>>((int)sizeof(SelLds<SEL_CAP_SMALL>)));
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_LARGE>>((int)sizeof(SelLds<SEL_CAP_LARGE>)));
   keep(raise_lds_limit<dw_kernel<DW_UPDATE>>(DW_LDS_BYTES));
@@ -2159,48 +1828,44 @@ int xfc_step_coo(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo, int
                    weight_decay, scale, workspace, workspace_bytes, stream);
 }
 
-constexpr int TOPK_SAMPLE = 2048;
-// K <= 8: the rows' bounds start from the K-th score over a sample of the first TOPK_SAMPLE labels (a small
-// logits pass and an exact selection) when every label group has enough tiles for that to pay; otherwise
-// from nothing.  Without it every workgroup's first tiles overflow the candidate buffers and are rescanned.
-static bool topk_seeded(int64_t L, int tiles_n, int n_groups) {
-  return L >= 8 * (int64_t)TOPK_SAMPLE && tiles_n >= 8 * n_groups;
-}
-// bytes of the K <= 8 pass with n_groups label groups: the groups' candidate lists, the rows' shared bounds,
-// and (seeded) the sample logits and their top K
-static size_t topk_need(int64_t B, int64_t K, int n_groups, bool seeded) {
-  size_t need = (size_t)n_groups * B * K * 8 + (size_t)round_up(B, 4) * 4;
-  if (seeded) need += (size_t)B * TOPK_SAMPLE * 2 + (size_t)B * K * 12;
-  return need;
-}
-// Label groups of the K <= 8 pass: enough to give every CU a workgroup, fewer when the workspace holds no more
-// (8 at least; the seeding is dropped before the last groups are).  A smaller batch has fewer row tiles and so
-// more groups: the need is not monotone in B.
-static void topk_plan(int64_t B, int64_t L, int64_t K, size_t ws_limit, int& tiles_m, int& tiles_n, int& n_groups,
-                      int& grid, bool& seeded) {
-  tiles_m = ceil_div(B, row_tile(B));
-  tiles_n = ceil_div(L, FwdCore::BN);
-  int per = num_cus() / (8 * tiles_m);  // groups per XCD
-  if (per < 1) per = 1;
-  n_groups = 8 * per;
-  const int cap = (int)round_up(tiles_n, 8);
-  if (n_groups > cap) n_groups = cap;
-  for (;; n_groups -= 8) {
-    seeded = topk_seeded(L, tiles_n, n_groups);
-    if (topk_need(B, K, n_groups, seeded) <= ws_limit) break;
-    if (seeded && topk_need(B, K, n_groups, false) <= ws_limit) { seeded = false; break; }
-    if (n_groups <= 8) break;  // the caller compares the need of this plan with what it was given
+// The K <= 8 pass.  Up to 32 rows whose fragments fit the LDS the weights stream past them (score_small_kernel), above that
+// the forward pass's main loop runs (both sides of the line: score_wide_kernel); each leaves the largest score of every block.
+struct TopkPlan {
+  bool small;
+  int block;          // labels per block
+  int64_t range, ldb; // labels handled at a time, blocks of a row of the maxima (a multiple of 4)
+};
+static int64_t topk_blocks(int64_t labels, int block) { return round_up(ceil_div(labels, block), 4); }
+// With a workspace that does not hold all maxima the labels go in ranges, the K best of each carried to the next.
+static TopkPlan topk_plan(int64_t B, int64_t L, int64_t d, int64_t K, size_t ws_limit) {
+  TopkPlan p;
+  p.small = B <= SCORE_SMALL_ROWS && (B <= 16 ? score_small_lds<1>(d) : score_small_lds<2>(d)) <= FULL_LDS;
+  p.block = p.small ? SCORE_SMALL_BLOCK : SCORE_WIDE_BLOCK;
+  p.range = L;
+  // a tile of the wide kernel writes the maxima of all its blocks
+  p.ldb = p.small ? topk_blocks(L, p.block) : topk_blocks(round_up(L, FwdWide::BM), p.block);
+  if ((size_t)B * (size_t)p.ldb * 4 > ws_limit) {
+    const int64_t lists = B * K * 8, unit = p.small ? 4 : FwdWide::BM / SCORE_WIDE_BLOCK;
+    const int64_t fit = ws_limit > (size_t)lists ? (int64_t)((ws_limit - (size_t)lists) / ((size_t)B * 4)) : 0;
+    p.ldb = fit / unit * unit;
+    p.range = p.ldb * p.block;
   }
-  grid = tiles_m * n_groups;
+  return p;
+}
+// What the pass refuses to run without, and what it runs fastest with.  (The former is what an earlier form of it needed.)
+static size_t topk_least(int64_t B, int64_t K) { return (size_t)8 * B * K * 8 + (size_t)round_up(B, 4) * 4; }
+static size_t topk_need(int64_t B, int64_t L, int64_t K) {
+  // whichever kernel the width leads to
+  const size_t wide = (size_t)B * (size_t)topk_blocks(round_up(L, FwdWide::BM), SCORE_WIDE_BLOCK) * 4;
+  const size_t small = B <= SCORE_SMALL_ROWS ? (size_t)B * (size_t)topk_blocks(L, SCORE_SMALL_BLOCK) * 4 : 0;
+  const size_t need = wide > small ? wide : small, least = topk_least(B, K);
+  return need > least ? need : least;
 }
 
 size_t xfc_topk_workspace_bytes(int64_t B, int64_t L, int64_t K) {
   if (!dims_ok(B) || !dims_ok(L) || K < 1 || K > SEL_MAX_K || B == 0 || L == 0) return 0;
   if (K > TOPK_MAX) return (size_t)B * (size_t)round_up(L, 8) * 2;  // the logits of every row
-  int tm, tn, ng, grid;
-  bool seeded;
-  topk_plan(B, L, K, ~(size_t)0, tm, tn, ng, grid, seeded);
-  return topk_need(B, K, ng, seeded);
+  return topk_need(B, L, K);
 }
 
 size_t xfc_layer_workspace_bytes(int64_t max_batch, int64_t L, int64_t d, int64_t max_nnz) {
@@ -2251,48 +1916,43 @@ int xfc_topk(const void* X, int64_t ldx, const void* W, int64_t ldw, int64_t B, 
     }
     return XFC_OK;
   }
-  TopkArgs a;
-  int grid;
-  bool seeded;
-  topk_plan(B, L, K, workspace ? workspace_bytes : 0, a.tiles_m, a.tiles_n, a.n_groups, grid, seeded);
-  const size_t need = topk_need(B, K, a.n_groups, seeded);
-  if (!workspace || workspace_bytes < need) return XFC_ERR_WORKSPACE;
+  const TopkPlan p = topk_plan(B, L, d, K, workspace ? workspace_bytes : 0);
+  if (!workspace || workspace_bytes < topk_least(B, K) || p.range < 1) return XFC_ERR_WORKSPACE;
   if (!aligned16(workspace)) return XFC_ERR_ALIGN;
-  a.X = (const half_t*)X; a.ldx = ldx; a.W = (const half_t*)W; a.ldw = ldw;
-  a.M = (int)B; a.N = (int)L; a.K = (int)d; a.topk = K;
-  a.cand_v = reinterpret_cast<float*>(workspace);
-  a.cand_i = reinterpret_cast<int32_t*>(a.cand_v + (size_t)a.n_groups * B * K);
-  a.bound = reinterpret_cast<uint32_t*>(a.cand_i + (size_t)a.n_groups * B * K);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (seeded) {
-    // 16-byte aligned: the lists above are B * K * 8 * n_groups bytes (n_groups a multiple of 8), the bounds 16-byte padded
-    half_t* sample = reinterpret_cast<half_t*>(a.bound + round_up(B, 4));
-    int64_t* sample_i = reinterpret_cast<int64_t*>(sample + (size_t)B * TOPK_SAMPLE);
-    float* sample_v = reinterpret_cast<float*>(sample_i + (size_t)B * K);
-    int rc0 = launch_fwd(FWD_LINEAR, (const half_t*)X, ldx, (const half_t*)W, ldw, sample, TOPK_SAMPLE, (int)B, TOPK_SAMPLE,
-                         (int)d, TOPK_SAMPLE, 1.0f, 0.0f, st);
-    if (rc0) return rc0;
-    const SelArgs sa = {(const half_t*)sample, (int64_t)TOPK_SAMPLE, TOPK_SAMPLE, (int64_t)TOPK_SAMPLE, K, 1, sample_v, sample_i};
-    if ((rc0 = launch_select<SEL_CAP_SMALL>((int)B, sa, st))) return rc0;
-    hipLaunchKernelGGL(topk_seed_kernel, dim3((unsigned)ceil_div(B, 256)), dim3(256), 0, st, (const float*)sample_v, K,
-                       a.bound, B);
-    if ((rc0 = check_launch())) return rc0;
-  } else {
-    // a kernel, not a memset: the call may be recorded into a graph
-    hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)ceil_div(B, 256)), dim3(256), 0, st, a.bound, 0u, B);
-    if (int rc0 = check_launch()) return rc0;
+  for (int64_t l0 = 0; l0 < L; l0 += p.range) {
+    const int64_t n = L - l0 < p.range ? L - l0 : p.range;
+    ScoreArgs a;
+    a.X = (const half_t*)X; a.ldx = ldx; a.W = (const half_t*)W + l0 * ldw; a.ldw = ldw;
+    a.bmax = reinterpret_cast<float*>(workspace); a.ldb = p.ldb;
+    a.M = (int)B; a.N = (int)n; a.K = (int)d;
+    int rc;
+    if (p.small) {
+      rc = B <= 16 ? launch_score_small<1>(a, st) : launch_score_small<2>(a, st);
+    } else {
+      a.tiles_m = ceil_div(B, row_tile(B) <= 128 ? ScoreWide128::BN : ScoreWide::BN);
+      a.tiles_n = ceil_div(n, ScoreWide::BM);
+      const int64_t ids = (int64_t)a.tiles_m * round_up(a.tiles_n, 8);
+      if (ids > 0x7fffffff) return XFC_ERR_INVALID;
+      a.n_ids = (int)ids;
+      auto launch = [&](auto core) {
+        using C = typename decltype(core)::type;
+        return launch_k<score_wide_kernel<C>>(dim3((unsigned)fwd_grid(ids)), dim3(C::NT), C::LDS_BYTES, st, a);
+      };
+      rc = row_tile(B) <= 128 ? launch(std::type_identity<ScoreWide128>{}) : launch(std::type_identity<ScoreWide>{});
+    }
+    if (rc) return rc;
+    PickArgs k;
+    k.X = a.X; k.ldx = ldx; k.W = a.W; k.ldw = ldw; k.bmax = a.bmax; k.ldb = p.ldb;
+    k.n_blocks = ceil_div(n, p.block); k.N = (int)n; k.K = (int)d; k.first = l0; k.topk = K;
+    k.best = p.range < L ? reinterpret_cast<unsigned long long*>(a.bmax + (size_t)B * p.ldb) : nullptr;
+    k.begin = l0 == 0; k.end = l0 + n == L;
+    k.numy = numy; k.out_v = values; k.out_i = indices;
+    if (p.small) hipLaunchKernelGGL(topk_pick_kernel<SCORE_SMALL_BLOCK>, dim3((unsigned)B), dim3(512), 0, st, k);
+    else hipLaunchKernelGGL(topk_pick_kernel<SCORE_WIDE_BLOCK>, dim3((unsigned)B), dim3(512), 0, st, k);
+    if ((rc = check_launch())) return rc;
   }
-  const dim3 tg((unsigned)grid), tb(FwdCore::NT);
-  int rc;
-  switch (row_tile(B)) {
-    case 64: rc = launch_k<topk_kernel<FwdCore64>>(tg, tb, TopkLds<FwdCore64>::BYTES, st, a); break;
-    case 128: rc = launch_k<topk_kernel<FwdCore128>>(tg, tb, TopkLds<FwdCore128>::BYTES, st, a); break;
-    default: rc = launch_k<topk_kernel<FwdCore>>(tg, tb, TopkLds<FwdCore>::BYTES, st, a); break;
-  }
-  if (rc) return rc;
-  hipLaunchKernelGGL(topk_merge_kernel, dim3((unsigned)B), dim3(256), 0, st, a.cand_v, a.cand_i, (int)B, a.n_groups, K,
-                     numy, values, indices);
-  return check_launch();
+  return XFC_OK;
 }
 
 int xfc_copy(const void* src, void* dst, int64_t bytes, void* stream) {
