@@ -243,6 +243,18 @@ int xfc_topk(const void* X, int64_t ldx, const void* W, int64_t ldw,
              void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * xfc_topk with a second buffer.  For K > 8 it takes the largest logit of every 32 labels, from which the
+ * selection learns which few parts of a row to read: min(B, rows the workspace holds) x round_up(L, 256) / 16
+ * bytes, 16-byte aligned (what xfc_topk_workspace_bytes(B, L, 8) asks for is more than enough).  A smaller one, or none, is not used and the
+ * selection reads the rows (xfc_topk does that too unless its workspace has the room behind the logits).
+ * K <= 8: not used.  The results are the same either way.
+ */
+int xfc_topk_scratch(const void* X, int64_t ldx, const void* W, int64_t ldw,
+                     int64_t B, int64_t L, int64_t d, int64_t numy, int K,
+                     float* values, int64_t* indices, void* workspace, size_t workspace_bytes,
+                     void* scratch, size_t scratch_bytes, void* stream);
+
+/*
  * One workspace for every call of a layer: the largest need of xfc_step_csr (= xfc_fwd_grad_* + xfc_dx)
  * and of xfc_topk with K <= 8 over all batch sizes 1..max_batch, with at most max_nnz label pairs per
  * batch.  The per-call *_workspace_bytes() functions are not monotone in B, so sizing by max_batch alone

@@ -317,9 +317,10 @@ class XFCLayer:
         L = lib()
         ws = self.outsoft if K > 8 else self._ws
         with torch.cuda.device(self.device):
-            rc = L.xfc_topk(x.data_ptr(), x.stride(0), self.xfc_weight.data_ptr(), self.dims, bsz, self.numy,
-                            self.dims, self.numy if numy is None else int(numy), int(K), vals.data_ptr(),
-                            inds.data_ptr(), ws.data_ptr(), ws.numel() * ws.element_size(), _stream(x))
+            rc = L.xfc_topk_scratch(x.data_ptr(), x.stride(0), self.xfc_weight.data_ptr(), self.dims, bsz, self.numy,
+                                    self.dims, self.numy if numy is None else int(numy), int(K), vals.data_ptr(),
+                                    inds.data_ptr(), ws.data_ptr(), ws.numel() * ws.element_size(),
+                                    self._ws.data_ptr(), self._ws.numel(), _stream(x))
         check(rc, "xfc_topk")
         return vals, inds
 
