@@ -34,6 +34,9 @@ _SIGNATURES = {
     "xfc_sgd_momentum_master": (_int, [_vp, _vp, _vp, _vp, _i64, _f32, _f32, _f32, _vp]),
     "xfc_dw": (_int, [_vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _f32, _vp]),
     "xfc_sgd_momentum": (_int, [_vp, _vp, _vp, _i64, _f32, _f32, _f32, _vp]),
+    "xfc_dx_dw_update": (_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _f32, _f32, _f32, _f32,
+                                _vp, _sz, _vp]),
+    "xfc_dx_dw": (_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _f32, _f32, _vp, _sz, _vp]),
     "xfc_step_workspace_bytes": (_sz, [_i64, _i64, _i64, _i64]),
     "xfc_step_csr": (_int, [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64,
                             _f32, _f32, _f32, _f32, _vp, _sz, _vp]),

@@ -21,15 +21,10 @@ from .xfc import XFCLayer
 class _XFCStep(torch.autograd.Function):
     @staticmethod
     def forward(ctx, embed, layer, pos_x, pos_y, scale, lr, compute_loss, accumulate):
-        bsz = embed.shape[0]
         loss = torch.zeros(1, device=layer.device, dtype=torch.float32)
         if compute_loss:
             layer.fwd_grad(embed, pos_x, pos_y, loss_out=loss)
-            gi = layer.dx(bsz, None, scale)
-            if accumulate:
-                layer.dw_accumulate(embed)
-            else:
-                layer.dw_update(embed, lr=lr)
+            gi = layer.backward_pass(embed, None, scale, accumulate, lr)
         else:
             gi = layer.xfc_backward(embed, pos_x, pos_y, None, scale, accumulate, lr)
         # the layer's grad_input buffer is reused by the next step: keep this step's values

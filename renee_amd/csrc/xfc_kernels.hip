@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "../../include/xfc_mi355x.h"
+#include "back_step.hpp"
 #include "pipe_core.hpp"
 #include "small_step.hpp"
 #include "topk.hpp"
@@ -1531,6 +1532,57 @@ size_t small_step_ws_bytes(int64_t B, int64_t L, int64_t d) {
   return need;
 }
 
+// dX and dW (or the update) of a batch of up to 256 rows in one pass over the labels (back_step.hpp).  Fn::operator()<S>() is
+// called with the kernel's sizes for B rows; false if there is none: more rows do not fit the LDS beside two images of their G.
+// (Above 64
+// rows it is the faster one at every size measured; see xfc_dx_dw for the others.)
+template <int MODE, class Fn>
+bool back_step_for(int64_t B, Fn&& fn) {
+  if (B < 1 || B > BACK_MAX_ROWS) return false;
+  constexpr bool ADD = MODE == BACK_ADD;  // its addends take registers that X^T has otherwise
+  if (B <= 64) fn(BackStep<1, 2>{});
+  else if (B <= 128) fn(BackStep<2, ADD ? 2 : 4>{});
+  else if (B <= 192) fn(BackStep<3, ADD ? 2 : 4>{});
+  else fn(BackStep<4, ADD ? 2 : 4>{});
+  return true;
+}
+// Ranges of labels, each with a partial dX of its own: as many as there are CUs for their slices, in eighths for the XCDs;
+// fewer where the labels or the workspace run out (8 at least).
+int back_ranges(int64_t B, int64_t L, int64_t d, size_t ws_limit) {
+  const int64_t slices = ceil_div(d, BACK_DIMS), per = num_cus() / (8 * slices), most = round_up(ceil_div(L, BACK_TILE), 8);
+  int64_t ranges = 8 * (per > 1 ? per : 1);
+  if (ranges > most) ranges = most;
+  while (ranges > 8 && (size_t)ranges * (size_t)B * (size_t)d * 4 > ws_limit) ranges -= 8;
+  return (int)ranges;
+}
+size_t back_ws_bytes(int64_t B, int64_t L, int64_t d) {
+  if (B < 1 || B > BACK_MAX_ROWS || L < 1 || d < 1) return 0;
+  return (size_t)back_ranges(B, L, d, ~(size_t)0) * (size_t)B * (size_t)d * 4;
+}
+template <int MODE>
+int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size_t ws_bytes, hipStream_t st, bool* taken) {
+  *taken = false;
+  a.ranges = back_ranges(a.B, a.L, a.d, ws_bytes);
+  if (!ws || !aligned16(ws) || (size_t)a.ranges * a.B * a.d * 4 > ws_bytes) return XFC_OK;
+  a.slices = ceil_div(a.d, BACK_DIMS);
+  a.tiles = ceil_div(a.L, BACK_TILE);
+  a.part = reinterpret_cast<float*>(ws);
+  // What the pass reads and writes against the Infinity Cache (256 MB, G and the partial sums beside it).  (60,007 labels x 768
+  // dims, 256 rows: 87 us without the hint, 91 with; 700,001 x 768, 128 rows: 953 and 892.)
+  const bool nt = (int64_t)a.L * a.d * (MODE == BACK_UPDATE ? 4 : 6) > (int64_t)224 << 20;
+  int rc = XFC_OK;
+  *taken = back_step_for<MODE>(a.B, [&](auto s) {
+    using S = decltype(s);
+    const dim3 g((unsigned)(a.slices * a.ranges)), b(S::NT);
+    rc = nt ? launch_k<back_step_kernel<S, MODE, true>>(g, b, S::LDS_BYTES, st, a)
+            : launch_k<back_step_kernel<S, MODE, false>>(g, b, S::LDS_BYTES, st, a);
+    if (rc) return;
+    launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges, scale, 0.0f, st);
+    rc = check_launch();
+  });
+  return rc;
+}
+
 int launch_generic(const void* in1, int64_t as0, int64_t as1, const void* in2, int64_t bs0, int64_t bs1, void* out,
                    int64_t os0, int64_t os1, int M, int N, int K, float alpha, float beta, int sigmoid, int out_half,
                    hipStream_t st) {
@@ -1633,6 +1685,18 @@ int xfc_init(void) {
       small_step_for(rows, d, [&](auto s) { keep(raise_lds_limit<small_step_kernel<decltype(s)>>(decltype(s)::LDS_BYTES)); });
   keep(raise_lds_limit<score_small_kernel<1>>(FULL_LDS));
   keep(raise_lds_limit<score_small_kernel<2>>(FULL_LDS));
+  auto back_limits = [&](auto mode) {
+    constexpr int MODE = decltype(mode)::value;
+    for (int64_t rows : {64, 128, 192, 256})
+      back_step_for<MODE>(rows, [&](auto s) {
+        using S = decltype(s);
+        keep(raise_lds_limit<back_step_kernel<S, MODE, true>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, false>>(S::LDS_BYTES));
+      });
+  };
+  back_limits(std::integral_constant<int, BACK_UPDATE>{});
+  back_limits(std::integral_constant<int, BACK_OUT>{});
+  back_limits(std::integral_constant<int, BACK_ADD>{});
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_SMALL>>((int)sizeof(SelLds<SEL_CAP_SMALL>)));
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_LARGE>>((int)sizeof(SelLds<SEL_CAP_LARGE>)));
   keep(raise_lds_limit<dw_kernel<DW_UPDATE>>(DW_LDS_BYTES));
@@ -1889,9 +1953,61 @@ int xfc_sgd_momentum(void* W, void* Mo, const float* grad, int64_t count, float 
   return check_launch();
 }
 
+// Both gradients of a batch; what the one pass does not take runs as two, which also report what is wrong with a call.
+static bool back_ok(const void* G, int64_t ldg, const void* X, int64_t ldx, const void* W, int64_t ldw, const void* dX, int64_t B,
+                    int64_t L, int64_t d) {
+  return dims_ok(B) && dims_ok(L) && dims_ok(d) && B >= 1 && B <= BACK_MAX_ROWS && L >= 1 && d >= 8 && G && X && W && dX &&
+         ldg % 8 == 0 && ldg < (int64_t)1 << 27 && ldx % 8 == 0 && ldw % 8 == 0 && d % 8 == 0 && aligned16(G) && aligned16(X) && aligned16(W) &&
+         ldg >= round_up(L, 8);
+}
+static BackArgs back_args(const void* G, int64_t ldg, const void* X, int64_t ldx, const void* W, int64_t ldw, int64_t B, int64_t L,
+                          int64_t d) {
+  BackArgs a = {};
+  a.G = (const half_t*)G; a.ldg = ldg; a.X = (const half_t*)X; a.ldx = ldx; a.W = (half_t*)const_cast<void*>(W); a.ldw = ldw;
+  a.B = (int)B; a.L = (int)L; a.d = (int)d;
+  return a;
+}
+
+int xfc_dx_dw_update(const void* G, int64_t ldg, const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo, int64_t ldm, float* dX,
+                     int64_t lddx, int64_t B, int64_t L, int64_t d, float lr, float momentum, float weight_decay, float scale,
+                     void* workspace, size_t workspace_bytes, void* stream) {
+  if (back_ok(G, ldg, X, ldx, W, ldw, dX, B, L, d) && Mo && ldm % 8 == 0 && aligned16(Mo)) {
+    BackArgs a = back_args(G, ldg, X, ldx, W, ldw, B, L, d);
+    a.Mo = (half_t*)Mo; a.ldm = ldm; a.lr = lr; a.mu = momentum; a.wd = weight_decay;
+    bool taken;
+    const int rc = launch_back<BACK_UPDATE>(a, dX, lddx, scale, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream), &taken);
+    if (taken) return rc;
+  }
+  const int rc = xfc_dx(G, ldg, W, ldw, dX, lddx, B, L, d, scale, workspace, workspace_bytes, stream);
+  if (rc) return rc;
+  return xfc_dw_update(G, ldg, X, ldx, W, ldw, Mo, ldm, B, L, d, lr, momentum, weight_decay, nullptr, 0, stream);
+}
+
+int xfc_dx_dw(const void* G, int64_t ldg, const void* X, int64_t ldx, const void* W, int64_t ldw, float* grad, int64_t ld_grad,
+              float* dX, int64_t lddx, int64_t B, int64_t L, int64_t d, float beta, float scale, void* workspace,
+              size_t workspace_bytes, void* stream) {
+  // Up to 64 rows the two passes read a gradient that no cache holds a little faster (16 rows x 700,001 x 768: 1,043 against 1,089
+  // us; x 320,001 x 768: 497 against 493; x 60,007: 86 to 91 against 97), unless the width leaves their tiles of 256 dims partly
+  // empty (x 700,001 x 384: 609 against 529).
+  const bool slow = dims_ok(L) && dims_ok(d) && B <= 64 && d % 256 == 0 && L * d * 4 > (int64_t)128 << 20;
+  if (!slow && back_ok(G, ldg, X, ldx, W, ldw, dX, B, L, d) && grad && ld_grad % 4 == 0 && aligned16(grad)) {
+    BackArgs a = back_args(G, ldg, X, ldx, W, ldw, B, L, d);
+    a.out = grad; a.ldo = ld_grad; a.beta = beta;
+    bool taken;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const int rc = beta != 0.f ? launch_back<BACK_ADD>(a, dX, lddx, scale, workspace, workspace_bytes, st, &taken)
+                               : launch_back<BACK_OUT>(a, dX, lddx, scale, workspace, workspace_bytes, st, &taken);
+    if (taken) return rc;
+  }
+  const int rc = xfc_dx(G, ldg, W, ldw, dX, lddx, B, L, d, scale, workspace, workspace_bytes, stream);
+  if (rc) return rc;
+  return xfc_dw(G, ldg, X, ldx, grad, ld_grad, B, L, d, beta, stream);
+}
+
 size_t xfc_step_workspace_bytes(int64_t B, int64_t L, int64_t d, int64_t nnz) {
   const size_t dx = xfc_dx_workspace_bytes(B, L, d), small = dims_ok(B) && dims_ok(L) && dims_ok(d) ? small_step_ws_bytes(B, L, d) : 0;
-  return (size_t)round_up(xfc_fwd_grad_workspace_bytes(L, nnz), 256) + (dx > small ? dx : small);
+  const size_t back = dims_ok(B) && dims_ok(L) && dims_ok(d) ? back_ws_bytes(B, L, d) : 0, most = dx > small ? dx : small;
+  return (size_t)round_up(xfc_fwd_grad_workspace_bytes(L, nnz), 256) + (most > back ? most : back);
 }
 
 // The step in one pass, if the call is one that small_step_kernel takes: its sizes, every operand present and aligned as
@@ -1943,9 +2059,8 @@ static int step_impl(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo,
   if (taken) return rc;
   rc = fwd_grad_impl(X, ldx, W, ldw, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, B, L, d, nullptr, ws, off, st);
   if (rc) return rc;
-  rc = xfc_dx(G, ldg, W, ldw, dX, lddx, B, L, d, scale, ws + off, workspace_bytes - off, stream);
-  if (rc) return rc;
-  return xfc_dw_update(G, ldg, X, ldx, W, ldw, Mo, ldm, B, L, d, lr, momentum, weight_decay, nullptr, 0, stream);
+  return xfc_dx_dw_update(G, ldg, X, ldx, W, ldw, Mo, ldm, dX, lddx, B, L, d, lr, momentum, weight_decay, scale, ws + off,
+                          workspace_bytes - off, stream);
 }
 
 int xfc_step_csr(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo, int64_t ldm, const int32_t* rowptr,
@@ -2011,8 +2126,9 @@ size_t xfc_layer_workspace_bytes(int64_t max_batch, int64_t L, int64_t d, int64_
   size_t dx = 0, topk = 0;
   const int64_t k8 = L < TOPK_MAX ? L : TOPK_MAX;
   for (int64_t b = 1; b <= max_batch; ++b) {
-    const size_t a = xfc_dx_workspace_bytes(b, L, d), small = small_step_ws_bytes(b, L, d);
+    const size_t a = xfc_dx_workspace_bytes(b, L, d), small = small_step_ws_bytes(b, L, d), back = back_ws_bytes(b, L, d);
     if (a > dx) dx = a;
+    if (back > dx) dx = back;
     if (small > dx) dx = small;
     const size_t t = k8 > 0 ? xfc_topk_workspace_bytes(b, L, k8) : 0;
     if (t > topk) topk = t;

@@ -81,10 +81,6 @@ class BCELossMultiNode:
         if whole:                                                     # one call: small batches take a single pass
             lay._step_coo(embed_out, pos_x, pos_y, grad_input, self.scale_bwd, self.lr, out)
             return self.loss
-        bsz = embed_out.shape[0]
-        lay.dx(bsz, grad_input, self.scale_bwd, out=out)              # :602-608
-        if self.accum == 1:
-            lay.dw_update(embed_out, lr=self.lr, out=out)             # :620-634 and the optimizer step of :343
-        else:
-            lay.dw_accumulate(embed_out, out=out)                     # :623 / :629
+        # :602-608, and :620-634 with the optimizer step of :343, or :623 / :629
+        lay.backward_pass(embed_out, grad_input, self.scale_bwd, self.accum != 1, self.lr, out)
         return self.loss

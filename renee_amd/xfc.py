@@ -427,6 +427,38 @@ class XFCLayer:
         check(rc, "xfc_dw")
         self._g_live = self._g_live and out is not None
 
+    def backward_pass(self, embed, grad_input: torch.Tensor | None = None, scale: float = 1.0, accumulate: bool = False,
+                      lr: float | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
+        """dx, then dw_update (accumulate: dw_accumulate), through one entry point: small batches take one
+        pass over the labels for both (dl_base.py:602-634)."""
+        if self.master_weights and not accumulate:
+            gi = self.dx(embed.shape[0], grad_input, scale, out)
+            self.dw_update(embed, lr=lr, out=out)
+            return gi
+        x = self._x16(embed)
+        bsz = x.shape[0]
+        G = self._g_view(bsz, out)
+        gi = self._grad_input(bsz, grad_input)
+        ws = self._ws
+        first, grad = self.xfc_weight_grad is None, self.xfc_weight_grad
+        if accumulate and first:
+            grad = torch.empty(self.numy, self.dims, device=self.device, dtype=torch.float32)
+        with torch.cuda.device(self.device):
+            if accumulate:
+                rc = lib().xfc_dx_dw(G.data_ptr(), G.stride(0), x.data_ptr(), x.stride(0), self.xfc_weight.data_ptr(), self.dims,
+                                     grad.data_ptr(), self.dims, gi.data_ptr(), gi.stride(0), bsz, self.numy, self.dims, 0.0 if first else 1.0,
+                                     float(scale), ws.data_ptr(), ws.numel(), _stream(x))
+            else:
+                rc = lib().xfc_dx_dw_update(G.data_ptr(), G.stride(0), x.data_ptr(), x.stride(0), self.xfc_weight.data_ptr(),
+                                            self.dims, self.momentum_buffer.data_ptr(), self.dims, gi.data_ptr(), gi.stride(0),
+                                            bsz, self.numy, self.dims, self.lr if lr is None else float(lr), self.momentum,
+                                            self.weight_decay, float(scale), ws.data_ptr(), ws.numel(), _stream(x))
+        check(rc, "xfc_dx_dw" if accumulate else "xfc_dx_dw_update")
+        if accumulate:
+            self.xfc_weight_grad = grad
+        self._g_live = self._g_live and out is not None
+        return gi
+
     def optimizer_step(self, lr: float | None = None) -> None:
         """SGD-momentum on the accumulated fp32 grad, then drop it (dl_base.py:343-344)."""
         _require(self.xfc_weight_grad is not None, "no accumulated gradient")
@@ -492,15 +524,9 @@ class XFCLayer:
         grad_input, then dW.  With accumulate=False the optimizer step is fused
         into the dW pass; with accumulate=True dW is added to the fp32 grad and
         optimizer_step() finishes the step."""
-        bsz = embed_out.shape[0]
         if accumulate or self.master_weights:
             self.fwd_grad(embed_out, pos_x, pos_y)
-            gi = self.dx(bsz, grad_input, scale)
-            if accumulate:
-                self.dw_accumulate(embed_out)
-            else:
-                self.dw_update(embed_out, lr=lr)
-            return gi
+            return self.backward_pass(embed_out, grad_input, scale, accumulate, lr)
         return self._step_coo(embed_out, pos_x, pos_y, grad_input, scale, lr)
 
     def _step_coo(self, embed_out, pos_x, pos_y, grad_input=None, scale: float = 1.0, lr: float | None = None,
