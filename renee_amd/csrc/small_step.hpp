@@ -4,7 +4,7 @@
 // What bounds it.  The step's products are small (16 to 64 rows against each weight), its traffic is not: 8 bytes per
 // weight.  As three products the weights came from memory twice more, and each launch filled and drained the chip anew.
 // Whole steps, three passes -> one: 32 rows x 131,072 labels x 768 dims 245 -> 193 us (this kernel 172 to 188: 4.3 to 4.7 TB/s of
-// those 8 bytes); 64 x 4,097 x 768 41 -> 30 us; 32 x 400,001 x 768 753 -> 540 us; 8 x 40,001 x 128 96 -> 23 us; 64 x
+// those 8 bytes); 32 x 400,001 x 768 753 -> 540 us; 8 x 40,001 x 128 96 -> 23 us; 64 x
 // 400,001 x 384 471 -> 307 us.  What is left: the weights' and the momentum's loads come in pieces of 64 bytes, and a
 // small label count is one tile to a workgroup, a chain of loads, z, the two barriers and the update (17 to 27 us).
 //
@@ -91,8 +91,10 @@ __device__ __forceinline__ float sigmoidf_fast(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.44269504088896341f));
 }
 
-template <class S>
+// STEP false: G alone, the first half of the step (W is only read; Mo and part are not used).
+template <class S, bool STEP = true>
 __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(SmallArgs a) {
+  constexpr bool AHEAD = S::AHEAD || !STEP;  // without the momentum and the sums the next tile's weights always fit
   constexpr int NW = S::NW, SB = S::SB, RB = S::RB, P = S::P, D = S::D;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -107,7 +109,8 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
   uint32_t* const mask = reinterpret_cast<uint32_t*>(regions + NW * S::REGION + S::G_BYTES);  // [2][P][32], by tile parity
 
   // the first tile's weights; then everything that is set up once while they are on their way
-  half8 wcur[2][SB], wnext[2][SB], m[2][SB], mnext[2][SB];
+  half8 wcur[2][SB], wnext[2][SB];
+  [[maybe_unused]] half8 m[2][SB], mnext[2][SB];
   auto load = [&](const half_t* base, int64_t ld, int tile, half8 (&v)[2][SB]) {
 #pragma unroll
     for (int lb = 0; lb < 2; ++lb) {
@@ -128,7 +131,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
         xv[p][s][b] = *reinterpret_cast<const half8*>(a.X + (int64_t)(row < a.B ? row : a.B - 1) * a.ldx + dim0 + 32 * s + 8 * g);
       }
   load(a.W, a.ldw, blockIdx.x, wcur);
-  if constexpr (S::AHEAD) load(a.Mo, a.ldm, blockIdx.x, m);
+  if constexpr (AHEAD && STEP) load(a.Mo, a.ldm, blockIdx.x, m);
 
   // label pairs, a few per thread, kept for all tiles (label -1: none, or out of range)
   int plab[S::PAIRS], prow[S::PAIRS];
@@ -160,7 +163,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
   // Rows past the batch: zeros for dW, so that they add nothing; the last row again for z.  Zeros there too would make z of
   // a label with an infinite weight no number, hence G, and dW in all dims of that label (0 . NaN); this way G holds
   // nothing there that it does not hold for a row of the batch.
-  half8 xt[P][SB][2];  // A side of dW: dim 8 (i / 4) + 4 b + i % 4, rows 8 g ..+7
+  [[maybe_unused]] half8 xt[P][SB][2];  // A side of dW: dim 8 (i / 4) + 4 b + i % 4, rows 8 g ..+7
 #pragma unroll
   for (int p = 0; p < P; ++p)
 #pragma unroll
@@ -170,20 +173,26 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
         const int rel = 8 * (i >> 2) + 4 * b + (i & 3), row = 32 * p + rel;
         half8 v = xv[p][s][b];
         *reinterpret_cast<half8*>(xf + ((p * 2 + b) * SB + s) * 512) = v;
+        if constexpr (STEP) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = row < a.B ? v[e] : (half_t)0.f;
-        *reinterpret_cast<half8*>(stage + rel * 32 + 8 * g) = v;
+          for (int e = 0; e < 8; ++e) v[e] = row < a.B ? v[e] : (half_t)0.f;
+          *reinterpret_cast<half8*>(stage + rel * 32 + 8 * g) = v;
+        }
       }
-      S::lds_done();
+      if constexpr (STEP) {
+        S::lds_done();
 #pragma unroll
-      for (int b = 0; b < 2; ++b) xt[p][s][b] = S::read_tr(stage, t4, 8 * (lane & 3) + 4 * b);
-      S::lds_done();
+        for (int b = 0; b < 2; ++b) xt[p][s][b] = S::read_tr(stage, t4, 8 * (lane & 3) + 4 * b);
+        S::lds_done();
+      }
     }
-  float4v acc[RB][SB][2];
+  [[maybe_unused]] float4v acc[RB][SB][2];
+  if constexpr (STEP) {
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-    for (int s = 0; s < SB; ++s) acc[rb][s][0] = acc[rb][s][1] = float4v{0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < SB; ++s) acc[rb][s][0] = acc[rb][s][1] = float4v{0.f, 0.f, 0.f, 0.f};
+  }
   S::barrier();  // the masks are clear
 
   int parity = 0;
@@ -198,10 +207,10 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
           for (int e = 0; e < 8; ++e) wcur[lb][s][e] = l0 + 16 * lb + i < a.L ? wcur[lb][s][e] : (half_t)0.f;
     }
     const int next = tile + (int)gridDim.x;
-    if constexpr (S::AHEAD) {
+    if constexpr (AHEAD) {
       if (next < a.tiles) {
         load(a.W, a.ldw, next, wnext);
-        load(a.Mo, a.ldm, next, mnext);
+        if constexpr (STEP) load(a.Mo, a.ldm, next, mnext);
       }
     }
     uint32_t* const mk = mask + parity * S::MASK_WORDS;
@@ -223,7 +232,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
           const half8 x = *reinterpret_cast<const half8*>(xf + (r * SB + s) * 512);
 #pragma unroll
           for (int lb = 0; lb < 2; ++lb) z[r][lb] = S::mfma(x, wcur[lb][s], z[r][lb]);
-          if constexpr (!S::AHEAD) { if (r & 1) __builtin_amdgcn_sched_barrier(0); }  // reads moved up cost spills
+          if constexpr (!AHEAD) { if (r & 1) __builtin_amdgcn_sched_barrier(0); }  // reads moved up cost spills
         }
       float4v own = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -231,7 +240,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
         if (S::SKIP && u == wave) own = z[u >> 1][u & 1];
         else *reinterpret_cast<float4v*>(zpart + (S::SKIP && u > wave ? u - 1 : u) * 256) = z[u >> 1][u & 1];
       }
-      if constexpr (!S::AHEAD) load(a.Mo, a.ldm, tile, m);
+      if constexpr (!AHEAD && STEP) load(a.Mo, a.ldm, tile, m);
       S::barrier();
 #pragma unroll
       for (int uu = 0; uu < (S::UNITS + NW - 1) / NW; ++uu) {
@@ -261,12 +270,24 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
     for (int w = tid; w < S::MASK_WORDS; w += S::NT) mask[(parity ^ 1) * S::MASK_WORDS + w] = 0u;
     S::barrier();
 
+    if constexpr (!STEP) {  // (every wave has its part of z read before the barrier above)
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+        if (wave == rb && 16 * rb + i < a.B && l0 + 8 * g < a.n_store)
+          *reinterpret_cast<half8*>(a.G + (int64_t)(16 * rb + i) * a.ldg + l0 + 8 * g) =
+              *reinterpret_cast<const half8*>(gs + (16 * rb + i) * 32 + 8 * g);
+#pragma unroll
+      for (int lb = 0; lb < 2; ++lb)
+#pragma unroll
+        for (int s = 0; s < SB; ++s) wcur[lb][s] = wnext[lb][s];
+      continue;
+    }
     // dX^T += W^T . G^T; the waves' regions are their own again
 #pragma unroll
     for (int s = 0; s < SB; ++s)
 #pragma unroll
       for (int lb = 0; lb < 2; ++lb) *reinterpret_cast<half8*>(stage + s * 1024 + (16 * lb + i) * 32 + 8 * g) = wcur[lb][s];
-    if constexpr (!S::AHEAD) {
+    if constexpr (!AHEAD) {
       if (next < a.tiles) load(a.W, a.ldw, next, wcur);
     }
     {
@@ -285,7 +306,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
           const half8 wt = S::read_tr(stage + s * 1024, t4, 16 * c + 4 * (lane & 3));
 #pragma unroll
           for (int rb = 0; rb < RB; ++rb) acc[rb][s][c] = S::mfma(wt, bg[rb], acc[rb][s][c]);
-          if constexpr (!S::AHEAD) { if (c) __builtin_amdgcn_sched_barrier(0); }
+          if constexpr (!AHEAD) { if (c) __builtin_amdgcn_sched_barrier(0); }
         }
     }
 
@@ -306,7 +327,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
           for (int p = 0; p < P; ++p) dw[b] = S::mfma(xt[p][s][b], gt[p], dw[b]);
         }
         half8 wv = wcur[lb][s], mv = m[lb][s];
-        if constexpr (!S::AHEAD) wv = *reinterpret_cast<const half8*>(stage + s * 1024 + (16 * lb + i) * 32 + 8 * g);
+        if constexpr (!AHEAD) wv = *reinterpret_cast<const half8*>(stage + s * 1024 + (16 * lb + i) * 32 + 8 * g);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float wf = (float)wv[e];
@@ -319,10 +340,10 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
           *reinterpret_cast<half8*>(a.Mo + (int64_t)label * a.ldm + dim0 + 32 * s + 8 * g) = mv;
           *reinterpret_cast<half8*>(a.W + (int64_t)label * a.ldw + dim0 + 32 * s + 8 * g) = wv;
         }
-        if constexpr (!S::AHEAD) __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!AHEAD) __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if constexpr (S::AHEAD) {
+    if constexpr (AHEAD) {
 #pragma unroll
       for (int lb = 0; lb < 2; ++lb)
 #pragma unroll
@@ -331,6 +352,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
     S::lds_done();  // the reads of the region are over before the next tile's parts of z go there
   }
 
+  if constexpr (!STEP) return;
   float* const part = a.part + (int64_t)blockIdx.x * a.B * D;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {

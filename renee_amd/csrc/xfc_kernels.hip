@@ -1682,7 +1682,10 @@ int xfc_init(void) {
   small_limits(std::type_identity<FwdCore64>{}, std::type_identity<DxCore64>{});
   for (int64_t rows : {32, 64})
     for (int64_t d : {128, 256, 384, 512, 768, 1024})
-      small_step_for(rows, d, [&](auto s) { keep(raise_lds_limit<small_step_kernel<decltype(s)>>(decltype(s)::LDS_BYTES)); });
+      small_step_for(rows, d, [&](auto s) {
+        keep(raise_lds_limit<small_step_kernel<decltype(s)>>(decltype(s)::LDS_BYTES));
+        keep(raise_lds_limit<small_step_kernel<decltype(s), false>>(decltype(s)::LDS_BYTES));
+      });
   keep(raise_lds_limit<score_small_kernel<1>>(FULL_LDS));
   keep(raise_lds_limit<score_small_kernel<2>>(FULL_LDS));
   auto back_limits = [&](auto mode) {
@@ -1785,6 +1788,35 @@ size_t xfc_fwd_grad_workspace_bytes(int64_t L, int64_t nnz) {
   return fwd_ws_bytes(nnz);
 }
 
+// What small_step_kernel reads for G.
+static SmallArgs small_args(const void* X, int64_t ldx, const void* W, int64_t ldw, const int32_t* rowptr, const int32_t* colidx,
+                            const int64_t* pos_x, const int64_t* pos_y, int64_t nnz, void* G, int64_t ldg, int64_t B, int64_t L) {
+  SmallArgs a = {};
+  a.X = (const half_t*)X; a.ldx = ldx; a.W = (half_t*)const_cast<void*>(W); a.ldw = ldw;
+  a.G = (half_t*)G; a.ldg = ldg;
+  a.rowptr = rowptr; a.colidx = colidx; a.pos_x = pos_x; a.pos_y = pos_y;
+  a.nnz = (int)nnz; a.B = (int)B; a.L = (int)L; a.n_store = (int)round_up(L, 8); a.tiles = small_step_tiles(L);
+  return a;
+}
+
+// G of a small batch and its positives in one launch, if there is such a kernel for the call (whose arguments have been
+// checked): no loss, no more pairs than the workgroups' threads hold.  XFC_OK with *taken false otherwise.  It stands as long as
+// it is the faster one: 32 rows x 131,072 x 768 41 -> 33 us and x 4,097 launch-bound, 16 -> 13, but x 320,001 97 -> 101; with 64 rows
+// its two barriers a tile weigh more, x 20,011 16 -> 13 but x 60,007 21 -> 25.
+static int small_grad(const void* X, int64_t ldx, const void* W, int64_t ldw, const int32_t* rowptr, const int32_t* colidx,
+                      const int64_t* pos_x, const int64_t* pos_y, int64_t nnz, void* G, int64_t ldg, int64_t B, int64_t L, int64_t d,
+                      const float* loss, hipStream_t st, bool* taken) {
+  *taken = false;
+  if (loss || B > SMALL_MAX_ROWS || nnz > SMALL_MAX_PAIRS || L * d > (B <= 32 ? (int64_t)160 << 20 : (int64_t)16 << 20)) return XFC_OK;
+  const SmallArgs a = small_args(X, ldx, W, ldw, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, B, L);
+  int rc = XFC_OK;
+  *taken = small_step_for(B, d, [&](auto s) {
+    using S = decltype(s);
+    rc = launch_k<small_step_kernel<S, false>>(dim3((unsigned)small_step_grid<S>(L)), dim3(S::NT), S::LDS_BYTES, st, a);
+  });
+  return rc;
+}
+
 static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw, const int32_t* rowptr,
                          const int32_t* colidx, const int64_t* pos_x, const int64_t* pos_y, int64_t nnz, void* G,
                          int64_t ldg, int64_t B, int64_t L, int64_t d, float* loss, void* ws, size_t ws_bytes,
@@ -1797,6 +1829,8 @@ static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw,
     return XFC_ERR_ALIGN;
   if (ldg < L) return XFC_ERR_SHAPE;
   if (!ws || ws_bytes < fwd_ws_bytes(nnz)) return XFC_ERR_WORKSPACE;
+  bool taken;
+  if (int rc0 = small_grad(X, ldx, W, ldw, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, B, L, d, loss, st, &taken); taken) return rc0;
   double* loss_part = loss ? reinterpret_cast<double*>((reinterpret_cast<uintptr_t>(ws) + 7) & ~(uintptr_t)7) : nullptr;
   float* loss_pos = loss ? reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(ws) + LOSS_PART_BYTES) : nullptr;
   // label columns L .. round_up(L, 8) are written as zero so that G can be read in 16-byte
@@ -2020,17 +2054,17 @@ static int small_step(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo
   *taken = false;
   if (B < 1 || B > SMALL_MAX_ROWS || !dims_ok(L) || L < 1 || !dims_ok(d) || nnz < 0 || nnz > SMALL_MAX_PAIRS) return XFC_OK;
   if (!X || !W || !Mo || !G || !dX || (nnz > 0 && !((rowptr && colidx) || (pos_x && pos_y)))) return XFC_OK;
+  // With 33 to 64 rows of 768 dims the one pass fetches nothing ahead (see SmallStep::AHEAD), and each workgroup leaves 192 KB of
+  // partial sums for a few tiles: G by itself and both gradients after it are faster while W and Mo stay in the caches, 64 rows x
+  // 4,097 labels 32.6 -> 26.7 us, x 20,011 52.6 -> 44.4, but x 40,009 70 -> 74 and 33 rows x 40,009 61 -> 69.
+  if (B > 32 && d >= 768 && L * d <= (int64_t)16 << 20) return XFC_OK;
   if (ldx % 8 || ldw % 8 || ldm % 8 || ldg % 8 || ldg < round_up(L, 8) || !aligned16(X) || !aligned16(W) || !aligned16(Mo) ||
       !aligned16(G) || !aligned16(ws))
     return XFC_OK;
   const size_t need = small_step_ws_bytes(B, L, d);
   if (need == 0 || ws_bytes < need) return XFC_OK;
-  SmallArgs a;
-  a.X = (const half_t*)X; a.ldx = ldx; a.W = (half_t*)W; a.ldw = ldw; a.Mo = (half_t*)Mo; a.ldm = ldm;
-  a.G = (half_t*)G; a.ldg = ldg;
-  a.rowptr = rowptr; a.colidx = colidx; a.pos_x = pos_x; a.pos_y = pos_y;
-  a.nnz = (int)nnz; a.B = (int)B; a.L = (int)L; a.n_store = (int)round_up(L, 8); a.tiles = small_step_tiles(L);
-  a.lr = lr; a.mu = momentum; a.wd = weight_decay; a.part = reinterpret_cast<float*>(ws);
+  SmallArgs a = small_args(X, ldx, W, ldw, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, B, L);
+  a.Mo = (half_t*)Mo; a.ldm = ldm; a.lr = lr; a.mu = momentum; a.wd = weight_decay; a.part = reinterpret_cast<float*>(ws);
   int rc = XFC_OK;
   small_step_for(B, d, [&](auto s) {
     using S = decltype(s);
