@@ -22,6 +22,8 @@ class _XFCStep(torch.autograd.Function):
     @staticmethod
     def forward(ctx, embed, layer, pos_x, pos_y, scale, lr, compute_loss, accumulate):
         loss = torch.zeros(1, device=layer.device, dtype=torch.float32)
+        ctx.embed_dtype, ctx.embed_device = embed.dtype, embed.device
+        embed = layer._x16(embed)  # cast once for both passes
         if compute_loss:
             layer.fwd_grad(embed, pos_x, pos_y, loss_out=loss)
             gi = layer.backward_pass(embed, None, scale, accumulate, lr)
@@ -29,7 +31,6 @@ class _XFCStep(torch.autograd.Function):
             gi = layer.xfc_backward(embed, pos_x, pos_y, None, scale, accumulate, lr)
         # the layer's grad_input buffer is reused by the next step: keep this step's values
         ctx.save_for_backward(gi.clone())
-        ctx.embed_dtype, ctx.embed_device = embed.dtype, embed.device
         return loss.reshape(())
 
     @staticmethod

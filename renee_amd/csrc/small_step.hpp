@@ -42,8 +42,13 @@ struct SmallArgs {
   float* part;                                   // [gridDim.x][B][D] partial sums of G.W
 };
 
-// NW waves, SB blocks of 32 dims per wave, RB blocks of 16 rows (2 or 4)
-template <int NW_, int SB_, int RB_>
+// NW waves, SB blocks of 32 dims per wave, RB blocks of 16 rows (2 or 4); LINES: an instruction that loads or stores weights
+// or momentum covers 8 labels x 128 bytes (see back_step.hpp) instead of 16 x 64, and the loads say that nothing will want
+// them again.  That is for sizes that no cache holds until the next step: 32 rows x 131,072 x 768 188 -> 169 us, x 700,001 961 ->
+// 888, 64 x 700,001 x 512 696 -> 621 (whole lines without the hint 720, half lines with it 1,048 at 32 x 700,001 x 768).  Below,
+// half lines without the hint are faster, as the caches serve them: 64 x 20,011 x 512 33.0 against 34.5, 32 x 4,097 x 1024 24.8
+// against 28.1.
+template <int NW_, int SB_, int RB_, bool LINES_ = false>
 struct SmallStep {
   static constexpr int NW = NW_, SB = SB_, RB = RB_, P = RB / 2, NT = 64 * NW, D = NW * SB * 32;
   static constexpr int UNITS = 2 * RB;           // 16 x 16 blocks of z, each summed by one wave
@@ -62,6 +67,8 @@ struct SmallStep {
   // after that and the next tile's are fetched in their place.  Spills that are left: 22 registers at 64 rows x 768, 5 at
   // 32 x 128, 1 at 32 x 384.
   static constexpr bool AHEAD = RB == 2 && SB <= 3;
+  static constexpr bool LINES = LINES_;
+  static_assert(!LINES || SB % 2 == 0, "a line is two blocks of dims");
   static constexpr int BY_REGS = 4 * WAVES_PER_EU / NW, BY_LDS = 160 * 1024 / LDS_BYTES;
   static constexpr int PER_CU = BY_REGS < BY_LDS ? BY_REGS : BY_LDS;
   static_assert(LDS_BYTES <= 160 * 1024 && PER_CU >= 1, "LDS and register budget");
@@ -81,6 +88,22 @@ struct SmallStep {
   }
   __device__ __forceinline__ static float4v mfma(const half8& a, const half8& b, const float4v& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+  }
+  // v (16 bytes) of the lane eight away in its row of sixteen; and one of two
+  template <class V>
+  __device__ __forceinline__ static V across8(const V& v) {
+    uint4v q = __builtin_bit_cast(uint4v, v);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q[e] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)q[e], 0x128, 0xf, 0xf, true);  // row_ror:8
+    return __builtin_bit_cast(V, q);
+  }
+  template <class V>
+  __device__ __forceinline__ static V pick(bool first, const V& x, const V& y) {
+    uint4v p = __builtin_bit_cast(uint4v, x);
+    const uint4v q = __builtin_bit_cast(uint4v, y);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[e] = first ? p[e] : q[e];
+    return __builtin_bit_cast(V, p);
   }
 };
 
@@ -108,16 +131,25 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
   half_t* const gs = reinterpret_cast<half_t*>(regions + NW * S::REGION);
   uint32_t* const mask = reinterpret_cast<uint32_t*>(regions + NW * S::REGION + S::G_BYTES);  // [2][P][32], by tile parity
 
+  // Which label of a tile (of block lb) and which of the wave's dims a lane's s-th piece of weights and momentum holds.
+  constexpr bool LINES = S::LINES;
+  [[maybe_unused]] const int low = i & 7, second = i >> 3;
+  auto label_of = [&](int lb, int s) { return LINES ? 16 * lb + 8 * (s & 1) + low : 16 * lb + i; };
+  auto col_of = [&](int s) { return (LINES ? 32 * ((s & ~1) + second) : 32 * s) + 8 * g; };
+  auto at_stage = [&](int lb, int s) { return (LINES ? (s & ~1) + second : s) * 1024 + label_of(lb, s) * 32 + 8 * g; };
   // the first tile's weights; then everything that is set up once while they are on their way
   half8 wcur[2][SB], wnext[2][SB];
   [[maybe_unused]] half8 m[2][SB], mnext[2][SB];
   auto load = [&](const half_t* base, int64_t ld, int tile, half8 (&v)[2][SB]) {
 #pragma unroll
     for (int lb = 0; lb < 2; ++lb) {
-      const int label = tile * 32 + 16 * lb + i;
-      const half_t* p = base + (int64_t)(label < a.L ? label : a.L - 1) * ld + dim0 + 8 * g;
 #pragma unroll
-      for (int s = 0; s < SB; ++s) v[lb][s] = *reinterpret_cast<const half8*>(p + 32 * s);
+      for (int s = 0; s < SB; ++s) {
+        const int label = tile * 32 + label_of(lb, s);
+        const half8* p = reinterpret_cast<const half8*>(base + (int64_t)(label < a.L ? label : a.L - 1) * ld + dim0 + col_of(s));
+        if constexpr (LINES) v[lb][s] = __builtin_nontemporal_load(p);
+        else v[lb][s] = *p;
+      }
     }
   };
   half8 xv[P][SB][2];
@@ -204,7 +236,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
 #pragma unroll
         for (int s = 0; s < SB; ++s)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) wcur[lb][s][e] = l0 + 16 * lb + i < a.L ? wcur[lb][s][e] : (half_t)0.f;
+          for (int e = 0; e < 8; ++e) wcur[lb][s][e] = l0 + label_of(lb, s) < a.L ? wcur[lb][s][e] : (half_t)0.f;
     }
     const int next = tile + (int)gridDim.x;
     if constexpr (AHEAD) {
@@ -226,14 +258,21 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
 #pragma unroll
       for (int r = 0; r < RB; ++r) z[r][0] = z[r][1] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < SB; ++s)
+      for (int s = 0; s < SB; ++s) {
+        half8 w[2];  // the B side: label 16 lb + i, dims 32 s + 8 g ..+7
+#pragma unroll
+        for (int lb = 0; lb < 2; ++lb) {
+          w[lb] = wcur[lb][s];
+          if constexpr (LINES) w[lb] = S::pick(second == (s & 1), w[lb], S::across8(wcur[lb][s ^ 1]));
+        }
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
           const half8 x = *reinterpret_cast<const half8*>(xf + (r * SB + s) * 512);
 #pragma unroll
-          for (int lb = 0; lb < 2; ++lb) z[r][lb] = S::mfma(x, wcur[lb][s], z[r][lb]);
+          for (int lb = 0; lb < 2; ++lb) z[r][lb] = S::mfma(x, w[lb], z[r][lb]);
           if constexpr (!AHEAD) { if (r & 1) __builtin_amdgcn_sched_barrier(0); }  // reads moved up cost spills
         }
+      }
       float4v own = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < S::UNITS; ++u) {  // u = (p, b, lb)
@@ -286,7 +325,7 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
 #pragma unroll
     for (int s = 0; s < SB; ++s)
 #pragma unroll
-      for (int lb = 0; lb < 2; ++lb) *reinterpret_cast<half8*>(stage + s * 1024 + (16 * lb + i) * 32 + 8 * g) = wcur[lb][s];
+      for (int lb = 0; lb < 2; ++lb) *reinterpret_cast<half8*>(stage + at_stage(lb, s)) = wcur[lb][s];
     if constexpr (!AHEAD) {
       if (next < a.tiles) load(a.W, a.ldw, next, wcur);
     }
@@ -316,18 +355,17 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
       half8 gt[P];
 #pragma unroll
       for (int p = 0; p < P; ++p) gt[p] = S::read_tr(gs + p * 1024, t4, 16 * lb + 4 * (lane & 3));
-      const int label = l0 + 16 * lb + i;
-#pragma unroll
-      for (int s = 0; s < SB; ++s) {
-        float4v dw[2];
+      auto product = [&](int s, float4v (&dw)[2]) {  // label 16 lb + i, dims 32 s + 8 g ..+7
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
           dw[b] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int p = 0; p < P; ++p) dw[b] = S::mfma(xt[p][s][b], gt[p], dw[b]);
         }
+      };
+      auto update = [&](int s, const float4v (&dw)[2]) {  // a lane's s-th piece
         half8 wv = wcur[lb][s], mv = m[lb][s];
-        if constexpr (!AHEAD) wv = *reinterpret_cast<const half8*>(stage + s * 1024 + (16 * lb + i) * 32 + 8 * g);
+        if constexpr (!AHEAD) wv = *reinterpret_cast<const half8*>(stage + at_stage(lb, s));
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float wf = (float)wv[e];
@@ -336,11 +374,33 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
           mv[e] = (half_t)mf;
           wv[e] = (half_t)(wf - a.lr * mf);
         }
+        const int label = l0 + label_of(lb, s);
         if (label < a.L) {
-          *reinterpret_cast<half8*>(a.Mo + (int64_t)label * a.ldm + dim0 + 32 * s + 8 * g) = mv;
-          *reinterpret_cast<half8*>(a.W + (int64_t)label * a.ldw + dim0 + 32 * s + 8 * g) = wv;
+          *reinterpret_cast<half8*>(a.Mo + (int64_t)label * a.ldm + dim0 + col_of(s)) = mv;
+          *reinterpret_cast<half8*>(a.W + (int64_t)label * a.ldw + dim0 + col_of(s)) = wv;
         }
         if constexpr (!AHEAD) __builtin_amdgcn_sched_barrier(0);
+      };
+      if constexpr (LINES) {
+#pragma unroll
+        for (int s = 0; s < SB; s += 2) {
+          float4v dw[2][2], mine[2];
+          product(s, dw[0]);
+          product(s + 1, dw[1]);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) mine[b] = S::pick(second == h, dw[h][b], S::across8(dw[1 - h][b]));
+            update(s + h, mine);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < SB; ++s) {
+          float4v dw[2];
+          product(s, dw);
+          update(s, dw);
+        }
       }
     }
     if constexpr (AHEAD) {

@@ -1500,14 +1500,21 @@ int launch_dw(int mode, DwArgs a, hipStream_t st) {
 // exceed the LDS.  Wherever there is one it is the faster: 1.24 to 4.1 times over 8 to 64 rows and 4,097 to
 // 400,001 labels, least at 64 x 400,001 x 768 (768 -> 618 us).  384 dims and 64 rows take 12 waves of one block of dims:
 // with 4 waves of three, 41 spills, 456 us at 64 x 400,001 instead of 307.
+// large: W and M are more than the caches hold beside the rest (small_step_large); whole lines pay there for these (8, 32 and
+// 64 rows x 90,001 to 2,000,003 labels: 1.02 to 1.10 times as fast with 768 dims, 0.98 to 1.08 with 1024, 1.02 to 1.15 with 512
+// and 64 rows), not for 256 and 384 dims (0.84 to 1.12, most below 1) nor for 32 rows of 512 (0.87 to 1.11).
+inline bool small_step_large(int64_t L, int64_t d) { return L * d * 4 > (int64_t)224 << 20; }
 template <class Fn>
-bool small_step_for(int64_t B, int64_t d, Fn&& fn) {
+bool small_step_for(int64_t B, int64_t d, bool large, Fn&& fn) {
   if (B < 1 || B > SMALL_MAX_ROWS) return false;
   auto rows = [&](auto narrow, auto wide) {
     if (B <= 32) fn(narrow);
     else fn(wide);
     return true;
   };
+  if (large && B > 32 && d == 512) { fn(SmallStep<8, 2, 4, true>{}); return true; }
+  if (large && B <= 32 && d == 768) { fn(SmallStep<6, 4, 2, true>{}); return true; }
+  if (large && B <= 32 && d == 1024) { fn(SmallStep<8, 4, 2, true>{}); return true; }
   switch (d) {
     case 128: return rows(SmallStep<4, 1, 2>{}, SmallStep<4, 1, 4>{});
     case 256: return rows(SmallStep<8, 1, 2>{}, SmallStep<8, 1, 4>{});
@@ -1517,6 +1524,13 @@ bool small_step_for(int64_t B, int64_t d, Fn&& fn) {
     case 1024: if (B <= 32) { fn(SmallStep<8, 4, 2>{}); return true; } return false;
     default: return false;
   }
+}
+// The same for G alone: the weights are wanted again.
+template <class Fn>
+bool small_grad_for(int64_t B, int64_t d, Fn&& fn) {
+  return small_step_for(B, d, false, [&](auto s) {
+    if constexpr (!decltype(s)::LINES) fn(s);
+  });
 }
 inline int small_step_tiles(int64_t L) { return ceil_div(round_up(L, 8), 32); }
 // Workgroups, each with a partial dX of its own: as many as run at once.
@@ -1528,7 +1542,7 @@ int small_step_grid(int64_t L) {
 // Bytes of the partial sums, 0 if there is no such kernel.
 size_t small_step_ws_bytes(int64_t B, int64_t L, int64_t d) {
   size_t need = 0;
-  if (L > 0) small_step_for(B, d, [&](auto s) { need = (size_t)small_step_grid<decltype(s)>(L) * B * d * 4; });
+  if (L > 0) small_step_for(B, d, small_step_large(L, d), [&](auto s) { need = (size_t)small_step_grid<decltype(s)>(L) * B * d * 4; });
   return need;
 }
 
@@ -1682,10 +1696,10 @@ int xfc_init(void) {
   small_limits(std::type_identity<FwdCore64>{}, std::type_identity<DxCore64>{});
   for (int64_t rows : {32, 64})
     for (int64_t d : {128, 256, 384, 512, 768, 1024})
-      small_step_for(rows, d, [&](auto s) {
-        keep(raise_lds_limit<small_step_kernel<decltype(s)>>(decltype(s)::LDS_BYTES));
-        keep(raise_lds_limit<small_step_kernel<decltype(s), false>>(decltype(s)::LDS_BYTES));
-      });
+      for (bool large : {false, true}) {
+        small_step_for(rows, d, large, [&](auto s) { keep(raise_lds_limit<small_step_kernel<decltype(s)>>(decltype(s)::LDS_BYTES)); });
+        small_grad_for(rows, d, [&](auto s) { keep(raise_lds_limit<small_step_kernel<decltype(s), false>>(decltype(s)::LDS_BYTES)); });
+      }
   keep(raise_lds_limit<score_small_kernel<1>>(FULL_LDS));
   keep(raise_lds_limit<score_small_kernel<2>>(FULL_LDS));
   auto back_limits = [&](auto mode) {
@@ -1810,7 +1824,7 @@ static int small_grad(const void* X, int64_t ldx, const void* W, int64_t ldw, co
   if (loss || B > SMALL_MAX_ROWS || nnz > SMALL_MAX_PAIRS || L * d > (B <= 32 ? (int64_t)160 << 20 : (int64_t)16 << 20)) return XFC_OK;
   const SmallArgs a = small_args(X, ldx, W, ldw, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, B, L);
   int rc = XFC_OK;
-  *taken = small_step_for(B, d, [&](auto s) {
+  *taken = small_grad_for(B, d, [&](auto s) {
     using S = decltype(s);
     rc = launch_k<small_step_kernel<S, false>>(dim3((unsigned)small_step_grid<S>(L)), dim3(S::NT), S::LDS_BYTES, st, a);
   });
@@ -2066,7 +2080,7 @@ static int small_step(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo
   SmallArgs a = small_args(X, ldx, W, ldw, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, B, L);
   a.Mo = (half_t*)Mo; a.ldm = ldm; a.lr = lr; a.mu = momentum; a.wd = weight_decay; a.part = reinterpret_cast<float*>(ws);
   int rc = XFC_OK;
-  small_step_for(B, d, [&](auto s) {
+  small_step_for(B, d, small_step_large(L, d), [&](auto s) {
     using S = decltype(s);
     const int grid = small_step_grid<S>(L);
     rc = launch_k<small_step_kernel<S>>(dim3((unsigned)grid), dim3(S::NT), S::LDS_BYTES, st, a);

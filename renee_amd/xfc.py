@@ -525,6 +525,7 @@ class XFCLayer:
         into the dW pass; with accumulate=True dW is added to the fp32 grad and
         optimizer_step() finishes the step."""
         if accumulate or self.master_weights:
+            embed_out = self._x16(embed_out)  # cast once for both passes
             self.fwd_grad(embed_out, pos_x, pos_y)
             return self.backward_pass(embed_out, grad_input, scale, accumulate, lr)
         return self._step_coo(embed_out, pos_x, pos_y, grad_input, scale, lr)
