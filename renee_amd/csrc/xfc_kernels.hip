@@ -2131,6 +2131,10 @@ int xfc_step_coo(const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo, int
 
 // The K <= 8 pass.  Up to 32 rows whose fragments fit the LDS the weights stream past them (score_small_kernel), above that
 // the forward pass's main loop runs (both sides of the line: score_wide_kernel); each leaves the largest score of every block.
+// From some 400 MB of weights on, more than the caches hold, the main loop's whole lines are faster from the third row on: 32
+// rows x 1,500,001 x 768 468 against 430 us, 16 x 2,300,001 x 512 467 against 443, 8 x 2,500,003 x 256 286 against 261; 1 row x
+// 1,500,001 x 768 402 against 407.
+constexpr int64_t SCORE_SMALL_BYTES = (int64_t)400 << 20;
 struct TopkPlan {
   bool small;
   int block;          // labels per block
@@ -2140,7 +2144,7 @@ static int64_t topk_blocks(int64_t labels, int block) { return round_up(ceil_div
 // With a workspace that does not hold all maxima the labels go in ranges, the K best of each carried to the next.
 static TopkPlan topk_plan(int64_t B, int64_t L, int64_t d, int64_t K, size_t ws_limit) {
   TopkPlan p;
-  p.small = B <= SCORE_SMALL_ROWS && (B <= 16 ? score_small_lds<1>(d) : score_small_lds<2>(d)) <= FULL_LDS;
+  p.small = B <= SCORE_SMALL_ROWS && (B <= 2 || L * d * 2 <= SCORE_SMALL_BYTES) && (B <= 16 ? score_small_lds<1>(d) : score_small_lds<2>(d)) <= FULL_LDS;
   p.block = p.small ? SCORE_SMALL_BLOCK : SCORE_WIDE_BLOCK;
   p.range = L;
   // a tile of the wide kernel writes the maxima of all its blocks

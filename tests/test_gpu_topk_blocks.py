@@ -41,7 +41,7 @@ def _problem(dev, B, L, d, seed):
                                      (20, 3001, 3000, 5), (16, 3001, 3000, 5), (64, 9000, 32, 1), (65, 257, 40, 8), (128, 70001, 136, 5),
                                      (129, 513, 72, 5), (700, 12345, 64, 5),
                                      # runs of two and four units; more than 131,072 blocks
-                                     (16, 131077, 64, 5), (20, 270011, 64, 5), (40, 700001, 8, 5), (3, 2200003, 8, 8)])
+                                     (16, 131077, 64, 5), (20, 270011, 64, 5), (40, 700001, 8, 5), (3, 2200003, 8, 8), (2, 290001, 768, 5), (9, 290001, 768, 5)])
 def test_blocks_against_a_stable_sort(dev, B, L, d, K):
     X, W = _problem(dev, B, L, d, B + L + d)
     v, i = _run(X, W, K)
