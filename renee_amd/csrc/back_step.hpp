@@ -2,10 +2,10 @@
 // before the update, and dW = G^T.X, which is written out or consumed by the momentum update of those weights.
 //
 // What bounds it.  With so few rows the products are small beside the traffic; as two kernels the weights and G were read
-// twice.  dX and the update of 199 rows x 131,073 labels x 768 dims, reduction included: 233 -> 202 us (256 rows 212, 128 rows
-// 188: 4.9 TB/s of the 8 bytes per weight and G); without its stores the pass takes 150 at 199 and 256 rows, the LDS reads and
-// their latency between two barriers.  Whole steps of 65 to 256 rows x 4,001 to 2,000,003 labels x 64 to 1024 dims: 1.03 to
-// 1.7 times as fast; four accumulated micro-batches of 256 x 320,001 x 384 with the update 2.04 -> 1.81 ms.
+// twice.  dX and the update of 199 rows x 131,072 labels x 768 dims, reduction included: 239 -> 202 us (256 rows 249 -> 223, 128
+// rows 203 -> 183: 5.0 TB/s of the 8 bytes per weight and G); without its stores the pass took 150 at 199 and 256 rows, the LDS
+// reads and their latency between two barriers.  Whole steps of 65 to 256 rows x 4,001 to 2,812,281 labels x 64 to 1024 dims: 1.03
+// to 1.5 times as fast.
 //
 // Split.  A workgroup owns a slice of 128 dims and a range of labels, which it walks 64 at a time.  Its eight waves are two
 // groups of 64 dims by four quarters; a quarter takes 16 of the tile's labels for dW and their update, and a quarter of the
@@ -36,9 +36,9 @@ struct BackArgs {
   half_t* W; int64_t ldw;                     // read only but for BACK_UPDATE
   half_t* Mo; int64_t ldm; float lr, mu, wd;  // BACK_UPDATE
   float* out; int64_t ldo; float beta;        // BACK_OUT, BACK_ADD
-  float* part;                                // [ranges][B][d] partial sums of G.W
+  float* part;                                // [ranges * parts][B][d] partial sums of G.W
   int B, L, d;
-  int slices, ranges, tiles;                  // ranges a multiple of 8; tiles of 64 labels
+  int slices, ranges, parts, tiles;           // ranges a multiple of 8; tiles of 64 labels
 };
 
 template <bool NT, class T>
@@ -94,7 +94,9 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
   const int slice = local % a.slices, range = (local / a.slices) * 8 + xcd;
   const int dim0 = slice * BACK_DIMS + dg * 64;
-  const int t0 = (int)((int64_t)a.tiles * range / a.ranges), t1 = (int)((int64_t)a.tiles * (range + 1) / a.ranges);
+  const int part0 = range * a.parts, part1 = part0 + a.parts;
+  auto first_tile = [&](int part) { return (int)((int64_t)a.tiles * part / (a.ranges * a.parts)); };
+  const int t0 = first_tile(part0), t1 = first_tile(part1);
   const int low = i & 7, second = i >> 3;  // of the whole-line layout: label (and low + 8), which 32 dims (fp32: which 16)
 
   // What a thread fetches.  Labels, rows and dims past the end repeat the last ones; they are cleared in the LDS, or belong
@@ -188,6 +190,28 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
   for (int rb = 0; rb < RQ; ++rb)
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[rb][c] = float4v{0.f, 0.f, 0.f, 0.f};
+  // The sums of a part leave when the tile before `upto` ends it (they may be none, as may the tiles of a part).
+  int part = part0, end = first_tile(part0 + 1);
+  auto leave = [&](int upto) {
+    while (part < part1 && end == upto) {
+      int row = RQ * qt * 16 + i, at = dim0 + 4 * g;
+      asm volatile("" : "+v"(row), "+v"(at));  // opaque: addresses made here and not kept through the loop
+      float* dst = a.part + ((int64_t)part * a.B + row) * a.d + at;
+#pragma unroll
+      for (int rb = 0; rb < RQ; ++rb) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          if (row < a.B && at + 16 * c < a.d) *reinterpret_cast<float4v*>(dst + 16 * c) = acc[rb][c];
+          acc[rb][c] = float4v{0.f, 0.f, 0.f, 0.f};
+        }
+        row += 16;
+        dst += 16 * (int64_t)a.d;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      end = first_tile(++part + 1);
+    }
+  };
+  leave(t0);
 
   int parity = 0;
   // Loads and stores of a wave between its fetches of G and the barrier that makes them known: of tiles that are whole.
@@ -214,18 +238,31 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
     if (tile + 1 < t1) fetch_g(tile + 1, gs + parity * S::G_HALVES);
     fetch(tile + BACK_AHEAD, q);
     exact = l0 + BACK_TILE <= a.L && dim0 + 64 <= a.d;  // every lane stores
-    // dX^T += W^T . G^T, this quarter's rows
+    // dX^T += W^T . G^T, this quarter's rows: the tile's 64 labels by themselves, then one addition.  (An MFMA rounds its sum
+    // once per 16 of k, and the error of a long sum grows with the root of its roundings: see back_plan.)
+    {
+      half8 bg[2][RQ];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      half8 bg[RQ];
+      for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int rb = 0; rb < RQ; ++rb)
-        bg[rb] = *reinterpret_cast<const half8*>(gi + (k * S::ROWS + (RQ * qt + rb) * 16 + i) * 32 + 8 * g);
+        for (int rb = 0; rb < RQ; ++rb)
+          bg[k][rb] = *reinterpret_cast<const half8*>(gi + (k * S::ROWS + (RQ * qt + rb) * 16 + i) * 32 + 8 * g);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const half8 wt = S::read_tr(wi + ((k * 2 + dg) * 2 + (c >> 1)) * 1024, t4, 16 * (c & 1) + 4 * (lane & 3));
+        float4v t[RQ];
 #pragma unroll
-        for (int rb = 0; rb < RQ; ++rb) acc[rb][c] = S::mfma(wt, bg[rb], acc[rb][c]);
+        for (int rb = 0; rb < RQ; ++rb) t[rb] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const half8 wt = S::read_tr(wi + ((k * 2 + dg) * 2 + (c >> 1)) * 1024, t4, 16 * (c & 1) + 4 * (lane & 3));
+#pragma unroll
+          for (int rb = 0; rb < RQ; ++rb) t[rb] = S::mfma(wt, bg[k][rb], t[rb]);
+        }
+#pragma unroll
+        for (int rb = 0; rb < RQ; ++rb) {
+          acc[rb][c] += t[rb];
+          asm volatile("" : "+v"(acc[rb][c]));  // added here: the sums of all blocks, kept for later, would not fit the registers
+        }
       }
     }
     // dW^T = X^T . G, this quarter's labels
@@ -281,24 +318,12 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
             *reinterpret_cast<float4v*>(a.out + (int64_t)(label + 8 * h) * a.ldo + col32(s)) = v;
         }
     }
+    leave(tile + 1);
   };
   for (int t = t0; t < t1; t += BACK_AHEAD) {
 #pragma unroll
     for (int s = 0; s < BACK_AHEAD; ++s)
       if (t + s < t1) work(t + s, ahead[s]);  // (the barriers: every wave has the same tiles)
-  }
-
-  float* const part = a.part + (int64_t)range * a.B * a.d;
-#pragma unroll
-  for (int rb = 0; rb < RQ; ++rb) {
-    const int row = (RQ * qt + rb) * 16 + i;
-    if (row < a.B) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int dim = dim0 + 16 * c + 4 * g;
-        if (dim < a.d) *reinterpret_cast<float4v*>(part + (int64_t)row * a.d + dim) = acc[rb][c];
-      }
-    }
   }
 }
 

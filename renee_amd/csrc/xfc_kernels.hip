@@ -1553,30 +1553,43 @@ size_t small_step_ws_bytes(int64_t B, int64_t L, int64_t d) {
 template <int MODE, class Fn>
 bool back_step_for(int64_t B, Fn&& fn) {
   if (B < 1 || B > BACK_MAX_ROWS) return false;
-  constexpr bool ADD = MODE == BACK_ADD;  // its addends take registers that X^T has otherwise
+  // what the addends and the update leave of the registers
+  constexpr bool ADD = MODE == BACK_ADD, UPDATE = MODE == BACK_UPDATE;
   if (B <= 64) fn(BackStep<1, 2>{});
   else if (B <= 128) fn(BackStep<2, ADD ? 2 : 4>{});
-  else if (B <= 192) fn(BackStep<3, ADD ? 2 : 4>{});
-  else fn(BackStep<4, ADD ? 2 : 4>{});
+  else if (B <= 192) fn(BackStep<3, ADD ? 2 : UPDATE ? 3 : 4>{});
+  else fn(BackStep<4, ADD ? 0 : UPDATE ? 2 : 4>{});
   return true;
 }
-// Ranges of labels, each with a partial dX of its own: as many as there are CUs for their slices, in eighths for the XCDs;
-// fewer where the labels or the workspace run out (8 at least).
-int back_ranges(int64_t B, int64_t L, int64_t d, size_t ws_limit) {
+// Ranges of labels, one per workgroup: as many as there are CUs for their slices, in eighths for the XCDs; fewer where the
+// labels or the workspace run out (8 at least).  On long label axes a range leaves a partial dX for each of its parts, so that
+// no sum has more roundings than xfc_dx's (a tile's 64 labels are one addition here, four there).  Error of dX against float64
+// by xfc_dx, by one chain of MFMAs per range, now: 199 rows x 131,072 x 768 2.8, 3.8, 1.7e-7, 256 x 320,001 x 384 3.4, 4.2,
+// 1.9e-7, 5 x 60,007 x 3072 2.7, 5.6, 1.7e-7.
+struct BackPlan { int ranges, parts; };
+BackPlan back_plan(int64_t B, int64_t L, int64_t d, size_t ws_limit) {
   const int64_t slices = ceil_div(d, BACK_DIMS), per = num_cus() / (8 * slices), most = round_up(ceil_div(L, BACK_TILE), 8);
   int64_t ranges = 8 * (per > 1 ? per : 1);
   if (ranges > most) ranges = most;
-  while (ranges > 8 && (size_t)ranges * (size_t)B * (size_t)d * 4 > ws_limit) ranges -= 8;
-  return (int)ranges;
+  const size_t one = (size_t)B * (size_t)d * 4;
+  while (ranges > 8 && (size_t)ranges * one > ws_limit) ranges -= 8;
+  int tiles_m, tiles_n, sums, k_per_split;
+  dx_plan((int)B, (int)d, (int)L, tiles_m, tiles_n, sums, k_per_split);
+  int64_t parts = ceil_div(sums, 4 * ranges);
+  while (parts > 1 && (size_t)(ranges * parts) * one > ws_limit) --parts;
+  return {(int)ranges, (int)parts};
 }
 size_t back_ws_bytes(int64_t B, int64_t L, int64_t d) {
   if (B < 1 || B > BACK_MAX_ROWS || L < 1 || d < 1) return 0;
-  return (size_t)back_ranges(B, L, d, ~(size_t)0) * (size_t)B * (size_t)d * 4;
+  const BackPlan p = back_plan(B, L, d, ~(size_t)0);
+  return (size_t)p.ranges * (size_t)p.parts * (size_t)B * (size_t)d * 4;
 }
 template <int MODE>
 int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size_t ws_bytes, hipStream_t st, bool* taken) {
   *taken = false;
-  a.ranges = back_ranges(a.B, a.L, a.d, ws_bytes);
+  const BackPlan p = back_plan(a.B, a.L, a.d, ws_bytes);
+  a.ranges = p.ranges;
+  a.parts = p.parts;
   if (!ws || !aligned16(ws) || (size_t)a.ranges * a.B * a.d * 4 > ws_bytes) return XFC_OK;
   a.slices = ceil_div(a.d, BACK_DIMS);
   a.tiles = ceil_div(a.L, BACK_TILE);
@@ -1591,7 +1604,7 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
     rc = nt ? launch_k<back_step_kernel<S, MODE, true>>(g, b, S::LDS_BYTES, st, a)
             : launch_k<back_step_kernel<S, MODE, false>>(g, b, S::LDS_BYTES, st, a);
     if (rc) return;
-    launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges, scale, 0.0f, st);
+    launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges * a.parts, scale, 0.0f, st);
     rc = check_launch();
   });
   return rc;

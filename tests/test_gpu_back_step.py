@@ -101,3 +101,29 @@ def test_what_the_two_calls_refuse_is_refused(dev):
     assert call(ldg=192) == 6                     # shorter than the labels
     assert call(nbytes=ws.numel() - 16) == 4      # less than 8 partial sums
     assert call() == 0
+
+
+# the last: more partial sums than ranges, which only wide or very long operands have
+@pytest.mark.parametrize("B,L,d", [(128, 131072, 768), (199, 131072, 768), (256, 320001, 384), (256, 40001, 1024), (5, 60007, 3072)])
+def test_dx_is_as_close_to_float64_as_by_itself(dev, B, L, d):
+    """The sums of dX may not be longer than xfc_dx's: their error (of random roundings, so with some allowance for chance, a
+    tenth) against float64 is the measure.  G all of one sign, as after the first steps, W not."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(B + L)
+    G = torch.zeros(B, (L + 7) // 8 * 8, dtype=torch.float16, device=dev)
+    G[:, :L] = torch.rand(B, L, generator=g, device=dev)
+    X = torch.randn(B, d, generator=g, device=dev).half()
+    W = (torch.randn(L, d, generator=g, device=dev) * 0.02).half()
+    M = torch.zeros_like(W)
+    want = torch.zeros(B, d, dtype=torch.float64, device=dev)
+    for l0 in range(0, L, 16384):
+        want += G[:, l0:min(L, l0 + 16384)].double() @ W[l0:l0 + 16384].double()
+    ws = torch.empty(max(lib().xfc_step_workspace_bytes(B, L, d, 0), lib().xfc_dx_workspace_bytes(B, L, d)), dtype=torch.uint8, device=dev)
+    one, two = torch.empty(B, d, device=dev), torch.empty(B, d, device=dev)
+    print(f"dX: B={B} L={L} d={d}", flush=True)
+    check(lib().xfc_dx(G.data_ptr(), G.stride(0), W.data_ptr(), d, two.data_ptr(), d, B, L, d, 1.0, ws.data_ptr(), ws.numel(), _st()), "xfc_dx")
+    check(lib().xfc_dx_dw_update(G.data_ptr(), G.stride(0), X.data_ptr(), d, W.data_ptr(), d, M.data_ptr(), d, one.data_ptr(), d, B, L, d,
+                                 0.0, 0.9, 0.0, 1.0, ws.data_ptr(), ws.numel(), _st()), "xfc_dx_dw_update")
+    error = [float((t.double() - want).norm() / want.norm()) for t in (one, two)]
+    print(f"  {error[0]:.2e}, xfc_dx {error[1]:.2e}", flush=True)
+    assert error[0] <= 1.1 * error[1]
