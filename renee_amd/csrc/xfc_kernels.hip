@@ -2049,8 +2049,13 @@ int xfc_dx_dw(const void* G, int64_t ldg, const void* X, int64_t ldx, const void
               size_t workspace_bytes, void* stream) {
   // Up to 64 rows the two passes read a gradient that no cache holds a little faster (16 rows x 700,001 x 768: 1,043 against 1,089
   // us; x 320,001 x 768: 497 against 493; x 60,007: 86 to 91 against 97), unless the width leaves their tiles of 256 dims partly
-  // empty (x 700,001 x 384: 609 against 529).
-  const bool slow = dims_ok(L) && dims_ok(d) && B <= 64 && d % 256 == 0 && L * d * 4 > (int64_t)128 << 20;
+  // empty (x 700,001 x 384: 609 against 529).  A gradient that is only written leaves the one pass with little to save, the
+  // second reading of G: on long axes it is the slower from 129 rows on where its slices do not come out even with the CUs (768
+  // dims, six of them on 240: 192 rows x 1,500,001 1.58 against 1.69 ms, 256 rows 1.77 against 1.98; 1024 dims, all CUs: 192 x
+  // 700,001 1.04 against 1.00).
+  const bool sizes = dims_ok(B) && dims_ok(L) && dims_ok(d) && d > 0, whole = sizes && d % 256 == 0;
+  const bool even = sizes && (num_cus() / 8) % ceil_div(d, BACK_DIMS) == 0;
+  const bool slow = whole && ((B <= 64 && L * d * 4 > (int64_t)128 << 20) || (beta == 0.f && B > 128 && !even && L * d > (int64_t)400 << 20));
   if (!slow && back_ok(G, ldg, X, ldx, W, ldw, dX, B, L, d) && grad && ld_grad % 4 == 0 && aligned16(grad)) {
     BackArgs a = back_args(G, ldg, X, ldx, W, ldw, B, L, d);
     a.out = grad; a.ldo = ld_grad; a.beta = beta;

@@ -127,3 +127,21 @@ def test_dx_is_as_close_to_float64_as_by_itself(dev, B, L, d):
     error = [float((t.double() - want).norm() / want.norm()) for t in (one, two)]
     print(f"  {error[0]:.2e}, xfc_dx {error[1]:.2e}", flush=True)
     assert error[0] <= 1.1 * error[1]
+
+
+def test_a_first_gradient_on_a_long_axis_takes_two_passes(dev):
+    """129 to 256 rows, 768 dims, a gradient that is only written: the two passes, which are faster there, to the last bit."""
+    B, L, d = 192, 560007, 768
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    G = torch.zeros(B, (L + 7) // 8 * 8, dtype=torch.float16, device=dev)
+    G[:, :L] = torch.rand(B, L, generator=g, device=dev)
+    X = torch.randn(B, d, generator=g, device=dev).half()
+    W = torch.randn(L, d, generator=g, device=dev).half()
+    ws = torch.empty(max(lib().xfc_step_workspace_bytes(B, L, d, 0), lib().xfc_dx_workspace_bytes(B, L, d)), dtype=torch.uint8, device=dev)
+    dX, grad = torch.empty(2, B, d, device=dev), torch.empty(2, L, d, device=dev)
+    check(lib().xfc_dx_dw(G.data_ptr(), G.stride(0), X.data_ptr(), d, W.data_ptr(), d, grad[0].data_ptr(), d, dX[0].data_ptr(), d, B, L, d,
+                          0.0, 1.0, ws.data_ptr(), ws.numel(), _st()), "xfc_dx_dw")
+    check(lib().xfc_dx(G.data_ptr(), G.stride(0), W.data_ptr(), d, dX[1].data_ptr(), d, B, L, d, 1.0, ws.data_ptr(), ws.numel(), _st()), "xfc_dx")
+    check(lib().xfc_dw(G.data_ptr(), G.stride(0), X.data_ptr(), d, grad[1].data_ptr(), d, B, L, d, 0.0, _st()), "xfc_dw")
+    assert torch.equal(dX[0], dX[1]) and torch.equal(grad[0], grad[1])
