@@ -1829,12 +1829,14 @@ static SmallArgs small_args(const void* X, int64_t ldx, const void* W, int64_t l
 // G of a small batch and its positives in one launch, if there is such a kernel for the call (whose arguments have been
 // checked): no loss, no more pairs than the workgroups' threads hold.  XFC_OK with *taken false otherwise.  It stands as long as
 // it is the faster one: 32 rows x 131,072 x 768 41 -> 33 us and x 4,097 launch-bound, 16 -> 13, but x 320,001 97 -> 101; with 64 rows
-// its two barriers a tile weigh more, x 20,011 16 -> 13 but x 60,007 21 -> 25.
+// its two barriers a tile weigh more, x 20,011 16 -> 13 but x 60,007 21 -> 25, and at 128 dims x 100,003 16.6 -> 15.1 but x 131,072
+// 16.4 -> 17.9.
 static int small_grad(const void* X, int64_t ldx, const void* W, int64_t ldw, const int32_t* rowptr, const int32_t* colidx,
                       const int64_t* pos_x, const int64_t* pos_y, int64_t nnz, void* G, int64_t ldg, int64_t B, int64_t L, int64_t d,
                       const float* loss, hipStream_t st, bool* taken) {
   *taken = false;
-  if (loss || B > SMALL_MAX_ROWS || nnz > SMALL_MAX_PAIRS || L * d > (B <= 32 ? (int64_t)160 << 20 : (int64_t)16 << 20)) return XFC_OK;
+  if (loss || B > SMALL_MAX_ROWS || nnz > SMALL_MAX_PAIRS) return XFC_OK;
+  if (B <= 32 ? L * d > (int64_t)160 << 20 : L * d > (int64_t)16 << 20 || L > 100 << 10) return XFC_OK;
   const SmallArgs a = small_args(X, ldx, W, ldw, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, B, L);
   int rc = XFC_OK;
   *taken = small_grad_for(B, d, [&](auto s) {

@@ -37,3 +37,18 @@ def test_grad_of_a_small_batch(dev, B, d, L):
     colidx = torch.tensor([c for r in rows for c in r], dtype=torch.int32)
     lay.outsoft.fill_(float("nan"))
     assert torch.equal(lay.fwd_grad(X.to(dev), rowptr=rowptr.to(dev), colidx=colidx.to(dev)), G)
+
+
+def test_many_labels_of_128_dims_go_through_the_product(dev):
+    """64 rows x 131,072 x 128: one launch is the slower there.  The pass with the loss always runs the product, so that its G has
+    the same bits (the other sums the logit in another order)."""
+    B, L, d = 64, 131072, 128
+    X, W = synth.make_X(B, d, 1, dev, torch.float32).half(), (synth.make_W(L, d, 1, dev, torch.float32) * 40).half()
+    lay = XFCLayer(L, d, B, dev, weight=W)
+    px, py = torch.arange(B, device=dev), torch.arange(B, device=dev) * 7
+    G = lay.fwd_grad(X, px, py).clone()
+    H = lay.fwd_grad(X, px, py, loss_out=torch.zeros(1, device=dev)).clone()
+    assert float((G - H).abs().max()) <= 2.0 ** -11 + 2e-5
+    G[px, py] = 0  # the positives' logits are summed in an order of their own
+    H[px, py] = 0
+    assert torch.equal(G, H)
