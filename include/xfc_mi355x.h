@@ -260,7 +260,8 @@ int xfc_topk(const void* X, int64_t ldx, const void* W, int64_t ldw,
  * xfc_topk with a second buffer.  For K > 8 it takes the largest logit of every 32 labels, from which the
  * selection learns which few parts of a row to read: min(B, rows the workspace holds) x round_up(L, 256) / 16
  * bytes, 16-byte aligned (what xfc_topk_workspace_bytes(B, L, 8) asks for is more than enough).  A smaller one, or none, is not used and the
- * selection reads the rows (xfc_topk does that too unless its workspace has the room behind the logits).
+ * selection reads the rows (xfc_topk does that too unless its workspace has the room behind the logits), as it does for K > 6144
+ * and for rows of fewer than 2048 or 2 K such blocks.
  * K <= 8: not used.  The results are the same either way.
  */
 int xfc_topk_scratch(const void* X, int64_t ldx, const void* W, int64_t ldw,

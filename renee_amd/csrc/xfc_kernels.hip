@@ -494,6 +494,10 @@ constexpr int SEL_BINS = 2048;  // histogram over the top 11 bits of the 16-bit 
 // LDS, one row per CU at a time) for K up to SEL_MAX_K
 constexpr int SEL_CAP_SMALL = 2048, SEL_CAP_LARGE = 16384;
 constexpr int SEL_SMALL_MAX_K = SEL_CAP_SMALL / 2;
+// At least K blocks reach the bound that the maxima give, on random logits up to a quarter more: the list of them has room for
+// twice SEL_SMALL_MAX_K in the place of the histogram and, at the end of the large buffer, for 8192.  (64 rows x 1,310,720 x 64,
+// K = 2049: 442 -> 157 us against full passes over the rows, which a list of 2048 led to; K = 8192, where it would not do: 508 -> 493.)
+constexpr int SEL_LIST_LARGE = 8192, SEL_BLOCKS_MAX_K = SEL_LIST_LARGE * 3 / 4;
 constexpr int SEL_BLOCKS_MIN = 2048;  // rows with fewer blocks of logits are selected without their maxima
 static_assert(2 * SEL_MAX_K <= SEL_CAP_LARGE, "ranks per row");
 
@@ -523,8 +527,9 @@ struct SelLds {
 // buffer the row has been read 1 + 1/sample_stride times instead of twice, and if not the full passes run.
 // With the maxima of the row's blocks of LOGIT_BLOCK (n_blocks > 0) they are that subset: the histogram is theirs, and only
 // blocks whose maximum reaches the bound are read at all, about K of them.  A block that holds a value that is no number has
-// no maximum to go by (one with the sign set ranks last); a row with such a block takes the full passes.  (512 rows x 1,310,720
-// logits, K = 100: 368 us with the sampled pass, now 54; the forward pass that leaves the maxima takes as long as without.)
+// no maximum to go by (one with the sign set ranks last); a row with such a block, or with more blocks at the bound than there is
+// room for, goes on with the sampled pass.  (512 rows x 1,310,720 logits, K = 100: 368 us with the sampled pass, 54 with the
+// maxima; the forward pass that leaves them takes as long as without.)
 template <int SEL_CAP>
 __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const half_t* __restrict__ logits, int64_t ldl, int L,
                                                                    int64_t numy, int K, int sample_stride,
@@ -585,10 +590,11 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const half_t* 
       if (second) piece(q1, i + (int)STEP);
     }
   };
-  auto push = [&](uint32_t key, int idx) {
+  auto push_below = [&](int room, uint32_t key, int idx) {
     const int slot = atomicAdd(&S.n_cand, 1);
-    if (slot < SEL_CAP) S.cand[slot] = ((unsigned long long)(0xffffu - key) << 32) | (uint32_t)idx;
+    if (slot < room) S.cand[slot] = ((unsigned long long)(0xffffu - key) << 32) | (uint32_t)idx;
   };
+  auto push = [&](uint32_t key, int idx) { push_below(SEL_CAP, key, idx); };
   // Finds, over hist[0..nb), the highest bin b with (count in bins above b) + base < K <= that + hist[b];
   // writes S.bin = b and S.above = base + count above b.  nb is a multiple of 64; executed by wave 0.
   auto find_bin = [&](int nb, int base) {
@@ -650,32 +656,36 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const half_t* 
       find_bin(SEL_BINS, 0);
       __syncthreads();
       const uint32_t kthr = (uint32_t)S.bin << 5;
-      // the blocks that reach the bound, in the place of the histogram, then their logits, four threads to a block
+      // the blocks that reach the bound, in a list, then their logits, four threads to a block
+      constexpr bool LARGE = SEL_CAP > SEL_CAP_SMALL;
+      constexpr int LIST = LARGE ? SEL_LIST_LARGE : SEL_BINS, ROOM = LARGE ? SEL_CAP - LIST / 2 : SEL_CAP;
+      int* const list = LARGE ? reinterpret_cast<int*>(S.cand + ROOM) : S.hist;
       if (tid == 0) S.n_blocks = 0;
       __syncthreads();
       for_each_from(maxima, n_blocks, kthr, [&](uint32_t, int b) {
         const int slot = atomicAdd(&S.n_blocks, 1);
-        if (slot < SEL_BINS) S.hist[slot] = b;
+        if (slot < LIST) list[slot] = b;
       });
       __syncthreads();
       const int hits = S.n_blocks;
-      for (int t = tid; t < hits * 4 && hits <= SEL_BINS; t += SEL_THREADS) {
-        const int i = S.hist[t >> 2] * LOGIT_BLOCK + (t & 3) * 8;
+      for (int t = tid; t < hits * 4 && hits <= LIST; t += SEL_THREADS) {
+        const int i = list[t >> 2] * LOGIT_BLOCK + (t & 3) * 8;
         if (i < L) {
           const uint4v q = *reinterpret_cast<const uint4v*>(row + i);
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             const uint32_t key = sel_key((q[e >> 1] >> (16 * (e & 1))) & 0xffffu);
-            if (i + e < L && key >= kthr) push(key, i + e);
+            if (i + e < L && key >= kthr) push_below(ROOM, key, i + e);
           }
         }
       }
       __syncthreads();
-      done = hits <= SEL_BINS && S.n_cand <= SEL_CAP;
+      done = hits <= LIST && S.n_cand <= ROOM;
       __syncthreads();
     }
     if (!done) reset();
-  } else if (sample_stride > 1) {
+  }
+  if (!done && sample_stride > 1) {
     for_each_block(sample_stride, [&](uint32_t key, int) { atomicAdd(&S.hist[key >> 5], 1); });
     __syncthreads();
     find_bin(SEL_BINS, 0);  // the host only asks for a sample that holds at least K elements
@@ -756,7 +766,9 @@ __global__ void __launch_bounds__(SEL_THREADS) topk_select_kernel(const half_t* 
     }
   }
   __syncthreads();
-  if (done && S.n_cand > 4 * K) {
+  int fewest = 512;  // what would be sorted with a closer bound, a power of two that holds little more than K
+  while (fewest < K + K / 16) fewest <<= 1;
+  if (done && S.n_cand > (K < 128 ? 4 * K : fewest)) {
     // a loose bound: the K-th largest candidate's bin gives a closer one, and fewer to sort
     unsigned long long mine[SEL_CAP / SEL_THREADS];
     const int had = S.n_cand;
@@ -2231,7 +2243,7 @@ static int topk_impl(const void* X, int64_t ldx, const void* W, int64_t ldw, int
     const int64_t n_blocks = ceil_div(L, LOGIT_BLOCK), ldb = round_up(L, FwdWide::BM) / LOGIT_BLOCK;
     const size_t logits = (size_t)round_up((int64_t)((size_t)block * (size_t)ldl * 2), 16), maxima = (size_t)block * (size_t)ldb * 2;
     half_t* bmax = nullptr;
-    if (n_blocks >= 2 * (int64_t)K && n_blocks >= SEL_BLOCKS_MIN) {
+    if (K <= SEL_BLOCKS_MAX_K && n_blocks >= 2 * (int64_t)K && n_blocks >= SEL_BLOCKS_MIN) {
       if (scratch && scratch_bytes >= maxima && aligned16(scratch)) bmax = (half_t*)scratch;
       else if (workspace_bytes >= logits + maxima) bmax = (half_t*)((unsigned char*)workspace + logits);
     }

@@ -81,3 +81,31 @@ def test_loose_bounds_and_rows_without_one(dev, B):
     W16 = W.half()
     W16.view(torch.int16)[5000:5040, 0] = -512 + 5  # 0xfe05: no number, sign set
     _check(X.half().to(dev), W16.to(dev), K)
+
+
+# more blocks at the bound than the small list holds, at its most, and more than the maxima are used for; NaN on top
+@pytest.mark.parametrize("B,L,K", [(3, 300007, 2049), (2, 400009, 4096), (2, 400009, 6144), (1, 600011, 6145), (1, 700001, 8192)])
+def test_long_lists_of_blocks(dev, B, L, K):
+    g = torch.Generator().manual_seed(K)
+    X, W = torch.randn(B, 16, generator=g).half().to(dev), torch.randn(L, 16, generator=g).half().to(dev)
+    _check(X, W, K)
+    W[777] = float("nan")
+    _check(X, W, K)
+    W[:, 1:] = 0.0  # many ties
+    W[:, 0] = torch.randint(-40, 40, (L,), generator=g).half().to(dev)
+    _check(X, W, K)
+
+
+@pytest.mark.parametrize("K,used", [(1024, True), (6144, True), (6145, False), (8192, False)])
+def test_maxima_are_made_where_they_serve(dev, K, used):
+    """A selection whose list of blocks could not hold K does not pay for the maxima: the second buffer stays as it was."""
+    B, L, d = 2, 600011, 16
+    g = torch.Generator().manual_seed(1)
+    X, W = torch.randn(B, d, generator=g).half().to(dev), torch.randn(L, d, generator=g).half().to(dev)
+    h = lib()
+    ws = torch.empty(h.xfc_topk_workspace_bytes(B, L, K), dtype=torch.uint8, device=dev)
+    sc = torch.full((B * ((L + 255) // 256) * 16,), 0x5a, dtype=torch.uint8, device=dev)
+    v, i = torch.empty(B, K, device=dev), torch.empty(B, K, dtype=torch.int64, device=dev)
+    check(h.xfc_topk_scratch(X.data_ptr(), d, W.data_ptr(), d, B, L, d, L, K, v.data_ptr(), i.data_ptr(), ws.data_ptr(), ws.numel(),
+                             sc.data_ptr(), sc.numel(), torch.cuda.current_stream().cuda_stream), "xfc_topk_scratch")
+    assert bool((sc != 0x5a).any()) == used
