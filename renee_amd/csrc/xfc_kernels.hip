@@ -496,7 +496,7 @@ constexpr int SEL_CAP_SMALL = 2048, SEL_CAP_LARGE = 16384;
 constexpr int SEL_SMALL_MAX_K = SEL_CAP_SMALL / 2;
 // At least K blocks reach the bound that the maxima give, on random logits up to a quarter more: the list of them has room for
 // twice SEL_SMALL_MAX_K in the place of the histogram and, at the end of the large buffer, for 8192.  (64 rows x 1,310,720 x 64,
-// K = 2049: 442 -> 157 us against full passes over the rows, which a list of 2048 led to; K = 8192, where it would not do: 508 -> 493.)
+// K = 2049: 403 -> 143 us against full passes over the rows, which a list of 2048 led to; K = 8192, where it would not do: 649 -> 630.)
 constexpr int SEL_LIST_LARGE = 8192, SEL_BLOCKS_MAX_K = SEL_LIST_LARGE * 3 / 4;
 constexpr int SEL_BLOCKS_MIN = 2048;  // rows with fewer blocks of logits are selected without their maxima
 static_assert(2 * SEL_MAX_K <= SEL_CAP_LARGE, "ranks per row");
