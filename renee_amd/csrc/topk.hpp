@@ -16,6 +16,7 @@
 namespace xfc {
 
 constexpr int TOPK_MAX = 8;
+constexpr int64_t TOPK_RANGE_MAX = (int64_t)1 << 30;  // labels of a range: the kernels' 32-bit indices run somewhat past its end
 typedef float float2v __attribute__((ext_vector_type(2)));
 
 // Floats as unsigned keys in the same order, and back.
@@ -62,7 +63,7 @@ struct ScoreArgs {
   const half_t* X; int64_t ldx;  // M rows of K
   const half_t* W; int64_t ldw;  // N labels of K
   float* bmax; int64_t ldb;      // [M][ldb]: the largest score of every block
-  int M, N, K;
+  int M, N, K;                   // N at most TOPK_RANGE_MAX
   int tiles_m, tiles_n, n_ids;   // wide: n_ids = tiles_m * round_up(tiles_n, 8)
   int run;                       // small: units in a row that a wave takes, 1, 2 or 4
 };
@@ -148,7 +149,7 @@ __global__ void __launch_bounds__(C::NT) score_wide_kernel(ScoreArgs a) {
 constexpr int SCORE_SMALL_ROWS = 32, SCORE_SMALL_BLOCK = 16, SCORE_SMALL_WAVES = 8, SCORE_STEPS = 4, SCORE_SLOTS = 3;
 
 template <int RB>
-constexpr int score_small_lds(int64_t K) { return (int)((K + 31) / 32) * RB * 1024; }
+constexpr int64_t score_small_lds(int64_t K) { return (K + 31) / 32 * RB * 1024; }
 
 // Two workgroups to a CU.
 template <int RB>

@@ -1650,7 +1650,7 @@ int launch_score_small(ScoreArgs a, hipStream_t st) {
     fprintf(stderr, "xfc: cannot raise the dynamic LDS limit to %d bytes: %s\n", FULL_LDS, hipGetErrorString(e));
     return XFC_ERR_HIP;
   }
-  return launch_k<score_small_kernel<RB>>(dim3((unsigned)(want < most ? want : most)), dim3(64 * NW), score_small_lds<RB>(a.K), st, a);
+  return launch_k<score_small_kernel<RB>>(dim3((unsigned)(want < most ? want : most)), dim3(64 * NW), (int)score_small_lds<RB>(a.K), st, a);
 }
 
 struct SelArgs {
@@ -2181,10 +2181,10 @@ static TopkPlan topk_plan(int64_t B, int64_t L, int64_t d, int64_t K, size_t ws_
   p.range = L;
   // a tile of the wide kernel writes the maxima of all its blocks
   p.ldb = p.small ? topk_blocks(L, p.block) : topk_blocks(round_up(L, FwdWide::BM), p.block);
-  if ((size_t)B * (size_t)p.ldb * 4 > ws_limit) {
-    const int64_t lists = B * K * 8, unit = p.small ? 4 : FwdWide::BM / SCORE_WIDE_BLOCK;
+  if ((size_t)B * (size_t)p.ldb * 4 > ws_limit || L > TOPK_RANGE_MAX) {
+    const int64_t lists = B * K * 8, unit = p.small ? 4 : FwdWide::BM / SCORE_WIDE_BLOCK, most = TOPK_RANGE_MAX / p.block;
     const int64_t fit = ws_limit > (size_t)lists ? (int64_t)((ws_limit - (size_t)lists) / ((size_t)B * 4)) : 0;
-    p.ldb = fit / unit * unit;
+    p.ldb = (fit < most ? fit : most) / unit * unit;
     p.range = p.ldb * p.block;
   }
   return p;

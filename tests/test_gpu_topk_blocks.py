@@ -82,3 +82,35 @@ def test_scores_that_are_no_numbers_are_passed_over(dev, B):
     v, i = _run(Xd, W.half().to(dev), K, numy=2500)
     assert i.cpu().tolist() == [[2047, 100] + [2499] * 6] * B
     assert v.cpu()[:, :2].tolist() == [[3.0, 2.0]] * B and bool(torch.isneginf(v[:, 2:]).all())
+
+
+@pytest.mark.parametrize("B", [1, 3])
+def test_label_counts_at_the_end_of_32_bits(dev, B):
+    """The largest label count there is, in ranges: the last label, one on each side of a range's end, and ties to the lower."""
+    L, d, K = 2 ** 31 - 1, 8, 6
+    if torch.cuda.mem_get_info()[0] < 45 << 30:
+        pytest.skip("needs 45 GB")
+    W = torch.zeros(L, d, dtype=torch.float16, device=dev)
+    best = {L - 1: 4.0, 2 ** 30 - 1: 3.0, 2 ** 30: 3.0, 5: 2.0}
+    for label, score in best.items():
+        W[label, 0] = score
+    X = torch.zeros(B, d, dtype=torch.float16, device=dev)
+    X[:, 0] = 1.0
+    v, i = _run(X, W, K)
+    assert i.cpu().tolist() == [[L - 1, 2 ** 30 - 1, 2 ** 30, 5, 0, 1]] * B
+    assert v.cpu().tolist() == [[4.0, 3.0, 3.0, 2.0, 0.0, 0.0]] * B
+
+
+def test_a_width_whose_fragments_exceed_32_bits_of_bytes(dev):
+    """2^25 dims, 17 rows: X as fragments would take 2 GB, no LDS and no positive int; the main loop takes the call."""
+    B, L, d, K = 17, 3, 2 ** 25, 3
+    g = torch.Generator(device=dev)
+    g.manual_seed(1)
+    X, W = torch.zeros(B, d, dtype=torch.float16, device=dev), torch.zeros(L, d, dtype=torch.float16, device=dev)
+    at = torch.randint(0, d, (64,), generator=g, device=dev)
+    at[0] = d - 1
+    X[:, at] = torch.randint(-2, 3, (B, 64), generator=g, device=dev).half()
+    W[:, at] = torch.randint(-2, 3, (L, 64), generator=g, device=dev).half()
+    v, i = _run(X, W, K)
+    ev, ei = _expect(X[:, at.unique()], W[:, at.unique()], K)
+    assert torch.equal(v, ev) and torch.equal(i, ei)
