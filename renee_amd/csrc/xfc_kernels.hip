@@ -17,6 +17,7 @@
 #include "pipe_core.hpp"
 #include "small_step.hpp"
 #include "topk.hpp"
+#include "topk_lists.hpp"
 #include "wide_core.hpp"
 
 namespace xfc {
@@ -1704,6 +1705,9 @@ int xfc_init(void) {
   keep(raise_lds_limit<fwd_wide_kernel<FWD_LINEAR, false, false, true>>(FwdWide::LDS_BYTES));
   keep(raise_lds_limit<score_wide_kernel<ScoreWide>>(ScoreWide::LDS_BYTES));
   keep(raise_lds_limit<score_wide_kernel<ScoreWide128>>(ScoreWide128::LDS_BYTES));
+  keep(raise_lds_limit<topk_list_kernel<ListCore>>(TopkLds<ListCore>::BYTES));
+  keep(raise_lds_limit<topk_list_kernel<ListCore128>>(TopkLds<ListCore128>::BYTES));
+  keep(raise_lds_limit<topk_list_kernel<ListCore64>>(TopkLds<ListCore64>::BYTES));
   keep(raise_lds_limit<dx_wide_kernel>(DxWide::LDS_BYTES));
   auto small_limits = [&](auto core_tag, auto dx_tag) {
     using C = typename decltype(core_tag)::type;
@@ -2189,7 +2193,44 @@ static TopkPlan topk_plan(int64_t B, int64_t L, int64_t d, int64_t K, size_t ws_
   }
   return p;
 }
-// What the pass refuses to run without, and what it runs fastest with.  (The former is what an earlier form of it needed.)
+
+constexpr int TOPK_SAMPLE = 2048;
+// The pass with lists (topk_lists.hpp).  Label groups: enough to give every CU a workgroup, fewer when the workspace holds no
+// more (8 at least; the seeding is dropped before the last groups are).  The rows' bounds start from the K-th score over a sample
+// of the first TOPK_SAMPLE labels (a small logits pass and an exact selection) when every label group has enough tiles for that
+// to pay; otherwise from nothing.  Without it every workgroup's first tiles overflow the candidate buffers and are rescanned.
+struct ListPlan { int tiles_m, tiles_n, groups; bool seeded; size_t need; };
+static ListPlan topk_list_plan(int64_t B, int64_t L, int64_t K, size_t ws_limit) {
+  ListPlan p;
+  p.tiles_m = ceil_div(B, row_tile(B));
+  p.tiles_n = ceil_div(L, ListCore::BN);
+  const int per = num_cus() / (8 * p.tiles_m);  // groups per XCD
+  const int cap = (int)round_up(p.tiles_n, 8);
+  p.groups = 8 * (per > 1 ? per : 1) < cap ? 8 * (per > 1 ? per : 1) : cap;
+  for (;; p.groups -= 8) {
+    // the groups' lists, the rows' shared bounds, and the sample's logits and their top K
+    const size_t lists = (size_t)p.groups * B * K * 8 + (size_t)round_up(B, 4) * 4, sample = (size_t)B * TOPK_SAMPLE * 2 + (size_t)B * K * 12;
+    p.seeded = L >= 8 * (int64_t)TOPK_SAMPLE && p.tiles_n >= 8 * p.groups && lists + sample <= ws_limit;
+    p.need = lists + (p.seeded ? sample : 0);
+    if (p.need <= ws_limit || p.groups <= 8) return p;
+  }
+}
+// Lists or maxima.  A workspace that holds the maxima of a third of the labels or more takes those range by range (1024 rows x 131,072
+// x 768, K = 5, three ranges 345 us, lists 386; 16 rows, four: 132 and 103); with less, launches and half-filled rounds add up (64
+// rows x 131,072, K = 1, nine: 196 and 92; x 700,001, K = 5, ten: 377 and 247; what the least takes, see topk_lists.hpp).  Lists of
+// more places cost the larger row tiles more: 65 to 512 rows with K from 4 on go up to nine ranges (128 rows x 700,001 x 64, nine: 155
+// and 213; 512 x 131,072 x 768, eight: 651 and 712; ten: 128 x 700,001 x 768 387 and 359).  With room for all of them lists
+// are the faster where storing and reading the maxima of very many labels weighs more than keeping lists of one to three places: up
+// to 128 rows, K = 1 from some 1.25 million labels on (64 rows x 1,500,001 x 512 319 against 285 us, x 2,812,281 x 768 830 against 733;
+// x 1,000,003 x 768 no difference), K = 2 and 3 from some 2 million on (64 x 2,812,281 x 768 1.12 and 1.08 times as fast, x 512 1.12
+// and 1.06), at widths whose weights take their time either way (x 2,812,281 x 256, K = 3: 0.88).
+static bool topk_by_lists(const TopkPlan& p, int64_t B, int64_t L, int64_t d, int64_t K) {
+  if (L > TOPK_RANGE_MAX) return false;
+  if (p.range < L) return (K >= 4 && B > 64 && B <= 512 ? 9 : 3) * p.range < L;
+  if (B > 128 || d < 256) return false;
+  return K == 1 ? L > 1250000 : K <= 3 && L > 2000000 && d <= 768 && (K == 2 || d >= 512);
+}
+// What the pass refuses to run without (lists of eight label groups), and what it runs fastest with.
 static size_t topk_least(int64_t B, int64_t K) { return (size_t)8 * B * K * 8 + (size_t)round_up(B, 4) * 4; }
 static size_t topk_need(int64_t B, int64_t L, int64_t K) {
   // whichever kernel the width leads to
@@ -2219,6 +2260,48 @@ size_t xfc_layer_workspace_bytes(int64_t max_batch, int64_t L, int64_t d, int64_
   }
   const size_t step = (size_t)round_up(xfc_fwd_grad_workspace_bytes(L, max_nnz), 256) + dx;
   return step > topk ? step : topk;
+}
+
+static int topk_lists(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, int B, int L, int d, int64_t numy, int K, float* values,
+                      int64_t* indices, void* workspace, size_t workspace_bytes, hipStream_t st) {
+  const ListPlan p = topk_list_plan(B, L, K, workspace_bytes);
+  if (workspace_bytes < p.need) return XFC_ERR_WORKSPACE;
+  ListArgs a;
+  a.X = X; a.ldx = ldx; a.W = W; a.ldw = ldw;
+  a.M = B; a.N = L; a.K = d; a.topk = K;
+  a.tiles_m = p.tiles_m; a.tiles_n = p.tiles_n; a.n_groups = p.groups;
+  a.cand_v = reinterpret_cast<float*>(workspace);
+  a.cand_i = reinterpret_cast<int32_t*>(a.cand_v + (size_t)p.groups * B * K);
+  a.bound = reinterpret_cast<uint32_t*>(a.cand_i + (size_t)p.groups * B * K);
+  const dim3 rows((unsigned)ceil_div(B, 256));
+  int rc;
+  if (p.seeded) {
+    // 16-byte aligned: the lists above are B * K * 8 * groups bytes (a multiple of 8 groups), the bounds 16-byte padded
+    half_t* sample = reinterpret_cast<half_t*>(a.bound + round_up(B, 4));
+    int64_t* sample_i = reinterpret_cast<int64_t*>(sample + (size_t)B * TOPK_SAMPLE);
+    float* sample_v = reinterpret_cast<float*>(sample_i + (size_t)B * K);
+    rc = launch_fwd(FWD_LINEAR, X, ldx, W, ldw, sample, TOPK_SAMPLE, B, TOPK_SAMPLE, d, TOPK_SAMPLE, 1.0f, 0.0f, st);
+    if (rc) return rc;
+    const SelArgs sa = {sample, (int64_t)TOPK_SAMPLE, TOPK_SAMPLE, (int64_t)TOPK_SAMPLE, K, 1, nullptr, 0, 0, sample_v, sample_i};
+    if ((rc = launch_select<SEL_CAP_SMALL>(B, sa, st))) return rc;
+    hipLaunchKernelGGL(topk_seed_kernel, rows, dim3(256), 0, st, (const float*)sample_v, K, a.bound, (int64_t)B);
+  } else {
+    // a kernel, not a memset: the call may be recorded into a graph
+    hipLaunchKernelGGL(fill_u32_kernel, rows, dim3(256), 0, st, a.bound, 0u, (int64_t)B);
+  }
+  if ((rc = check_launch())) return rc;
+  auto launch = [&](auto core) {
+    using C = typename decltype(core)::type;
+    return launch_k<topk_list_kernel<C>>(dim3((unsigned)(p.tiles_m * p.groups)), dim3(C::NT), TopkLds<C>::BYTES, st, a);
+  };
+  switch (row_tile(B)) {
+    case 64: rc = launch(std::type_identity<ListCore64>{}); break;
+    case 128: rc = launch(std::type_identity<ListCore128>{}); break;
+    default: rc = launch(std::type_identity<ListCore>{}); break;
+  }
+  if (rc) return rc;
+  hipLaunchKernelGGL(topk_merge_kernel, dim3((unsigned)B), dim3(256), 0, st, a.cand_v, a.cand_i, B, p.groups, K, numy, values, indices);
+  return check_launch();
 }
 
 static int topk_impl(const void* X, int64_t ldx, const void* W, int64_t ldw, int64_t B, int64_t L, int64_t d, int64_t numy,
@@ -2266,10 +2349,14 @@ static int topk_impl(const void* X, int64_t ldx, const void* W, int64_t ldw, int
     }
     return XFC_OK;
   }
-  const TopkPlan p = topk_plan(B, L, d, K, workspace ? workspace_bytes : 0);
-  if (!workspace || workspace_bytes < topk_least(B, K) || p.range < 1) return XFC_ERR_WORKSPACE;
+  if (!workspace || workspace_bytes < topk_least(B, K)) return XFC_ERR_WORKSPACE;
   if (!aligned16(workspace)) return XFC_ERR_ALIGN;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const TopkPlan p = topk_plan(B, L, d, K, workspace_bytes);
+  if (topk_by_lists(p, B, L, d, K))
+    return topk_lists((const half_t*)X, ldx, (const half_t*)W, ldw, (int)B, (int)L, (int)d, numy, K, values, indices, workspace,
+                      workspace_bytes, st);
+  if (p.range < 1) return XFC_ERR_WORKSPACE;
   for (int64_t l0 = 0; l0 < L; l0 += p.range) {
     const int64_t n = L - l0 < p.range ? L - l0 : p.range;
     ScoreArgs a;
