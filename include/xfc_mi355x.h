@@ -249,7 +249,7 @@ int xfc_step_coo(const void* X, int64_t ldx, void* W, int64_t ldw, void* M, int6
  * B x L x 4 / 16 (up to 32 rows) or / 32 bytes, and NOT monotone in B; a smaller workspace is accepted down to
  * 64*B*K + 4*round_up(B,4) bytes (the same result): the labels then go in a few ranges, or, below a third (65 to 512 rows, K >= 4:
  * a ninth) of it, through a pass that keeps lists of the K best per label group, as many groups as fit (16 rows x 700,001 x 768, K = 5: 0.21 ms with all of
- * 11 MB, 0.23 with 0.23 MB, 3.8 with the least, 5.2 KB).  Use xfc_layer_workspace_bytes() for a buffer that serves every batch size.
+ * 2.8 MB, 0.23 with 0.23 MB, 3.8 with the least, 5.2 KB).  Use xfc_layer_workspace_bytes() for a buffer that serves every batch size.
  */
 size_t xfc_topk_workspace_bytes(int64_t B, int64_t L, int64_t K);
 int xfc_topk(const void* X, int64_t ldx, const void* W, int64_t ldw,

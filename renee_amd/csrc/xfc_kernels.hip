@@ -2223,12 +2223,14 @@ static ListPlan topk_list_plan(int64_t B, int64_t L, int64_t K, size_t ws_limit)
 // are the faster where storing and reading the maxima of very many labels weighs more than keeping lists of one to three places: up
 // to 128 rows, K = 1 from some 1.25 million labels on (64 rows x 1,500,001 x 512 319 against 285 us, x 2,812,281 x 768 830 against 733;
 // x 1,000,003 x 768 no difference), K = 2 and 3 from some 2 million on (64 x 2,812,281 x 768 1.12 and 1.08 times as fast, x 512 1.12
-// and 1.06), at widths whose weights take their time either way (x 2,812,281 x 256, K = 3: 0.88).
+// and 1.06), at widths whose weights take their time either way (x 2,812,281 x 256, K = 3: 0.88); up to 3 rows of 768 dims for every
+// K, where one workgroup a row reads all its maxima (1 row x 2,812,281 x 768, K = 5: 740 against 706 us).
 static bool topk_by_lists(const TopkPlan& p, int64_t B, int64_t L, int64_t d, int64_t K) {
   if (L > TOPK_RANGE_MAX) return false;
   if (p.range < L) return (K >= 4 && B > 64 && B <= 512 ? 9 : 3) * p.range < L;
   if (B > 128 || d < 256) return false;
-  return K == 1 ? L > 1250000 : K <= 3 && L > 2000000 && d <= 768 && (K == 2 || d >= 512);
+  if (K == 1) return L > 1250000;
+  return L > 2000000 && d <= 768 && (K == 2 ? d >= 512 || B <= 64 : K == 3 ? d >= 512 : d > 512 && B <= 3);
 }
 // What the pass refuses to run without (lists of eight label groups), and what it runs fastest with.
 static size_t topk_least(int64_t B, int64_t K) { return (size_t)8 * B * K * 8 + (size_t)round_up(B, 4) * 4; }
