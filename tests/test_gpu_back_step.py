@@ -100,6 +100,7 @@ def test_what_the_two_calls_refuse_is_refused(dev):
     assert call(ldg=196) == 3                     # not a multiple of 8
     assert call(ldg=192) == 6                     # shorter than the labels
     assert call(nbytes=ws.numel() - 16) == 4      # less than 8 partial sums
+    assert call(m=0) == 1                         # no momentum
     assert call() == 0
 
 
@@ -126,6 +127,7 @@ def test_dx_is_as_close_to_float64_as_by_itself(dev, B, L, d):
                                  0.0, 0.9, 0.0, 1.0, ws.data_ptr(), ws.numel(), _st()), "xfc_dx_dw_update")
     error = [float((t.double() - want).norm() / want.norm()) for t in (one, two)]
     print(f"  {error[0]:.2e}, xfc_dx {error[1]:.2e}", flush=True)
+    assert not torch.equal(one, two)  # the joint pass has run, and not the two in its place
     assert error[0] <= 1.1 * error[1]
 
 

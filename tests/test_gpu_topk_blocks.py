@@ -114,3 +114,27 @@ def test_a_width_whose_fragments_exceed_32_bits_of_bytes(dev):
     v, i = _run(X, W, K)
     ev, ei = _expect(X[:, at.unique()], W[:, at.unique()], K)
     assert torch.equal(v, ev) and torch.equal(i, ei)
+
+
+# streamed past 16 and 32 rows, the main loop on 128 and 256; widths that end inside a k-step of 32 and a stage of 64
+@pytest.mark.parametrize("B,L,d", [(7, 4001, 72), (16, 20011, 768), (32, 5003, 200), (20, 9001, 1032), (40, 9001, 104), (128, 7001, 768),
+                                   (129, 5003, 136), (300, 9001, 776)])
+def test_the_second_look_has_the_bits_of_the_first(dev, B, L, d):
+    """What the K best blocks rest on: a row's best score, formed again, is the largest of the maxima to the last bit.  Operands whose
+    sums round; with K = 1 and room for all maxima these lie at the start of the workspace."""
+    g = torch.Generator().manual_seed(B + d)
+    X, W = torch.randn(B, d, generator=g).half().to(dev), torch.randn(L, d, generator=g).half().to(dev)
+    h = lib()
+    small = B <= 32 and -(-d // 32) * (1024 if B <= 16 else 2048) <= 160 * 1024
+    blocks = -(-L // 16) if small else -(-L // 256) * 8
+    ldb = -(-blocks // 4) * 4
+    nbytes = max(h.xfc_topk_workspace_bytes(B, L, 1), B * ldb * 4)
+    ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
+    v, i = torch.empty(B, 1, device=dev), torch.empty(B, 1, dtype=torch.int64, device=dev)
+    print(f"bits: B={B} L={L} d={d}", flush=True)
+    check(h.xfc_topk(X.data_ptr(), d, W.data_ptr(), d, B, L, d, L, 1, v.data_ptr(), i.data_ptr(), ws.data_ptr(), nbytes,
+                     torch.cuda.current_stream().cuda_stream), "xfc_topk")
+    maxima = ws.view(torch.float32)[:B * ldb].view(B, ldb)[:, :-(-L // (16 if small else 32))]
+    assert torch.equal(maxima.max(dim=1).values, v[:, 0])
+    z = X.double() @ W.double().t()
+    assert float((z.max(dim=1).values - v[:, 0].double()).abs().max()) <= 1e-5 * float(z.abs().max())
