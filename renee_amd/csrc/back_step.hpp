@@ -23,7 +23,7 @@
 //
 // Register layouts: those of small_step.hpp, i = lane % 16, g = lane / 16.
 #pragma once
-#include "pipe_core.hpp"
+#include "wave16.hpp"
 
 namespace xfc {
 
@@ -49,37 +49,16 @@ __device__ __forceinline__ T load(const T* p) {
 
 // up to 64 RQ rows; XR of the 2 RQ blocks of 32 rows of X^T in registers
 template <int RQ_, int XR_>
-struct BackStep {
+struct BackStep : Wave16 {
   static constexpr int RQ = RQ_, XR = XR_, NT = 512, ROWS = 64 * RQ, RP = 2 * RQ;
   static constexpr int G_HALVES = ROWS * BACK_TILE, W_HALVES = BACK_DIMS * BACK_TILE, X_HALVES = (RP - XR) * 32 * BACK_DIMS;
   static constexpr int LDS_BYTES = (X_HALVES + 2 * (G_HALVES + W_HALVES)) * 2;
   static constexpr int G_FETCH = ROWS / 64;  // fetch instructions (16 rows x 32 labels of G) of a wave per tile
   static_assert(LDS_BYTES <= 160 * 1024 && ROWS <= BACK_MAX_ROWS && XR <= RP, "budget");
-  static __device__ __forceinline__ void lds_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-  static __device__ __forceinline__ void barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-  // Transposing read of a [k][32] image: lane t of each 16 supplies 4 columns of row t / 4 and receives column t of 4 rows.
-  static __device__ __forceinline__ half8 read_tr(const half_t* base, int k, int col) {
-    const fp16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16((XFC_LDS fp16x4_t*)(base + k * 32 + col));
-    const fp16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16((XFC_LDS fp16x4_t*)(base + (k + 4) * 32 + col));
-    half8 f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { f[e] = (half_t)lo[e]; f[4 + e] = (half_t)hi[e]; }
-    return f;
-  }
-  static __device__ __forceinline__ float4v mfma(const half8& a, const half8& b, const float4v& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-  // v of the lane eight away in the row of sixteen
-  static __device__ __forceinline__ float4v across8(const float4v& v) {
-    float4v r;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) r[e] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v[e]), 0x128, 0xf, 0xf, true));  // row_ror:8
-    return r;
-  }
 };
 
-// NT: the arrays that are read and written (BACK_UPDATE: W and Mo, BACK_ADD: out) are loaded as what will not be wanted again,
-// for sizes that no cache holds until the next step.
+// NT: the arrays that are read and written (BACK_UPDATE: W and Mo, BACK_ADD: out; BACK_OUT has none) are loaded as what will not
+// be wanted again, for sizes that no cache holds until the next step.
 template <class S, int MODE, bool NT>
 __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
   constexpr int RQ = S::RQ, RP = S::RP, XR = S::XR;

@@ -3,10 +3,10 @@
 //
 // What bounds it.  The step's products are small (16 to 64 rows against each weight), its traffic is not: 8 bytes per
 // weight.  As three products the weights came from memory twice more, and each launch filled and drained the chip anew.
-// Whole steps, three passes -> one: 32 rows x 131,072 labels x 768 dims 245 -> 193 us (this kernel 172 to 188: 4.3 to 4.7 TB/s of
-// those 8 bytes); 32 x 400,001 x 768 753 -> 540 us; 8 x 40,001 x 128 96 -> 23 us; 64 x
-// 400,001 x 384 471 -> 307 us.  What is left: the weights' and the momentum's loads come in pieces of 64 bytes, and a
-// small label count is one tile to a workgroup, a chain of loads, z, the two barriers and the update (17 to 27 us).
+// Whole steps, three passes -> one: 32 rows x 131,072 labels x 768 dims 245 -> 193 us and with whole lines (LINES below) 171
+// (this kernel 166: 4.9 TB/s of those 8 bytes); 8 x 40,001 x 128 96 -> 23 us; 64 x 400,001 x 384 471 -> 307 us.  What is left:
+// where whole lines do not pay, the weights' and the momentum's loads come in pieces of 64 bytes, and a small label count is
+// one tile to a workgroup, a chain of loads, z, the two barriers and the update (17 to 27 us).
 //
 // Split.  A workgroup takes tiles of 32 labels; each of its NW waves owns D / NW of the dims of all of them, for all three
 // products, so that a weight is loaded by one lane, used from its registers for z and for the update, and stored by the
@@ -23,7 +23,7 @@
 //            8 g ..+7 of label 16 lb + i: those of the weights it holds
 //   dX       lane holds dims 4 g ..+3 of row 16 rb + i, accumulated over all tiles of the workgroup
 #pragma once
-#include "pipe_core.hpp"
+#include "wave16.hpp"
 
 namespace xfc {
 
@@ -49,7 +49,7 @@ struct SmallArgs {
 // half lines without the hint are faster, as the caches serve them: 64 x 20,011 x 512 33.0 against 34.5, 32 x 4,097 x 1024 24.8
 // against 28.1.
 template <int NW_, int SB_, int RB_, bool LINES_ = false>
-struct SmallStep {
+struct SmallStep : Wave16 {
   static constexpr int NW = NW_, SB = SB_, RB = RB_, P = RB / 2, NT = 64 * NW, D = NW * SB * 32;
   static constexpr int UNITS = 2 * RB;           // 16 x 16 blocks of z, each summed by one wave
   static constexpr bool SKIP = UNITS == NW;      // one block per wave: its own part need not go through the LDS
@@ -65,7 +65,7 @@ struct SmallStep {
   // dims a wave, the registers do not hold them beside the sums (40 to 60 spilled, 749 us instead of 618 at 64 rows x
   // 400,001 labels x 768): there the momentum's loads wait until z has left its registers, and the weights move to the LDS
   // after that and the next tile's are fetched in their place.  Spills that are left: 22 registers at 64 rows x 768, 5 at
-  // 32 x 128, 1 at 32 x 384.
+  // 32 x 128, 2 at 32 x 384.
   static constexpr bool AHEAD = RB == 2 && SB <= 3;
   static constexpr bool LINES = LINES_;
   static_assert(!LINES || SB % 2 == 0, "a line is two blocks of dims");
@@ -74,37 +74,6 @@ struct SmallStep {
   static_assert(LDS_BYTES <= 160 * 1024 && PER_CU >= 1, "LDS and register budget");
   static_assert(UNITS % NW == 0 || UNITS < NW, "blocks of z divide among the waves");
   static_assert(RB <= NW, "one wave stores 16 rows of G");
-
-  __device__ __forceinline__ static void barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-  __device__ __forceinline__ static void lds_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-  // Transposing read of a [k][32] image: lane t of each 16 supplies 4 columns of row t / 4 and receives column t of 4 rows.
-  __device__ __forceinline__ static half8 read_tr(const half_t* base, int k, int col) {
-    const fp16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4f16((XFC_LDS fp16x4_t*)(base + k * 32 + col));
-    const fp16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4f16((XFC_LDS fp16x4_t*)(base + (k + 4) * 32 + col));
-    half8 f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { f[e] = (half_t)lo[e]; f[4 + e] = (half_t)hi[e]; }
-    return f;
-  }
-  __device__ __forceinline__ static float4v mfma(const half8& a, const half8& b, const float4v& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-  // v (16 bytes) of the lane eight away in its row of sixteen; and one of two
-  template <class V>
-  __device__ __forceinline__ static V across8(const V& v) {
-    uint4v q = __builtin_bit_cast(uint4v, v);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) q[e] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)q[e], 0x128, 0xf, 0xf, true);  // row_ror:8
-    return __builtin_bit_cast(V, q);
-  }
-  template <class V>
-  __device__ __forceinline__ static V pick(bool first, const V& x, const V& y) {
-    uint4v p = __builtin_bit_cast(uint4v, x);
-    const uint4v q = __builtin_bit_cast(uint4v, y);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) p[e] = first ? p[e] : q[e];
-    return __builtin_bit_cast(V, p);
-  }
 };
 
 // 1 / (1 + 2^(-z log2 e)) with the bare v_exp_f32 / v_rcp_f32: the exponential may flush to zero or

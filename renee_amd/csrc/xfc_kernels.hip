@@ -1510,8 +1510,9 @@ int launch_dw(int mode, DwArgs a, hipStream_t st) {
 // The one-pass step of small batches (small_step.hpp).  Fn::operator()<S>() is called with the kernel for d dims and B
 // rows; false if there is none: these six widths are the ones that are built (each is two kernels; 64, 192, 320, 640 and
 // others would divide among waves in 32s too, and run as three passes), and 64 rows of 1024 dims with the waves' regions
-// exceed the LDS.  Wherever there is one it is the faster: 1.24 to 4.1 times over 8 to 64 rows and 4,097 to
-// 400,001 labels, least at 64 x 400,001 x 768 (768 -> 618 us).  384 dims and 64 rows take 12 waves of one block of dims:
+// exceed the LDS.  Wherever there is one it is the faster than three passes: 1.24 to 4.1 times over 8 to 64 rows and 4,097 to
+// 400,001 labels, least at 64 x 400,001 x 768 (768 -> 618 us); than G in one launch and the joint backward pass after it, but
+// for 33 to 64 rows of 768 dims while W and M stay in the caches (see small_step).  384 dims and 64 rows take 12 waves of one block of dims:
 // with 4 waves of three, 41 spills, 456 us at 64 x 400,001 instead of 307.
 // large: W and M are more than the caches hold beside the rest (small_step_large); whole lines pay there for these (8, 32 and
 // 64 rows x 90,001 to 2,000,003 labels: 1.02 to 1.10 times as fast with 768 dims, 0.98 to 1.08 with 1024, 1.02 to 1.15 with 512
@@ -1614,7 +1615,7 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
   *taken = back_step_for<MODE>(a.B, [&](auto s) {
     using S = decltype(s);
     const dim3 g((unsigned)(a.slices * a.ranges)), b(S::NT);
-    rc = nt ? launch_k<back_step_kernel<S, MODE, true>>(g, b, S::LDS_BYTES, st, a)
+    rc = nt ? launch_k<back_step_kernel<S, MODE, MODE != BACK_OUT>>(g, b, S::LDS_BYTES, st, a)
             : launch_k<back_step_kernel<S, MODE, false>>(g, b, S::LDS_BYTES, st, a);
     if (rc) return;
     launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges * a.parts, scale, 0.0f, st);
@@ -1736,7 +1737,7 @@ int xfc_init(void) {
     for (int64_t rows : {64, 128, 192, 256})
       back_step_for<MODE>(rows, [&](auto s) {
         using S = decltype(s);
-        keep(raise_lds_limit<back_step_kernel<S, MODE, true>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, MODE != BACK_OUT>>(S::LDS_BYTES));
         keep(raise_lds_limit<back_step_kernel<S, MODE, false>>(S::LDS_BYTES));
       });
   };
