@@ -40,6 +40,11 @@ __device__ __attribute__((aligned(16))) const uint32_t g_zero16[4] = {0u, 0u, 0u
 // Row of C held by accumulator register r of a 32x32 block, for this lane.
 __device__ __forceinline__ int c_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 
+// vmcnt.  gfx950 has one counter for a wave's vector-memory operations, and it counts them down in the order of their issue,
+// loads, fetches to the LDS and stores alike: "at most N outstanding" proves every operation done that has N or more behind it.
+// The compiler relies on the same (a load with two stores behind it is waited for with vmcnt(2)), and so do the counted waits
+// here and in back_step.hpp: operations that nobody counted, spills say, can only make them wait longer.
+//
 // Waits until at most N of this wave's vector-memory operations are outstanding, then joins the
 // workgroup barrier.  Written as one asm block: a plain __syncthreads() carries a fence that makes
 // the compiler drain every outstanding global->LDS fetch first, which would serialise the ring.
@@ -394,8 +399,8 @@ struct PipeCore {
         }
         const int n_slot = c_slot + 1 == STAGES ? 0 : c_slot + 1;
         // this wave's LDS reads of stage c are complete (lgkmcnt) and its share of stage c+1 has landed.
-        // After an epilogue the wave's stores share the counter with the fetches and may retire out of
-        // order with them, so the first wait after one drains everything.
+        // After an epilogue the wave's stores stand behind those fetches, as many as the tile's edges left, so
+        // the first wait after one drains everything (waiting for the certain ones only gained nothing).
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), in a form the compiler's own wait bookkeeping sees
         if (drain_all) { wait_lds_vmcnt_barrier<0>(); drain_all = false; }
         else wait_lds_vmcnt_barrier<(STAGES - 2) * LOADS_PER_STAGE>();

@@ -6,9 +6,10 @@
 // lies in one of the K best blocks, because every block ahead of its own holds a label ahead of it.  The second kernel's
 // scores are the first one's to the last bit (the same MFMAs in the same order), so a tie is a tie in both.
 //
-// What it replaced: lists of the K best kept per workgroup in the LDS beside a ring of two slots, a filter against shared
-// bounds in every tile's epilogue and exact retakes of the tiles that overflowed it, then a merge of the lists.  Here an
-// epilogue is one maximum per two scores, the ring keeps its third slot, and no tile depends on what came before.
+// What it replaced, but where these stay the faster (topk_lists.hpp): lists of the K best kept per workgroup in the LDS beside a
+// ring of two slots, a filter against shared bounds in every tile's epilogue and exact retakes of the tiles that overflowed it,
+// then a merge of the lists.  Here an epilogue is one maximum per two scores, the ring keeps its third slot, and no tile depends
+// on what came before.
 #pragma once
 #include "pipe_core.hpp"
 #include "wide_core.hpp"
@@ -69,7 +70,8 @@ struct ScoreArgs {
 };
 
 // ---------------------------------------------------------------------------------------------
-// more than SCORE_SMALL_ROWS rows: the forward pass's main loop, blocks of 32 labels
+// more than SCORE_SMALL_ROWS rows, or from the third on with weights that no cache holds: the forward pass's main loop, blocks
+// of 32 labels
 // ---------------------------------------------------------------------------------------------
 // Bound as the forward pass is, by the matrix pipes above 128 rows (1024 rows x 2,812,281 labels x 768: 3.75 ms, 1.18 PFLOP/s; the
 // whole call 4.27 -> 3.74 ms) and by the stream of weights on the 128-row tile (65 rows x 700,001 x 768: 195 us, 5.5 TB/s, the whole
@@ -139,7 +141,7 @@ __global__ void __launch_bounds__(C::NT) score_wide_kernel(ScoreArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// up to SCORE_SMALL_ROWS rows: the weights stream past the rows, blocks of 16 labels
+// up to SCORE_SMALL_ROWS rows of weights that the caches hold, two of any: the weights stream past the rows, blocks of 16 labels
 // ---------------------------------------------------------------------------------------------
 // Bound by the stream of weights.  X lies in the LDS as MFMA fragments, RB blocks of 16 rows; a wave takes units of 16
 // labels, loads them straight into the A side's registers (16 rows x 64 bytes an instruction) and keeps two to three

@@ -379,8 +379,8 @@ struct WideCore {
           if (k_left < BK) clear_tail(k_left);
         }
         // this wave's LDS reads of stage c are complete (lgkmcnt) and its share of stage c+1 has landed.
-        // After an epilogue the wave's stores share the counter with the fetches and may retire out of
-        // order with them, so the first wait after one drains everything.
+        // After an epilogue the wave's stores stand behind those fetches, as many as the tile's edges left, so
+        // the first wait after one drains everything (see pipe_core.hpp).
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), in a form the compiler's own wait bookkeeping sees
         if (drain_all) { wait_lds_vmcnt_barrier<0>(); drain_all = false; }
         else wait_lds_vmcnt_barrier<A_CH>();

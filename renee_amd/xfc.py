@@ -297,7 +297,7 @@ class XFCLayer:
     def topk(self, embed: torch.Tensor, K: int = 5, numy: int | None = None, overwrite_g: bool = False):
         """Exact top-K labels per row over all labels (FullPredictor's scoring loop, dl_base.py:736-756,
         with the pad clamp of :782 when numy < the stored label count).  Returns (values fp32, indices
-        int64), each (batch, K); ties go to the lower label id.  K <= 8192: up to 8 in one fused pass,
+        int64), each (batch, K); ties go to the lower label id.  K <= 8192: up to 8 without writing the logits,
         above that (the final evaluation's K = 100, dl_base.py:817-818; torch.topk at :756) by an exact
         selection over the fp16 logits, which are written to `outsoft` as the reference's scorer does
         (dl_base.py:745).
