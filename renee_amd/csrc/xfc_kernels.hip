@@ -2072,9 +2072,15 @@ int xfc_dx_dw(const void* G, int64_t ldg, const void* X, int64_t ldx, const void
   // second reading of G: on long axes it is the slower from 129 rows on where its slices do not come out even with the CUs (768
   // dims, six of them on 240: 192 rows x 1,500,001 1.58 against 1.69 ms, 256 rows 1.77 against 1.98; 1024 dims, all CUs: 192 x
   // 700,001 1.04 against 1.00).
-  const bool sizes = dims_ok(B) && dims_ok(L) && dims_ok(d) && d > 0, whole = sizes && d % 256 == 0;
-  const bool even = sizes && (num_cus() / 8) % ceil_div(d, BACK_DIMS) == 0;
-  const bool slow = whole && ((B <= 64 && L * d * 4 > (int64_t)128 << 20) || (beta == 0.f && B > 128 && !even && L * d > (int64_t)400 << 20));
+  // 33 to 128 rows of 256 to 512 dims have a stretch of middle sizes, whose gradient and weights the Infinity Cache holds between
+  // two passes, where these write a first gradient the faster (whole steps, joint pass over two: 33 to 64 rows 1.07 to 1.09 x
+  // 384 dims x 131,072 labels, 1.05 x 512 x 60,007, 1.04 x 256 x 131,072; 100 rows 1.03 to 1.05 x 512, 0.97 to 1.01 x 384).
+  // Adding to a gradient has none: two passes 7 to 15 % the slower x 40,007 x 384 and 512, the same up to 131,072.
+  const bool sizes = dims_ok(B) && dims_ok(L) && dims_ok(d) && d > 0;
+  const int64_t weights = sizes ? L * d : 0, Mi = (int64_t)1 << 20;
+  const bool whole = sizes && d % 256 == 0, even = sizes && (num_cus() / 8) % ceil_div(d, BACK_DIMS) == 0;
+  const bool middle = beta == 0.f && B > 32 && B <= (d < 384 ? 64 : 128) && d >= 256 && d <= 512 && weights > 20 * Mi && weights <= 52 * Mi;
+  const bool slow = middle || (whole && ((B <= 64 && weights > 32 * Mi) || (beta == 0.f && B > 128 && !even && weights > 400 * Mi)));
   if (!slow && back_ok(G, ldg, X, ldx, W, ldw, dX, B, L, d) && grad && ld_grad % 4 == 0 && aligned16(grad)) {
     BackArgs a = back_args(G, ldg, X, ldx, W, ldw, B, L, d);
     a.out = grad; a.ldo = ld_grad; a.beta = beta;

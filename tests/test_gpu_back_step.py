@@ -131,9 +131,10 @@ def test_dx_is_as_close_to_float64_as_by_itself(dev, B, L, d):
     assert error[0] <= 1.1 * error[1]
 
 
-def test_a_first_gradient_on_a_long_axis_takes_two_passes(dev):
-    """129 to 256 rows, 768 dims, a gradient that is only written: the two passes, which are faster there, to the last bit."""
-    B, L, d = 192, 560007, 768
+@pytest.mark.parametrize("B,L,d", [(192, 560007, 768), (100, 131072, 384), (48, 60007, 512)])
+def test_gradients_that_take_two_passes(dev, B, L, d):
+    """129 to 256 rows of 768 dims on a long axis and 33 to 128 of middle sizes: the two passes, which are faster there, to the
+    last bit."""
     g = torch.Generator(device=dev)
     g.manual_seed(3)
     G = torch.zeros(B, (L + 7) // 8 * 8, dtype=torch.float16, device=dev)
