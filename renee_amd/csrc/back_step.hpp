@@ -2,9 +2,10 @@
 // before the update, and dW = G^T.X, which is written out or consumed by the momentum update of those weights.
 //
 // What bounds it.  With so few rows the products are small beside the traffic; as two kernels the weights and G were read
-// twice.  dX and the update of 199 rows x 131,072 labels x 768 dims, reduction included: 239 -> 202 us (256 rows 249 -> 223, 128
-// rows 203 -> 183: 5.0 TB/s of the 8 bytes per weight and G); without its stores the pass took 150 at 199 and 256 rows, the LDS
-// reads and their latency between two barriers.  Whole steps of 65 to 256 rows x 4,001 to 2,812,281 labels x 64 to 1024 dims: 1.03
+// twice.  dX and the update of 199 rows x 131,072 labels x 768 dims, reduction included: 239 -> 199 us (256 rows 248 -> 220, 128
+// rows 202 -> 183: 5.0 TB/s of the 8 bytes per weight and G); without its stores the pass took 150 at 199 and 256 rows, the LDS
+// reads and their latency between two barriers.  Above 192 rows the sums of one tile that dX is made from (one rounding each into
+// the running sum) take the registers of half of X^T: 211 -> 220 us at 256 rows, dX as close to float64 as xfc_dx's.  Whole steps of 65 to 256 rows x 4,001 to 2,812,281 labels x 64 to 1024 dims: 1.03
 // to 1.5 times as fast.
 //
 // Split.  A workgroup owns a slice of 128 dims and a range of labels, which it walks 64 at a time.  Its eight waves are two
