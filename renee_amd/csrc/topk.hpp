@@ -80,7 +80,7 @@ struct ScoreArgs {
 constexpr int SCORE_WIDE_BLOCK = 32;
 
 using ScoreWide = WideCore<256, 256, 2, 2, true>;
-using ScoreWide128 = WideCore<256, 128, 2, 2, true>;
+using ScoreWide128 = WideCore<256, 128, 2, 2, true, true>;
 
 template <class C>
 __global__ void __launch_bounds__(C::NT) score_wide_kernel(ScoreArgs a) {

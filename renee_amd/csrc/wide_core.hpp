@@ -33,6 +33,12 @@
 namespace xfc {
 
 // address = uniform 64-bit base + per-lane 32-bit offset; LDS address = uniform lds + the constant at
+// SPILLED: the base may have been in a vector register's lane (scalar registers are spilled there).  Five instructions must stand
+// between the v_readlane_b32 that brings it back and a vector-memory instruction that reads it, and the compiler does not see that
+// there is one in the asm; a scalar move waits by itself, so the base goes through one.  (It stands where M0 wants one instruction
+// before the fetch anyway, but the two registers cost the 1024-row top-K pass, which spills none of them, 1.2 %.  tests/test_host.py
+// looks the built kernels over.)
+template <bool NT = false, bool SPILLED = false>
 __device__ __forceinline__ void wide_load16(int64_t ubase, uint32_t voff, uint32_t lds, int at) {
   // an integer operand whose halves are marked uniform: the "s" constraint alone is not always honoured
   const uint64_t b0 = (uint64_t)ubase;
@@ -41,7 +47,17 @@ __device__ __forceinline__ void wide_load16(int64_t ubase, uint32_t voff, uint32
   const uint32_t b_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b0);
   const uint64_t b = ((uint64_t)b_hi << 32) | (uint64_t)b_lo;
   const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds);
-  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m), "v"(voff), "s"(b), "n"(at) : "memory", "m0", "scc");
+  if constexpr (SPILLED) {
+    uint64_t t;
+    if constexpr (NT)
+      asm volatile("s_add_u32 m0, %1, %4\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0 nt" : "=&s"(t) : "s"(m), "v"(voff), "s"(b), "n"(at) : "memory", "m0", "scc");
+    else
+      asm volatile("s_add_u32 m0, %1, %4\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(t) : "s"(m), "v"(voff), "s"(b), "n"(at) : "memory", "m0", "scc");
+  } else if constexpr (NT) {
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(m), "v"(voff), "s"(b), "n"(at) : "memory", "m0", "scc");
+  } else {
+    asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m), "v"(voff), "s"(b), "n"(at) : "memory", "m0", "scc");
+  }
 }
 
 // Swizzles: the 16 lanes (b128) or 32 lanes (b64) the LDS serves at a time must spread over all 64 banks.
@@ -53,10 +69,11 @@ __device__ __forceinline__ int wide_mc_swz(int k) { return ((k & 3) << 1) | (((k
 
 // The A side comes from HBM: its ring has three slots, and it is fetched half a stage earlier than the B side, whose
 // ring has two.  The B side is K-contiguous.
-template <int BM_, int BN_, int WM_, int WN_, bool A_KC_>
+// SPILLED_: some of the fetches' addresses are spilled (see wide_load16).
+template <int BM_, int BN_, int WM_, int WN_, bool A_KC_, bool SPILLED_ = false>
 struct WideCore {
   static constexpr int BM = BM_, BN = BN_, BK = 64, WM = WM_, WN = WN_;
-  static constexpr bool A_KC = A_KC_;
+  static constexpr bool A_KC = A_KC_, SPILLED = SPILLED_;
   static constexpr int NW = WM * WN, NT = 64 * NW;
   static constexpr int TM = BM / WM, TN = BN / WN;   // a wave's tile
   static constexpr int FM = TM / 16, FN = TN / 16;   // in 16 x 16 blocks
@@ -157,7 +174,7 @@ struct WideCore {
       for (int i = 0; i < CH; ++i)
         if (piece_k(i, wave, lane) >= n) *reinterpret_cast<uint4v*>(region + (i * NW + wave) * 512 + lane * 8) = uint4v{0u, 0u, 0u, 0u};
     }
-    __device__ __forceinline__ void issue(int i, uint32_t wave_region) const { wide_load16(at[i], voff[i], wave_region, i * NW * 1024); }
+    __device__ __forceinline__ void issue(int i, uint32_t wave_region) const { wide_load16<false, SPILLED>(at[i], voff[i], wave_region, i * NW * 1024); }
     __device__ __forceinline__ void bump(int i) { at[i] += kstep; }
   };
   // A fill cursor: the stage of the work list an operand's next fetches belong to.

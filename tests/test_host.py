@@ -218,7 +218,6 @@ def test_empty_batch_is_accepted_without_touching_the_device():
 # before every wave is past its last read of the stage it held.
 # ---------------------------------------------------------------------------------------------------
 def _pipecore_instantiations():
-    import re
 
     src = open(os.path.join(ROOT, "renee_amd", "csrc", "xfc_kernels.hip")).read()
     found = {}
@@ -338,3 +337,55 @@ def test_layer_workspace_covers_every_batch_size_up_to_max_batch():
     assert saw_non_monotone  # the case this function exists for does occur in the sweep
     # K below 8 never needs more than K = 8
     assert h.xfc_topk_workspace_bytes(256, 70001, 5) <= h.xfc_layer_workspace_bytes(300, 70001, 16, 64 * 300)
+
+
+def test_built_kernels_keep_the_distance_from_a_vector_write_of_a_scalar_register_to_its_use_as_an_address():
+    """Five instructions must stand between a vector instruction that writes a scalar register (the compiler's v_readlane_b32 of a
+    spilled one) and a vector-memory instruction that reads it; the compiler keeps that distance for its own instructions but
+    does not see those in inline asm.  (In the 128-row top-K kernel global_load_lds_dwordx4 v98, s[4:5] stood three behind
+    v_readlane_b32 s5.)  The built library's code is looked over, straight on through its branches."""
+    import shutil
+    import subprocess
+
+    from renee_amd.build import LIB_PATH
+
+    objdump = shutil.which("llvm-objdump", path="/opt/rocm/llvm/bin:/opt/rocm/lib/llvm/bin:" + os.environ.get("PATH", ""))
+    bundler = shutil.which("clang-offload-bundler", path="/opt/rocm/llvm/bin:/opt/rocm/lib/llvm/bin:" + os.environ.get("PATH", ""))
+    if not objdump or not bundler:
+        pytest.skip("no disassembler")
+    import tempfile
+
+    with tempfile.TemporaryDirectory() as tmp:
+        fat, code = os.path.join(tmp, "fat"), os.path.join(tmp, "code")
+        subprocess.run([objdump.replace("objdump", "objcopy"), f"--dump-section=.hip_fatbin={fat}", LIB_PATH, os.path.join(tmp, "copy")], check=True)
+        subprocess.run([bundler, "--unbundle", "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--input={fat}", f"--output={code}"],
+                       check=True)
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", "--no-leading-addr", code], check=True, stdout=subprocess.PIPE, text=True).stdout
+
+    def scalars(operands):
+        out = set()
+        for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", operands):
+            out |= set(range(int(lo), int(hi) + 1))
+        return out | {int(n) for n in re.findall(r"\bs(\d+)\b", operands)}
+
+    kernels = accesses = 0
+    kernel, recent = "", []  # the scalar registers that vector instructions wrote, instruction by instruction
+    for line in text.splitlines():
+        if line.endswith(">:"):
+            kernel, recent = line, []
+            kernels += 1
+            continue
+        line = line.split("//")[0].strip()
+        if not line:
+            continue
+        op, _, operands = line.partition(" ")
+        if re.match(r"(global|flat|scratch|buffer)_", op):
+            accesses += 1
+            close = set().union(*recent[-5:]) if recent else set()
+            assert not close & scalars(operands), (kernel, line)
+        if op == "s_nop":
+            recent += [set()] * (int(operands, 0) + 1)
+        else:
+            recent.append(scalars(operands.split(",")[0]) if op.startswith("v_") else set())
+        recent = recent[-8:]
+    assert kernels > 50 and accesses > 10000
