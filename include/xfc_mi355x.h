@@ -190,9 +190,9 @@ int xfc_sgd_momentum_master(float* W32, float* M32, void* W16, const float* grad
 
 /*
  * xfc_dx followed by xfc_dw_update (dW accumulated: by xfc_dw), with the same arguments and results: dX is formed
- * from the weights before the update.  Batches of up to 256 rows take one pass over the labels, which reads W and
- * G once, where it is the faster and the workspace holds its partial sums; the others, and every call that the two would refuse, run as
- * the two.  Workspace: what xfc_dx takes; xfc_step_workspace_bytes() and xfc_layer_workspace_bytes() cover the one pass.
+ * from the weights before the update.  Batches of up to 256 rows, and of up to 512 with the update, widths that are
+ * multiples of 128 and ldm = ldw, take one pass over the labels, which reads W and G once, where it is the faster and the
+ * workspace holds its partial sums; the others, and every call that the two would refuse, run as the two.  Workspace: what xfc_dx takes; xfc_step_workspace_bytes() and xfc_layer_workspace_bytes() cover the one pass.
  */
 int xfc_dx_dw_update(const void* G, int64_t ldg, const void* X, int64_t ldx, void* W, int64_t ldw,
                      void* M, int64_t ldm, float* dX, int64_t lddx, int64_t B, int64_t L, int64_t d,

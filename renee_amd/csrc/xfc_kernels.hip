@@ -14,6 +14,7 @@
 
 #include "../../include/xfc_mi355x.h"
 #include "back_step.hpp"
+#include "back_wide.hpp"
 #include "pipe_core.hpp"
 #include "small_step.hpp"
 #include "topk.hpp"
@@ -1593,9 +1594,33 @@ BackPlan back_plan(int64_t B, int64_t L, int64_t d, size_t ws_limit) {
   while (parts > 1 && (size_t)(ranges * parts) * one > ws_limit) --parts;
   return {(int)ranges, (int)parts};
 }
+// The same for more rows (back_wide.hpp), the update only and widths of whole slices: there it is the faster at every size measured
+// (whole steps of 257 to 512 rows x 4,097 to 2,812,281 labels x 128 to 1024 dims: 1.11 to 1.41 times, least at 260 x 131,073 x 768,
+// most at 300 x 1,310,720 x 128; the two passes read the weights and G twice).  With 193 to 256 rows the kernel above is (131,073
+// x 768: 303 us by that one, 306 by this).
+template <class Fn>
+bool back_wide_for(int64_t B, int64_t d, Fn&& fn) {
+  if (B <= BACK_MAX_ROWS || B > BACK_WIDE_ROWS || d % BACK_DIMS) return false;
+  if (B <= 320) fn(BackWide<5>{});
+  else if (B <= 384) fn(BackWide<6>{});
+  else if (B <= 448) fn(BackWide<7>{});
+  else fn(BackWide<8>{});
+  return true;
+}
+// A workgroup per CU.  Parts as above, but a tile's labels are part of the chain of MFMAs, as in xfc_dx: as many chains as that has,
+// less an eighth of the ranges, since these come out a little closer to float64 than as many of xfc_dx's (512 rows x 131,072 x 768:
+// 42 chains 3.7e-7, xfc_dx's 40 3.9e-7).
+BackPlan back_wide_plan(int64_t B, int64_t L, int64_t d) {
+  const int64_t slices = d / BACK_DIMS, per = num_cus() / slices, tiles = ceil_div(L, BACK_TILE);
+  const int64_t ranges = per < 1 ? 1 : per < tiles ? per : tiles;
+  int tiles_m, tiles_n, sums, k_per_split;
+  dx_plan((int)B, (int)d, (int)L, tiles_m, tiles_n, sums, k_per_split);
+  const int64_t parts = ceil_div(sums - ranges / 8, ranges);
+  return {(int)ranges, (int)(parts > 1 ? parts : 1)};
+}
 size_t back_ws_bytes(int64_t B, int64_t L, int64_t d) {
-  if (B < 1 || B > BACK_MAX_ROWS || L < 1 || d < 1) return 0;
-  const BackPlan p = back_plan(B, L, d, ~(size_t)0);
+  if (B < 1 || B > BACK_WIDE_ROWS || L < 1 || d < 1 || (B > BACK_MAX_ROWS && d % BACK_DIMS)) return 0;
+  const BackPlan p = B > BACK_MAX_ROWS ? back_wide_plan(B, L, d) : back_plan(B, L, d, ~(size_t)0);
   return (size_t)p.ranges * (size_t)p.parts * (size_t)B * (size_t)d * 4;
 }
 template <int MODE>
@@ -1617,6 +1642,36 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
     const dim3 g((unsigned)(a.slices * a.ranges)), b(S::NT);
     rc = nt ? launch_k<back_step_kernel<S, MODE, MODE != BACK_OUT>>(g, b, S::LDS_BYTES, st, a)
             : launch_k<back_step_kernel<S, MODE, false>>(g, b, S::LDS_BYTES, st, a);
+    if (rc) return;
+    launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges * a.parts, scale, 0.0f, st);
+    rc = check_launch();
+  });
+  return rc;
+}
+
+int launch_back_wide(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size_t ws_bytes, hipStream_t st, bool* taken) {
+  *taken = false;
+  if (a.ldm != a.ldw || a.ldw >= (int64_t)1 << 27 || !ws || !aligned16(ws) || back_ws_bytes(a.B, a.L, a.d) > ws_bytes) return XFC_OK;
+  int rc = XFC_OK;
+  *taken = back_wide_for(a.B, a.d, [&](auto s) {
+    using S = decltype(s);
+    const BackPlan p = back_wide_plan(a.B, a.L, a.d);
+    a.ranges = p.ranges;
+    a.parts = p.parts;
+    a.slices = a.d / BACK_DIMS;
+    a.tiles = ceil_div(a.L, BACK_TILE);
+    a.part = reinterpret_cast<float*>(ws);
+    const dim3 g((unsigned)round_up(a.slices * a.ranges, 8)), b(S::NT);
+    // Non-temporal loads where weights, momentum and G are more than the Infinity Cache holds (whole steps, without and with: 300
+    // rows x 60,001 labels x 768 dims 147 and 152 us, 512 rows 184 and 182, 512 x 131,072 x 256 167 and 158).  Non-temporal stores
+    // as well where the weights and the momentum are up to about twice that, and G less than half of it: they leave the cache to
+    // the weights that the next forward pass reads (512 x 131,073 x 768 383 -> 366 us, 90,001 263 -> 253, 180,001 the same,
+    // 1,310,720 3277 -> 3370; 512 x 300,001 x 256 354 -> 366).
+    const int64_t state = (int64_t)a.L * a.d * 4, Mi = (int64_t)1 << 20;
+    const bool loads = state + (int64_t)a.L * a.B * 2 > 224 * Mi, stores = state > 224 * Mi && state <= 560 * Mi && a.B <= a.d;
+    rc = stores ? launch_k<back_wide_kernel<S, true, true>>(g, b, S::LDS_BYTES, st, a)
+         : loads ? launch_k<back_wide_kernel<S, true, false>>(g, b, S::LDS_BYTES, st, a)
+                 : launch_k<back_wide_kernel<S, false, false>>(g, b, S::LDS_BYTES, st, a);
     if (rc) return;
     launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges * a.parts, scale, 0.0f, st);
     rc = check_launch();
@@ -1741,6 +1796,13 @@ int xfc_init(void) {
         keep(raise_lds_limit<back_step_kernel<S, MODE, false>>(S::LDS_BYTES));
       });
   };
+  for (int64_t rows : {320, 384, 448, 512})
+    back_wide_for(rows, BACK_DIMS, [&](auto s) {
+      using S = decltype(s);
+      keep(raise_lds_limit<back_wide_kernel<S, false, false>>(S::LDS_BYTES));
+      keep(raise_lds_limit<back_wide_kernel<S, true, false>>(S::LDS_BYTES));
+      keep(raise_lds_limit<back_wide_kernel<S, true, true>>(S::LDS_BYTES));
+    });
   back_limits(std::integral_constant<int, BACK_UPDATE>{});
   back_limits(std::integral_constant<int, BACK_OUT>{});
   back_limits(std::integral_constant<int, BACK_ADD>{});
@@ -2035,8 +2097,8 @@ int xfc_sgd_momentum(void* W, void* Mo, const float* grad, int64_t count, float 
 
 // Both gradients of a batch; what the one pass does not take runs as two, which also report what is wrong with a call.
 static bool back_ok(const void* G, int64_t ldg, const void* X, int64_t ldx, const void* W, int64_t ldw, const void* dX, int64_t B,
-                    int64_t L, int64_t d) {
-  return dims_ok(B) && dims_ok(L) && dims_ok(d) && B >= 1 && B <= BACK_MAX_ROWS && L >= 1 && d >= 8 && G && X && W && dX &&
+                    int64_t L, int64_t d, int64_t rows = BACK_MAX_ROWS) {
+  return dims_ok(B) && dims_ok(L) && dims_ok(d) && B >= 1 && B <= rows && L >= 1 && d >= 8 && G && X && W && dX &&
          ldg % 8 == 0 && ldg < (int64_t)1 << 27 && ldx % 8 == 0 && ldw % 8 == 0 && d % 8 == 0 && aligned16(G) && aligned16(X) && aligned16(W) &&
          ldg >= round_up(L, 8);
 }
@@ -2051,11 +2113,13 @@ static BackArgs back_args(const void* G, int64_t ldg, const void* X, int64_t ldx
 int xfc_dx_dw_update(const void* G, int64_t ldg, const void* X, int64_t ldx, void* W, int64_t ldw, void* Mo, int64_t ldm, float* dX,
                      int64_t lddx, int64_t B, int64_t L, int64_t d, float lr, float momentum, float weight_decay, float scale,
                      void* workspace, size_t workspace_bytes, void* stream) {
-  if (back_ok(G, ldg, X, ldx, W, ldw, dX, B, L, d) && Mo && ldm % 8 == 0 && aligned16(Mo)) {
+  if (back_ok(G, ldg, X, ldx, W, ldw, dX, B, L, d, BACK_WIDE_ROWS) && Mo && ldm % 8 == 0 && aligned16(Mo)) {
     BackArgs a = back_args(G, ldg, X, ldx, W, ldw, B, L, d);
     a.Mo = (half_t*)Mo; a.ldm = ldm; a.lr = lr; a.mu = momentum; a.wd = weight_decay;
     bool taken;
-    const int rc = launch_back<BACK_UPDATE>(a, dX, lddx, scale, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream), &taken);
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    const int rc = B > BACK_MAX_ROWS ? launch_back_wide(a, dX, lddx, scale, workspace, workspace_bytes, st, &taken)
+                                     : launch_back<BACK_UPDATE>(a, dX, lddx, scale, workspace, workspace_bytes, st, &taken);
     if (taken) return rc;
   }
   const int rc = xfc_dx(G, ldg, W, ldw, dX, lddx, B, L, d, scale, workspace, workspace_bytes, stream);

@@ -429,8 +429,8 @@ class XFCLayer:
 
     def backward_pass(self, embed, grad_input: torch.Tensor | None = None, scale: float = 1.0, accumulate: bool = False,
                       lr: float | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
-        """dx, then dw_update (accumulate: dw_accumulate), through one entry point: small batches take one
-        pass over the labels for both (dl_base.py:602-634)."""
+        """dx, then dw_update (accumulate: dw_accumulate), through one entry point: batches of up to 512
+        rows take one pass over the labels for both (dl_base.py:602-634)."""
         if self.master_weights and not accumulate:
             gi = self.dx(embed.shape[0], grad_input, scale, out)
             self.dw_update(embed, lr=lr, out=out)

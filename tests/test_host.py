@@ -339,11 +339,12 @@ def test_layer_workspace_covers_every_batch_size_up_to_max_batch():
     assert h.xfc_topk_workspace_bytes(256, 70001, 5) <= h.xfc_layer_workspace_bytes(300, 70001, 16, 64 * 300)
 
 
-def test_built_kernels_keep_the_distance_from_a_vector_write_of_a_scalar_register_to_its_use_as_an_address():
+def test_built_kernels_keep_the_distances_that_the_compiler_does_not_see_in_inline_asm():
     """Five instructions must stand between a vector instruction that writes a scalar register (the compiler's v_readlane_b32 of a
     spilled one) and a vector-memory instruction that reads it; the compiler keeps that distance for its own instructions but
     does not see those in inline asm.  (In the 128-row top-K kernel global_load_lds_dwordx4 v98, s[4:5] stood three behind
-    v_readlane_b32 s5.)  The built library's code is looked over, straight on through its branches."""
+    v_readlane_b32 s5.)  Likewise two between a vector instruction and an MFMA that reads what it wrote (v_accvgpr_read_b32 of a fragment
+that did not fit the ordinary registers).  The built library's code is looked over, straight on through its branches."""
     import shutil
     import subprocess
 
@@ -362,17 +363,23 @@ def test_built_kernels_keep_the_distance_from_a_vector_write_of_a_scalar_registe
                        check=True)
         text = subprocess.run([objdump, "-d", "--no-show-raw-insn", "--no-leading-addr", code], check=True, stdout=subprocess.PIPE, text=True).stdout
 
+    def vectors(operands):
+        out = set()
+        for kind, lo, hi in re.findall(r"\b([va])\[(\d+):(\d+)\]", operands):
+            out |= {(kind, n) for n in range(int(lo), int(hi) + 1)}
+        return out | {(kind, int(n)) for kind, n in re.findall(r"\b([va])(\d+)\b", operands)}
+
     def scalars(operands):
         out = set()
         for lo, hi in re.findall(r"\bs\[(\d+):(\d+)\]", operands):
             out |= set(range(int(lo), int(hi) + 1))
         return out | {int(n) for n in re.findall(r"\bs(\d+)\b", operands)}
 
-    kernels = accesses = 0
-    kernel, recent = "", []  # the scalar registers that vector instructions wrote, instruction by instruction
+    kernels = accesses = products = 0
+    kernel, recent, wrote = "", [], []  # the scalar and the vector registers that vector instructions wrote, instruction by instruction
     for line in text.splitlines():
         if line.endswith(">:"):
-            kernel, recent = line, []
+            kernel, recent, wrote = line, [], []
             kernels += 1
             continue
         line = line.split("//")[0].strip()
@@ -383,9 +390,16 @@ def test_built_kernels_keep_the_distance_from_a_vector_write_of_a_scalar_registe
             accesses += 1
             close = set().union(*recent[-5:]) if recent else set()
             assert not close & scalars(operands), (kernel, line)
+        if op.startswith("v_mfma"):
+            products += 1
+            close = set().union(*wrote[-2:]) if wrote else set()
+            assert not close & vectors(operands.partition(",")[2]), (kernel, line)
+        plain = op.startswith("v_") and not op.startswith("v_mfma")
         if op == "s_nop":
             recent += [set()] * (int(operands, 0) + 1)
+            wrote += [set()] * (int(operands, 0) + 1)
         else:
-            recent.append(scalars(operands.split(",")[0]) if op.startswith("v_") else set())
-        recent = recent[-8:]
-    assert kernels > 50 and accesses > 10000
+            recent.append(scalars(operands.split(",")[0]) if plain else set())
+            wrote.append(vectors(operands.split(",")[0]) if plain else set())
+        recent, wrote = recent[-8:], wrote[-4:]
+    assert kernels > 50 and accesses > 10000 and products > 4000
