@@ -23,6 +23,10 @@
 //   branches around fetches between MFMAs cost 15 % of a product that runs from the L2, fetch addresses made of a base and
 //   two offsets (five scalar instructions a fetch) 6 % of dX, the third slot for the operand from HBM 9 % of the forward
 //   pass (1.31 -> 1.19 ms), a fill cursor with a byte of state per slot 4 % of both.
+// Then: what a stage does once (the turns of the rings, counts, the bumps, which the compiler had moved there) out of the gap
+// between the sub-steps and behind their last bumps, tile to tile addresses by one difference, and an epilogue's stores counted
+// instead of waited for: forward pass 1.055 -> 1.030 ms, dX 0.880 -> 0.865, top-5 of 1024 x 2,812,281 3.70 -> 3.65 ms, the logits of
+// top-100 at 512 x 1,310,720 1.113 -> 1.083.
 // Eight waves of 128 x 64 run no faster (1359 against 1360 TFLOP/s at 8192^3), read half again as many LDS bytes, and
 // leave 128 registers for everything that is not an accumulator.
 #pragma once
@@ -108,6 +112,19 @@ struct WideCore {
     int r0, rmax;
   };
 
+  // A uniform value that is to be made here and not where it is used.
+  __device__ __forceinline__ static void pin(int& v) {
+    v = __builtin_amdgcn_readfirstlane(v);
+    asm volatile("" : "+s"(v));
+  }
+  __device__ __forceinline__ static void pin(uint32_t& v) {
+    v = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+    asm volatile("" : "+s"(v));
+  }
+  __device__ __forceinline__ static void pin(int64_t& v) {
+    v = uniform64(v);
+    asm volatile("" : "+s"(v));
+  }
   // Addresses of the CH 16-byte pieces a thread fetches for one operand each stage.  Every fetch is
   // "uniform 64-bit address + per-thread 32-bit offset": the base advances along k with scalar adds, so a
   // steady-state stage costs no vector ALU work.
@@ -175,7 +192,10 @@ struct WideCore {
         if (piece_k(i, wave, lane) >= n) *reinterpret_cast<uint4v*>(region + (i * NW + wave) * 512 + lane * 8) = uint4v{0u, 0u, 0u, 0u};
     }
     __device__ __forceinline__ void issue(int i, uint32_t wave_region) const { wide_load16<false, SPILLED>(at[i], voff[i], wave_region, i * NW * 1024); }
-    __device__ __forceinline__ void bump(int i) { at[i] += kstep; }
+    __device__ __forceinline__ void bump(int i) {
+      at[i] += kstep;
+      pin(at[i]);
+    }
   };
   // A fill cursor: the stage of the work list an operand's next fetches belong to.
   template <bool IS_A>
@@ -186,25 +206,43 @@ struct WideCore {
     uint32_t ring, dst;  // LDS address of this wave's first piece in slot 0 and in the stage's slot
     int item, k_left;    // k of the item from this stage on
     int64_t ld;
+    int64_t end = 0;     // where the item's tile starts, moved on by its stages; 0: its addresses do not lead to the next one's
     template <class GetItem>
     __device__ __forceinline__ void open(GetItem& get, int wave, int lane) {
       Operand o[2];
       int kb, ke;
       get(item, o[0], o[1], kb, ke);
       const Operand& me = o[IS_A ? 0 : 1];
-      load.init(me, kb, wave, lane);
+      constexpr bool KC = IS_A ? A_KC : true;
+      // From one tile that lies inside the operand to another all addresses move by the same (made anew they are 150
+      // instructions between two stages).
+      const bool inside = me.r0 + (IS_A ? BM : BN) <= me.rmax && (ke - kb) % BK == 0;
+      const int64_t start = uniform64(reinterpret_cast<int64_t>(me.p) + (KC ? me.r0 * me.ld + kb : kb * me.ld + me.r0) * 2);
+      if (inside && end != 0) {
+        const int64_t by = uniform64(start - end);
+#pragma unroll
+        for (int i = 0; i < CH; ++i) load.at[i] += by;
+      } else {
+        load.init(me, kb, wave, lane);
+      }
+      end = inside ? uniform64(start + (ke - kb) / BK * load.kstep) : 0;
       ld = me.ld;
       k_left = ke - kb;
       if (k_left < BK) load.retarget(k_left, ld, wave, lane);
     }
     __device__ __forceinline__ void piece(int i) const { load.issue(i, dst); }
     __device__ __forceinline__ void bump(int i) { load.bump(i); }
-    // To the next stage, whose addresses bump() has made.  Past the last one the cursor stays: later fetches repeat it,
-    // nobody reads the copies, and the count of outstanding fetches per stage stays what the waits assume.
-    template <class GetItem>
-    __device__ __forceinline__ void advance(GetItem& get, int item_end, int wave, int lane) {
+    // To the next stage, whose addresses bump() has made: what every stage has, for a place among the MFMAs (and pinned there), and
+    // what the end of an item needs.  Past the last one the cursor stays: later fetches repeat it, nobody reads the copies, and
+    // the count of outstanding fetches per stage stays what the waits assume.
+    __device__ __forceinline__ void step() {
       dst = dst == ring + (SLOTS - 1) * BYTES ? ring : dst + BYTES;
       k_left -= BK;
+      pin(dst);
+      pin(k_left);
+    }
+    template <class GetItem>
+    __device__ __forceinline__ void turn(GetItem& get, int item_end, int wave, int lane) {
       if (k_left < BK) {
         if (k_left > 0) {
           load.retarget(k_left, ld, wave, lane);
@@ -297,15 +335,16 @@ struct WideCore {
   //   get(item, oa, ob, k_begin, k_end)  fills the operands and the k range of an item (k_end > k_begin,
   //                                      k_begin a multiple of BK)
   //   epilogue(item, acc)                consumes the finished accumulators; it may use global memory and LDS
-  //                                      outside the ring's LDS_BYTES
+  //                                      outside the ring's LDS_BYTES, and returns whether this wave has made STORES stores at least
   // All threads of the workgroup call this together.
   //
   // Schedule per stage c: under the MFMAs of its first sub-step the fragments of the second are read and the A side
   // fetches its part of stage c+2, into the slot that stage c-1 left.  Between the sub-steps the wave waits for
   // its part of stage c+1 to have landed (all but the fetches just issued) and joins the barrier; past it, every wave has
   // finished reading stage c, so under the MFMAs of the second sub-step the B side's slot is refilled, with its part
-  // of stage c+2, and the first fragments of stage c+1 are read.
-  template <class GetItem, class Epilogue>
+  // of stage c+2, and the first fragments of stage c+1 are read.  What a stage does once, the ring's turns and counts, stands
+  // behind a sub-step's last bump, where the matrix pipe does not wait for it.
+  template <int STORES = 0, class GetItem, class Epilogue>
   __device__ __forceinline__ static void run(int item_begin, int item_end, half_t* lds, GetItem get, Epilogue epilogue) {
     if (item_begin >= item_end) return;
     const int lane = threadIdx.x & 63;
@@ -328,21 +367,23 @@ struct WideCore {
       get(item, oa, ob, kb, ke);
       return ke - kb;
     };
-    const half_t *sa = a_ring, *sb = b_ring;  // the stage being multiplied
+    int sa = 0, sb = 0;  // the slots of the stage being multiplied, in halves
     // Zeros in place of what that stage holds past its last k (n of them are left).  Each wave clears the pieces it
     // fetched, between its own wait for them and the barrier.
     auto clear_tail = [&](int n) {
       wait_vmcnt<0>();
-      Cursor<true>::Load::clear_tail(const_cast<half_t*>(sa), n, wave, lane);
-      Cursor<false>::Load::clear_tail(const_cast<half_t*>(sb), n, wave, lane);
+      Cursor<true>::Load::clear_tail(a_ring + sa, n, wave, lane);
+      Cursor<false>::Load::clear_tail(b_ring + sb, n, wave, lane);
     };
     auto issue_one = [&]() {
 #pragma unroll
       for (int j = 0; j < A_CH; ++j) ca.piece(j), ca.bump(j);
 #pragma unroll
       for (int j = 0; j < B_CH; ++j) cb.piece(j), cb.bump(j);
-      ca.advance(get, item_end, wave, lane);
-      cb.advance(get, item_end, wave, lane);
+      ca.step();
+      ca.turn(get, item_end, wave, lane);
+      cb.step();
+      cb.turn(get, item_end, wave, lane);
     };
     issue_one();
     int k_left = length(item_begin);  // k of the item from the stage being multiplied on
@@ -353,9 +394,9 @@ struct WideCore {
 
     Frags f0, f1;  // the fragments of a stage's first and second sub-step
 #pragma unroll
-    for (int j = 0; j < NR; ++j) read_one(j, sa, sb, 0, wm, wn, lane, f0);
+    for (int j = 0; j < NR; ++j) read_one(j, a_ring + sa, b_ring + sb, 0, wm, wn, lane, f0);
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    bool drain_all = false;
+    int behind = 0;  // an item's first wait: 1, after the epilogue's STORES stores or more; 2, after an unknown number
     // (lambdas, not calls: written out, the compiler deals the forward kernel's scalar registers in another order)
     auto a_piece = [&](int j) { ca.piece(j); };
     auto a_bump = [&](int j) { ca.bump(j); };
@@ -366,9 +407,20 @@ struct WideCore {
 #pragma unroll
       for (int n = 0; n < NM; ++n) {
         mfma<decltype(first_tag)::value>(n, f0, acc);
-        if (n % READ_EVERY == 0 && n / READ_EVERY < NR) read_one(n / READ_EVERY, sa, sb, 1, wm, wn, lane, f1);
+        if (n % READ_EVERY == 0 && n / READ_EVERY < NR) read_one(n / READ_EVERY, a_ring + sa, b_ring + sb, 1, wm, wn, lane, f1);
         if (n % A_EVERY == A_EVERY - 1 && n / A_EVERY < A_CH) a_piece(n / A_EVERY);
         if (n % A_EVERY == 1 && n > A_EVERY && n / A_EVERY - 1 < A_CH) a_bump(n / A_EVERY - 1);
+        if (n == NM - 5) ca.step();
+        if (n == NM - 4) {
+          sa = sa == (A_SLOTS - 1) * A_HALVES ? 0 : sa + A_HALVES;
+          pin(sa);
+        }
+        if (n == NM - 3) {
+          sb = sb == (B_SLOTS - 1) * B_HALVES ? 0 : sb + B_HALVES;
+          k_left -= BK;
+          pin(sb);
+          pin(k_left);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -376,40 +428,46 @@ struct WideCore {
 #pragma unroll
       for (int n = 0; n < NM; ++n) {
         mfma<false>(n, f1, acc);
-        if (n % READ_EVERY == 0 && n / READ_EVERY < NR) read_one(n / READ_EVERY, sa, sb, 0, wm, wn, lane, f0);
+        if (n % READ_EVERY == 0 && n / READ_EVERY < NR) read_one(n / READ_EVERY, a_ring + sa, b_ring + sb, 0, wm, wn, lane, f0);
         if (n % B_EVERY == B_EVERY - 1 && n / B_EVERY < B_CH) b_piece(n / B_EVERY);
         if (n % B_EVERY == 1 && n > B_EVERY && n / B_EVERY - 1 < B_CH) b_bump(n / B_EVERY - 1);
+        if (n == NM - 4) cb.step();
         __builtin_amdgcn_sched_barrier(0);
       }
     };
     for (int item = item_begin; item < item_end; ++item) {
-      const int nk = (k_left + BK - 1) / BK;
-      for (int kt = 0; kt < nk; ++kt) {
-        if (kt == 0) sub_step0(std::true_type{});
+      bool first = true, more;
+      do {
+        if (first) sub_step0(std::true_type{});
         else sub_step0(std::false_type{});
-        ca.advance(get, item_end, wave, lane);
-        sa = sa == a_ring + (A_SLOTS - 1) * A_HALVES ? a_ring : sa + A_HALVES;
-        sb = sb == b_ring + (B_SLOTS - 1) * B_HALVES ? b_ring : sb + B_HALVES;
-        k_left -= BK;
+        first = false;
+        more = k_left > 0;
+        ca.turn(get, item_end, wave, lane);
         if (k_left < BK) {
           if (k_left <= 0) k_left = item + 1 < item_end ? length(item + 1) : BK;
           if (k_left < BK) clear_tail(k_left);
         }
-        // this wave's LDS reads of stage c are complete (lgkmcnt) and its share of stage c+1 has landed.
-        // After an epilogue the wave's stores stand behind those fetches, as many as the tile's edges left, so
-        // the first wait after one drains everything (see pipe_core.hpp).
+        // this wave's LDS reads of stage c are complete (lgkmcnt) and its share of stage c+1 has landed.  After an epilogue the
+        // wave's stores stand behind those fetches: where their number is known they are not waited for here (they have
+        // another stage until a fetch behind them is), else, a tile's edges, the first wait drains everything.
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), in a form the compiler's own wait bookkeeping sees
-        if (drain_all) { wait_lds_vmcnt_barrier<0>(); drain_all = false; }
-        else wait_lds_vmcnt_barrier<A_CH>();
+        if (behind == 0) wait_lds_vmcnt_barrier<A_CH>();
+        else if (behind == 1) wait_lds_vmcnt_barrier<A_CH + STORES>();
+        else wait_lds_vmcnt_barrier<0>();
+        behind = 0;
         sub_step1();
-        cb.advance(get, item_end, wave, lane);
+        cb.turn(get, item_end, wave, lane);
         // No LDS read stays pending across the loop edge (the reads above finished long before the
         // MFMAs were all issued): the compiler then knows the next stage's first MFMAs need no wait.
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-      }
+      } while (more);
       settle(acc);
-      epilogue(item, acc);
-      drain_all = true;
+      if constexpr (STORES > 0) {
+        behind = epilogue(item, acc) ? 1 : 2;
+      } else {
+        epilogue(item, acc);
+        behind = 2;
+      }
     }
     wait_vmcnt<0>();
   }

@@ -120,13 +120,13 @@ __global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
   // A lane owns one batch row and eight consecutive labels of every 32: 16-byte stores straight from the registers,
   // 64 bytes per row and instruction, the other 64 of the line with the next.  Of a tile's 54,000 cycles this takes
   // 10,000: the two transcendentals of a sigmoid occupy a SIMD for 32 cycles per 64 elements, which with the conversions
-  // is 9,200 (2,900 without the sigmoid), and the stores hide under them; the wait for the last of them to be written,
-  // in the next tile's first stage, is another 1,900.  Stores of whole lines (8 rows x 128 or 4 x 256 bytes per
+  // is 9,200 (2,900 without the sigmoid), and the stores hide under them; the wait for the last of them to be written
+  // was another 1,900 in the next tile's first stage, which now passes them by their count.  Stores of whole lines (8 rows x 128 or 4 x 256 bytes per
   // instruction) take as long: all CUs together store at 7.3 TB/s into the caches whatever the shape.
   auto epilogue = [&](int item, float4v (&acc)[C::FM][C::FN]) {
     int mt, nt;
     xcd_map(item * G + w, a.tiles_m, mt, nt);
-    if (nt >= a.tiles_n) return;
+    if (nt >= a.tiles_n) return false;
     const int row_l = mt * C::BN + wn * C::TN + (lane & 15);
     const int col_l = nt * C::BM + wm * C::TM + 8 * (lane >> 4);
     // A tile that crosses the label count is compiled as a path of its own: the common one carries no column checks.
@@ -207,10 +207,14 @@ __global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
         }
       }
     };
-    if (nt * C::BM + C::BM > a.N) body(std::true_type{});
-    else body(std::false_type{});
+    if (nt * C::BM + C::BM > a.N) {
+      body(std::true_type{});
+      return false;
+    }
+    body(std::false_type{});
+    return mt * C::BN + (wn + 1) * C::TN <= a.M;
   };
-  C::run(0, n_items, lds, get, epilogue);
+  C::template run<C::FN * C::FM / 2>(0, n_items, lds, get, epilogue);
   if constexpr (LOSS) {
     // deterministic: lanes -> wave (butterfly), waves -> workgroup (LDS, fixed order), one partial per workgroup
 #pragma unroll
