@@ -39,7 +39,8 @@ struct BackArgs {
   float* out; int64_t ldo; float beta;        // BACK_OUT, BACK_ADD
   float* part;                                // [ranges * parts][B][d] partial sums of G.W
   int B, L, d;
-  int slices, ranges, parts, tiles;           // ranges a multiple of 8; tiles of 64 labels
+  int slices, ranges, parts, tiles;           // ranges a multiple of 8 (back_wide.hpp: any number); tiles of 64 labels
+  bool back;                                  // back_wide.hpp: the last labels first
 };
 
 template <bool NT, class T>

@@ -105,10 +105,11 @@ __global__ void __launch_bounds__(S::NT, 1) back_wide_kernel(BackArgs a) {
   if (id >= a.slices * a.ranges) return;
   const int slice = id % a.slices, range = id / a.slices, dim0 = slice * BACK_DIMS;
   const int part0 = range * a.parts, part1 = part0 + a.parts;
-  // Its tiles: every a.ranges-th from the range's number on, counted from 0 here.
+  // Its tiles: every a.ranges-th from the range's number on, counted from 0 here (a.back: from the last one on).
   const int t1 = (a.tiles - range + a.ranges - 1) / a.ranges, most = (a.tiles + a.ranges - 1) / a.ranges;
   const int whole = a.L - (a.tiles - 1) * BACK_TILE;                                     // labels of the last tile
-  const int edge = whole < BACK_TILE && (a.tiles - 1) % a.ranges == range ? t1 - 1 : -1;  // if it is not whole and here
+  const int edge = whole < BACK_TILE && (a.tiles - 1) % a.ranges == range ? (a.back ? 0 : t1 - 1) : -1;  // if it is not whole and here
+  const int label0 = (range + (a.back ? (t1 - 1) * a.ranges : 0)) * BACK_TILE, step = (a.back ? -a.ranges : a.ranges) * BACK_TILE;
   // Rows of the batch in an image: in their order, but for the last wave's, which are the batch's last 16 RB rounded up to eights;
   // those of them that another wave has, and those past the batch, are zeros.
   const int eights = (a.B + 7) >> 3, q0 = wave < 3 ? S::G_FETCH * wave : eights - S::G_FETCH;  // the wave's first eight
@@ -119,16 +120,21 @@ __global__ void __launch_bounds__(S::NT, 1) back_wide_kernel(BackArgs a) {
   auto g_col = [&](int eight, int lane) XFC_INLINE { return 8 * ((lane & 7) ^ S::g_swz(8 * eight + (lane >> 3))); };
   const uint32_t lds_g = gs + (uint32_t)wave * (uint32_t)(S::G_FETCH * 1024);
   uint32_t gv[3];  // of even and odd eights; gv[2]: of the last, which may be part of one
+  auto whole_g = [&]() XFC_INLINE {
+    int lane_ = lane;
+    asm volatile("" : "+v"(lane_));  // opaque: made once or twice, nothing of it is to be kept
 #pragma unroll
-  for (int h = 0; h < 2; ++h) gv[h] = (uint32_t)(lane >> 3) * (uint32_t)(a.ldg * 2) + 2u * g_col(h, lane);
-  const int last = a.B - 1 - 8 * (q0 + S::G_FETCH - 1);
-  gv[2] = (uint32_t)((lane >> 3) < last ? lane >> 3 : last) * (uint32_t)(a.ldg * 2) + 2u * g_col(1, lane);
+    for (int h = 0; h < 2; ++h) gv[h] = (uint32_t)(lane_ >> 3) * (uint32_t)(a.ldg * 2) + 2u * g_col(h, lane_);
+    const int last = a.B - 1 - 8 * (q0 + S::G_FETCH - 1);
+    gv[2] = (uint32_t)((lane_ >> 3) < last ? lane_ >> 3 : last) * (uint32_t)(a.ldg * 2) + 2u * g_col(1, lane_);
+  };
+  whole_g();
   const uint32_t w_col = 16u * (uint32_t)((lane & 15) ^ S::w_swz(8 * wave + (lane >> 4)));
   const uint32_t wv = (uint32_t)(lane >> 4) * (uint32_t)(a.ldw * 2) + w_col;
-  const int64_t w_row = uniform64(a.ldw * 2), w_step = uniform64((int64_t)a.ranges * BACK_TILE * a.ldw * 2);
-  const int64_t g_step = (int64_t)a.ranges * BACK_TILE * 2, g_eight = uniform64(a.ldg * 16);
-  int64_t at_g = uniform64(reinterpret_cast<int64_t>(a.G + (int64_t)(8 * q0) * a.ldg + (int64_t)range * BACK_TILE));
-  int64_t at_w = uniform64(reinterpret_cast<int64_t>(a.W + (int64_t)range * BACK_TILE * a.ldw + dim0));  // of the tile being multiplied
+  const int64_t w_row = uniform64(a.ldw * 2), w_step = uniform64((int64_t)step * a.ldw * 2);
+  const int64_t g_step = (int64_t)step * 2, g_eight = uniform64(a.ldg * 16);
+  int64_t at_g = uniform64(reinterpret_cast<int64_t>(a.G + (int64_t)(8 * q0) * a.ldg + label0));
+  int64_t at_w = uniform64(reinterpret_cast<int64_t>(a.W + (int64_t)label0 * a.ldw + dim0));  // of the tile being multiplied
   const int64_t w_to_m = uniform64(reinterpret_cast<int64_t>(a.Mo) - reinterpret_cast<int64_t>(a.W));
   // To be called before the fetches of G of the tile that is not whole: labels past the end repeat others that are there.
   auto edge_g = [&]() XFC_INLINE {
@@ -203,6 +209,7 @@ __global__ void __launch_bounds__(S::NT, 1) back_wide_kernel(BackArgs a) {
     fetch_w(f, std::integral_constant<int, 0>{}, 0, false);
     fetch_w(f, std::integral_constant<int, 1>{}, 0, false);
   });
+  if (edge == 0 && t1 > 1) whole_g();
   if (edge == 1) edge_g();
   wait_vmcnt<0>();
   if (ragged || edge == 0) clear_g(0, lds_g);

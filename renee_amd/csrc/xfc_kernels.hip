@@ -1673,6 +1673,10 @@ int launch_back_wide(BackArgs a, float* dX, int64_t lddx, float scale, void* ws,
     // 1,310,720 3277 -> 3370; 512 x 300,001 x 256 354 -> 366).
     const int64_t state = (int64_t)a.L * a.d * 4, Mi = (int64_t)1 << 20;
     const bool loads = state + (int64_t)a.L * a.B * 2 > 224 * Mi, stores = state > 224 * Mi && state <= 560 * Mi && a.B <= a.d;
+    // The forward pass has left the caches the last labels' G and weights: those first (512 x 327,680 x 768 838 -> 825 us, 262,144 x
+    // 256 303 -> 286, 1,310,720 x 768 3233 -> 3217), but where the stores pass the caches by (131,072 x 768: 333 -> 336) or these
+    // hold everything (300 x 60,001 x 768: 147 -> 160).
+    a.back = loads && !stores;
     rc = stores ? launch_k<back_wide_kernel<S, true, true>>(g, b, S::LDS_BYTES, st, a)
          : loads ? launch_k<back_wide_kernel<S, true, false>>(g, b, S::LDS_BYTES, st, a)
                  : launch_k<back_wide_kernel<S, false, false>>(g, b, S::LDS_BYTES, st, a);
