@@ -59,9 +59,9 @@ struct BackStep : Wave16 {
   static_assert(LDS_BYTES <= 160 * 1024 && ROWS <= BACK_MAX_ROWS && XR <= RP, "budget");
 };
 
-// NT: the arrays that are read and written (BACK_UPDATE: W and Mo, BACK_ADD: out; BACK_OUT has none) are loaded as what will not
-// be wanted again, for sizes that no cache holds until the next step.
-template <class S, int MODE, bool NT>
+// NT, NTS: the arrays that are written (BACK_UPDATE: W and Mo, otherwise out) are loaded, and stored, as what will not be wanted
+// again, for sizes that no cache holds until the next step.
+template <class S, int MODE, bool NT, bool NTS>
 __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
   constexpr int RQ = S::RQ, RP = S::RP, XR = S::XR;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
@@ -281,8 +281,8 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
           wv[e] = (half_t)(wf - a.lr * mf);
         }
         if (label + 8 * h < a.L && col < a.d) {
-          *reinterpret_cast<half8*>(a.Mo + (int64_t)(label + 8 * h) * a.ldm + col) = mv;
-          *reinterpret_cast<half8*>(a.W + (int64_t)(label + 8 * h) * a.ldw + col) = wv;
+          store<NTS>(reinterpret_cast<half8*>(a.Mo + (int64_t)(label + 8 * h) * a.ldm + col), mv);
+          store<NTS>(reinterpret_cast<half8*>(a.W + (int64_t)(label + 8 * h) * a.ldw + col), wv);
         }
       }
     } else {
@@ -296,7 +296,7 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
           for (int e = 0; e < 4; ++e) v[e] = second == h ? dw[s][h][e] : far[e];
           if constexpr (MODE == BACK_ADD) v += a.beta * now.o[s][h];
           if (label + 8 * h < a.L && col32(s) < a.d)
-            *reinterpret_cast<float4v*>(a.out + (int64_t)(label + 8 * h) * a.ldo + col32(s)) = v;
+            store<NTS>(reinterpret_cast<float4v*>(a.out + (int64_t)(label + 8 * h) * a.ldo + col32(s)), v);
         }
     }
     leave(tile + 1);

@@ -37,6 +37,12 @@ typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
 __device__ __attribute__((aligned(16))) const uint32_t g_zero16[4] = {0u, 0u, 0u, 0u};
 
+template <bool NT, class T>
+__device__ __forceinline__ void store(T* p, const T& v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
 // Row of C held by accumulator register r of a 32x32 block, for this lane.
 __device__ __forceinline__ int c_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
 

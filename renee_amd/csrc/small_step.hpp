@@ -43,8 +43,8 @@ struct SmallArgs {
 };
 
 // NW waves, SB blocks of 32 dims per wave, RB blocks of 16 rows (2 or 4); LINES: an instruction that loads or stores weights
-// or momentum covers 8 labels x 128 bytes (see back_step.hpp) instead of 16 x 64, and the loads say that nothing will want
-// them again.  That is for sizes that no cache holds until the next step: 32 rows x 131,072 x 768 188 -> 169 us, x 700,001 961 ->
+// or momentum covers 8 labels x 128 bytes (see back_step.hpp) instead of 16 x 64, and the loads and stores say that nothing will
+// want them again.  That is for sizes that no cache holds until the next step: 32 rows x 131,072 x 768 188 -> 169 us, x 700,001 961 ->
 // 888, 64 x 700,001 x 512 696 -> 621 (whole lines without the hint 720, half lines with it 1,048 at 32 x 700,001 x 768).  Below,
 // half lines without the hint are faster, as the caches serve them: 64 x 20,011 x 512 33.0 against 34.5, 32 x 4,097 x 1024 24.8
 // against 28.1.
@@ -345,8 +345,8 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
         }
         const int label = l0 + label_of(lb, s);
         if (label < a.L) {
-          *reinterpret_cast<half8*>(a.Mo + (int64_t)label * a.ldm + dim0 + col_of(s)) = mv;
-          *reinterpret_cast<half8*>(a.W + (int64_t)label * a.ldw + dim0 + col_of(s)) = wv;
+          store<S::LINES>(reinterpret_cast<half8*>(a.Mo + (int64_t)label * a.ldm + dim0 + col_of(s)), mv);
+          store<S::LINES>(reinterpret_cast<half8*>(a.W + (int64_t)label * a.ldw + dim0 + col_of(s)), wv);
         }
         if constexpr (!AHEAD) __builtin_amdgcn_sched_barrier(0);
       };

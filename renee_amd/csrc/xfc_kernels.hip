@@ -999,7 +999,8 @@ struct DwArgs {
 
 // Persistent, one workgroup per CU: workgroup w takes tile ids w, w + gridDim.x, ...; the dim tiles of
 // one label tile have neighbouring ids on one XCD, so its slice of G is fetched from HBM once.
-template <int MODE>
+// NTS: what is written is stored as what will not be wanted again (see launch_dw).
+template <int MODE, bool NTS>
 __global__ void __launch_bounds__(DwCore::NT) dw_kernel(DwArgs a) {
   using C = DwCore;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
@@ -1097,8 +1098,8 @@ __global__ void __launch_bounds__(DwCore::NT) dw_kernel(DwArgs a) {
           o0 += a.beta * p0;
           o1 += a.beta * p1;
         }
-        if (in) *reinterpret_cast<float4v*>(orow + col) = o0;
-        if (in1) *reinterpret_cast<float4v*>(orow + col1) = o1;
+        if (in) store<NTS>(reinterpret_cast<float4v*>(orow + col), o0);
+        if (in1) store<NTS>(reinterpret_cast<float4v*>(orow + col1), o1);
       } else if constexpr (MODE == DW_UPDATE_MASTER) {
         // the reference's regime (fp32 parameter and FusedSGD state, dl_base.py:185, main.py:178-179) with the
         // per-step fp16 cast of W (dl_base.py:562) written from the same pass
@@ -1129,12 +1130,12 @@ __global__ void __launch_bounds__(DwCore::NT) dw_kernel(DwArgs a) {
           float* wp = a.W32 + (int64_t)row * a.ldw32;
           float* mp = a.M32 + (int64_t)row * a.ldm32;
           half_t* hp = a.Wt + (int64_t)row * a.ldw;
-          *reinterpret_cast<float4v*>(mp + col) = mv[0];
-          *reinterpret_cast<float4v*>(wp + col) = wv[0];
+          store<NTS>(reinterpret_cast<float4v*>(mp + col), mv[0]);
+          store<NTS>(reinterpret_cast<float4v*>(wp + col), wv[0]);
           *reinterpret_cast<half4*>(hp + col) = half4{w16[0], w16[1], w16[2], w16[3]};
           if (in1) {
-            *reinterpret_cast<float4v*>(mp + col1) = mv[1];
-            *reinterpret_cast<float4v*>(wp + col1) = wv[1];
+            store<NTS>(reinterpret_cast<float4v*>(mp + col1), mv[1]);
+            store<NTS>(reinterpret_cast<float4v*>(wp + col1), wv[1]);
             *reinterpret_cast<half4*>(hp + col1) = half4{w16[4], w16[5], w16[6], w16[7]};
           }
         }
@@ -1155,8 +1156,8 @@ __global__ void __launch_bounds__(DwCore::NT) dw_kernel(DwArgs a) {
             mv[e] = (half_t)mf;
             wv[e] = (half_t)(wf - a.lr * mf);
           }
-          *reinterpret_cast<half8*>(a.Mo + (int64_t)row * a.ldm + col) = mv;
-          *reinterpret_cast<half8*>(a.Wt + (int64_t)row * a.ldw + col) = wv;
+          store<NTS>(reinterpret_cast<half8*>(a.Mo + (int64_t)row * a.ldm + col), mv);
+          store<NTS>(reinterpret_cast<half8*>(a.Wt + (int64_t)row * a.ldw + col), wv);
         }
       }
     }
@@ -1507,9 +1508,19 @@ int launch_dw(int mode, DwArgs a, hipStream_t st) {
   int64_t grid = (int64_t)round_up(num_cus(), 8);  // one resident workgroup per CU
   if (grid > ids) grid = ids / 8 * 8 > 0 ? ids / 8 * 8 : ids;
   const dim3 g((unsigned)grid), b(DwCore::NT);
-  if (mode == DW_UPDATE) return launch_k<dw_kernel<DW_UPDATE>>(g, b, DW_LDS_BYTES, st, a);
-  if (mode == DW_UPDATE_MASTER) return launch_k<dw_kernel<DW_UPDATE_MASTER>>(g, b, DW_LDS_BYTES, st, a);
-  return launch_k<dw_kernel<DW_OUT>>(g, b, DW_LDS_BYTES, st, a);
+  // Non-temporal stores where what is written would push out of the caches what the next kernels read, from about their size on.  A
+  // gradient: six-argument calls of 512 rows x 131,072 labels x 768 dims 384 -> 347 us, 128 rows 212 -> 178, 512 x 200,000 x 256 303
+  // -> 261, x 80,000 x 768 258 -> 241, but x 32,768 118 -> 120.  Master weights: steps of 512 x 655,363 x 768 2868 -> 2813, 64 x
+  // 200,001 717 -> 668, 256 x 131,072 x 256 201 -> 193, but 256 x 20,001 x 768 115 -> 123.  fp16 state: 1024 x 2,812,281 x 768 13.81 ->
+  // 13.67 ms, x 700,001 3.48 -> 3.44, but 800 x 200,001 x 512 684 -> 688, 700 x 131,072 x 256 228 -> 235.
+  const int64_t weights = (int64_t)a.M * a.N, Mi = (int64_t)1 << 20;
+  auto launch = [&](auto mode_tag, int64_t least) {
+    constexpr int MODE = decltype(mode_tag)::value;
+    return weights > least ? launch_k<dw_kernel<MODE, true>>(g, b, DW_LDS_BYTES, st, a) : launch_k<dw_kernel<MODE, false>>(g, b, DW_LDS_BYTES, st, a);
+  };
+  if (mode == DW_UPDATE) return launch(std::integral_constant<int, DW_UPDATE>{}, 140 * Mi);
+  if (mode == DW_UPDATE_MASTER) return launch(std::integral_constant<int, DW_UPDATE_MASTER>{}, 28 * Mi);
+  return launch(std::integral_constant<int, DW_OUT>{}, 40 * Mi);
 }
 
 // The one-pass step of small batches (small_step.hpp).  Fn::operator()<S>() is called with the kernel for d dims and B
@@ -1640,12 +1651,19 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
   // What the pass reads and writes against the Infinity Cache (256 MB, G and the partial sums beside it).  (60,007 labels x 768
   // dims, 256 rows: 87 us without the hint, 91 with; 700,001 x 768, 128 rows: 953 and 892.)
   const bool nt = (int64_t)a.L * a.d * (MODE == BACK_UPDATE ? 4 : 6) > (int64_t)224 << 20;
+  // The same for the stores: whole steps of 256 rows x 131,072 labels x 768 dims 287 -> 259 us, 128 x 320,001 539 -> 498, 100 x
+  // 400,001 x 384 354 -> 326, 256 x 1,310,720 x 768 2.73 -> 2.53 ms; four micro-batches of 200 x 200,001 x 384 1163 -> 1076 us.
+  // With an update of 193 to 255 rows only from some 480 MB on: 199 x 131,072 x 768 the same, 200 x 200,001 x 512 296 -> 301, x
+  // 90,001 x 768 198 -> 200, x 700,001 x 768 1338 -> 1288.
+  const bool nts = nt && (MODE != BACK_UPDATE || a.B <= 192 || a.B == 256 || (int64_t)a.L * a.d * 4 > (int64_t)480 << 20);
   int rc = XFC_OK;
   *taken = back_step_for<MODE>(a.B, [&](auto s) {
     using S = decltype(s);
     const dim3 g((unsigned)(a.slices * a.ranges)), b(S::NT);
-    rc = nt ? launch_k<back_step_kernel<S, MODE, MODE != BACK_OUT>>(g, b, S::LDS_BYTES, st, a)
-            : launch_k<back_step_kernel<S, MODE, false>>(g, b, S::LDS_BYTES, st, a);
+    constexpr bool NT = MODE != BACK_OUT, LOADS = MODE == BACK_UPDATE && S::RQ == 4;
+    rc = nts           ? launch_k<back_step_kernel<S, MODE, NT, true>>(g, b, S::LDS_BYTES, st, a)
+         : LOADS && nt ? launch_k<back_step_kernel<S, MODE, LOADS, false>>(g, b, S::LDS_BYTES, st, a)
+                       : launch_k<back_step_kernel<S, MODE, false, false>>(g, b, S::LDS_BYTES, st, a);
     if (rc) return;
     launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges * a.parts, scale, 0.0f, st);
     rc = check_launch();
@@ -1800,8 +1818,9 @@ int xfc_init(void) {
     for (int64_t rows : {64, 128, 192, 256})
       back_step_for<MODE>(rows, [&](auto s) {
         using S = decltype(s);
-        keep(raise_lds_limit<back_step_kernel<S, MODE, MODE != BACK_OUT>>(S::LDS_BYTES));
-        keep(raise_lds_limit<back_step_kernel<S, MODE, false>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, MODE != BACK_OUT, true>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, MODE == BACK_UPDATE && S::RQ == 4, false>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, false, false>>(S::LDS_BYTES));
       });
   };
   for (int64_t rows : {320, 384, 448, 512})
@@ -1816,9 +1835,13 @@ int xfc_init(void) {
   back_limits(std::integral_constant<int, BACK_ADD>{});
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_SMALL>>((int)sizeof(SelLds<SEL_CAP_SMALL>)));
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_LARGE>>((int)sizeof(SelLds<SEL_CAP_LARGE>)));
-  keep(raise_lds_limit<dw_kernel<DW_UPDATE>>(DW_LDS_BYTES));
-  keep(raise_lds_limit<dw_kernel<DW_OUT>>(DW_LDS_BYTES));
-  keep(raise_lds_limit<dw_kernel<DW_UPDATE_MASTER>>(DW_LDS_BYTES));
+  auto dw_limits = [&](auto mode) {
+    keep(raise_lds_limit<dw_kernel<decltype(mode)::value, false>>(DW_LDS_BYTES));
+    keep(raise_lds_limit<dw_kernel<decltype(mode)::value, true>>(DW_LDS_BYTES));
+  };
+  dw_limits(std::integral_constant<int, DW_UPDATE>{});
+  dw_limits(std::integral_constant<int, DW_OUT>{});
+  dw_limits(std::integral_constant<int, DW_UPDATE_MASTER>{});
   (void)num_cus();
   if (static_scratch_ptr() == nullptr) return XFC_ERR_HIP;
   if (e != hipSuccess) {
