@@ -206,26 +206,33 @@ struct WideCore {
     uint32_t ring, dst;  // LDS address of this wave's first piece in slot 0 and in the stage's slot
     int item, k_left;    // k of the item from this stage on
     int64_t ld;
-    int64_t end = 0;     // where the item's tile starts, moved on by its stages; 0: its addresses do not lead to the next one's
-    template <class GetItem>
+    int64_t shift;        // of the first address from where the item's tile starts
+    bool inside = false;  // the tile lies inside the operand, its k are whole stages, and shift is known
+    // MOVE: from one tile that lies inside the operand to another all addresses move by the same (made anew they are 150
+    // instructions between two stages).  Not from the first one: what that takes would stand in front of every kernel's first
+    // stage, 0.3 us of a small one's 20.
+    template <bool MOVE, class GetItem>
     __device__ __forceinline__ void open(GetItem& get, int wave, int lane) {
       Operand o[2];
       int kb, ke;
       get(item, o[0], o[1], kb, ke);
       const Operand& me = o[IS_A ? 0 : 1];
-      constexpr bool KC = IS_A ? A_KC : true;
-      // From one tile that lies inside the operand to another all addresses move by the same (made anew they are 150
-      // instructions between two stages).
-      const bool inside = me.r0 + (IS_A ? BM : BN) <= me.rmax && (ke - kb) % BK == 0;
-      const int64_t start = uniform64(reinterpret_cast<int64_t>(me.p) + (KC ? me.r0 * me.ld + kb : kb * me.ld + me.r0) * 2);
-      if (inside && end != 0) {
-        const int64_t by = uniform64(start - end);
+      if constexpr (MOVE) {
+        constexpr bool KC = IS_A ? A_KC : true;
+        const bool was = inside;
+        inside = me.r0 + (IS_A ? BM : BN) <= me.rmax && (ke - kb) % BK == 0;
+        const int64_t start = uniform64(reinterpret_cast<int64_t>(me.p) + (KC ? me.r0 * me.ld + kb : kb * me.ld + me.r0) * 2);
+        if (was && inside) {
+          const int64_t by = uniform64(start + shift - load.at[0]);
 #pragma unroll
-        for (int i = 0; i < CH; ++i) load.at[i] += by;
+          for (int i = 0; i < CH; ++i) load.at[i] += by;
+        } else {
+          load.init(me, kb, wave, lane);
+          shift = uniform64(load.at[0] - start);
+        }
       } else {
         load.init(me, kb, wave, lane);
       }
-      end = inside ? uniform64(start + (ke - kb) / BK * load.kstep) : 0;
       ld = me.ld;
       k_left = ke - kb;
       if (k_left < BK) load.retarget(k_left, ld, wave, lane);
@@ -241,14 +248,14 @@ struct WideCore {
       pin(dst);
       pin(k_left);
     }
-    template <class GetItem>
+    template <bool MOVE, class GetItem>
     __device__ __forceinline__ void turn(GetItem& get, int item_end, int wave, int lane) {
       if (k_left < BK) {
         if (k_left > 0) {
           load.retarget(k_left, ld, wave, lane);
         } else if (item + 1 < item_end) {
           ++item;
-          open(get, wave, lane);
+          open<MOVE>(get, wave, lane);
         } else {
           k_left += BK;
 #pragma unroll
@@ -359,8 +366,8 @@ struct WideCore {
     ca.ring = ca.dst = lds_addr(a_ring) + (uint32_t)wave * 1024u;
     cb.ring = cb.dst = lds_addr(b_ring) + (uint32_t)wave * 1024u;
     ca.item = cb.item = item_begin;
-    ca.open(get, wave, lane);
-    cb.open(get, wave, lane);
+    ca.template open<false>(get, wave, lane);
+    cb.template open<false>(get, wave, lane);
     auto length = [&](int item) {  // k of an item
       Operand oa, ob;
       int kb, ke;
@@ -375,22 +382,25 @@ struct WideCore {
       Cursor<true>::Load::clear_tail(a_ring + sa, n, wave, lane);
       Cursor<false>::Load::clear_tail(b_ring + sb, n, wave, lane);
     };
-    auto issue_one = [&]() {
+    int k_left = length(item_begin);  // k of the item from the stage being multiplied on
+    // The first two stages' fetches, and the wait for the first (a loop: every line of code in front of the first MFMA costs a
+    // small kernel an instruction fetch).
+#pragma nounroll
+    for (int stage = 0; stage < 2; ++stage) {
 #pragma unroll
       for (int j = 0; j < A_CH; ++j) ca.piece(j), ca.bump(j);
 #pragma unroll
       for (int j = 0; j < B_CH; ++j) cb.piece(j), cb.bump(j);
       ca.step();
-      ca.turn(get, item_end, wave, lane);
+      ca.template turn<false>(get, item_end, wave, lane);
       cb.step();
-      cb.turn(get, item_end, wave, lane);
-    };
-    issue_one();
-    int k_left = length(item_begin);  // k of the item from the stage being multiplied on
-    if (k_left < BK) clear_tail(k_left);
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    wait_vmcnt_barrier<0>();
-    issue_one();
+      cb.template turn<false>(get, item_end, wave, lane);
+      if (stage == 0) {
+        if (k_left < BK) clear_tail(k_left);
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+        wait_vmcnt_barrier<0>();
+      }
+    }
 
     Frags f0, f1;  // the fragments of a stage's first and second sub-step
 #pragma unroll
@@ -442,7 +452,7 @@ struct WideCore {
         else sub_step0(std::false_type{});
         first = false;
         more = k_left > 0;
-        ca.turn(get, item_end, wave, lane);
+        ca.template turn<true>(get, item_end, wave, lane);
         if (k_left < BK) {
           if (k_left <= 0) k_left = item + 1 < item_end ? length(item + 1) : BK;
           if (k_left < BK) clear_tail(k_left);
@@ -456,7 +466,7 @@ struct WideCore {
         else wait_lds_vmcnt_barrier<0>();
         behind = 0;
         sub_step1();
-        cb.turn(get, item_end, wave, lane);
+        cb.template turn<true>(get, item_end, wave, lane);
         // No LDS read stays pending across the loop edge (the reads above finished long before the
         // MFMAs were all issued): the compiler then knows the next stage's first MFMAs need no wait.
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)

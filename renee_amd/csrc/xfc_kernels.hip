@@ -1653,9 +1653,9 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
   const bool nt = (int64_t)a.L * a.d * (MODE == BACK_UPDATE ? 4 : 6) > (int64_t)224 << 20;
   // The same for the stores: whole steps of 256 rows x 131,072 labels x 768 dims 287 -> 259 us, 128 x 320,001 539 -> 498, 100 x
   // 400,001 x 384 354 -> 326, 256 x 1,310,720 x 768 2.73 -> 2.53 ms; four micro-batches of 200 x 200,001 x 384 1163 -> 1076 us.
-  // With an update of 193 to 255 rows only from some 480 MB on: 199 x 131,072 x 768 the same, 200 x 200,001 x 512 296 -> 301, x
-  // 90,001 x 768 198 -> 200, x 700,001 x 768 1338 -> 1288.
-  const bool nts = nt && (MODE != BACK_UPDATE || a.B <= 192 || a.B == 256 || (int64_t)a.L * a.d * 4 > (int64_t)480 << 20);
+  // With an update of 193 to 224 rows, where some of the waves fetch no rows of G, only from some 480 MB on: 224 x 131,072 x 768 269
+  // -> 273 us (240 277 -> 253), 200 x 200,001 x 512 296 -> 301, x 90,001 x 768 198 -> 200, x 700,001 x 768 1338 -> 1288.
+  const bool nts = nt && (MODE != BACK_UPDATE || a.B <= 192 || a.B > 224 || (int64_t)a.L * a.d * 4 > (int64_t)480 << 20);
   int rc = XFC_OK;
   *taken = back_step_for<MODE>(a.B, [&](auto s) {
     using S = decltype(s);
