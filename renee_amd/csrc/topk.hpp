@@ -301,15 +301,31 @@ __device__ __forceinline__ uint32_t wave_max32(uint32_t v) {
   step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
-// The same of 64-bit keys, uniform: by their upper halves, and by the lower ones of those that share the largest.
-// (By shuffles of whole keys, six steps through the LDS, topk_pick_kernel took 23.6 us at 16 x 131,072 and K = 5, now 14.)
+// The same of 64-bit keys, uniform: by their upper halves, and by the lower ones of those that share the largest, if there are
+// several.  (By shuffles of whole keys, six steps through the LDS, topk_pick_kernel took 23.6 us at 16 x 131,072 and K = 5, then 14.)
 __device__ __forceinline__ unsigned long long wave_max(unsigned long long k) {
   const uint32_t hi = wave_max32((uint32_t)(k >> 32));
-  const uint32_t lo = wave_max32((uint32_t)(k >> 32) == hi ? (uint32_t)k : 0u);
+  const unsigned long long with = __ballot((uint32_t)(k >> 32) == hi);
+  uint32_t lo;
+  if ((with & (with - 1)) == 0) lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)k, __builtin_ctzll(with));
+  else lo = wave_max32((uint32_t)(k >> 32) == hi ? (uint32_t)k : 0u);
   return ((unsigned long long)hi << 32) | lo;
 }
+// The K largest of the wave's keys, all different but for 0, in lanes 0 .. K - 1 (0 where there are fewer).
+__device__ __forceinline__ unsigned long long wave_top(unsigned long long key, int K, int lane) {
+  unsigned long long top = 0;
+  if (__ballot(key != 0) == 0) return top;
+  for (int r = 0; r < K; ++r) {
+    const unsigned long long m = wave_max(key);
+    if (m == 0) break;
+    if (lane == r) top = m;
+    if (key == m) key = 0;
+  }
+  return top;
+}
 
-// One workgroup per row.  Bound by reading the blocks' maxima and the chosen blocks' weights (1024 rows x 87,885 blocks, K = 5: 122 us,
+// One workgroup per row.  With few blocks or many rows bound by its instructions (25 us at 700 rows x 282 blocks, where seven of
+// a thread's eight fetches brought nothing and six of the eight waves put zeros in order): what has nothing to do is left out.  Else by reading the blocks' maxima and the chosen blocks' weights (1024 rows x 87,885 blocks, K = 5: 122 us,
 // 5 TB/s), on small batches by latency (16 x 8,192 blocks: 14 us): each thread finds the best of its blocks,
 // the K best threads are looked at again block by block (a wave each), and the K best blocks' scores are formed by MFMAs
 // that hold the row in all sixteen columns.  Keys are (score, id) as topk_entry makes them, all different but for 0.
@@ -324,7 +340,8 @@ __global__ void __launch_bounds__(512) topk_pick_kernel(PickArgs a) {
   const int K = a.topk;
   const float* maxima = a.bmax + (int64_t)row * a.ldb;
   const int quads = (a.n_blocks + 3) / 4;
-  auto quad = [&](int q) { return *reinterpret_cast<const float4v*>(maxima + 4 * (int64_t)(q < quads ? q : quads - 1)); };
+  // (a row's maxima are less than 2^32 bytes: a lane keeps one offset per load)
+  auto quad = [&](int q) { return *reinterpret_cast<const float4v*>(reinterpret_cast<const char*>(maxima) + 16u * (uint32_t)(q < quads ? q : quads - 1)); };
   // the best key below `bound` of blocks 4 q ..+3, whose maxima are v
   auto best_of = [&](int q, const float4v& v, unsigned long long bound) {
     unsigned long long best = 0;
@@ -338,19 +355,12 @@ __global__ void __launch_bounds__(512) topk_pick_kernel(PickArgs a) {
   // out[0..K) = the K largest of the workgroup's keys, in order; all threads of the workgroup call it
   auto top_of_all = [&](unsigned long long key, unsigned long long* out) {
     __syncthreads();
-    for (int r = 0; r < K; ++r) {
-      const unsigned long long m = wave_max(key);
-      if (lane == 0) list[wave * TOPK_MAX + r] = m;
-      if (key == m) key = 0;
-    }
+    const unsigned long long own = wave_top(key, K, lane);
+    if (lane < K) list[wave * TOPK_MAX + lane] = own;
     __syncthreads();
     if (wave == 0) {
-      unsigned long long k = lane < NW * K ? list[(lane / K) * TOPK_MAX + lane % K] : 0ull;
-      for (int r = 0; r < K; ++r) {
-        const unsigned long long m = wave_max(k);
-        if (lane == 0) out[r] = m;
-        if (k == m) k = 0;
-      }
+      const unsigned long long top = wave_top((lane & (TOPK_MAX - 1)) < K ? list[lane] : 0ull, K, lane);
+      if (lane < K) out[lane] = top;
     }
     __syncthreads();
   };
@@ -359,12 +369,14 @@ __global__ void __launch_bounds__(512) topk_pick_kernel(PickArgs a) {
   unsigned long long bound = ~0ull;  // blocks at or above it have been taken
   for (;;) {
     unsigned long long mine = 0;
-    for (int q = tid; q < quads; q += 512 * FETCH) {
+    for (int q = tid; q - lane < quads; q += 512 * FETCH) {
+      const int n = (quads - (q - lane) + 511) / 512;  // of the wave's fetches, those that bring anything new
       float4v v[FETCH];
 #pragma unroll
       for (int f = 0; f < FETCH; ++f) v[f] = quad(q + 512 * f);
 #pragma unroll
       for (int f = 0; f < FETCH; ++f) {
+        if (f >= n) break;
         const unsigned long long k = best_of(q + 512 * f, v[f], bound);
         mine = k > mine ? k : mine;
       }
