@@ -43,6 +43,8 @@ DW_UPDATE_TRAFFIC_BYTES = {2: (2.000 * 2815091.2 + 1.000 * 3932160.0) * 1024.0,
                            1: (2.000 * 285002.6 + 1.000 * 393216.0) * 1024.0,
                            3: (2.000 * 8609197.2 + 1.000 * 8436843.0) * 1024.0,
                            4: (2.000 * 49335013.9 + 1.000 * 50331648.0) * 1024.0}
+# the same of the one pass that makes both gradients and the update of up to 512 rows
+BACK_PASS_TRAFFIC_BYTES = {2: (2.000 * 2706564.4 + 1.000 * 3996673.8) * 1024.0}
 
 
 def _oracle_steps(B, L, d, c, seed, n_max, budget_s, warm):
@@ -167,14 +169,28 @@ def time_config(cfg: int, steps: int, warmup: int, seed: int, dev, wall_clock: b
            "ms_events": {"mean": ms_events, "median": per_step[steps // 2], "min": per_step[0]},
            "wall_s_incl_restore": wall_with_restore}
     if wall_clock:
-        # the contract's figure: K steps back to back between two synchronisations, nothing else in between
+        # the contract's figure: K steps back to back between two synchronisations, nothing else in between, through the
+        # entry point for a whole step (which takes both gradients and the update in one pass where that is the faster)
+        for _ in range(warmup + 1):
+            restore()
+            layer.step_csr(X, rowptr, colidx)
         restore()
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         for _ in range(steps):
-            step()
+            layer.step_csr(X, rowptr, colidx)
         torch.cuda.synchronize()
         out["wall_ms_per_step"] = (time.perf_counter() - t0) * 1e3 / steps
+        # both gradients and the update through their common entry point, in step order
+        ev = [[torch.cuda.Event(enable_timing=True) for _ in range(2)] for _ in range(steps)]
+        for e in ev:
+            restore()
+            layer.fwd_grad(X, rowptr=rowptr, colidx=colidx)
+            e[0].record()
+            layer.backward_pass(X)
+            e[1].record()
+        torch.cuda.synchronize()
+        out["backward_pass_ms"] = sum(e[0].elapsed_time(e[1]) for e in ev) / steps
         # the plain copy kernel on the same buffers: what an HBM read + write stream reaches on this box
         restore()
         torch.cuda.synchronize()
@@ -383,6 +399,17 @@ def main() -> int:
     upd_bytes = 8.0 * L * d  # read W, read M, write W, write M in fp16
     achieved = upd_bytes / (k_ms[2] * 1e-3) / 1e9
     traffic = DW_UPDATE_TRAFFIC_BYTES.get(args.config)
+    dw_roofline = {"kernel": "dw_kernel<DW_UPDATE> (dW GEMM + SGD-momentum update)", "bound": "hbm",
+                   "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
+                   "traffic": traffic,
+                   "achieved_incl_measured_traffic": None if traffic is None else traffic / (k_ms[2] * 1e-3) / 1e9,
+                   "copy_kernel_gbs_same_run": r.get("copy_gbs")}
+    roofline = dw_roofline  # of the step's longest kernel
+    if args.config in BACK_PASS_TRAFFIC_BYTES:
+        back_s, traffic = r["backward_pass_ms"] * 1e-3, BACK_PASS_TRAFFIC_BYTES[args.config]
+        roofline = dict(dw_roofline, kernel="back_wide_kernel (dX and dW GEMMs + SGD-momentum update, incl. the reduce of dX's partial sums)",
+                        achieved=upd_bytes / back_s / 1e9, frac=upd_bytes / back_s / 1e9 / HBM_PEAK_GBS, traffic=traffic,
+                        achieved_incl_measured_traffic=traffic / back_s / 1e9, tflops=2 * gemm_flop / back_s / 1e12)
     wall_ms = r["wall_ms_per_step"]
     wall_tf = 3 * gemm_flop / (wall_ms * 1e-3) / 1e12
     out = {
@@ -398,25 +425,23 @@ def main() -> int:
                    "batch": B, "d": d, "labels": L, "lr": 0.05, "momentum": 0.9,
                    "timed_state": "the K timed steps run back to back from W ~ N(0,0.02) as initialised and the "
                                   "momentum of step 1"},
-        "timing": "ms_per_step / value: wall clock over the K steps between two device synchronisations; "
-                  "ms_per_step_events and kernels_ms: per-step HIP event intervals on the launch stream with W and M "
-                  "restored before each step outside the interval",
+        "timing": "ms_per_step / value: wall clock over the K steps between two device synchronisations, each one call "
+                  "of XFCLayer.step_csr; ms_per_step_events and kernels_ms: per-step HIP event intervals on the launch "
+                  "stream with the step as three calls (fwd_grad, dx, dw_update) and W and M restored before each step "
+                  "outside the interval; backward_pass_ms: dx and dw_update as the one call that step_csr makes",
         "ms_per_step_events": r["ms_events"],
         "step_tflops": wall_tf,
         "mfma_peak_frac": wall_tf / MFMA_F16_PEAK_TFLOPS,
         "copy_gbs": r.get("copy_gbs"),
         "unfused_update": r.get("unfused_update"),
         "kernels_ms": s["kernels_ms"],
+        "backward_pass_ms": r.get("backward_pass_ms"),
         "fwd_grad_with_loss_ms": r.get("fwd_grad_with_loss_ms"),
         "kernels_tflops": {"fwd_grad": gemm_flop / k_ms[0] / 1e9, "dx": gemm_flop / k_ms[1] / 1e9,
                            "dw_update": gemm_flop / k_ms[2] / 1e9},
-        "roofline": {"kernel": "dw_kernel<DW_UPDATE> (dW GEMM + SGD-momentum update)", "bound": "hbm",
-                     "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": traffic,
-                     "achieved_incl_measured_traffic": None if traffic is None else traffic / (k_ms[2] * 1e-3) / 1e9,
-                     "copy_kernel_gbs_same_run": r.get("copy_gbs")},
-        # the two MFMA-bound kernels of the step, each against the dense fp16 matrix peak on 2*B*L*d flop
-        "rooflines": [
+        "roofline": roofline,
+        # the kernels of the step's three single calls: dW + update against HBM, the two MFMA-bound ones against the dense fp16 matrix peak on 2*B*L*d flop
+        "rooflines": [dw_roofline] + [
             {"kernel": "fwd_wide_kernel (logits GEMM + sigmoid epilogue, incl. positives_kernel)",
              "bound": "mfma", "achieved": gemm_flop / k_ms[0] / 1e9, "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
              "frac": gemm_flop / k_ms[0] / 1e9 / MFMA_F16_PEAK_TFLOPS},
