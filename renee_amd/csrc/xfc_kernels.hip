@@ -1655,12 +1655,14 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
   // 400,001 x 384 354 -> 326, 256 x 1,310,720 x 768 2.73 -> 2.53 ms; four micro-batches of 200 x 200,001 x 384 1163 -> 1076 us.
   // With an update of 193 to 224 rows, where some of the waves fetch no rows of G, only from some 480 MB on: 224 x 131,072 x 768 269
   // -> 273 us (240 277 -> 253), 200 x 200,001 x 512 296 -> 301, x 90,001 x 768 198 -> 200, x 700,001 x 768 1338 -> 1288.
-  const bool nts = nt && (MODE != BACK_UPDATE || a.B <= 192 || a.B > 224 || (int64_t)a.L * a.d * 4 > (int64_t)480 << 20);
+  // Nor with an update of up to 64 dims and a few rows: 9 x 1,990,020 x 64, with loss, 380 -> 400 us, 1,300,020 261 -> 273, 33
+  // 397 -> 404, 48 the same, but 64 421 -> 397, 33 x 1,000,003 x 128 316 -> 271.
+  const bool nts = nt && (MODE != BACK_UPDATE || ((a.d > 64 || a.B > 48) && (a.B <= 192 || a.B > 224 || (int64_t)a.L * a.d * 4 > (int64_t)480 << 20)));
   int rc = XFC_OK;
   *taken = back_step_for<MODE>(a.B, [&](auto s) {
     using S = decltype(s);
     const dim3 g((unsigned)(a.slices * a.ranges)), b(S::NT);
-    constexpr bool NT = MODE != BACK_OUT, LOADS = MODE == BACK_UPDATE && S::RQ == 4;
+    constexpr bool NT = MODE != BACK_OUT, LOADS = MODE == BACK_UPDATE && (S::RQ == 1 || S::RQ == 4);
     rc = nts           ? launch_k<back_step_kernel<S, MODE, NT, true>>(g, b, S::LDS_BYTES, st, a)
          : LOADS && nt ? launch_k<back_step_kernel<S, MODE, LOADS, false>>(g, b, S::LDS_BYTES, st, a)
                        : launch_k<back_step_kernel<S, MODE, false, false>>(g, b, S::LDS_BYTES, st, a);
@@ -1819,7 +1821,7 @@ int xfc_init(void) {
       back_step_for<MODE>(rows, [&](auto s) {
         using S = decltype(s);
         keep(raise_lds_limit<back_step_kernel<S, MODE, MODE != BACK_OUT, true>>(S::LDS_BYTES));
-        keep(raise_lds_limit<back_step_kernel<S, MODE, MODE == BACK_UPDATE && S::RQ == 4, false>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, MODE == BACK_UPDATE && (S::RQ == 1 || S::RQ == 4), false>>(S::LDS_BYTES));
         keep(raise_lds_limit<back_step_kernel<S, MODE, false, false>>(S::LDS_BYTES));
       });
   };

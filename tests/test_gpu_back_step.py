@@ -39,7 +39,9 @@ def _reference(G, X, W, d, L, scale):
 @pytest.mark.parametrize("B,L,d,pad", [(1, 1, 8, 0), (3, 64, 72, 8), (64, 65, 128, 0), (65, 63, 136, 8), (100, 1003, 64, 0),
                                        (128, 4097, 768, 0), (129, 513, 200, 16), (192, 777, 384, 0), (193, 70001, 64, 0),
                                        (199, 9001, 1024, 0), (256, 20011, 768, 8), (255, 130, 120, 0),
-                                       (100, 80001, 768, 0)])  # too large for the caches: loads with the hint
+                                       (100, 80001, 768, 0),   # too large for the caches: loads and stores with the hint
+                                       (48, 1100003, 56, 8),   # loads alone
+                                       (49, 950003, 64, 0)])
 def test_update_in_one_pass(dev, B, L, d, pad):
     G, X, W, M = _operands(dev, B, L, d, pad)
     lr, mu, wd, scale = 0.1, 0.9, 0.01, 2.0
