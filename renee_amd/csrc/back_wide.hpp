@@ -28,6 +28,7 @@
 // ten slots after the last MFMA or more, bases of fetches and stores that may have been spilled go through a scalar move.
 #pragma once
 #include "back_step.hpp"
+#include "back_wide_order.hpp"
 #include "wide_core.hpp"
 
 namespace xfc {
@@ -36,23 +37,11 @@ constexpr int BACK_WIDE_ROWS = 512;
 
 // Up to 64 RB rows.
 template <int RB_>
-struct BackWide {
-  static constexpr int RB = RB_, NT = 256, ROWS = 64 * RB, RP = 2 * RB;
+struct BackWide : BackWideOrder<RB_> {
+  static constexpr int RB = RB_, NT = 256, ROWS = 64 * RB;
   static constexpr int G_BYTES = ROWS * BACK_TILE * 2, W_BYTES = BACK_DIMS * BACK_TILE;  // an image of G; of half a tile's weights
   static constexpr int LDS_BYTES = 2 * G_BYTES + 4 * W_BYTES;
-  static constexpr int G_FETCH = 2 * RB;  // fetch instructions (8 rows x 64 labels of G) of a wave per tile
-  // The slots of half a tile: a wave's MFMAs, dW's and then dX's.
-  static constexpr int DW = 4 * RP, N = DW + 8 * RB;
-  static constexpr int BAR = N - 18;                // the barrier stands before this one
-  static constexpr int AHEAD = 3;                   // fragments of G are read so many groups of four slots ahead
-  static constexpr int TAIL = (N - BAR - 3) / 3 + 1;  // fetches behind the barrier: every third slot has one
-  static constexpr int PACE = RB >= 6 ? 1 : RB == 5 ? 2 : 3;      // pieces of the update per slot, 16 for each 16 labels, then their stores
-  static constexpr int UPD = DW + 10, STORE0 = UPD + 16 / PACE, STORE1 = UPD + 33 / PACE;
-  // Vector-memory operations a wave has at least behind the fetches of the weights it waits for, in a tile's first half and second
-  static constexpr int STORES = (STORE0 < BAR ? 2 : 0) + (STORE1 < BAR ? 2 : 0);
-  static constexpr int BEHIND0 = G_FETCH + STORES, BEHIND1 = STORES;
   static_assert(LDS_BYTES <= 160 * 1024 && ROWS <= BACK_WIDE_ROWS, "budget");
-  static_assert(TAIL >= 4 && 3 * (G_FETCH + 3) - (N - BAR - 2) < BAR && STORE1 < N && STORE0 - 4 < BAR && 4 * AHEAD < N - BAR, "schedule");
 
   // XOR on the 16-byte chunks of a row of G's image (128 bytes), and of the weights' (256)
   static __device__ __forceinline__ int g_swz(int row) {
@@ -315,19 +304,16 @@ __global__ void __launch_bounds__(S::NT, 1) back_wide_kernel(BackArgs a) {
       each<N>([&](auto slot) XFC_INLINE {
         constexpr int n = decltype(slot)::value;
         if constexpr (n == S::BAR) {
+          if (tile == edge) wait_vmcnt<S::wait(h, true)>();
           if constexpr (h == 0) {
-            if (tile == edge) {
-              wait_vmcnt<S::BEHIND0>();
-              clear_w(1);
-            }
-            wait_lds_vmcnt_barrier<S::BEHIND0>();
-          } else {
-            if (ragged || tile + 1 == edge) {
-              wait_vmcnt<S::BEHIND1>();
-              clear_g(tile + 1, lds_next);
-              if (tile + 1 == edge) clear_w(0);
-            }
-            wait_lds_vmcnt_barrier<S::BEHIND1>();
+            if (tile == edge) clear_w(1);
+          } else if (ragged || tile + 1 == edge) {
+            wait_vmcnt<S::wait(h, false)>();
+            clear_g(tile + 1, lds_next);
+            if (tile + 1 == edge) clear_w(0);
+          }
+          wait_lds_vmcnt_barrier<S::wait(h, false)>();
+          if constexpr (h == 1) {
             if (tile + 2 == edge) edge_g();
           }
         }
@@ -361,11 +347,10 @@ __global__ void __launch_bounds__(S::NT, 1) back_wide_kernel(BackArgs a) {
         if constexpr (n == S::STORE0 - 6) wq[1] = S::read16(own_at + h * S::W_BYTES + 4096);
         if constexpr (n == S::STORE0 - 4) mq[1] = S::read16(own_at + (2 + h) * S::W_BYTES + 4096);
         // fetches
-        constexpr int f = n > S::BAR ? n - S::BAR - 2 : n + N - S::BAR - 2;  // from the barrier's first on
-        if constexpr (f >= 0 && f % 3 == 0) {
-          if constexpr (n > S::BAR && f / 3 < 4) fetch_w(std::integral_constant<int, f / 3>{}, std::integral_constant<int, h>{}, tile, true);
-          else if constexpr (n > S::BAR && h == 1) fetch_g(std::integral_constant<int, f / 3 - 4>{}, lds_here, tile + 3 < t1);
-          else if constexpr (n < S::BAR && h == 0 && f / 3 - 4 < S::G_FETCH) fetch_g(std::integral_constant<int, f / 3 - 4>{}, lds_next, tile + 2 < t1);
+        if constexpr (constexpr int f = S::w_fetch(n); f >= 0) fetch_w(std::integral_constant<int, f>{}, std::integral_constant<int, h>{}, tile, true);
+        if constexpr (constexpr int j = S::g_fetch(h, n); j >= 0) {
+          if constexpr (h == 1) fetch_g(std::integral_constant<int, j>{}, lds_here, tile + 3 < t1);
+          else fetch_g(std::integral_constant<int, j>{}, lds_next, tile + 2 < t1);
         }
         if constexpr (n >= S::UPD && n <= S::STORE1)
           each<S::PACE>([&](auto u) XFC_INLINE { update(std::integral_constant<int, S::PACE * (n - S::UPD) + decltype(u)::value>{}); });
