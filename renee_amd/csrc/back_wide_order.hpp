@@ -1,8 +1,12 @@
-// The order of back_wide.hpp's fetches, stores and counted waits, as arithmetic on a slot's number: the kernel takes its schedule
-// from here, and tests/test_back_wide_order.py replays it on the host.  Plain C++, nothing of the GPU.
+// The order of back_wide.hpp's fetches, stores and counted waits, as arithmetic on a slot's number, and the lengths of its sums: the
+// kernel and its launch take both from here, and tests/test_back_wide_order.py goes through them on the host.  Plain C++, nothing of the GPU.
 #pragma once
 
 namespace xfc {
+
+// Into how many partial sums of dX a range of labels is divided: a tile's labels are part of one chain of MFMAs, as in xfc_dx, and
+// there are as many chains as xfc_dx has (`sums`) or more.
+constexpr int back_wide_parts(int ranges, int sums) { return (sums + ranges - 1) / ranges; }
 
 // For up to 64 RB rows.
 template <int RB_>

@@ -1622,16 +1622,15 @@ bool back_wide_for(int64_t B, int64_t d, Fn&& fn) {
   else fn(BackWide<8>{});
   return true;
 }
-// A workgroup per CU.  Parts as above, but a tile's labels are part of the chain of MFMAs, as in xfc_dx: as many chains as that has,
-// less an eighth of the ranges, since these come out a little closer to float64 than as many of xfc_dx's (512 rows x 131,072 x 768:
-// 42 chains 3.7e-7, xfc_dx's 40 3.9e-7).
+// A workgroup per CU, and at least as many chains as xfc_dx has, for no longer ones.  (With fewer the error of dX grows, as the root
+// of their lengths: 512 rows x 2,812,281 x 768, 128 of xfc_dx's, 126 here 1.01 times its 9.9e-7, 168 0.86; 300 x 2,080,392 x 1280, 125
+// 1.015 and 150 0.92.  The longer reduction takes 0.4 % of that step, 7.22 -> 7.24 ms.)
 BackPlan back_wide_plan(int64_t B, int64_t L, int64_t d) {
   const int64_t slices = d / BACK_DIMS, per = num_cus() / slices, tiles = ceil_div(L, BACK_TILE);
   const int64_t ranges = per < 1 ? 1 : per < tiles ? per : tiles;
   int tiles_m, tiles_n, sums, k_per_split;
   dx_plan((int)B, (int)d, (int)L, tiles_m, tiles_n, sums, k_per_split);
-  const int64_t parts = ceil_div(sums - ranges / 8, ranges);
-  return {(int)ranges, (int)(parts > 1 ? parts : 1)};
+  return {(int)ranges, back_wide_parts((int)ranges, sums)};
 }
 size_t back_ws_bytes(int64_t B, int64_t L, int64_t d) {
   if (B < 1 || B > BACK_WIDE_ROWS || L < 1 || d < 1 || (B > BACK_MAX_ROWS && d % BACK_DIMS)) return 0;

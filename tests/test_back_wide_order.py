@@ -13,16 +13,23 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "renee_amd", "csrc")
 
 
-@pytest.fixture(scope="module")
-def orders(tmp_path_factory):
-    """Per RB: G's fetches of a tile, how many of them stand behind the second half's barrier, wait[half][edge] and, slot by slot of
-    the two halves, what happens there."""
+def _compiled(tmp_path_factory, text, numbers):
+    """The lines that the program `text`, compiled beside the kernels' sources, prints when it reads `numbers`."""
     gxx = shutil.which("g++") or shutil.which("clang++", path="/opt/rocm/llvm/bin:/opt/rocm/lib/llvm/bin")
     if gxx is None:
         pytest.skip("no host compiler")
     tmp = tmp_path_factory.mktemp("order")
     src, exe = tmp / "order.cpp", tmp / "order"
-    src.write_text('#include <cstdio>\n#include "back_wide_order.hpp"\n'
+    src.write_text(text)
+    subprocess.run([gxx, "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    return subprocess.run([str(exe)], check=True, input=" ".join(map(str, numbers)), stdout=subprocess.PIPE, text=True).stdout.splitlines()
+
+
+@pytest.fixture(scope="module")
+def orders(tmp_path_factory):
+    """Per RB: G's fetches of a tile, how many of them stand behind the second half's barrier, wait[half][edge] and, slot by slot of
+    the two halves, what happens there."""
+    src_text = ('#include <cstdio>\n#include "back_wide_order.hpp"\n'
                    'template <int RB> void show() {\n'
                    '  using S = xfc::BackWideOrder<RB>;\n'
                    '  printf("order %d %d %d %d %d %d %d\\n", RB, S::G_FETCH, S::TAIL - 4, S::wait(0, false), S::wait(0, true), S::wait(1, false), S::wait(1, true));\n'
@@ -35,9 +42,8 @@ def orders(tmp_path_factory):
                    '      if (n == S::STORE1) printf("%d store 1\\n", h);\n'
                    '    }\n}\n'
                    'int main() { show<5>(); show<6>(); show<7>(); show<8>(); }\n')
-    subprocess.run([gxx, "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(src), "-o", str(exe)], check=True)
     out = {}
-    for line in subprocess.run([str(exe)], check=True, stdout=subprocess.PIPE, text=True).stdout.splitlines():
+    for line in _compiled(tmp_path_factory, src_text, []):
         v = line.split()
         if v[0] == "order":
             rb, g_fetch, tail, w0, e0, w1, e1 = (int(x) for x in v[1:])
@@ -124,3 +130,26 @@ def test_the_replay_finds_stores_that_were_counted_but_not_made(orders):
     assert all(late[8][whole] == {0, 1, 2, 3} for whole in range(1, 33)) and all(late[8][whole] == {2, 3} for whole in range(33, 49))
     assert all(late[rb][whole] == {2, 3} for rb, most in ((5, 32), (6, 16), (7, 32)) for whole in range(1, most + 1))
     assert not any(late[rb][whole] for rb in late for whole in range(49, 64))
+
+
+def test_no_chain_of_dx_is_longer_than_xfc_dx_has(tmp_path_factory):
+    """Rows, labels and dims of up to 32 slices of 128: the longest chain of MFMAs of a partial sum of dX against xfc_dx's, whose number of
+    sums is that of its workspace."""
+    from renee_amd._lib import lib
+
+    shapes = [(B, L, 128 * slices) for B in (257, 300, 384, 400, 449, 512) for slices in (1, 2, 3, 4, 5, 6, 8, 10, 12, 24, 32)
+              for L in (1, 63, 64, 65, 200, 448, 513, 1396, 1827, 1912, 4097, 20011, 131073, 320001, 655363, 1310720, 1537820, 2080392, 2812281)]
+    sums = [lib().xfc_gemm_workspace_bytes(B, d, L) // (B * d * 4) for B, L, d in shapes]
+    tiles = [-(-L // 64) for _, L, _ in shapes]
+    ranges = [min(256 // (d // 128), t) for (_, _, d), t in zip(shapes, tiles)]  # a workgroup per CU
+    text = ('#include <cstdio>\n#include "back_wide_order.hpp"\n'
+            'int main() { int r, s; while (scanf("%d %d", &r, &s) == 2) printf("%d\\n", xfc::back_wide_parts(r, s)); }\n')
+    parts = [int(line) for line in _compiled(tmp_path_factory, text, [n for rs in zip(ranges, sums) for n in rs])]
+    assert len(parts) == len(shapes)
+    for shape, t, r, s, p in zip(shapes, tiles, ranges, sums, parts):
+        most = -(-t // r)  # tiles of a range; part q of it has those from most * q / p on
+        lengths = [most * (q + 1) // p - most * q // p for q in range(p)]
+        assert p >= 1 and sum(lengths) == most, shape
+        assert 64 * max(lengths) <= -(-(-(-shape[1] // s)) // 64) * 64, shape
+    src = open(os.path.join(CSRC, "xfc_kernels.hip")).read()
+    assert src.count("return {(int)ranges, back_wide_parts((int)ranges, sums)};") == 1
