@@ -5,8 +5,11 @@
 namespace xfc {
 
 // Into how many partial sums of dX a range of labels is divided: a tile's labels are part of one chain of MFMAs, as in xfc_dx, and
-// there are as many chains as xfc_dx has (`sums`) or more.
-constexpr int back_wide_parts(int ranges, int sums) { return (sums + ranges - 1) / ranges; }
+// there are as many chains as xfc_dx has (`sums`) or more, but none without a tile.
+constexpr int back_wide_parts(int tiles, int ranges, int sums) {
+  const int want = (sums + ranges - 1) / ranges, most = (tiles + ranges - 1) / ranges;
+  return want < most ? want : most;
+}
 
 // For up to 64 RB rows.
 template <int RB_>

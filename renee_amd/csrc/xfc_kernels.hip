@@ -1630,7 +1630,7 @@ BackPlan back_wide_plan(int64_t B, int64_t L, int64_t d) {
   const int64_t ranges = per < 1 ? 1 : per < tiles ? per : tiles;
   int tiles_m, tiles_n, sums, k_per_split;
   dx_plan((int)B, (int)d, (int)L, tiles_m, tiles_n, sums, k_per_split);
-  return {(int)ranges, back_wide_parts((int)ranges, sums)};
+  return {(int)ranges, back_wide_parts((int)tiles, (int)ranges, sums)};
 }
 size_t back_ws_bytes(int64_t B, int64_t L, int64_t d) {
   if (B < 1 || B > BACK_WIDE_ROWS || L < 1 || d < 1 || (B > BACK_MAX_ROWS && d % BACK_DIMS)) return 0;

@@ -132,9 +132,9 @@ def test_the_replay_finds_stores_that_were_counted_but_not_made(orders):
     assert not any(late[rb][whole] for rb in late for whole in range(49, 64))
 
 
-def test_no_chain_of_dx_is_longer_than_xfc_dx_has(tmp_path_factory):
+def test_no_chain_of_dx_is_longer_than_xfc_dx_has_and_none_is_empty(tmp_path_factory):
     """Rows, labels and dims of up to 32 slices of 128: the longest chain of MFMAs of a partial sum of dX against xfc_dx's, whose number of
-    sums is that of its workspace."""
+    sums is that of its workspace.  (Sums without a tile made a step of 512 rows x 64 labels x 768 dims take 108 us, 67 as two passes.)"""
     from renee_amd._lib import lib
 
     shapes = [(B, L, 128 * slices) for B in (257, 300, 384, 400, 449, 512) for slices in (1, 2, 3, 4, 5, 6, 8, 10, 12, 24, 32)
@@ -143,13 +143,13 @@ def test_no_chain_of_dx_is_longer_than_xfc_dx_has(tmp_path_factory):
     tiles = [-(-L // 64) for _, L, _ in shapes]
     ranges = [min(256 // (d // 128), t) for (_, _, d), t in zip(shapes, tiles)]  # a workgroup per CU
     text = ('#include <cstdio>\n#include "back_wide_order.hpp"\n'
-            'int main() { int r, s; while (scanf("%d %d", &r, &s) == 2) printf("%d\\n", xfc::back_wide_parts(r, s)); }\n')
-    parts = [int(line) for line in _compiled(tmp_path_factory, text, [n for rs in zip(ranges, sums) for n in rs])]
+            'int main() { int t, r, s; while (scanf("%d %d %d", &t, &r, &s) == 3) printf("%d\\n", xfc::back_wide_parts(t, r, s)); }\n')
+    parts = [int(line) for line in _compiled(tmp_path_factory, text, [n for trs in zip(tiles, ranges, sums) for n in trs])]
     assert len(parts) == len(shapes)
     for shape, t, r, s, p in zip(shapes, tiles, ranges, sums, parts):
         most = -(-t // r)  # tiles of a range; part q of it has those from most * q / p on
         lengths = [most * (q + 1) // p - most * q // p for q in range(p)]
-        assert p >= 1 and sum(lengths) == most, shape
+        assert p >= 1 and min(lengths) >= 1 and sum(lengths) == most, shape
         assert 64 * max(lengths) <= -(-(-(-shape[1] // s)) // 64) * 64, shape
     src = open(os.path.join(CSRC, "xfc_kernels.hip")).read()
-    assert src.count("return {(int)ranges, back_wide_parts((int)ranges, sums)};") == 1
+    assert src.count("return {(int)ranges, back_wide_parts((int)tiles, (int)ranges, sums)};") == 1
