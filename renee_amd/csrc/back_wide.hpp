@@ -65,14 +65,11 @@ template <int N, class F>
 __device__ __forceinline__ void each(F&& f) { each_of(std::make_integer_sequence<int, N>{}, f); }
 
 // address = uniform 64-bit base + per-lane 32-bit offset (a store's data may not be overwritten by the next two instructions)
-template <bool NT, class V>
+template <class V>
 __device__ __forceinline__ void wide_store16(int64_t ubase, uint32_t voff, const V& v) {
   const uint64_t b = (uint64_t)uniform64(ubase);
   uint64_t t;  // see wide_load16
-  if constexpr (NT)
-    asm volatile("s_mov_b64 %0, %3\n\tglobal_store_dwordx4 %1, %2, %0 nt\n\ts_nop 1" : "=&s"(t) : "v"(voff), "v"(v), "s"(b) : "memory");
-  else
-    asm volatile("s_mov_b64 %0, %3\n\tglobal_store_dwordx4 %1, %2, %0\n\ts_nop 1" : "=&s"(t) : "v"(voff), "v"(v), "s"(b) : "memory");
+  asm volatile("s_mov_b64 %0, %3\n\tglobal_store_dwordx4 %1, %2, %0\n\ts_nop 1" : "=&s"(t) : "v"(voff), "v"(v), "s"(b) : "memory");
 }
 __device__ __forceinline__ void lane_load16(const void* p, uint32_t lds, int at) {
   const uint32_t m = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds);
@@ -81,7 +78,8 @@ __device__ __forceinline__ void lane_load16(const void* p, uint32_t lds, int at)
 
 #define XFC_INLINE __attribute__((always_inline))
 
-template <class S, bool NTL, bool NTS>
+// NT: weights and momentum are loaded as what will not be wanted again, for sizes that no cache holds until the next step.
+template <class S, bool NT>
 __global__ void __launch_bounds__(S::NT, 1) back_wide_kernel(BackArgs a) {
   constexpr int RB = S::RB, RP = S::RP, DW = S::DW, N = S::N;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
@@ -170,7 +168,7 @@ __global__ void __launch_bounds__(S::NT, 1) back_wide_kernel(BackArgs a) {
       at += left < 0 ? left * w_row : 0;
       v = (uint32_t)((lane_ >> 4) < left ? lane_ >> 4 : left > 0 ? left : 0) * (uint32_t)(a.ldw * 2) + w_col;
     }
-    wide_load16<NTL, true>(at, v, (f < 2 ? ws : ms) + half * S::W_BYTES + wave * 2048, e * 1024);
+    wide_load16<NT, true>(at, v, (f < 2 ? ws : ms) + half * S::W_BYTES + wave * 2048, e * 1024);
   };
 
   // X^T, A side of dW: rows 8 g ..+7 of each 32, dim 8 (i / 4) + 4 b + i % 4 of the wave's 32.  By way of G's images, 64 dims each.
@@ -290,8 +288,8 @@ __global__ void __launch_bounds__(S::NT, 1) back_wide_kernel(BackArgs a) {
         constexpr int lb = decltype(lb_)::value;
         const int64_t to = at_w + (32 * h + 16 * lb) * w_row;
         auto out = [&]() XFC_INLINE {
-          wide_store16<NTS>(to + w_to_m, w_out, mq[lb]);
-          wide_store16<NTS>(to, w_out, wq[lb]);
+          wide_store16(to + w_to_m, w_out, mq[lb]);
+          wide_store16(to, w_out, wq[lb]);
         };
         if (tile != edge) {
           out();

@@ -1686,19 +1686,15 @@ int launch_back_wide(BackArgs a, float* dX, int64_t lddx, float scale, void* ws,
     a.part = reinterpret_cast<float*>(ws);
     const dim3 g((unsigned)round_up(a.slices * a.ranges, 8)), b(S::NT);
     // Non-temporal loads where weights, momentum and G are more than the Infinity Cache holds (whole steps, without and with: 300
-    // rows x 60,001 labels x 768 dims 147 and 152 us, 512 rows 184 and 182, 512 x 131,072 x 256 167 and 158).  Non-temporal stores
-    // as well where the weights and the momentum are up to about twice that, and G less than half of it: they leave the cache to
-    // the weights that the next forward pass reads (512 x 131,073 x 768 383 -> 366 us, 90,001 263 -> 253, 180,001 the same,
-    // 1,310,720 3277 -> 3370; 512 x 300,001 x 256 354 -> 366).
-    const int64_t state = (int64_t)a.L * a.d * 4, Mi = (int64_t)1 << 20;
-    const bool loads = state + (int64_t)a.L * a.B * 2 > 224 * Mi, stores = state > 224 * Mi && state <= 560 * Mi && a.B <= a.d;
-    // The forward pass has left the caches the last labels' G and weights: those first (512 x 327,680 x 768 838 -> 825 us, 262,144 x
-    // 256 303 -> 286, 1,310,720 x 768 3233 -> 3217), but where the stores pass the caches by (131,072 x 768: 333 -> 336) or these
-    // hold everything (300 x 60,001 x 768: 147 -> 160).
-    a.back = loads && !stores;
-    rc = stores ? launch_k<back_wide_kernel<S, true, true>>(g, b, S::LDS_BYTES, st, a)
-         : loads ? launch_k<back_wide_kernel<S, true, false>>(g, b, S::LDS_BYTES, st, a)
-                 : launch_k<back_wide_kernel<S, false, false>>(g, b, S::LDS_BYTES, st, a);
+    // rows x 60,001 labels x 768 dims 147 and 152 us, 512 rows 184 and 182, 512 x 131,072 x 256 167 and 158).  There the forward pass has left the
+    // caches the last labels' G and weights: those first (512 x 327,680 x 768 838 -> 825 us, 262,144 x 256 303 -> 286, 1,310,720 x
+    // 768 3233 -> 3217), but not where these hold everything (300 x 60,001 x 768: 147 -> 160).
+    // Non-temporal stores, which leave the cache to the weights that the next forward pass reads, in the other order, gain up to 2 % in steps
+    // back to back and lose as much elsewhere.  Steps by themselves, each followed by 0.6 ms of matrix products over 96 MB, and each
+    // waited for, with such stores and as it is: 512 x 131,073 x 768 364 and 370, 1002 and 991, 395 and 378 us; 512 x 180,001 x 768 489
+    // and 483, 1116 and 1107, 509 and 495; 300 x 300,001 x 384 411 and 403, 1019 and 1011, 430 and 423.
+    a.back = (int64_t)a.L * a.d * 4 + (int64_t)a.L * a.B * 2 > (int64_t)224 << 20;
+    rc = a.back ? launch_k<back_wide_kernel<S, true>>(g, b, S::LDS_BYTES, st, a) : launch_k<back_wide_kernel<S, false>>(g, b, S::LDS_BYTES, st, a);
     if (rc) return;
     launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges * a.parts, scale, 0.0f, st);
     rc = check_launch();
@@ -1827,9 +1823,8 @@ int xfc_init(void) {
   for (int64_t rows : {320, 384, 448, 512})
     back_wide_for(rows, BACK_DIMS, [&](auto s) {
       using S = decltype(s);
-      keep(raise_lds_limit<back_wide_kernel<S, false, false>>(S::LDS_BYTES));
-      keep(raise_lds_limit<back_wide_kernel<S, true, false>>(S::LDS_BYTES));
-      keep(raise_lds_limit<back_wide_kernel<S, true, true>>(S::LDS_BYTES));
+      keep(raise_lds_limit<back_wide_kernel<S, false>>(S::LDS_BYTES));
+      keep(raise_lds_limit<back_wide_kernel<S, true>>(S::LDS_BYTES));
     });
   back_limits(std::integral_constant<int, BACK_UPDATE>{});
   back_limits(std::integral_constant<int, BACK_OUT>{});
