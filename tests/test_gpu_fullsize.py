@@ -158,8 +158,9 @@ def test_config4_streaming_shape(dev):
 def test_smaller_batches_fit_a_layer_sized_for_max_batch(dev):
     """A layer built for max_batch serves every smaller batch on the workspace it allocated once
     (dl_base.py:175-187, :318-340), also where the smaller batch's own plan needs more scratch than
-    max_batch's: dX at 260 rows of a 512-row layer (more label slices than 512 rows take), and the fused
-    top-5 at 256 rows of a 300-row layer with few feature dims (more label groups)."""
+    max_batch's: dX by itself at 260 rows of a 512-row layer (more label slices than 512 rows take; the
+    whole step takes dX and the update in one pass, with a plan of its own), and the fused top-5 at 256
+    rows of a 300-row layer with few feature dims (more label groups)."""
     L, d = 1310720, 768
     lay = XFCLayer(L, d, 512, dev, seed=5)
     B = 260
@@ -167,6 +168,8 @@ def test_smaller_batches_fit_a_layer_sized_for_max_batch(dev):
     P = synth.make_positives(B, L, 20, 5.0, 1.0, 5)
     px, py = (t.to(dev) for t in P.coo())
     W0 = lay.xfc_weight.clone()
+    lay.fwd_grad(X, px, py)
+    by_itself = lay.dx(B, scale=1.0).clone()
     dX = lay.xfc_backward(X, px, py, scale=1.0).clone()
     ref = torch.zeros(B, d, device=dev)
     for l0 in range(0, L, CHUNK):
@@ -177,6 +180,7 @@ def test_smaller_batches_fit_a_layer_sized_for_max_batch(dev):
         Gr[px[m], py[m] - l0] -= 1.0
         ref += Gr @ Wc
     assert float((dX - ref).norm() / ref.norm()) <= TOL
+    assert float((by_itself - ref).norm() / ref.norm()) <= TOL
     del lay, W0
     torch.cuda.empty_cache()
     L, d = 70001, 16
