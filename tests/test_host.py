@@ -339,14 +339,11 @@ def test_layer_workspace_covers_every_batch_size_up_to_max_batch():
     assert h.xfc_topk_workspace_bytes(256, 70001, 5) <= h.xfc_layer_workspace_bytes(300, 70001, 16, 64 * 300)
 
 
-def test_built_kernels_keep_the_distances_that_the_compiler_does_not_see_in_inline_asm():
-    """Five instructions must stand between a vector instruction that writes a scalar register (the compiler's v_readlane_b32 of a
-    spilled one) and a vector-memory instruction that reads it; the compiler keeps that distance for its own instructions but
-    does not see those in inline asm.  (In the 128-row top-K kernel global_load_lds_dwordx4 v98, s[4:5] stood three behind
-    v_readlane_b32 s5.)  Likewise two between a vector instruction and an MFMA that reads what it wrote (v_accvgpr_read_b32 of a fragment
-that did not fit the ordinary registers).  The built library's code is looked over, straight on through its branches."""
+def _built_code():
+    """The instructions of the library's kernels: {kernel: [(address, operation, operands, address branched to or None)]}."""
     import shutil
     import subprocess
+    import tempfile
 
     from renee_amd.build import LIB_PATH
 
@@ -354,14 +351,34 @@ that did not fit the ordinary registers).  The built library's code is looked ov
     bundler = shutil.which("clang-offload-bundler", path="/opt/rocm/llvm/bin:/opt/rocm/lib/llvm/bin:" + os.environ.get("PATH", ""))
     if not objdump or not bundler:
         pytest.skip("no disassembler")
-    import tempfile
-
     with tempfile.TemporaryDirectory() as tmp:
         fat, code = os.path.join(tmp, "fat"), os.path.join(tmp, "code")
         subprocess.run([objdump.replace("objdump", "objcopy"), f"--dump-section=.hip_fatbin={fat}", LIB_PATH, os.path.join(tmp, "copy")], check=True)
         subprocess.run([bundler, "--unbundle", "--type=o", "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--input={fat}", f"--output={code}"],
                        check=True)
-        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", "--no-leading-addr", code], check=True, stdout=subprocess.PIPE, text=True).stdout
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", code], check=True, stdout=subprocess.PIPE, text=True).stdout
+    kernels, current, start = {}, None, 0
+    for line in text.splitlines():
+        head = re.fullmatch(r"([0-9a-f]+) <(.+)>:", line)
+        if head:
+            start, current = int(head.group(1), 16), kernels.setdefault(head.group(2), [])
+            continue
+        instruction, _, comment = line.partition("//")
+        if current is None or not instruction.strip() or not comment:
+            continue
+        op, _, operands = instruction.strip().partition(" ")
+        to = re.search(r"<.*?(?:\+0x([0-9a-f]+))?>$", comment) if op.startswith(("s_branch", "s_cbranch")) else None
+        current.append((int(comment.split(":")[0], 16), op, operands, start + int(to.group(1) or "0", 16) if to else None))
+    return kernels
+
+
+def test_built_kernels_keep_the_distances_that_the_compiler_does_not_see_in_inline_asm():
+    """Five instructions must stand between a vector instruction that writes a scalar register (the compiler's v_readlane_b32 of a
+    spilled one) and a vector-memory instruction that reads it; the compiler keeps that distance for its own instructions but
+    does not see those in inline asm.  (In the 128-row top-K kernel global_load_lds_dwordx4 v98, s[4:5] stood three behind
+    v_readlane_b32 s5.)  Likewise two between a vector instruction and an MFMA that reads what it wrote (v_accvgpr_read_b32 of a fragment
+    that did not fit the ordinary registers).  The built library's code is looked over, backwards from each such instruction along
+    every way that leads to it, branches taken and not."""
 
     def vectors(operands):
         out = set()
@@ -375,31 +392,31 @@ that did not fit the ordinary registers).  The built library's code is looked ov
             out |= set(range(int(lo), int(hi) + 1))
         return out | {int(n) for n in re.findall(r"\bs(\d+)\b", operands)}
 
-    kernels = accesses = products = 0
-    kernel, recent, wrote = "", [], []  # the scalar and the vector registers that vector instructions wrote, instruction by instruction
-    for line in text.splitlines():
-        if line.endswith(">:"):
-            kernel, recent, wrote = line, [], []
-            kernels += 1
-            continue
-        line = line.split("//")[0].strip()
-        if not line:
-            continue
-        op, _, operands = line.partition(" ")
-        if re.match(r"(global|flat|scratch|buffer)_", op):
-            accesses += 1
-            close = set().union(*recent[-5:]) if recent else set()
-            assert not close & scalars(operands), (kernel, line)
-        if op.startswith("v_mfma"):
-            products += 1
-            close = set().union(*wrote[-2:]) if wrote else set()
-            assert not close & vectors(operands.partition(",")[2]), (kernel, line)
-        plain = op.startswith("v_") and not op.startswith("v_mfma")
-        if op == "s_nop":
-            recent += [set()] * (int(operands, 0) + 1)
-            wrote += [set()] * (int(operands, 0) + 1)
-        else:
-            recent.append(scalars(operands.split(",")[0]) if plain else set())
-            wrote.append(vectors(operands.split(",")[0]) if plain else set())
-        recent, wrote = recent[-8:], wrote[-4:]
-    assert kernels > 50 and accesses > 10000 and products > 4000
+    accesses = products = joins = 0
+    kernels = _built_code()
+    for kernel, code in kernels.items():
+        place = {at: n for n, (at, *_) in enumerate(code)}
+        before = [[n - 1] if n and code[n - 1][1] not in ("s_branch", "s_endpgm", "s_setpc_b64") else [] for n in range(len(code))]
+        for n, (_, op, _, to) in enumerate(code):
+            if to is not None:
+                before[place[to]].append(n)
+                joins += 1
+
+        def clear(n, left, reads, of):
+            """No vector instruction among the last `left` before n, whichever way, writes what is read."""
+            for m in before[n]:
+                _, op, operands, _ = code[m]
+                plain = op.startswith("v_") and not op.startswith("v_mfma")
+                assert not (plain and reads & of(operands.split(",")[0])), (kernel, code[n], code[m])
+                rest = left - (int(operands, 0) + 1 if op == "s_nop" else 1)
+                if rest > 0:
+                    clear(m, rest, reads, of)
+
+        for n, (_, op, operands, _) in enumerate(code):
+            if re.match(r"(global|flat|scratch|buffer)_", op):
+                accesses += 1
+                clear(n, 5, scalars(operands), scalars)
+            if op.startswith("v_mfma"):
+                products += 1
+                clear(n, 2, vectors(operands.partition(",")[2]), vectors)
+    assert len(kernels) > 50 and accesses > 10000 and products > 4000 and joins > 1000
