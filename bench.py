@@ -38,13 +38,13 @@ HBM_PEAK_GBS = 8000.0           # MI355X HBM3E, AMD's published figure
 
 # HBM bytes per launch of the dW+update kernel: rocprofv3 --pmc FETCH_SIZE (KiB, x2.000 from the 1 GiB
 # copy in the same run) + WRITE_SIZE (KiB, x1.000); see profiles/xfc_step_cfg2_hbm_traffic_pmc.md.
-DW_UPDATE_TRAFFIC_BYTES = {2: (2.000 * 2815091.2 + 1.000 * 3932160.0) * 1024.0,
+DW_UPDATE_TRAFFIC_BYTES = {2: (2.000 * 2634108.7 + 1.000 * 3932160.9) * 1024.0,
                            # the other configurations: profiles/xfc_step_other_configs_hbm_traffic_pmc.md
-                           1: (2.000 * 285002.6 + 1.000 * 393216.0) * 1024.0,
-                           3: (2.000 * 8609197.2 + 1.000 * 8436843.0) * 1024.0,
-                           4: (2.000 * 49335013.9 + 1.000 * 50331648.0) * 1024.0}
+                           1: (2.000 * 284904.1 + 1.000 * 393216.0) * 1024.0,
+                           3: (2.000 * 7261453.5 + 1.000 * 8436843.4) * 1024.0,
+                           4: (2.000 * 42552528.6 + 1.000 * 50331648.4) * 1024.0}
 # the same of the one pass that makes both gradients and the update of up to 512 rows
-BACK_PASS_TRAFFIC_BYTES = {2: (2.000 * 2706564.4 + 1.000 * 3996673.8) * 1024.0}
+BACK_PASS_TRAFFIC_BYTES = {2: (2.000 * 2706516.5 + 1.000 * 3996676.3) * 1024.0}
 
 
 def _oracle_steps(B, L, d, c, seed, n_max, budget_s, warm):

@@ -16,7 +16,7 @@
 // Schedule.  Half a tile is 16 RB MFMAs of a wave, dW's and then dX's; each is followed by its share of the rest: fragments of G
 // twelve MFMAs ahead, every third one a fetch, the update of the half's 32 labels under dX's.  One barrier a half, before the
 // last 18 MFMAs; the fetches of the next half's weights and momentum and of the next tile's G follow it, and the next half's first
-// fragments.  A wave waits for the fetches by count: vector-memory operations retire in order.
+// fragments.  A wave waits for the fetches by count: vector-memory operations retire in order.  The order itself is back_wide_order.hpp's.
 // Stores of 16 labels x 64 bytes, half lines that the neighbouring wave completes, cost nothing against whole lines here.
 //
 // Layouts.  G's image: rows of 64 labels, read along the labels (dX) and transposed (dW).  The 16-byte chunk c of row r lies at

@@ -49,7 +49,7 @@ __device__ __forceinline__ int c_row(int r, int lane) { return 8 * (r >> 2) + 4 
 // vmcnt.  gfx950 has one counter for a wave's vector-memory operations, and it counts them down in the order of their issue,
 // loads, fetches to the LDS and stores alike: "at most N outstanding" proves every operation done that has N or more behind it.
 // The compiler relies on the same (a load with two stores behind it is waited for with vmcnt(2)), and so do the counted waits
-// here and in back_step.hpp: operations that nobody counted, spills say, can only make them wait longer.
+// here, in wide_core.hpp, back_step.hpp and back_wide_order.hpp: operations that nobody counted, spills say, can only make them wait longer.
 //
 // Waits until at most N of this wave's vector-memory operations are outstanding, then joins the
 // workgroup barrier.  Written as one asm block: a plain __syncthreads() carries a fence that makes

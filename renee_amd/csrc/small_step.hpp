@@ -45,7 +45,9 @@ struct SmallArgs {
 // NW waves, SB blocks of 32 dims per wave, RB blocks of 16 rows (2 or 4); LINES: an instruction that loads or stores weights
 // or momentum covers 8 labels x 128 bytes (see back_step.hpp) instead of 16 x 64, and the loads and stores say that nothing will
 // want them again.  That is for sizes that no cache holds until the next step: 32 rows x 131,072 x 768 188 -> 169 us, x 700,001 961 ->
-// 888, 64 x 700,001 x 512 696 -> 621 (whole lines without the hint 720, half lines with it 1,048 at 32 x 700,001 x 768).  Below,
+// 888, 64 x 700,001 x 512 696 -> 621 (whole lines without the hint 720, half lines with it 1,048 at 32 x 700,001 x 768).  The stores' hint
+// alone, 32 x 131,072 x 768: back to back 171 -> 158, each step followed by a copy of 512 MiB 374 -> 361 or by 0.6 ms of matrix products
+// 767 -> 763, a new state's first 182 -> 179, waited for 165 -> 183, when whoever runs next need not write back what the caches hold.  Below,
 // half lines without the hint are faster, as the caches serve them: 64 x 20,011 x 512 33.0 against 34.5, 32 x 4,097 x 1024 24.8
 // against 28.1.
 template <int NW_, int SB_, int RB_, bool LINES_ = false>

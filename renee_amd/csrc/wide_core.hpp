@@ -15,8 +15,8 @@
 //
 // What bounds it.  A SIMD's matrix pipe takes 16 cycles for such an MFMA and 4 to issue it; with one wave per SIMD the
 // pipe stays busy as long as no more than three other instructions stand between two MFMAs.  Counters at 512 x 1,310,720
-// x 768 put dX at 2048 MFMA cycles of 2919 per stage (PipeCore: of 3100), the rest being the stage barrier (370), issue
-// slots of the fetches (address and M0 arithmetic included) and some 40 scalar instructions of loop control.  The other
+// x 768 put dX at 2048 MFMA cycles of 2850 per stage (PipeCore: of 3100), the rest being the stage barrier and issue
+// slots of the fetches (address and M0 arithmetic included).  The other
 // bound is power: with random operands the chip lowers its clock (1.6 to 1.9 GHz here) the more the busier the pipes and
 // the HBM are, so fewer LDS bytes and fewer stalled cycles count twice.  Measured on one card, back to back:
 //   forward pass 1.21 -> 1.11 ms, dX 1.046 -> 0.926 ms (batch 512, 1,310,720 labels, d = 768) against PipeCore;
@@ -25,8 +25,8 @@
 //   pass (1.31 -> 1.19 ms), a fill cursor with a byte of state per slot 4 % of both.
 // Then: what a stage does once (the turns of the rings, counts, the bumps, which the compiler had moved there) out of the gap
 // between the sub-steps and behind their last bumps, tile to tile addresses by one difference, and an epilogue's stores counted
-// instead of waited for: forward pass 1.055 -> 1.030 ms, dX 0.880 -> 0.865, top-5 of 1024 x 2,812,281 3.70 -> 3.65 ms, the logits of
-// top-100 at 512 x 1,310,720 1.113 -> 1.083.
+// instead of waited for: forward pass 1.055 -> 1.030 ms, dX 0.880 -> 0.865, the logits of top-100 at 512 x 1,310,720 1.113 ->
+// 1.083 (top-5 of 1024 x 2,812,281 3.70 and 3.65 ms, no more than its runs differ by).
 // Eight waves of 128 x 64 run no faster (1359 against 1360 TFLOP/s at 8192^3), read half again as many LDS bytes, and
 // leave 128 registers for everything that is not an accumulator.
 #pragma once

@@ -1512,7 +1512,8 @@ int launch_dw(int mode, DwArgs a, hipStream_t st) {
   // gradient: six-argument calls of 512 rows x 131,072 labels x 768 dims 384 -> 347 us, 128 rows 212 -> 178, 512 x 200,000 x 256 303
   // -> 261, x 80,000 x 768 258 -> 241, but x 32,768 118 -> 120.  Master weights: steps of 512 x 655,363 x 768 2868 -> 2813, 64 x
   // 200,001 717 -> 668, 256 x 131,072 x 256 201 -> 193, but 256 x 20,001 x 768 115 -> 123.  fp16 state: 1024 x 2,812,281 x 768 13.81 ->
-  // 13.67 ms, x 700,001 3.48 -> 3.44, but 800 x 200,001 x 512 684 -> 688, 700 x 131,072 x 256 228 -> 235.
+  // 13.67 ms, x 700,001 3.48 -> 3.44, but 800 x 200,001 x 512 684 -> 688, 700 x 131,072 x 256 228 -> 235.  Not only back to back: the
+  // calls of 512 rows x 131,072 each followed by a copy of 512 MiB 567 -> 522, by 0.6 ms of matrix products 1011 -> 978, waited for 409 -> 373.
   const int64_t weights = (int64_t)a.M * a.N, Mi = (int64_t)1 << 20;
   auto launch = [&](auto mode_tag, int64_t least) {
     constexpr int MODE = decltype(mode_tag)::value;
@@ -1610,8 +1611,8 @@ BackPlan back_plan(int64_t B, int64_t L, int64_t d, size_t ws_limit) {
   return {(int)ranges, (int)parts};
 }
 // The same for more rows (back_wide.hpp), the update only and widths of whole slices: there it is the faster at every size measured
-// (whole steps of 257 to 512 rows x 4,097 to 2,812,281 labels x 128 to 1024 dims: 1.11 to 1.41 times, least at 260 x 131,073 x 768,
-// most at 300 x 1,310,720 x 128; the two passes read the weights and G twice).  With 193 to 256 rows the kernel above is (131,073
+// (whole steps of 257 to 512 rows x 1 to 2,812,281 labels x 128 to 3072 dims: 1.05 to 1.44 times, least at 400 x 131,073 x 1280,
+// most at 320 x 400,001 x 128; the two passes read the weights and G twice).  With 193 to 256 rows the kernel above is (131,073
 // x 768: 303 us by that one, 306 by this).
 template <class Fn>
 bool back_wide_for(int64_t B, int64_t d, Fn&& fn) {
@@ -1656,6 +1657,9 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
   // -> 273 us (240 277 -> 253), 200 x 200,001 x 512 296 -> 301, x 90,001 x 768 198 -> 200, x 700,001 x 768 1338 -> 1288.
   // Nor with an update of up to 64 dims and a few rows: 9 x 1,990,020 x 64, with loss, 380 -> 400 us, 1,300,020 261 -> 273, 33
   // 397 -> 404, 48 the same, but 64 421 -> 397, 33 x 1,000,003 x 128 316 -> 271.
+  // Not only back to back: steps of 256 x 131,072 x 768 each followed by a copy of 512 MiB 483 -> 451, by 0.6 ms of matrix products 890
+  // -> 868, waited for 277 -> 274; of 100 x 400,001 x 384 566 -> 543 and 956 -> 941, but waited for 346 -> 385: what is stored through
+  // the caches is written back by whoever runs next.
   const bool nts = nt && (MODE != BACK_UPDATE || ((a.d > 64 || a.B > 48) && (a.B <= 192 || a.B > 224 || (int64_t)a.L * a.d * 4 > (int64_t)480 << 20)));
   int rc = XFC_OK;
   *taken = back_step_for<MODE>(a.B, [&](auto s) {
