@@ -8,13 +8,20 @@
 // the running sum) take the registers of half of X^T: 211 -> 220 us at 256 rows, dX as close to float64 as xfc_dx's.  Whole steps of 65 to 256 rows x 4,001 to 2,812,281 labels x 64 to 1024 dims: 1.03
 // to 1.5 times as fast.
 //
-// Split.  A workgroup owns a slice of 128 dims and a range of labels, which it walks 64 at a time.  Its eight waves are two
+// Split.  A workgroup owns a slice of 128 dims and every a.ranges-th tile of 64 labels, from the last one on.  Its eight waves are two
 // groups of 64 dims by four quarters; a quarter takes 16 of the tile's labels for dW and their update, and a quarter of the
 // rows for dX.  The weights cross between the quarters, and G between all, through the LDS, with one barrier a tile (two
 // images of each); X^T stays in the registers as far as they reach, the rest lies in the LDS as MFMA fragments, and dX stays in
 // the registers.  The weights and the momentum of the next two tiles are on their way, fetched unconditionally (past the last
 // tile it again), so that the waits count the loads exactly; G goes straight to the LDS, a tile ahead.  The slices of a range
 // run side by side on one XCD and meet in its L2 for G.
+//
+// Order.  The whole chip walks from the last labels to the first, as the forward pass has left the caches the last ones' G and weights
+// (up to 256 MB of them), and ends with those that the next forward pass begins with.  Each range a stretch of its own, from its first
+// label on -> this, whole steps: 256 rows x 131,072 labels x 768 dims 272 -> 263 us, 100 x 400,001 x 384 331 -> 322, 90 x 2,000,000 x
+// 128 639 -> 585, two micro-batches of 200 x 200,001 x 384 626 -> 596.  The fetches of G are dealt to the waves one by one, so that
+// with 193 to 255 rows, or 129 to 191, all have some: 199 x 131,072 x 768 with the loss 291 -> 283, and with the non-temporal stores, which
+// until then did not pay there, 261; 200 x 200,001 x 512 297 -> 267.  The first ones are sent before X^T is turned.
 //
 // Whole lines.  An instruction that loads or stores weights or momentum covers 8 labels x 128 bytes: lanes with i < 8 have
 // dims 8 g ..+7 of label i, the others dims 32 + 8 g ..+7 of label i - 8.  The products come out 16 labels x 32 dims at a
@@ -59,9 +66,9 @@ struct BackStep : Wave16 {
   static_assert(LDS_BYTES <= 160 * 1024 && ROWS <= BACK_MAX_ROWS && XR <= RP, "budget");
 };
 
-// NT, NTS: the arrays that are written (BACK_UPDATE: W and Mo, otherwise out) are loaded, and stored, as what will not be wanted
-// again, for sizes that no cache holds until the next step.
-template <class S, int MODE, bool NT, bool NTS>
+// NT: the arrays that are written (BACK_UPDATE: W and Mo, otherwise out) are loaded and stored as what will not be wanted again, for
+// sizes that no cache holds until the next step.
+template <class S, int MODE, bool NT>
 __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
   constexpr int RQ = S::RQ, RP = S::RP, XR = S::XR;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
@@ -76,8 +83,10 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
   const int slice = local % a.slices, range = (local / a.slices) * 8 + xcd;
   const int dim0 = slice * BACK_DIMS + dg * 64;
   const int part0 = range * a.parts, part1 = part0 + a.parts;
-  auto first_tile = [&](int part) { return (int)((int64_t)a.tiles * part / (a.ranges * a.parts)); };
-  const int t0 = first_tile(part0), t1 = first_tile(part1);
+  // Its tiles: every a.ranges-th from the range's number on, counted from the last one.
+  const int t1 = (a.tiles - range + a.ranges - 1) / a.ranges, most = (a.tiles + a.ranges - 1) / a.ranges;
+  auto l0_of = [&](int tile) { return (range + (t1 - 1 - tile) * a.ranges) * BACK_TILE; };
+  auto first_tile = [&](int part) { return part < part1 ? (int)((int64_t)most * (part - part0) / a.parts) : t1; };
   const int low = i & 7, second = i >> 3;  // of the whole-line layout: label (and low + 8), which 32 dims (fp32: which 16)
 
   // What a thread fetches.  Labels, rows and dims past the end repeat the last ones; they are cleared in the LDS, or belong
@@ -89,10 +98,10 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
   const int col = dim0 + 32 * second + 8 * g, colc = col < a.d ? col : a.d - 8;
   auto col32 = [&](int s) { return dim0 + 32 * s + 16 * second + 4 * g; };
   auto fetch = [&](int tile, Ahead& q) {
-    tile = tile < t1 ? tile : t1 - 1;
+    const int l0 = l0_of(tile < t1 ? tile : t1 - 1);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int label = tile * BACK_TILE + 16 * qt + 8 * h + low;
+      const int label = l0 + 16 * qt + 8 * h + low;
       const int64_t l = label < a.L ? label : a.L - 1;
       q.w[h] = load<NT && MODE == BACK_UPDATE>(reinterpret_cast<const half8*>(a.W + l * a.ldw + colc));
       if constexpr (MODE == BACK_UPDATE) q.m[h] = load<NT>(reinterpret_cast<const half8*>(a.Mo + l * a.ldm + colc));
@@ -109,9 +118,10 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
   // batch stay the zeros they were at the start, or come as such, and so do labels past the last eight.  The fetches are the
   // wave's last ones but for `after` loads and the tile's stores.
   auto fetch_g = [&](int tile, half_t* image) {
+    const int l0 = l0_of(tile);
 #pragma unroll
     for (int j = 0; j < S::G_FETCH; ++j) {
-      const int n = wave * S::G_FETCH + j, row0 = (n >> 1) * 16, k = n & 1, at = tile * BACK_TILE + 32 * k;
+      const int n = 8 * j + wave, row0 = (n >> 1) * 16, k = n & 1, at = l0 + 32 * k;
       if (row0 < a.B) {
         half_t* const dst = image + (k * S::ROWS + row0) * 32;
         if (row0 + 16 <= a.B && at + 32 <= a.L) {
@@ -123,9 +133,10 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
       }
     }
   };
-  if (t0 < t1) {
+  if (t1 > 0) {
 #pragma unroll
-    for (int t = 0; t < BACK_AHEAD; ++t) fetch(t0 + t, ahead[t]);
+    for (int t = 0; t < BACK_AHEAD; ++t) fetch(t, ahead[t]);
+    fetch_g(0, gs);
   }
 
   // X^T, A side of dW: rows 8 g ..+7 of each 32, dim 8 (i / 4) + 4 b + i % 4 of a block (in fp32: 16 b + i).  Rows past the
@@ -164,7 +175,6 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
     for (int q = tid; q < 4 * S::ROWS * 4; q += S::NT)
       if ((q >> 2) % S::ROWS >= a.B) *reinterpret_cast<half8*>(gs + q * 8) = half8{};
     S::barrier();  // X^T is whole, the images of the weights are free
-    if (t0 < t1) fetch_g(t0, gs);
   }
   float4v acc[RQ][4];  // rows 16 (RQ qt + rb) + i, dims 16 c + 4 g ..+3 of the group's 64
 #pragma unroll
@@ -192,14 +202,14 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
       end = first_tile(++part + 1);
     }
   };
-  leave(t0);
+  leave(0);
 
   int parity = 0;
   // Loads and stores of a wave between its fetches of G and the barrier that makes them known: of tiles that are whole.
   constexpr int AFTER = MODE == BACK_UPDATE ? 8 : MODE == BACK_ADD ? 10 : 6;
   bool exact = false;
   auto work = [&](int tile, Ahead& q) {
-    const int l0 = tile * BACK_TILE, label = l0 + 16 * qt + low;
+    const int l0 = l0_of(tile), label = l0 + 16 * qt + low;
     half_t* const gi = gs + parity * S::G_HALVES;
     half_t* const wi = ws + parity * S::W_HALVES;
     parity ^= 1;
@@ -281,8 +291,8 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
           wv[e] = (half_t)(wf - a.lr * mf);
         }
         if (label + 8 * h < a.L && col < a.d) {
-          store<NTS>(reinterpret_cast<half8*>(a.Mo + (int64_t)(label + 8 * h) * a.ldm + col), mv);
-          store<NTS>(reinterpret_cast<half8*>(a.W + (int64_t)(label + 8 * h) * a.ldw + col), wv);
+          store<NT>(reinterpret_cast<half8*>(a.Mo + (int64_t)(label + 8 * h) * a.ldm + col), mv);
+          store<NT>(reinterpret_cast<half8*>(a.W + (int64_t)(label + 8 * h) * a.ldw + col), wv);
         }
       }
     } else {
@@ -296,12 +306,12 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
           for (int e = 0; e < 4; ++e) v[e] = second == h ? dw[s][h][e] : far[e];
           if constexpr (MODE == BACK_ADD) v += a.beta * now.o[s][h];
           if (label + 8 * h < a.L && col32(s) < a.d)
-            store<NTS>(reinterpret_cast<float4v*>(a.out + (int64_t)(label + 8 * h) * a.ldo + col32(s)), v);
+            store<NT>(reinterpret_cast<float4v*>(a.out + (int64_t)(label + 8 * h) * a.ldo + col32(s)), v);
         }
     }
     leave(tile + 1);
   };
-  for (int t = t0; t < t1; t += BACK_AHEAD) {
+  for (int t = 0; t < t1; t += BACK_AHEAD) {
 #pragma unroll
     for (int s = 0; s < BACK_AHEAD; ++s)
       if (t + s < t1) work(t + s, ahead[s]);  // (the barriers: every wave has the same tiles)

@@ -1648,27 +1648,22 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
   a.slices = ceil_div(a.d, BACK_DIMS);
   a.tiles = ceil_div(a.L, BACK_TILE);
   a.part = reinterpret_cast<float*>(ws);
-  // What the pass reads and writes against the Infinity Cache (256 MB, G and the partial sums beside it).  (60,007 labels x 768
-  // dims, 256 rows: 87 us without the hint, 91 with; 700,001 x 768, 128 rows: 953 and 892.)
-  const bool nt = (int64_t)a.L * a.d * (MODE == BACK_UPDATE ? 4 : 6) > (int64_t)224 << 20;
-  // The same for the stores: whole steps of 256 rows x 131,072 labels x 768 dims 287 -> 259 us, 128 x 320,001 539 -> 498, 100 x
-  // 400,001 x 384 354 -> 326, 256 x 1,310,720 x 768 2.73 -> 2.53 ms; four micro-batches of 200 x 200,001 x 384 1163 -> 1076 us.
-  // With an update of 193 to 224 rows, where some of the waves fetch no rows of G, only from some 480 MB on: 224 x 131,072 x 768 269
-  // -> 273 us (240 277 -> 253), 200 x 200,001 x 512 296 -> 301, x 90,001 x 768 198 -> 200, x 700,001 x 768 1338 -> 1288.
-  // Nor with an update of up to 64 dims and a few rows: 9 x 1,990,020 x 64, with loss, 380 -> 400 us, 1,300,020 261 -> 273, 33
-  // 397 -> 404, 48 the same, but 64 421 -> 397, 33 x 1,000,003 x 128 316 -> 271.
+  // Non-temporal loads and stores of the arrays that are written, from where these push out of the Infinity Cache (256 MB) what the
+  // forward pass left there of G and the weights.  Whole steps with the hint from 224 MiB of weights and momentum on and with it
+  // as here, over three states in turn, over one, and over one with 0.6 ms of matrix products before each (us): 256 rows x 60,001 labels x
+  // 768 dims 148, 133, 796 -> 133, 132, 789; 100 x 70,001 x 768 142, 132, 763 -> 132, 131, 765; 200 x 120,001 x 384 146, 130, 783 -> 138,
+  // 137, 770; but 256 x 40,001 x 768 (117 MiB) 117, 99, 746 -> 107, 106, 740.  A gradient: two micro-batches of 128 x 50,001 x 384 (110
+  // MiB with W) 167, 158, 793 -> 169, 161, 794, of 100 x 90,001 x 384 (198) 270, 260, 907 -> 269, 263, 904.
   // Not only back to back: steps of 256 x 131,072 x 768 each followed by a copy of 512 MiB 483 -> 451, by 0.6 ms of matrix products 890
   // -> 868, waited for 277 -> 274; of 100 x 400,001 x 384 566 -> 543 and 956 -> 941, but waited for 346 -> 385: what is stored through
-  // the caches is written back by whoever runs next.
-  const bool nts = nt && (MODE != BACK_UPDATE || ((a.d > 64 || a.B > 48) && (a.B <= 192 || a.B > 224 || (int64_t)a.L * a.d * 4 > (int64_t)480 << 20)));
+  // the caches is written back by whoever runs next.  (Those are of the pass from the first labels on.)
+  const bool nt = (int64_t)a.L * a.d * (MODE == BACK_UPDATE ? 4 : 6) > (int64_t)(MODE == BACK_UPDATE ? 144 : 224) << 20;
   int rc = XFC_OK;
   *taken = back_step_for<MODE>(a.B, [&](auto s) {
     using S = decltype(s);
     const dim3 g((unsigned)(a.slices * a.ranges)), b(S::NT);
-    constexpr bool NT = MODE != BACK_OUT, LOADS = MODE == BACK_UPDATE && (S::RQ == 1 || S::RQ == 4);
-    rc = nts           ? launch_k<back_step_kernel<S, MODE, NT, true>>(g, b, S::LDS_BYTES, st, a)
-         : LOADS && nt ? launch_k<back_step_kernel<S, MODE, LOADS, false>>(g, b, S::LDS_BYTES, st, a)
-                       : launch_k<back_step_kernel<S, MODE, false, false>>(g, b, S::LDS_BYTES, st, a);
+    rc = nt ? launch_k<back_step_kernel<S, MODE, true>>(g, b, S::LDS_BYTES, st, a)
+            : launch_k<back_step_kernel<S, MODE, false>>(g, b, S::LDS_BYTES, st, a);
     if (rc) return;
     launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges * a.parts, scale, 0.0f, st);
     rc = check_launch();
@@ -1819,9 +1814,8 @@ int xfc_init(void) {
     for (int64_t rows : {64, 128, 192, 256})
       back_step_for<MODE>(rows, [&](auto s) {
         using S = decltype(s);
-        keep(raise_lds_limit<back_step_kernel<S, MODE, MODE != BACK_OUT, true>>(S::LDS_BYTES));
-        keep(raise_lds_limit<back_step_kernel<S, MODE, MODE == BACK_UPDATE && (S::RQ == 1 || S::RQ == 4), false>>(S::LDS_BYTES));
-        keep(raise_lds_limit<back_step_kernel<S, MODE, false, false>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, true>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, false>>(S::LDS_BYTES));
       });
   };
   for (int64_t rows : {320, 384, 448, 512})
