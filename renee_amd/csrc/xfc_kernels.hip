@@ -40,9 +40,12 @@ __device__ __forceinline__ void xcd_map(int id, int n_inner, int& inner, int& ou
 // ---------------------------------------------------------------------------------------------
 enum FwdMode { FWD_LINEAR = 0, FWD_SIGMOID = 1, FWD_SIGMOID_PLAIN = 2 };  // PLAIN: alpha 1, beta 0
 
-// Batches above 128 rows: 256 labels (the A side, contiguous in the output) x 256 rows, W running ahead.
+// Batches above 128 rows, as a rule: 256 labels (the A side, contiguous in the output) x 256 rows, W running ahead.
 using FwdWide = WideCore<256, 256, 2, 2, true>;
 static_assert(FwdWide::LDS_BYTES <= 160 * 1024, "LDS budget");
+// The same loop on 128 labels x 128 rows, two workgroups to a CU (see fwd_plan).
+using FwdWide128 = WideCore<128, 128, 2, 2, true>;
+static_assert(2 * FwdWide128::LDS_BYTES <= 160 * 1024, "two to a CU");
 // Batches of up to 128 and 64 rows (the reference's B = 32 plumbing case, --accum micro-batches, the last partial batch
 // of an epoch), where a 256-row tile would spend most of its MFMAs on padding: W streams from HBM, eight waves, three
 // ring slots.
@@ -98,9 +101,8 @@ struct FwdArgs {
 
 // Persistent: workgroup w takes tile ids w, w + gridDim.x, ... (gridDim.x a multiple of 8, so an
 // id keeps its XCD and the row tiles of one label tile run side by side on one L2).
-template <int MODE, bool BETA, bool LOSS = false, bool BMAX = false>
-__global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
-  using C = FwdWide;
+template <class C, int MODE, bool BETA, bool LOSS = false, bool BMAX = false>
+__global__ void __launch_bounds__(C::NT, 160 * 1024 / C::LDS_BYTES) fwd_wide_kernel(FwdArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   half_t* lds = reinterpret_cast<half_t*>(smem_raw);
   const int G = gridDim.x, w = blockIdx.x;
@@ -109,11 +111,11 @@ __global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
   const int wm = wave / C::WN, wn = wave % C::WN;
   double loss_acc = 0.0;  // LOSS: this lane's share of sum softplus(z)
 
-  auto get = [&](int item, C::Operand& oa, C::Operand& ob, int& kb, int& ke) {
+  auto get = [&](int item, typename C::Operand& oa, typename C::Operand& ob, int& kb, int& ke) {
     int mt, nt;
     xcd_map(item * G + w, a.tiles_m, mt, nt);
-    oa = C::Operand{a.W, a.ldw, nt < a.tiles_n ? nt * C::BM : 0, a.N};
-    ob = C::Operand{a.X, a.ldx, mt * C::BN, a.M};
+    oa = typename C::Operand{a.W, a.ldw, nt < a.tiles_n ? nt * C::BM : 0, a.N};
+    ob = typename C::Operand{a.X, a.ldx, mt * C::BN, a.M};
     kb = 0;
     ke = a.K;
   };
@@ -191,7 +193,7 @@ __global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
             }
           }
           if constexpr (BMAX) {
-            static_assert(MODE == FWD_LINEAR && C::FM == 8, "four blocks of logits, eight columns of each in a lane");
+            static_assert(MODE == FWD_LINEAR && (C::FM == 8 || C::FM == 4), "four blocks of logits or two, eight columns of each in a lane");
             half8 m8 = v8;
 #pragma unroll
             for (int e = 0; e < 8; ++e) m8[e] = !EDGE || col + e < a.N ? v8[e] : (half_t)-__builtin_huge_valf();
@@ -201,8 +203,9 @@ __global__ void __launch_bounds__(FwdWide::NT) fwd_wide_kernel(FwdArgs a) {
         }
         if constexpr (BMAX) {
           // lanes 16 g .. 16 g + 15 end up with block g of their row
-          const half_t m = pk_larger(pk_fold16(pk_fold32(largest[0], largest[2]), pk_fold32(largest[1], largest[3])));
-          if (row_in) a.bmax[(int64_t)row * a.ldb + (nt * C::BM + wm * C::TM) / LOGIT_BLOCK + (lane >> 4)] = m;
+          constexpr int BACK = C::FM / 2 - 2;  // (of two blocks the upper half of the lanes holds what the lower does)
+          const half_t m = pk_larger(pk_fold16(pk_fold32(largest[0], largest[BACK]), pk_fold32(largest[1], largest[1 + BACK])));
+          if (row_in && (lane >> 4) < C::FM / 2) a.bmax[(int64_t)row * a.ldb + (nt * C::BM + wm * C::TM) / LOGIT_BLOCK + (lane >> 4)] = m;
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -1379,21 +1382,66 @@ size_t fwd_ws_bytes(int64_t nnz) { return LOSS_PART_BYTES + (size_t)round_up((nn
 // Row-tile height for a batch of M rows (see FwdWide / FwdCore / FwdCore64).
 inline int row_tile(int64_t M) { return M <= 64 ? 64 : M <= 128 ? 128 : 256; }
 
-// Workgroups of the forward pass: one resident per CU (the number of tile ids is a multiple of 8).
-inline int64_t fwd_grid(int64_t ids) {
-  const int64_t grid = round_up(num_cus(), 8) < MAX_FWD_GRID ? round_up(num_cus(), 8) : MAX_FWD_GRID;
+// Workgroups of a persistent pass over tiles: one resident per CU (the number of tile ids is a multiple of 8).
+inline int64_t fwd_grid(int64_t ids, int per_cu = 1) {
+  const int64_t all = per_cu * round_up(num_cus(), 8), grid = all < MAX_FWD_GRID ? all : MAX_FWD_GRID;
   return grid < ids ? grid : ids;
 }
 
+// Which tile the forward pass takes: the labels [0, first) go by `tile`, those after them, if any, by FWD_WIDE128.
+enum FwdTile { FWD_64, FWD_128, FWD_WIDE, FWD_WIDE128 };
+struct FwdPlan {
+  FwdTile tile;
+  int64_t first;
+};
+inline int64_t fwd_ids(FwdTile t, int64_t M, int64_t n) {
+  const int64_t rows = t == FWD_64 ? 64 : t == FWD_WIDE ? 256 : 128, labels = t == FWD_WIDE128 ? 128 : 256;
+  return ceil_div(M, rows) * round_up(ceil_div(n, labels), 8);
+}
+// Large tiles move the fewest bytes through the fetch path, small ones fill the chip with few labels, leave no last round nearly
+// empty, and two of them on a CU work at each other's epilogues.  Time in rounds of the large tile, of 256 tiles on as many CUs: a round is
+// 8.6 us at 64 dims, 16.5 at 384, 26 at 768, 32 at 1024, 256 small tiles 0.31 of it (with the loss, whose epilogue is the longer,
+// 0.28); on the 128-row tile of the eight-wave loop a round is 14.5 to 22 us at 768 dims, and 256 small tiles 0.58 of it.  Measured
+// (fwd_grad without pairs, large and small, us): 200 rows x 8,001 labels x 768 dims 27.7 and 10.9, x 30,001 30.7 and 19.7, x
+// 60,001 34.6 and 35.7, x 131,073 84 and 73, 256 x 131,072 63 and 81, 512 x 60,001 57 and 70, x 20,001 x 256 21.1 and 13.5, 300 x
+// 131,073 x 384 80 and 61, 1024 x 131,072 x 768 219 and 262; 100 rows x 4,097 x 768 14.2 and 10.3, x 60,001 20.7 and 22.8, x 80,001 39.2 and
+// 34.3, x 250,001 85 and 96.  Where whole rounds of large tiles leave few labels over, those go by small tiles in a launch of their
+// own, 7.5 us and more: whole steps of 512 rows x 131,073 labels x 768 dims 379 -> 370 us, 256 rows 281 -> 273, 512 x 100,001 299 -> 290, with
+// the loss 512 x 131,073 414 -> 396.  Whole steps of few labels: 200 x 8,001 62.8 -> 45.4, 300 x 16,001 79 -> 68; top-100 of 200 x 20,001
+// 40.4 -> 29.3.
+FwdPlan fwd_plan(int64_t M, int64_t n, int64_t d, bool loss) {
+  if (M <= 64) return {FWD_64, n};
+  const int64_t cus = num_cus();
+  auto rounds = [&](FwdTile t, int64_t labels) { return (double)ceil_div(fwd_ids(t, M, labels), cus); };
+  if (M <= 128) return {0.58 * rounds(FWD_WIDE128, n) < rounds(FWD_128, n) ? FWD_WIDE128 : FWD_128, n};
+  const double small = loss ? 0.28 : 0.31, launch = 7.5 / (7.0 + 1.58 * (double)ceil_div(d, FwdWide::BK));
+  const double large = rounds(FWD_WIDE, n);
+  FwdPlan best = {FWD_WIDE, n};
+  double least = large;
+  if (small * rounds(FWD_WIDE128, n) < least) best = {FWD_WIDE128, n}, least = small * rounds(FWD_WIDE128, n);
+  // whole rounds, in label tiles that the 8 XCDs divide
+  const int64_t first = ((int64_t)large - 1) * cus / ceil_div(M, FwdWide::BN) / 8 * 8 * FwdWide::BM;
+  if (first > 0 && first < n && large - 1.0 + launch + small * rounds(FWD_WIDE128, n - first) < least) best = {FWD_WIDE, first};
+  return best;
+}
+// Workgroups of the pass, each with a partial sum of the loss.
+int64_t fwd_grid(const FwdPlan& p, int64_t M) { return fwd_grid(fwd_ids(p.tile, M, p.first), p.tile == FWD_WIDE128 ? 2 : 1); }
+int64_t fwd_rest_grid(const FwdPlan& p, int64_t M, int64_t n) {
+  if (p.first >= n) return 0;
+  const int64_t ids = fwd_ids(FWD_WIDE128, M, n - p.first), left = MAX_FWD_GRID - fwd_grid(p, M), grid = fwd_grid(ids, 2);
+  return grid < left ? grid : left;
+}
+
+template <class C>
 int launch_fwd_wide(int mode, const FwdArgs& a, dim3 g, hipStream_t st) {
-  constexpr int LDS = FwdWide::LDS_BYTES;
-  const dim3 b(FwdWide::NT);
-  if (a.loss_part) return launch_k<fwd_wide_kernel<FWD_SIGMOID_PLAIN, false, true>>(g, b, LDS, st, a);
-  if (mode == FWD_SIGMOID && a.beta != 0.f) return launch_k<fwd_wide_kernel<FWD_SIGMOID, true>>(g, b, LDS, st, a);
-  if (mode == FWD_SIGMOID && a.alpha == 1.0f) return launch_k<fwd_wide_kernel<FWD_SIGMOID_PLAIN, false>>(g, b, LDS, st, a);
-  if (mode == FWD_SIGMOID) return launch_k<fwd_wide_kernel<FWD_SIGMOID, false>>(g, b, LDS, st, a);
-  if (a.bmax) return launch_k<fwd_wide_kernel<FWD_LINEAR, false, false, true>>(g, b, LDS, st, a);
-  return launch_k<fwd_wide_kernel<FWD_LINEAR, false>>(g, b, LDS, st, a);
+  constexpr int LDS = C::LDS_BYTES;
+  const dim3 b(C::NT);
+  if (a.loss_part) return launch_k<fwd_wide_kernel<C, FWD_SIGMOID_PLAIN, false, true>>(g, b, LDS, st, a);
+  if (mode == FWD_SIGMOID && a.beta != 0.f) return launch_k<fwd_wide_kernel<C, FWD_SIGMOID, true>>(g, b, LDS, st, a);
+  if (mode == FWD_SIGMOID && a.alpha == 1.0f) return launch_k<fwd_wide_kernel<C, FWD_SIGMOID_PLAIN, false>>(g, b, LDS, st, a);
+  if (mode == FWD_SIGMOID) return launch_k<fwd_wide_kernel<C, FWD_SIGMOID, false>>(g, b, LDS, st, a);
+  if (a.bmax) return launch_k<fwd_wide_kernel<C, FWD_LINEAR, false, false, true>>(g, b, LDS, st, a);
+  return launch_k<fwd_wide_kernel<C, FWD_LINEAR, false>>(g, b, LDS, st, a);
 }
 
 template <class C>
@@ -1411,23 +1459,40 @@ int launch_fwd_c(int mode, const FwdArgs& a, dim3 g, hipStream_t st) {
 int launch_fwd(int mode, const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, half_t* out, int64_t ldo, int M,
                int N, int K, int n_store, float alpha, float beta, hipStream_t st, double* loss_part = nullptr,
                half_t* bmax = nullptr, int64_t ldb = 0) {
+  const FwdPlan p = fwd_plan(M, n_store, K, loss_part != nullptr);
   FwdArgs a;
   a.X = X; a.ldx = ldx; a.W = W; a.ldw = ldw; a.out = out; a.ldo = ldo;
-  a.M = M; a.N = N; a.K = K; a.n_store = n_store; a.alpha = alpha; a.beta = beta;
+  a.M = M; a.N = p.first < N ? (int)p.first : N; a.K = K; a.n_store = (int)p.first; a.alpha = alpha; a.beta = beta;
   a.loss_part = loss_part;
   a.bmax = bmax; a.ldb = ldb;
-  a.tiles_m = ceil_div(M, row_tile(M));
-  a.tiles_n = ceil_div(n_store, FwdWide::BM);
-  const int64_t ids = (int64_t)a.tiles_m * round_up(a.tiles_n, 8);
-  if (ids <= 0) return XFC_OK;
-  if (ids > 0x7fffffff) return XFC_ERR_INVALID;
-  a.n_ids = (int)ids;
-  const dim3 g((unsigned)fwd_grid(ids));
-  switch (row_tile(M)) {
-    case 64: return launch_fwd_c<FwdCore64>(mode, a, g, st);
-    case 128: return launch_fwd_c<FwdCore>(mode, a, g, st);
-    default: return launch_fwd_wide(mode, a, g, st);
+  auto tiles = [&](FwdTile t, int64_t n) {
+    a.tiles_n = ceil_div(n, t == FWD_WIDE128 ? FwdWide128::BM : FwdWide::BM);
+    const int64_t ids = fwd_ids(t, M, n);
+    a.tiles_m = (int)(ids / round_up(a.tiles_n, 8));
+    a.n_ids = (int)ids;
+    return ids <= 0x7fffffff;
+  };
+  if (M <= 0 || n_store <= 0) return XFC_OK;
+  if (!tiles(p.tile, p.first)) return XFC_ERR_INVALID;
+  const int64_t grid = fwd_grid(p, M), rest = fwd_rest_grid(p, M, n_store);
+  const dim3 g((unsigned)grid);
+  int rc;
+  switch (p.tile) {
+    case FWD_64: rc = launch_fwd_c<FwdCore64>(mode, a, g, st); break;
+    case FWD_128: rc = launch_fwd_c<FwdCore>(mode, a, g, st); break;
+    case FWD_WIDE: rc = launch_fwd_wide<FwdWide>(mode, a, g, st); break;
+    default: rc = launch_fwd_wide<FwdWide128>(mode, a, g, st); break;
   }
+  if (rc || rest == 0) return rc;
+  // the labels that whole rounds have left (a multiple of 256 lies before them)
+  a.W += p.first * ldw;
+  a.out += p.first;
+  a.N = N - (int)p.first;
+  a.n_store = n_store - (int)p.first;
+  if (loss_part) a.loss_part += grid;
+  if (bmax) a.bmax += p.first / LOGIT_BLOCK;
+  tiles(FWD_WIDE128, a.n_store);
+  return launch_fwd_wide<FwdWide128>(mode, a, dim3((unsigned)rest), st);
 }
 
 // Split count for dX: a multiple of 8 slices of the label axis (workgroup ids are dealt round-robin over
@@ -1775,12 +1840,17 @@ int xfc_abi_version(void) { return XFC_ABI_VERSION; }
 int xfc_init(void) {
   hipError_t e = hipSuccess;
   auto keep = [&](hipError_t r) { if (e == hipSuccess) e = r; };
-  keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID_PLAIN, false, true>>(FwdWide::LDS_BYTES));
-  keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID, true>>(FwdWide::LDS_BYTES));
-  keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID, false>>(FwdWide::LDS_BYTES));
-  keep(raise_lds_limit<fwd_wide_kernel<FWD_SIGMOID_PLAIN, false>>(FwdWide::LDS_BYTES));
-  keep(raise_lds_limit<fwd_wide_kernel<FWD_LINEAR, false>>(FwdWide::LDS_BYTES));
-  keep(raise_lds_limit<fwd_wide_kernel<FWD_LINEAR, false, false, true>>(FwdWide::LDS_BYTES));
+  auto wide_limits = [&](auto core_tag) {
+    using C = typename decltype(core_tag)::type;
+    keep(raise_lds_limit<fwd_wide_kernel<C, FWD_SIGMOID_PLAIN, false, true>>(C::LDS_BYTES));
+    keep(raise_lds_limit<fwd_wide_kernel<C, FWD_SIGMOID, true>>(C::LDS_BYTES));
+    keep(raise_lds_limit<fwd_wide_kernel<C, FWD_SIGMOID, false>>(C::LDS_BYTES));
+    keep(raise_lds_limit<fwd_wide_kernel<C, FWD_SIGMOID_PLAIN, false>>(C::LDS_BYTES));
+    keep(raise_lds_limit<fwd_wide_kernel<C, FWD_LINEAR, false>>(C::LDS_BYTES));
+    keep(raise_lds_limit<fwd_wide_kernel<C, FWD_LINEAR, false, false, true>>(C::LDS_BYTES));
+  };
+  wide_limits(std::type_identity<FwdWide>{});
+  wide_limits(std::type_identity<FwdWide128>{});
   keep(raise_lds_limit<score_wide_kernel<ScoreWide>>(ScoreWide::LDS_BYTES));
   keep(raise_lds_limit<score_wide_kernel<ScoreWide128>>(ScoreWide128::LDS_BYTES));
   keep(raise_lds_limit<topk_list_kernel<ListCore>>(TopkLds<ListCore>::BYTES));
@@ -1969,6 +2039,7 @@ static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw,
   // label columns L .. round_up(L, 8) are written as zero so that G can be read in 16-byte
   // pieces along the label axis by the dX and dW kernels (ldg is a multiple of 8, so they exist)
   const int64_t n_store = round_up(L, 8);
+  const FwdPlan plan = fwd_plan(B, n_store, d, loss != nullptr);
   int rc = launch_fwd(FWD_SIGMOID, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)G, ldg, (int)B, (int)L, (int)d,
                       (int)n_store, 1.0f, 0.0f, st, loss_part);
   if (rc) return rc;
@@ -1979,14 +2050,13 @@ static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw,
                          rowptr, colidx, pos_x, pos_y, nnz, (int)B, L, (int)d, (half_t*)G, ldg, loss_pos);
     };
     if (!loss) launch(positives_kernel<POS_G>);
-    else if (row_tile(B) == FwdWide::BN) launch(positives_kernel<POS_LOSS_WIDE>);
+    else if (plan.tile == FWD_WIDE || plan.tile == FWD_WIDE128) launch(positives_kernel<POS_LOSS_WIDE>);
     else launch(positives_kernel<POS_LOSS>);
     if ((rc = check_launch())) return rc;
   }
   if (loss) {
-    const int64_t ids = (int64_t)ceil_div(B, row_tile(B)) * round_up(ceil_div(n_store, FwdWide::BM), 8);
-    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(1024), 0, st, (const double*)loss_part, (int)fwd_grid(ids),
-                       (const float*)loss_pos, nnz, loss);
+    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(1024), 0, st, (const double*)loss_part,
+                       (int)(fwd_grid(plan, B) + fwd_rest_grid(plan, B, n_store)), (const float*)loss_pos, nnz, loss);
     return check_launch();
   }
   return XFC_OK;
