@@ -66,11 +66,12 @@ struct BackStep : Wave16 {
   static_assert(LDS_BYTES <= 160 * 1024 && ROWS <= BACK_MAX_ROWS && XR <= RP, "budget");
 };
 
-// NT: the arrays that are written (BACK_UPDATE: W and Mo, otherwise out) are loaded and stored as what will not be wanted again, for
-// sizes that no cache holds until the next step.
-template <class S, int MODE, bool NT>
+// HOW the arrays that are written (BACK_UPDATE: W and Mo, otherwise out) are stored; PAST: and loaded, as what will not be wanted
+// again.  THROUGH: the partial sums as well.
+template <class S, int MODE, int HOW>
 __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
   constexpr int RQ = S::RQ, RP = S::RP, XR = S::XR;
+  constexpr bool NT = HOW == PAST;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   half_t* const gs = reinterpret_cast<half_t*>(smem_raw);  // [2 images][2 halves of the tile][ROWS][32]
   half_t* const ws = gs + 2 * S::G_HALVES;                 // [2 images][2 halves of the tile][4 blocks of 32 dims][32][32]
@@ -192,7 +193,7 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
       for (int rb = 0; rb < RQ; ++rb) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          if (row < a.B && at + 16 * c < a.d) *reinterpret_cast<float4v*>(dst + 16 * c) = acc[rb][c];
+          if (row < a.B && at + 16 * c < a.d) store<HOW == THROUGH ? THROUGH : CACHED>(reinterpret_cast<float4v*>(dst + 16 * c), acc[rb][c]);
           acc[rb][c] = float4v{0.f, 0.f, 0.f, 0.f};
         }
         row += 16;
@@ -291,8 +292,8 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
           wv[e] = (half_t)(wf - a.lr * mf);
         }
         if (label + 8 * h < a.L && col < a.d) {
-          store<NT>(reinterpret_cast<half8*>(a.Mo + (int64_t)(label + 8 * h) * a.ldm + col), mv);
-          store<NT>(reinterpret_cast<half8*>(a.W + (int64_t)(label + 8 * h) * a.ldw + col), wv);
+          store<HOW>(reinterpret_cast<half8*>(a.Mo + (int64_t)(label + 8 * h) * a.ldm + col), mv);
+          store<HOW>(reinterpret_cast<half8*>(a.W + (int64_t)(label + 8 * h) * a.ldw + col), wv);
         }
       }
     } else {
@@ -306,7 +307,7 @@ __global__ void __launch_bounds__(S::NT, 2) back_step_kernel(BackArgs a) {
           for (int e = 0; e < 4; ++e) v[e] = second == h ? dw[s][h][e] : far[e];
           if constexpr (MODE == BACK_ADD) v += a.beta * now.o[s][h];
           if (label + 8 * h < a.L && col32(s) < a.d)
-            store<NT>(reinterpret_cast<float4v*>(a.out + (int64_t)(label + 8 * h) * a.ldo + col32(s)), v);
+            store<HOW>(reinterpret_cast<float4v*>(a.out + (int64_t)(label + 8 * h) * a.ldo + col32(s)), v);
         }
     }
     leave(tile + 1);

@@ -37,10 +37,23 @@ typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
 __device__ __attribute__((aligned(16))) const uint32_t g_zero16[4] = {0u, 0u, 0u, 0u};
 
-template <bool NT, class T>
+// How an output is stored.  CACHED: it stays in the L2 until something pushes it out or the kernel ends, which waits for what its
+// eight L2s (32 MB) still hold to be written back.  THROUGH: past the L2 to the Infinity Cache at once (agent scope): nothing is left
+// to write back, for outputs about as large as the L2s or smaller; more of them, or pieces of lines, pass the fabric faster when the L2
+// has gathered them.  PAST: as what will not be wanted again, past the Infinity Cache too, for outputs that it would not hold.
+enum StoreHow { CACHED = 0, PAST = 1, THROUGH = 2 };
+template <int HOW, class T>
 __device__ __forceinline__ void store(T* p, const T& v) {
-  if constexpr (NT) __builtin_nontemporal_store(v, p);
-  else *p = v;
+  static_assert(HOW != THROUGH || sizeof(T) == 16 || sizeof(T) == 8 || sizeof(T) == 4, "piece");
+  if constexpr (HOW == PAST) {
+    __builtin_nontemporal_store(v, p);
+  } else if constexpr (HOW == THROUGH) {  // (a store's data may not be overwritten by the next two instructions)
+    if constexpr (sizeof(T) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+    else if constexpr (sizeof(T) == 8) asm volatile("global_store_dwordx2 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+    else asm volatile("global_store_dword %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+  } else {
+    *p = v;
+  }
 }
 
 // Row of C held by accumulator register r of a 32x32 block, for this lane.

@@ -347,8 +347,8 @@ __global__ void __launch_bounds__(S::NT, S::WAVES_PER_EU) small_step_kernel(Smal
         }
         const int label = l0 + label_of(lb, s);
         if (label < a.L) {
-          store<S::LINES>(reinterpret_cast<half8*>(a.Mo + (int64_t)label * a.ldm + dim0 + col_of(s)), mv);
-          store<S::LINES>(reinterpret_cast<half8*>(a.W + (int64_t)label * a.ldw + dim0 + col_of(s)), wv);
+          store<S::LINES ? PAST : CACHED>(reinterpret_cast<half8*>(a.Mo + (int64_t)label * a.ldm + dim0 + col_of(s)), mv);
+          store<S::LINES ? PAST : CACHED>(reinterpret_cast<half8*>(a.W + (int64_t)label * a.ldw + dim0 + col_of(s)), wv);
         }
         if constexpr (!AHEAD) __builtin_amdgcn_sched_barrier(0);
       };

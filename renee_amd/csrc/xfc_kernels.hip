@@ -97,6 +97,7 @@ struct FwdArgs {
   double* loss_part;                // LOSS: one partial sum per workgroup
   half_t* bmax; int64_t ldb;        // BMAX: [M][ldb] the largest stored value of every LOGIT_BLOCK columns
   int tiles_m, tiles_n, n_ids;      // n_ids = tiles_m * round_up(tiles_n, 8)
+  bool through;                     // out is stored through the L2 (see launch_fwd)
 };
 
 // Persistent: workgroup w takes tile ids w, w + gridDim.x, ... (gridDim.x a multiple of 8, so an
@@ -185,7 +186,8 @@ __global__ void __launch_bounds__(C::NT, 160 * 1024 / C::LDS_BYTES) fwd_wide_ker
           if (row_in) {
             if (!EDGE || col + 8 <= a.n_store) {
               // (a non-temporal store of half a line is written back before the other half comes: 1.19 against 1.14 ms)
-              *reinterpret_cast<half8*>(dst + 32 * p) = v8;
+              if (C::FM == 4 && a.through) store<THROUGH>(reinterpret_cast<half8*>(dst + 32 * p), v8);
+              else *reinterpret_cast<half8*>(dst + 32 * p) = v8;
             } else {
 #pragma unroll
               for (int e = 0; e < 8; ++e)
@@ -340,7 +342,8 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
               // uniform part + per-lane part computed once per tile: no per-strip vector multiply
               half_t* dst = a.out + ((int64_t)(m0 + wm * C::TM + fm * 32 + 8 * q) * a.ldo + n0 + wn * C::TN) + lane_off[p];
               if (!EDGE || col + 8 <= a.n_store) {
-                __builtin_nontemporal_store(v8, reinterpret_cast<half8*>(dst));  // G is not re-read before it leaves the L2
+                if (a.through) store<THROUGH>(reinterpret_cast<half8*>(dst), v8);
+                else store<PAST>(reinterpret_cast<half8*>(dst), v8);  // G is not re-read before it leaves the L2
               } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
@@ -846,6 +849,7 @@ struct DxArgs {
 };
 
 // One workgroup per (output tile, slice of the label axis); the tiles of one slice get ids on one XCD.
+template <int HOW>
 __global__ void __launch_bounds__(DxWide::NT) dx_wide_kernel(DxArgs a) {
   using C = DxWide;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
@@ -860,7 +864,7 @@ __global__ void __launch_bounds__(DxWide::NT) dx_wide_kernel(DxArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be
   const int wm = wave / C::WN, wn = wave % C::WN;
   float* part = a.part + (int64_t)split * a.M * a.N;
-  auto store = [&](float4v (&acc)[C::FM][C::FN]) {
+  auto leave = [&](float4v (&acc)[C::FM][C::FN]) {
 #pragma unroll
     for (int fn = 0; fn < C::FN; ++fn) {
       const int row = m0 + wn * C::TN + fn * 16 + (lane & 15);
@@ -868,7 +872,7 @@ __global__ void __launch_bounds__(DxWide::NT) dx_wide_kernel(DxArgs a) {
 #pragma unroll
         for (int fm = 0; fm < C::FM; ++fm) {
           const int col = n0 + wm * C::TM + fm * 16 + 4 * (lane >> 4);
-          if (col < a.N) *reinterpret_cast<float4v*>(part + (int64_t)row * a.N + col) = acc[fm][fn];
+          if (col < a.N) store<HOW>(reinterpret_cast<float4v*>(part + (int64_t)row * a.N + col), acc[fm][fn]);
         }
       }
     }
@@ -876,7 +880,7 @@ __global__ void __launch_bounds__(DxWide::NT) dx_wide_kernel(DxArgs a) {
   if (k_end <= k_begin) {  // a slice past the end of the label axis contributes zeros
     float4v acc[C::FM][C::FN];
     C::zero(acc);
-    store(acc);
+    leave(acc);
     return;
   }
   auto get = [&](int, C::Operand& oa, C::Operand& ob, int& kb, int& ke) {
@@ -885,12 +889,12 @@ __global__ void __launch_bounds__(DxWide::NT) dx_wide_kernel(DxArgs a) {
     kb = k_begin;
     ke = k_end;
   };
-  auto epilogue = [&](int, float4v (&acc)[C::FM][C::FN]) { store(acc); };
+  auto epilogue = [&](int, float4v (&acc)[C::FM][C::FN]) { leave(acc); };
   C::run(0, 1, lds, get, epilogue);
 }
 
 // The same on the smaller row tiles.
-template <class C>
+template <class C, int HOW>
 __global__ void __launch_bounds__(C::NT) dx_kernel(DxArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   half_t* lds = reinterpret_cast<half_t*>(smem_raw);
@@ -904,7 +908,7 @@ __global__ void __launch_bounds__(C::NT) dx_kernel(DxArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform, and known to be
   const int wm = wave / C::WN, wn = wave % C::WN;
   float* part = a.part + (int64_t)split * a.M * a.N;
-  auto store = [&](float16v (&acc)[C::FM][C::FN]) {
+  auto leave = [&](float16v (&acc)[C::FM][C::FN]) {
 #pragma unroll
     for (int fm = 0; fm < C::FM; ++fm)
 #pragma unroll
@@ -914,7 +918,7 @@ __global__ void __launch_bounds__(C::NT) dx_kernel(DxArgs a) {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int row = m0 + wm * C::TM + fm * 32 + c_row(r, lane);
-            if (row < a.M) part[(int64_t)row * a.N + col] = acc[fm][fn][r];
+            if (row < a.M) store<HOW>(part + (int64_t)row * a.N + col, (float)acc[fm][fn][r]);
           }
         }
       }
@@ -922,7 +926,7 @@ __global__ void __launch_bounds__(C::NT) dx_kernel(DxArgs a) {
   if (k_end <= k_begin) {  // a slice past the end of the label axis contributes zeros
     float16v acc[C::FM][C::FN];
     C::zero(acc);
-    store(acc);
+    leave(acc);
     return;
   }
   auto get = [&](int, typename C::Operand& oa, typename C::Operand& ob, int& kb, int& ke) {
@@ -931,7 +935,7 @@ __global__ void __launch_bounds__(C::NT) dx_kernel(DxArgs a) {
     kb = k_begin;
     ke = k_end;
   };
-  auto epilogue = [&](int, float16v (&acc)[C::FM][C::FN]) { store(acc); };
+  auto epilogue = [&](int, float16v (&acc)[C::FM][C::FN]) { leave(acc); };
   C::run(0, 1, lds, get, epilogue);
 }
 
@@ -1002,8 +1006,8 @@ struct DwArgs {
 
 // Persistent, one workgroup per CU: workgroup w takes tile ids w, w + gridDim.x, ...; the dim tiles of
 // one label tile have neighbouring ids on one XCD, so its slice of G is fetched from HBM once.
-// NTS: what is written is stored as what will not be wanted again (see launch_dw).
-template <int MODE, bool NTS>
+// HOW what is written is stored: see launch_dw.
+template <int MODE, int HOW>
 __global__ void __launch_bounds__(DwCore::NT) dw_kernel(DwArgs a) {
   using C = DwCore;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
@@ -1101,8 +1105,8 @@ __global__ void __launch_bounds__(DwCore::NT) dw_kernel(DwArgs a) {
           o0 += a.beta * p0;
           o1 += a.beta * p1;
         }
-        if (in) store<NTS>(reinterpret_cast<float4v*>(orow + col), o0);
-        if (in1) store<NTS>(reinterpret_cast<float4v*>(orow + col1), o1);
+        if (in) store<HOW>(reinterpret_cast<float4v*>(orow + col), o0);
+        if (in1) store<HOW>(reinterpret_cast<float4v*>(orow + col1), o1);
       } else if constexpr (MODE == DW_UPDATE_MASTER) {
         // the reference's regime (fp32 parameter and FusedSGD state, dl_base.py:185, main.py:178-179) with the
         // per-step fp16 cast of W (dl_base.py:562) written from the same pass
@@ -1133,13 +1137,13 @@ __global__ void __launch_bounds__(DwCore::NT) dw_kernel(DwArgs a) {
           float* wp = a.W32 + (int64_t)row * a.ldw32;
           float* mp = a.M32 + (int64_t)row * a.ldm32;
           half_t* hp = a.Wt + (int64_t)row * a.ldw;
-          store<NTS>(reinterpret_cast<float4v*>(mp + col), mv[0]);
-          store<NTS>(reinterpret_cast<float4v*>(wp + col), wv[0]);
-          *reinterpret_cast<half4*>(hp + col) = half4{w16[0], w16[1], w16[2], w16[3]};
+          store<HOW>(reinterpret_cast<float4v*>(mp + col), mv[0]);
+          store<HOW>(reinterpret_cast<float4v*>(wp + col), wv[0]);
+          store<HOW == THROUGH ? THROUGH : CACHED>(reinterpret_cast<half4*>(hp + col), half4{w16[0], w16[1], w16[2], w16[3]});
           if (in1) {
-            store<NTS>(reinterpret_cast<float4v*>(mp + col1), mv[1]);
-            store<NTS>(reinterpret_cast<float4v*>(wp + col1), wv[1]);
-            *reinterpret_cast<half4*>(hp + col1) = half4{w16[4], w16[5], w16[6], w16[7]};
+            store<HOW>(reinterpret_cast<float4v*>(mp + col1), mv[1]);
+            store<HOW>(reinterpret_cast<float4v*>(wp + col1), wv[1]);
+            store<HOW == THROUGH ? THROUGH : CACHED>(reinterpret_cast<half4*>(hp + col1), half4{w16[4], w16[5], w16[6], w16[7]});
           }
         }
       } else {
@@ -1159,8 +1163,8 @@ __global__ void __launch_bounds__(DwCore::NT) dw_kernel(DwArgs a) {
             mv[e] = (half_t)mf;
             wv[e] = (half_t)(wf - a.lr * mf);
           }
-          store<NTS>(reinterpret_cast<half8*>(a.Mo + (int64_t)row * a.ldm + col), mv);
-          store<NTS>(reinterpret_cast<half8*>(a.Wt + (int64_t)row * a.ldw + col), wv);
+          store<HOW>(reinterpret_cast<half8*>(a.Mo + (int64_t)row * a.ldm + col), mv);
+          store<HOW>(reinterpret_cast<half8*>(a.Wt + (int64_t)row * a.ldw + col), wv);
         }
       }
     }
@@ -1465,6 +1469,9 @@ int launch_fwd(int mode, const half_t* X, int64_t ldx, const half_t* W, int64_t 
   a.M = M; a.N = p.first < N ? (int)p.first : N; a.K = K; a.n_store = (int)p.first; a.alpha = alpha; a.beta = beta;
   a.loss_part = loss_part;
   a.bmax = bmax; a.ldb = ldb;
+  // Few logits are written through: with whole steps of 40 rows x 30,001 labels x 64 dims 23.0 -> 22.3 us, 256 x 20,001 x 256 43.2 -> 42.3, 50 x
+  // 10,001 x 1024 41.4 -> 39.3, but (the wide loop's pieces are half lines) 512 x 20,001 x 768 97.2 -> 98.9, 100 x 60,001 109.9 -> 110.7.
+  a.through = (int64_t)M * n_store * 2 <= (int64_t)(p.tile == FWD_WIDE128 ? 10 : 8) << 20;
   auto tiles = [&](FwdTile t, int64_t n) {
     a.tiles_n = ceil_div(n, t == FWD_WIDE128 ? FwdWide128::BM : FwdWide::BM);
     const int64_t ids = fwd_ids(t, M, n);
@@ -1553,11 +1560,17 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
   if (grid <= 0 || M <= 0 || N <= 0) return XFC_OK;
   const dim3 g((unsigned)grid);
   int rc;
-  switch (row_tile(M)) {
-    case 64: rc = launch_k<dx_kernel<DxCore64>>(g, dim3(DxCore64::NT), DxCore64::LDS_BYTES, st, a); break;
-    case 128: rc = launch_k<dx_kernel<DxCore>>(g, dim3(DxCore::NT), DxCore::LDS_BYTES, st, a); break;
-    default: rc = launch_k<dx_wide_kernel>(g, dim3(DxWide::NT), DxWide::LDS_BYTES, st, a); break;
-  }
+  // Partial sums that the L2s hold much of are written through: six-argument calls of 512 rows x 20,000 labels x 768 dims 92.5 -> 90.0
+  // us, steps of 600 x 8,001 77.0 -> 75.4, x 20,001 115.4 -> 113.7, but 512 x 60,000 192.6 -> 194.2, 1024 x 60,001 x 256 179 -> 184.
+  auto launch = [&](auto how) {
+    constexpr int HOW = decltype(how)::value;
+    switch (row_tile(M)) {
+      case 64: return launch_k<dx_kernel<DxCore64, HOW>>(g, dim3(DxCore64::NT), DxCore64::LDS_BYTES, st, a);
+      case 128: return launch_k<dx_kernel<DxCore, HOW>>(g, dim3(DxCore::NT), DxCore::LDS_BYTES, st, a);
+      default: return launch_k<dx_wide_kernel<HOW>>(g, dim3(DxWide::NT), DxWide::LDS_BYTES, st, a);
+    }
+  };
+  rc = need <= (size_t)48 << 20 ? launch(std::integral_constant<int, THROUGH>{}) : launch(std::integral_constant<int, CACHED>{});
   if (rc) return rc;
   launch_dx_reduce(a.part, out, ldo, M, N, a.splits, alpha, beta, st);
   return check_launch();
@@ -1580,13 +1593,20 @@ int launch_dw(int mode, DwArgs a, hipStream_t st) {
   // 13.67 ms, x 700,001 3.48 -> 3.44, but 800 x 200,001 x 512 684 -> 688, 700 x 131,072 x 256 228 -> 235.  Not only back to back: the
   // calls of 512 rows x 131,072 each followed by a copy of 512 MiB 567 -> 522, by 0.6 ms of matrix products 1011 -> 978, waited for 409 -> 373.
   const int64_t weights = (int64_t)a.M * a.N, Mi = (int64_t)1 << 20;
-  auto launch = [&](auto mode_tag, int64_t least) {
+  // Small ones are written through (see StoreHow).  Over three states in turn and over one (us): master weights 64 rows x 5,001 labels x 768 dims 49.7, 50.3 -> 45.3, 46.7, 300 x 10,001 94, 86 -> 93, 73, but 100 x 20,001
+  // 97.6, 83.9 -> 99.2, 81.2; fp16 state 600 x 8,001 77.1, 77.4 -> 72.6, 73.8, 800 x 60,001 306, 305 -> 304, 301, but 1024 x 131,072 687 -> 694; six-argument calls of 128 x
+  // 40,000 80, 69 -> 79, 68, 512 x 40,000 152, 138 -> 149, 135.
+  auto launch = [&](auto mode_tag, int64_t through, int64_t past) {
     constexpr int MODE = decltype(mode_tag)::value;
-    return weights > least ? launch_k<dw_kernel<MODE, true>>(g, b, DW_LDS_BYTES, st, a) : launch_k<dw_kernel<MODE, false>>(g, b, DW_LDS_BYTES, st, a);
+    if (weights > past) return launch_k<dw_kernel<MODE, PAST>>(g, b, DW_LDS_BYTES, st, a);
+    if constexpr (MODE != DW_OUT) {
+      if (weights > through) return launch_k<dw_kernel<MODE, CACHED>>(g, b, DW_LDS_BYTES, st, a);
+    }
+    return launch_k<dw_kernel<MODE, THROUGH>>(g, b, DW_LDS_BYTES, st, a);
   };
-  if (mode == DW_UPDATE) return launch(std::integral_constant<int, DW_UPDATE>{}, 140 * Mi);
-  if (mode == DW_UPDATE_MASTER) return launch(std::integral_constant<int, DW_UPDATE_MASTER>{}, 28 * Mi);
-  return launch(std::integral_constant<int, DW_OUT>{}, 40 * Mi);
+  if (mode == DW_UPDATE) return launch(std::integral_constant<int, DW_UPDATE>{}, 48 * Mi, 140 * Mi);
+  if (mode == DW_UPDATE_MASTER) return launch(std::integral_constant<int, DW_UPDATE_MASTER>{}, 12 * Mi, 28 * Mi);
+  return launch(std::integral_constant<int, DW_OUT>{}, 40 * Mi, 40 * Mi);
 }
 
 // The one-pass step of small batches (small_step.hpp).  Fn::operator()<S>() is called with the kernel for d dims and B
@@ -1723,12 +1743,18 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
   // -> 868, waited for 277 -> 274; of 100 x 400,001 x 384 566 -> 543 and 956 -> 941, but waited for 346 -> 385: what is stored through
   // the caches is written back by whoever runs next.  (Those are of the pass from the first labels on.)
   const bool nt = (int64_t)a.L * a.d * (MODE == BACK_UPDATE ? 4 : 6) > (int64_t)(MODE == BACK_UPDATE ? 144 : 224) << 20;
+  // Small updates are written through.  Whole steps, over three states in turn and over one (us): 64 rows x 4,097 labels x 768 dims
+  // 25.2 -> 24.0, 100 x 10,001 40.5, 40.7 -> 39.1, 38.8, 200 x 20,001 66.5, 60.7 -> 65.7, 59.6; but 100 x 40,001 88.4, 80.1 -> 90.4, 77.8.  (Of
+  // a gradient it makes no difference: 200 x 5,001 to 256 x 40,001 x 384.)
+  const bool small = (int64_t)a.L * a.d * 4 <= (int64_t)64 << 20;
   int rc = XFC_OK;
   *taken = back_step_for<MODE>(a.B, [&](auto s) {
     using S = decltype(s);
     const dim3 g((unsigned)(a.slices * a.ranges)), b(S::NT);
-    rc = nt ? launch_k<back_step_kernel<S, MODE, true>>(g, b, S::LDS_BYTES, st, a)
-            : launch_k<back_step_kernel<S, MODE, false>>(g, b, S::LDS_BYTES, st, a);
+    constexpr int SMALL = MODE == BACK_UPDATE ? THROUGH : CACHED;
+    rc = nt      ? launch_k<back_step_kernel<S, MODE, PAST>>(g, b, S::LDS_BYTES, st, a)
+         : small ? launch_k<back_step_kernel<S, MODE, SMALL>>(g, b, S::LDS_BYTES, st, a)
+                 : launch_k<back_step_kernel<S, MODE, CACHED>>(g, b, S::LDS_BYTES, st, a);
     if (rc) return;
     launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges * a.parts, scale, 0.0f, st);
     rc = check_launch();
@@ -1856,7 +1882,8 @@ int xfc_init(void) {
   keep(raise_lds_limit<topk_list_kernel<ListCore>>(TopkLds<ListCore>::BYTES));
   keep(raise_lds_limit<topk_list_kernel<ListCore128>>(TopkLds<ListCore128>::BYTES));
   keep(raise_lds_limit<topk_list_kernel<ListCore64>>(TopkLds<ListCore64>::BYTES));
-  keep(raise_lds_limit<dx_wide_kernel>(DxWide::LDS_BYTES));
+  keep(raise_lds_limit<dx_wide_kernel<CACHED>>(DxWide::LDS_BYTES));
+  keep(raise_lds_limit<dx_wide_kernel<THROUGH>>(DxWide::LDS_BYTES));
   auto small_limits = [&](auto core_tag, auto dx_tag) {
     using C = typename decltype(core_tag)::type;
     using D = typename decltype(dx_tag)::type;
@@ -1867,7 +1894,8 @@ int xfc_init(void) {
     keep(raise_lds_limit<fwd_kernel<C, FWD_SIGMOID_PLAIN, false>>(LDS));
     keep(raise_lds_limit<fwd_kernel<C, FWD_LINEAR, false>>(LDS));
     keep(raise_lds_limit<fwd_kernel<C, FWD_LINEAR, false, false, true>>(LDS));
-    keep(raise_lds_limit<dx_kernel<D>>(D::LDS_BYTES));
+    keep(raise_lds_limit<dx_kernel<D, CACHED>>(D::LDS_BYTES));
+    keep(raise_lds_limit<dx_kernel<D, THROUGH>>(D::LDS_BYTES));
   };
   small_limits(std::type_identity<FwdCore>{}, std::type_identity<DxCore>{});
   small_limits(std::type_identity<FwdCore64>{}, std::type_identity<DxCore64>{});
@@ -1884,8 +1912,9 @@ int xfc_init(void) {
     for (int64_t rows : {64, 128, 192, 256})
       back_step_for<MODE>(rows, [&](auto s) {
         using S = decltype(s);
-        keep(raise_lds_limit<back_step_kernel<S, MODE, true>>(S::LDS_BYTES));
-        keep(raise_lds_limit<back_step_kernel<S, MODE, false>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, CACHED>>(S::LDS_BYTES));
+        keep(raise_lds_limit<back_step_kernel<S, MODE, PAST>>(S::LDS_BYTES));
+        if constexpr (MODE == BACK_UPDATE) keep(raise_lds_limit<back_step_kernel<S, MODE, THROUGH>>(S::LDS_BYTES));
       });
   };
   for (int64_t rows : {320, 384, 448, 512})
@@ -1900,8 +1929,10 @@ int xfc_init(void) {
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_SMALL>>((int)sizeof(SelLds<SEL_CAP_SMALL>)));
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_LARGE>>((int)sizeof(SelLds<SEL_CAP_LARGE>)));
   auto dw_limits = [&](auto mode) {
-    keep(raise_lds_limit<dw_kernel<decltype(mode)::value, false>>(DW_LDS_BYTES));
-    keep(raise_lds_limit<dw_kernel<decltype(mode)::value, true>>(DW_LDS_BYTES));
+    constexpr int MODE = decltype(mode)::value;
+    keep(raise_lds_limit<dw_kernel<MODE, THROUGH>>(DW_LDS_BYTES));
+    keep(raise_lds_limit<dw_kernel<MODE, PAST>>(DW_LDS_BYTES));
+    if constexpr (MODE != DW_OUT) keep(raise_lds_limit<dw_kernel<MODE, CACHED>>(DW_LDS_BYTES));
   };
   dw_limits(std::integral_constant<int, DW_UPDATE>{});
   dw_limits(std::integral_constant<int, DW_OUT>{});
