@@ -5,6 +5,7 @@
 //   dw    : dW = G^T . X, consumed in the tile by  M = mu*M + dW + wd*W ; W -= lr*M
 // plus the plain six-argument GEMM the reference extension exposes.
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 #include <stdio.h>
 
@@ -983,11 +984,16 @@ enum DwMode { DW_OUT = 0, DW_UPDATE = 1, DW_UPDATE_MASTER = 2 };  // MASTER: fp3
 // the other's GEMM, measured 7-11 % slower at every batch size: its stages move half again as much through LDS
 // and the fetch path per flop, and the update's streaming is bound by HBM either way.)
 using DwCore = PipeCore<256, 256, 64, 4, 2, 2, false, false, false, false, false, 4>;
+// 128 labels x 128 dims, eight waves of 32 x 64, two workgroups to a CU: see launch_dw.
+using DwCore128 = PipeCore<128, 128, 64, 4, 2, 2, false, false, false, false, false, 4>;
 constexpr int DW_STAGE_FLOATS = 8 * 64;  // per wave: 8 label rows x 64 dims
-constexpr int DW_LDS_BYTES = DwCore::LDS_BYTES + DwCore::NW * DW_STAGE_FLOATS * 4;
-static_assert(DW_LDS_BYTES <= 160 * 1024, "LDS budget");
-static_assert(DwCore::TM == 64 && DwCore::TN == 128, "the update epilogue walks 64 x 128 wave tiles");
-static_assert(DwCore::FN % 2 == 0, "epilogue walks pairs of 32-column blocks");
+template <class C>
+struct DwLds {
+  static constexpr int BYTES = C::LDS_BYTES + C::NW * DW_STAGE_FLOATS * 4, PER_CU = 160 * 1024 / BYTES;
+  static_assert(BYTES <= 160 * 1024, "LDS budget");
+  static_assert(C::FN % 2 == 0, "epilogue walks pairs of 32-column blocks");
+};
+static_assert(DwLds<DwCore>::PER_CU == 1 && DwLds<DwCore128>::PER_CU == 2, "workgroups on a CU");
 
 struct DwArgs {
   const half_t* G; int64_t ldg;   // K x M (batch rows x labels), label-contiguous
@@ -1004,12 +1010,11 @@ struct DwArgs {
   int tiles_m, tiles_n, n_ids;      // n_ids = tiles_n * round_up(tiles_m, 8)
 };
 
-// Persistent, one workgroup per CU: workgroup w takes tile ids w, w + gridDim.x, ...; the dim tiles of
+// Persistent, as many workgroups as the CUs hold: workgroup w takes tile ids w, w + gridDim.x, ...; the dim tiles of
 // one label tile have neighbouring ids on one XCD, so its slice of G is fetched from HBM once.
 // HOW what is written is stored: see launch_dw.
-template <int MODE, int HOW>
-__global__ void __launch_bounds__(DwCore::NT) dw_kernel(DwArgs a) {
-  using C = DwCore;
+template <class C, int MODE, int HOW>
+__global__ void __launch_bounds__(C::NT, C::NW * DwLds<C>::PER_CU / 4) dw_kernel(DwArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   half_t* lds = reinterpret_cast<half_t*>(smem_raw);
   const int G = gridDim.x, w = blockIdx.x;
@@ -1576,16 +1581,57 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
   return check_launch();
 }
 
-int launch_dw(int mode, DwArgs a, hipStream_t st) {
-  a.tiles_m = ceil_div(a.M, DwCore::BM);
-  a.tiles_n = ceil_div(a.N, DwCore::BN);
+// Large tiles move the fewest bytes through the fetch path and the L2s, small ones fill the chip with few labels, leave no last round
+// nearly empty, waste less of a width that is no multiple of 256, and two of them on a CU work at each other's epilogues.  Compared
+// by rounds of the large ones, four small tiles to one of them at a price: nothing while the update's traffic binds, up to a sixth
+// at 1024 rows, 0.05 more for a state that no cache holds (fp32: from 200 Mi weights on), a fifth for a gradient that none does and 256
+// rows or more.  Measured
+// (us, large and small).  Updates: 32 rows x 8,001 labels x 256 dims 10.9 and 5.7, 128 x 30,001 x 768 46 and 37, 600 x 4,097 x 768 22.3
+// and 11.8, 1024 x 20,001 x 1024 83 and 68, 384 x 700,001 x 384 583 and 537, 1024 x 1,000,001 x 128 728 and 636, but 512 x 655,363 x 768
+// 1000 and 1100, 1024 x 131,072 x 768 293 and 327.  Master weights: 300 x 20,001 x 1024 106 and 82, 512 x 131,072 x
+// 768 393 and 373, 512 x 700,001 x 384 1163 and 1064, whole steps of 512 x 450,001 x
+// 768 1943 and 1911, 128 x 450,001 1532 and 1556, 512 x 655,363 2581 and 2629 or 2828 and 2823, 1024 x 655,363 x 768 2262 and 2381.  Gradients: 128 x
+// 131,073 x 768 79.7 and 74.7, 300 x 8,001 x 768 13.2 and 10.0, 512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768 505 and 611.
+bool dw_small_tiles(int mode, int64_t labels, int64_t dims, int64_t rows, bool past) {
+  auto rounds = [&](int64_t tile) {  // (a last one nearly empty leaves the others the more of the memory: half of it counts)
+    const double n = (double)(ceil_div(dims, tile) * round_up(ceil_div(labels, tile), 8)), cus = num_cus();
+    return 0.5 * (n / cus + ceil(n / cus));
+  };
+  const double over = rows > 256 ? (double)((rows < 1024 ? rows : 1024) - 256) : 0.0;
+  double price = 1.0 + 0.0002 * over;
+  if (mode == DW_UPDATE && past) price += 0.05;
+  if (mode == DW_OUT && past && rows >= 256) price = 1.2;
+  if (mode == DW_UPDATE_MASTER) {
+    const int64_t Mi = (int64_t)1 << 20;
+    price = 0.99 + (rows > 512 || labels * dims > (rows <= 128 ? 200 : 380) * Mi ? 0.05 : 0.0);
+  }
+  return price * rounds(DwCore128::BM) < 4.0 * rounds(DwCore::BM);
+}
+template <class C>
+int launch_dw_tiles(int mode, DwArgs a, bool past, bool through, hipStream_t st) {
+  a.tiles_m = ceil_div(a.M, C::BM);
+  a.tiles_n = ceil_div(a.N, C::BN);
   const int64_t ids = (int64_t)a.tiles_n * round_up(a.tiles_m, 8);
   if (ids <= 0) return XFC_OK;
   if (ids > 0x7fffffff) return XFC_ERR_INVALID;
   a.n_ids = (int)ids;
-  int64_t grid = (int64_t)round_up(num_cus(), 8);  // one resident workgroup per CU
+  int64_t grid = (int64_t)DwLds<C>::PER_CU * round_up(num_cus(), 8);
   if (grid > ids) grid = ids / 8 * 8 > 0 ? ids / 8 * 8 : ids;
-  const dim3 g((unsigned)grid), b(DwCore::NT);
+  const dim3 g((unsigned)grid), b(C::NT);
+  constexpr int LDS = DwLds<C>::BYTES;
+  auto launch = [&](auto mode_tag) {
+    constexpr int MODE = decltype(mode_tag)::value;
+    if (past) return launch_k<dw_kernel<C, MODE, PAST>>(g, b, LDS, st, a);
+    if constexpr (MODE != DW_OUT) {
+      if (!through) return launch_k<dw_kernel<C, MODE, CACHED>>(g, b, LDS, st, a);
+    }
+    return launch_k<dw_kernel<C, MODE, THROUGH>>(g, b, LDS, st, a);
+  };
+  if (mode == DW_UPDATE) return launch(std::integral_constant<int, DW_UPDATE>{});
+  if (mode == DW_UPDATE_MASTER) return launch(std::integral_constant<int, DW_UPDATE_MASTER>{});
+  return launch(std::integral_constant<int, DW_OUT>{});
+}
+int launch_dw(int mode, const DwArgs& a, hipStream_t st) {
   // Non-temporal stores where what is written would push out of the caches what the next kernels read, from about their size on.  A
   // gradient: six-argument calls of 512 rows x 131,072 labels x 768 dims 384 -> 347 us, 128 rows 212 -> 178, 512 x 200,000 x 256 303
   // -> 261, x 80,000 x 768 258 -> 241, but x 32,768 118 -> 120.  Master weights: steps of 512 x 655,363 x 768 2868 -> 2813, 64 x
@@ -1596,17 +1642,10 @@ int launch_dw(int mode, DwArgs a, hipStream_t st) {
   // Small ones are written through (see StoreHow).  Over three states in turn and over one (us): master weights 64 rows x 5,001 labels x 768 dims 49.7, 50.3 -> 45.3, 46.7, 300 x 10,001 94, 86 -> 93, 73, but 100 x 20,001
   // 97.6, 83.9 -> 99.2, 81.2; fp16 state 600 x 8,001 77.1, 77.4 -> 72.6, 73.8, 800 x 60,001 306, 305 -> 304, 301, but 1024 x 131,072 687 -> 694; six-argument calls of 128 x
   // 40,000 80, 69 -> 79, 68, 512 x 40,000 152, 138 -> 149, 135.
-  auto launch = [&](auto mode_tag, int64_t through, int64_t past) {
-    constexpr int MODE = decltype(mode_tag)::value;
-    if (weights > past) return launch_k<dw_kernel<MODE, PAST>>(g, b, DW_LDS_BYTES, st, a);
-    if constexpr (MODE != DW_OUT) {
-      if (weights > through) return launch_k<dw_kernel<MODE, CACHED>>(g, b, DW_LDS_BYTES, st, a);
-    }
-    return launch_k<dw_kernel<MODE, THROUGH>>(g, b, DW_LDS_BYTES, st, a);
-  };
-  if (mode == DW_UPDATE) return launch(std::integral_constant<int, DW_UPDATE>{}, 48 * Mi, 140 * Mi);
-  if (mode == DW_UPDATE_MASTER) return launch(std::integral_constant<int, DW_UPDATE_MASTER>{}, 12 * Mi, 28 * Mi);
-  return launch(std::integral_constant<int, DW_OUT>{}, 40 * Mi, 40 * Mi);
+  const bool through = weights <= (mode == DW_UPDATE ? 48 : mode == DW_UPDATE_MASTER ? 12 : 40) * Mi;
+  const bool past = weights > (mode == DW_UPDATE ? 140 : mode == DW_UPDATE_MASTER ? 28 : 40) * Mi;
+  return dw_small_tiles(mode, a.M, a.N, a.K, past) ? launch_dw_tiles<DwCore128>(mode, a, past, through, st)
+                                                   : launch_dw_tiles<DwCore>(mode, a, past, through, st);
 }
 
 // The one-pass step of small batches (small_step.hpp).  Fn::operator()<S>() is called with the kernel for d dims and B
@@ -1928,15 +1967,20 @@ int xfc_init(void) {
   back_limits(std::integral_constant<int, BACK_ADD>{});
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_SMALL>>((int)sizeof(SelLds<SEL_CAP_SMALL>)));
   keep(raise_lds_limit<topk_select_kernel<SEL_CAP_LARGE>>((int)sizeof(SelLds<SEL_CAP_LARGE>)));
-  auto dw_limits = [&](auto mode) {
-    constexpr int MODE = decltype(mode)::value;
-    keep(raise_lds_limit<dw_kernel<MODE, THROUGH>>(DW_LDS_BYTES));
-    keep(raise_lds_limit<dw_kernel<MODE, PAST>>(DW_LDS_BYTES));
-    if constexpr (MODE != DW_OUT) keep(raise_lds_limit<dw_kernel<MODE, CACHED>>(DW_LDS_BYTES));
+  auto dw_limits = [&](auto core_tag, auto mode) {
+    using C = typename decltype(core_tag)::type;
+    constexpr int MODE = decltype(mode)::value, LDS = DwLds<C>::BYTES;
+    keep(raise_lds_limit<dw_kernel<C, MODE, THROUGH>>(LDS));
+    keep(raise_lds_limit<dw_kernel<C, MODE, PAST>>(LDS));
+    if constexpr (MODE != DW_OUT) keep(raise_lds_limit<dw_kernel<C, MODE, CACHED>>(LDS));
   };
-  dw_limits(std::integral_constant<int, DW_UPDATE>{});
-  dw_limits(std::integral_constant<int, DW_OUT>{});
-  dw_limits(std::integral_constant<int, DW_UPDATE_MASTER>{});
+  auto dw_all_limits = [&](auto core_tag) {
+    dw_limits(core_tag, std::integral_constant<int, DW_UPDATE>{});
+    dw_limits(core_tag, std::integral_constant<int, DW_OUT>{});
+    dw_limits(core_tag, std::integral_constant<int, DW_UPDATE_MASTER>{});
+  };
+  dw_all_limits(std::type_identity<DwCore>{});
+  dw_all_limits(std::type_identity<DwCore128>{});
   (void)num_cus();
   if (static_scratch_ptr() == nullptr) return XFC_ERR_HIP;
   if (e != hipSuccess) {
