@@ -343,7 +343,7 @@ __global__ void __launch_bounds__(C::NT) fwd_kernel(FwdArgs a) {
               // uniform part + per-lane part computed once per tile: no per-strip vector multiply
               half_t* dst = a.out + ((int64_t)(m0 + wm * C::TM + fm * 32 + 8 * q) * a.ldo + n0 + wn * C::TN) + lane_off[p];
               if (!EDGE || col + 8 <= a.n_store) {
-                if (a.through) store<THROUGH>(reinterpret_cast<half8*>(dst), v8);
+                if (!LOSS && a.through) store<THROUGH>(reinterpret_cast<half8*>(dst), v8);
                 else store<PAST>(reinterpret_cast<half8*>(dst), v8);  // G is not re-read before it leaves the L2
               } else {
 #pragma unroll
@@ -1566,7 +1566,8 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
   const dim3 g((unsigned)grid);
   int rc;
   // Partial sums that the L2s hold much of are written through: six-argument calls of 512 rows x 20,000 labels x 768 dims 92.5 -> 90.0
-  // us, steps of 600 x 8,001 77.0 -> 75.4, x 20,001 115.4 -> 113.7, but 512 x 60,000 192.6 -> 194.2, 1024 x 60,001 x 256 179 -> 184.
+  // us, steps of 600 x 8,001 77.0 -> 75.4, x 20,001 115.4 -> 113.7, but 512 x 60,000 192.6 -> 194.2, 1024 x 60,001 x 256 179 -> 184,
+  // and longer axes, whose pass is not waited for as long, too (dX by itself: 100 x 119,605 x 384 35.2 -> 37.2, 899 x 106,385 x 768 162 -> 167).
   auto launch = [&](auto how) {
     constexpr int HOW = decltype(how)::value;
     switch (row_tile(M)) {
@@ -1575,7 +1576,7 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
       default: return launch_k<dx_wide_kernel<HOW>>(g, dim3(DxWide::NT), DxWide::LDS_BYTES, st, a);
     }
   };
-  rc = need <= (size_t)48 << 20 ? launch(std::integral_constant<int, THROUGH>{}) : launch(std::integral_constant<int, CACHED>{});
+  rc = need <= (size_t)48 << 20 && K <= 40000 ? launch(std::integral_constant<int, THROUGH>{}) : launch(std::integral_constant<int, CACHED>{});
   if (rc) return rc;
   launch_dx_reduce(a.part, out, ldo, M, N, a.splits, alpha, beta, st);
   return check_launch();
@@ -1584,14 +1585,15 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
 // Large tiles move the fewest bytes through the fetch path and the L2s, small ones fill the chip with few labels, leave no last round
 // nearly empty, waste less of a width that is no multiple of 256, and two of them on a CU work at each other's epilogues.  Compared
 // by rounds of the large ones, four small tiles to one of them at a price: nothing while the update's traffic binds, up to a sixth
-// at 1024 rows, 0.05 more for a state that no cache holds (fp32: from 200 Mi weights on), a fifth for a gradient that none does and 256
-// rows or more.  Measured
+// (of a gradient a quarter) at 1024 rows, 0.05 more for a state that no cache holds (fp32: from 160 Mi weights on); of a gradient a fifth for one that none does and
+// 256 rows or more, two fifths for a large one of whole large tiles, whose rows a small tile writes in pieces of 512 bytes.  Measured
 // (us, large and small).  Updates: 32 rows x 8,001 labels x 256 dims 10.9 and 5.7, 128 x 30,001 x 768 46 and 37, 600 x 4,097 x 768 22.3
 // and 11.8, 1024 x 20,001 x 1024 83 and 68, 384 x 700,001 x 384 583 and 537, 1024 x 1,000,001 x 128 728 and 636, but 512 x 655,363 x 768
 // 1000 and 1100, 1024 x 131,072 x 768 293 and 327.  Master weights: 300 x 20,001 x 1024 106 and 82, 512 x 131,072 x
 // 768 393 and 373, 512 x 700,001 x 384 1163 and 1064, whole steps of 512 x 450,001 x
 // 768 1943 and 1911, 128 x 450,001 1532 and 1556, 512 x 655,363 2581 and 2629 or 2828 and 2823, 1024 x 655,363 x 768 2262 and 2381.  Gradients: 128 x
-// 131,073 x 768 79.7 and 74.7, 300 x 8,001 x 768 13.2 and 10.0, 512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768 505 and 611.
+// 131,073 x 768 79.7 and 74.7, 300 x 8,001 x 768 13.2 and 10.0, 512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768 505 and 611, 136 x 1,096,208 x
+// 256 243 and 334, 248 x 234,640 x 1024 204 and 227, 712 x 80,256 x 512 86.8 and 90.7, but 1024 x 20,000 x 1024 62 and 53, 256 x 400,000 x 384 156 and 147.
 bool dw_small_tiles(int mode, int64_t labels, int64_t dims, int64_t rows, bool past) {
   auto rounds = [&](int64_t tile) {  // (a last one nearly empty leaves the others the more of the memory: half of it counts)
     const double n = (double)(ceil_div(dims, tile) * round_up(ceil_div(labels, tile), 8)), cus = num_cus();
@@ -1600,11 +1602,13 @@ bool dw_small_tiles(int mode, int64_t labels, int64_t dims, int64_t rows, bool p
   const double over = rows > 256 ? (double)((rows < 1024 ? rows : 1024) - 256) : 0.0;
   double price = 1.0 + 0.0002 * over;
   if (mode == DW_UPDATE && past) price += 0.05;
-  if (mode == DW_OUT && past && rows >= 256) price = 1.2;
-  if (mode == DW_UPDATE_MASTER) {
-    const int64_t Mi = (int64_t)1 << 20;
-    price = 0.99 + (rows > 512 || labels * dims > (rows <= 128 ? 200 : 380) * Mi ? 0.05 : 0.0);
+  const int64_t Mi = (int64_t)1 << 20, weights = labels * dims;
+  if (mode == DW_OUT) {
+    if (past && dims % DwCore::BN == 0 && weights > 120 * Mi) price = 1.4;
+    else if (past && rows >= 256) price = 1.2;
+    else price += 0.0001 * over;
   }
+  if (mode == DW_UPDATE_MASTER) price = 0.99 + (rows > 512 || weights > (rows <= 128 ? 160 : 380) * Mi ? 0.05 : 0.0);
   return price * rounds(DwCore128::BM) < 4.0 * rounds(DwCore::BM);
 }
 template <class C>
@@ -1622,10 +1626,8 @@ int launch_dw_tiles(int mode, DwArgs a, bool past, bool through, hipStream_t st)
   auto launch = [&](auto mode_tag) {
     constexpr int MODE = decltype(mode_tag)::value;
     if (past) return launch_k<dw_kernel<C, MODE, PAST>>(g, b, LDS, st, a);
-    if constexpr (MODE != DW_OUT) {
-      if (!through) return launch_k<dw_kernel<C, MODE, CACHED>>(g, b, LDS, st, a);
-    }
-    return launch_k<dw_kernel<C, MODE, THROUGH>>(g, b, LDS, st, a);
+    if (through) return launch_k<dw_kernel<C, MODE, THROUGH>>(g, b, LDS, st, a);
+    return launch_k<dw_kernel<C, MODE, CACHED>>(g, b, LDS, st, a);
   };
   if (mode == DW_UPDATE) return launch(std::integral_constant<int, DW_UPDATE>{});
   if (mode == DW_UPDATE_MASTER) return launch(std::integral_constant<int, DW_UPDATE_MASTER>{});
@@ -1639,10 +1641,11 @@ int launch_dw(int mode, const DwArgs& a, hipStream_t st) {
   // 13.67 ms, x 700,001 3.48 -> 3.44, but 800 x 200,001 x 512 684 -> 688, 700 x 131,072 x 256 228 -> 235.  Not only back to back: the
   // calls of 512 rows x 131,072 each followed by a copy of 512 MiB 567 -> 522, by 0.6 ms of matrix products 1011 -> 978, waited for 409 -> 373.
   const int64_t weights = (int64_t)a.M * a.N, Mi = (int64_t)1 << 20;
-  // Small ones are written through (see StoreHow).  Over three states in turn and over one (us): master weights 64 rows x 5,001 labels x 768 dims 49.7, 50.3 -> 45.3, 46.7, 300 x 10,001 94, 86 -> 93, 73, but 100 x 20,001
-  // 97.6, 83.9 -> 99.2, 81.2; fp16 state 600 x 8,001 77.1, 77.4 -> 72.6, 73.8, 800 x 60,001 306, 305 -> 304, 301, but 1024 x 131,072 687 -> 694; six-argument calls of 128 x
-  // 40,000 80, 69 -> 79, 68, 512 x 40,000 152, 138 -> 149, 135.
-  const bool through = weights <= (mode == DW_UPDATE ? 48 : mode == DW_UPDATE_MASTER ? 12 : 40) * Mi;
+  // Small ones are written through (see StoreHow).  Over three states in turn and over one (us): master weights 64 rows x 5,001
+  // labels x 768 dims 49.7, 50.3 -> 45.3, 46.7, 300 x 10,001 94, 86 -> 93, 73, but 100 x 20,001 97.6, 83.9 -> 99.2, 81.2; fp16 state 600 x
+  // 8,001 77.1, 77.4 -> 72.6, 73.8, 800 x 60,001 306, 305 -> 304, 301, but 1024 x 131,072 687 -> 694.  Gradients, six-argument calls of 128 x
+  // 20,000 50.9 -> 47.9; by themselves, with G out of HBM, larger ones lose: 256 x 23,293 x 1024 32 -> 37, 512 x 27,823 x 1024 49 -> 61.
+  const bool through = weights <= (mode == DW_UPDATE ? 48 : mode == DW_UPDATE_MASTER ? 12 : 16) * Mi;
   const bool past = weights > (mode == DW_UPDATE ? 140 : mode == DW_UPDATE_MASTER ? 28 : 40) * Mi;
   return dw_small_tiles(mode, a.M, a.N, a.K, past) ? launch_dw_tiles<DwCore128>(mode, a, past, through, st)
                                                    : launch_dw_tiles<DwCore>(mode, a, past, through, st);
@@ -1972,7 +1975,7 @@ int xfc_init(void) {
     constexpr int MODE = decltype(mode)::value, LDS = DwLds<C>::BYTES;
     keep(raise_lds_limit<dw_kernel<C, MODE, THROUGH>>(LDS));
     keep(raise_lds_limit<dw_kernel<C, MODE, PAST>>(LDS));
-    if constexpr (MODE != DW_OUT) keep(raise_lds_limit<dw_kernel<C, MODE, CACHED>>(LDS));
+    keep(raise_lds_limit<dw_kernel<C, MODE, CACHED>>(LDS));
   };
   auto dw_all_limits = [&](auto core_tag) {
     dw_limits(core_tag, std::integral_constant<int, DW_UPDATE>{});
