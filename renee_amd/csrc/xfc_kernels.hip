@@ -1593,7 +1593,7 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
 // 768 393 and 373, 512 x 700,001 x 384 1163 and 1064, whole steps of 512 x 450,001 x
 // 768 1943 and 1911, 128 x 450,001 1532 and 1556, 512 x 655,363 2581 and 2629 or 2828 and 2823, 1024 x 655,363 x 768 2262 and 2381.  Gradients: 128 x
 // 131,073 x 768 79.7 and 74.7, 300 x 8,001 x 768 13.2 and 10.0, 512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768 505 and 611, 136 x 1,096,208 x
-// 256 243 and 334, 248 x 234,640 x 1024 204 and 227, 712 x 80,256 x 512 86.8 and 90.7, but 1024 x 20,000 x 1024 62 and 53, 256 x 400,000 x 384 156 and 147.
+// 256 243 and 334, 248 x 234,640 x 1024 204 and 227, 712 x 80,256 x 512 86.8 and 90.7, 32 x 1,000,000 x 128 90 and 100, but 64 rows 97 and 92, 1024 x 20,000 x 1024 62 and 53, 256 x 400,000 x 384 156 and 147.
 bool dw_small_tiles(int mode, int64_t labels, int64_t dims, int64_t rows, bool past) {
   auto rounds = [&](int64_t tile) {  // (a last one nearly empty leaves the others the more of the memory: half of it counts)
     const double n = (double)(ceil_div(dims, tile) * round_up(ceil_div(labels, tile), 8)), cus = num_cus();
@@ -1606,6 +1606,7 @@ bool dw_small_tiles(int mode, int64_t labels, int64_t dims, int64_t rows, bool p
   if (mode == DW_OUT) {
     if (past && dims % DwCore::BN == 0 && weights > 120 * Mi) price = 1.4;
     else if (past && rows >= 256) price = 1.2;
+    else if (past && rows <= 48 && dims > 64 && dims <= DwCore128::BN) price = 2.2;  // (half of a large tile empty: what it multiplies is little)
     else price += 0.0001 * over;
   }
   if (mode == DW_UPDATE_MASTER) price = 0.99 + (rows > 512 || weights > (rows <= 128 ? 160 : 380) * Mi ? 0.05 : 0.0);
