@@ -1,7 +1,8 @@
-"""Updates and partial sums of dX on both sides of the sizes up to which they are written through the L2, against float64, with leading
+"""Updates, gradients and partial sums of dX on both sides of the sizes up to which they are written through the L2, against float64, with leading
 dimensions past the width.  Checks and bounds are those of test_gpu_back_step.py and test_gpu_past_caches.py."""
 import pytest
 import test_gpu_back_step as back
+import test_gpu_dw_tiles as tiles
 import test_gpu_past_caches as past
 import torch
 from test_gpu_back_step import _st
@@ -23,7 +24,15 @@ def test_update(dev, state, B, L, least):
     past.test_update(dev, state, B, L, least)
 
 
-@pytest.mark.parametrize("B,L,d", [(40, 3001, 64), (130, 8001, 72), (600, 1001, 200), (512, 33001, 768), (140, 200001, 256)])  # 48 MiB of partial sums
+# 16 and 40 Mi weights lie between, the latter on large tiles up to 48 rows
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+@pytest.mark.parametrize("B,L,d", [(16, 21001, 768), (16, 22001, 768), (700, 22001, 768), (48, 320001, 128), (48, 340001, 128), (56, 340001, 128)])
+def test_gradient(dev, B, L, d, beta):
+    tiles.test_gradient(dev, B, L, d, beta)
+
+
+@pytest.mark.parametrize("B,L,d", [(40, 3001, 64), (130, 8001, 72), (600, 1001, 200), (512, 33001, 768), (140, 200001, 256),
+                                   (130, 39999, 72), (130, 40001, 72)])  # 48 MiB of partial sums, 40,000 labels
 def test_gradient_of_the_input(dev, B, L, d):
     g = torch.Generator(device=dev).manual_seed(B + L)
     G = torch.zeros(B, (L + 7) // 8 * 8, dtype=torch.float16, device=dev)
