@@ -350,8 +350,11 @@ __global__ void __launch_bounds__(256) topk_merge_kernel(const float* __restrict
 // top-K for 8 < K <= 8192: exact selection over rows of fp16 logits (one workgroup per row)
 
 // bound[r] = key of a value safely below the K-th largest of row r's sample scores.  The sample scores
-// are fp16 roundings (half an ulp from the fp32 score at most), so one part in 1024 plus the smallest fp16
-// step below the K-th rounded score is below the K-th fp32 score of the sample, hence of the whole row.
+// are fp16 roundings (half an ulp from the fp32 score at most) of sums made as the list kernels make them, the same MFMAs in
+// the same order, so one part in 1024 plus the smallest fp16 step below the K-th rounded score is below the K-th fp32 score of the
+// sample, hence of the whole row.  (Sums in another order differ by what they round off, relative to the products' magnitudes: where
+// these cancel, by more than that.  The wide loop's 16x16x32 MFMAs happen to give the same bits: 211,000 best scores of operands over up
+// to 21 binary orders of magnitude and of cancelling products.)
 __global__ void __launch_bounds__(256) topk_seed_kernel(const float* __restrict__ sample_v, int K, uint32_t* __restrict__ bound,
                                                         int64_t n) {
   const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;

@@ -1465,10 +1465,9 @@ int launch_fwd_c(int mode, const FwdArgs& a, dim3 g, hipStream_t st) {
   return launch_k<fwd_kernel<C, FWD_LINEAR, false>>(g, b, LDS, st, a);
 }
 
-int launch_fwd(int mode, const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, half_t* out, int64_t ldo, int M,
+int launch_fwd(const FwdPlan& p, int mode, const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, half_t* out, int64_t ldo, int M,
                int N, int K, int n_store, float alpha, float beta, hipStream_t st, double* loss_part = nullptr,
                half_t* bmax = nullptr, int64_t ldb = 0) {
-  const FwdPlan p = fwd_plan(M, n_store, K, loss_part != nullptr);
   FwdArgs a;
   a.X = X; a.ldx = ldx; a.W = W; a.ldw = ldw; a.out = out; a.ldo = ldo;
   a.M = M; a.N = p.first < N ? (int)p.first : N; a.K = K; a.n_store = (int)p.first; a.alpha = alpha; a.beta = beta;
@@ -2018,8 +2017,8 @@ int xfc_gemm(const void* in1, int64_t in1_rows, int64_t in1_cols, int64_t in1_s0
     const bool fast = out_s1 == 1 && out_s0 % 8 == 0 && aligned16(out) && in1_s0 % 8 == 0 && in2_s1 % 8 == 0 &&
                       K % 8 == 0 && aligned16(in1) && aligned16(in2) && K > 0;
     if (fast)
-      return launch_fwd(FWD_SIGMOID, (const half_t*)in1, in1_s0, (const half_t*)in2, in2_s1, (half_t*)out, out_s0,
-                        (int)M, (int)N, (int)K, (int)N, alpha, beta, st);
+      return launch_fwd(fwd_plan(M, N, K, false), FWD_SIGMOID, (const half_t*)in1, in1_s0, (const half_t*)in2, in2_s1, (half_t*)out,
+                        out_s0, (int)M, (int)N, (int)K, (int)N, alpha, beta, st);
     return launch_generic(in1, in1_s0, in1_s1, in2, in2_s0, in2_s1, out, out_s0, out_s1, (int)M, (int)N, (int)K, alpha,
                           beta, 1, 1, st);
   }
@@ -2059,8 +2058,8 @@ int xfc_logits(const void* X, int64_t ldx, const void* W, int64_t ldw, void* out
   if (ldx % 8 || ldw % 8 || ldo % 8 || d % 8 || !aligned16(X) || !aligned16(W) || !aligned16(out))
     return XFC_ERR_ALIGN;
   if (ldo < L) return XFC_ERR_SHAPE;
-  return launch_fwd(FWD_LINEAR, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)out, ldo, (int)B, (int)L, (int)d,
-                    (int)L, 1.0f, 0.0f, reinterpret_cast<hipStream_t>(stream));
+  return launch_fwd(fwd_plan(B, L, d, false), FWD_LINEAR, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)out, ldo, (int)B,
+                    (int)L, (int)d, (int)L, 1.0f, 0.0f, reinterpret_cast<hipStream_t>(stream));
 }
 
 size_t xfc_fwd_grad_workspace_bytes(int64_t L, int64_t nnz) {
@@ -2119,7 +2118,7 @@ static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw,
   // pieces along the label axis by the dX and dW kernels (ldg is a multiple of 8, so they exist)
   const int64_t n_store = round_up(L, 8);
   const FwdPlan plan = fwd_plan(B, n_store, d, loss != nullptr);
-  int rc = launch_fwd(FWD_SIGMOID, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)G, ldg, (int)B, (int)L, (int)d,
+  int rc = launch_fwd(plan, FWD_SIGMOID, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)G, ldg, (int)B, (int)L, (int)d,
                       (int)n_store, 1.0f, 0.0f, st, loss_part);
   if (rc) return rc;
   if (nnz > 0) {
@@ -2527,7 +2526,9 @@ static int topk_lists(const half_t* X, int64_t ldx, const half_t* W, int64_t ldw
     half_t* sample = reinterpret_cast<half_t*>(a.bound + round_up(B, 4));
     int64_t* sample_i = reinterpret_cast<int64_t*>(sample + (size_t)B * TOPK_SAMPLE);
     float* sample_v = reinterpret_cast<float*>(sample_i + (size_t)B * K);
-    rc = launch_fwd(FWD_LINEAR, X, ldx, W, ldw, sample, TOPK_SAMPLE, B, TOPK_SAMPLE, d, TOPK_SAMPLE, 1.0f, 0.0f, st);
+    // by the list kernels' own loop, whatever the rows: topk_seed_kernel counts on sums that are theirs to the last bit
+    const FwdPlan sums = {B <= 64 ? FWD_64 : FWD_128, TOPK_SAMPLE};
+    rc = launch_fwd(sums, FWD_LINEAR, X, ldx, W, ldw, sample, TOPK_SAMPLE, B, TOPK_SAMPLE, d, TOPK_SAMPLE, 1.0f, 0.0f, st);
     if (rc) return rc;
     const SelArgs sa = {sample, (int64_t)TOPK_SAMPLE, TOPK_SAMPLE, (int64_t)TOPK_SAMPLE, K, 1, nullptr, 0, 0, sample_v, sample_i};
     if ((rc = launch_select<SEL_CAP_SMALL>(B, sa, st))) return rc;
@@ -2579,8 +2580,8 @@ static int topk_impl(const void* X, int64_t ldx, const void* W, int64_t ldw, int
     }
     for (int64_t r0 = 0; r0 < B; r0 += block) {
       const int64_t rows = B - r0 < block ? B - r0 : block;
-      int rc = launch_fwd(FWD_LINEAR, (const half_t*)X + r0 * ldx, ldx, (const half_t*)W, ldw, (half_t*)workspace, ldl,
-                          (int)rows, (int)L, (int)d, (int)L, 1.0f, 0.0f, st, nullptr, bmax, ldb);
+      int rc = launch_fwd(fwd_plan(rows, L, d, false), FWD_LINEAR, (const half_t*)X + r0 * ldx, ldx, (const half_t*)W, ldw,
+                          (half_t*)workspace, ldl, (int)rows, (int)L, (int)d, (int)L, 1.0f, 0.0f, st, nullptr, bmax, ldb);
       if (rc) return rc;
       // sample every stride-th 16 KB block first when that still holds 16 K elements and points at about a
       // thousand candidates at most (half the sort buffer)

@@ -106,6 +106,27 @@ def test_the_best_of_very_many_labels(dev, B):
     assert torch.equal(v, w[:, :1]) and torch.equal(i, j[:, :1])
 
 
+# a workspace for all label groups (256 CUs) and the sample; K = 1 goes by lists at the last size whatever it is
+@pytest.mark.parametrize("B,L,K,groups", [(40, 540001, 1, 256), (100, 540001, 1, 256), (128, 540001, 3, 256), (129, 540001, 1, 256),
+                                          (700, 170001, 3, 80), (100, 1250007, 1, 0)])
+def test_bounds_from_a_sample_where_products_cancel(dev, B, L, K, groups):
+    """Scores of identical labels, each the sum of products and of their negatives: none is more than what the sums round off, so that
+    a sample summed in another order than the lists might lie above every one of them.  The first labels win, whatever they score."""
+    d = 256
+    g = torch.Generator().manual_seed(B)
+    x, w, order = torch.randn(B, d // 2, generator=g).half() * 8, torch.randn(d // 2, generator=g).half() * 8, torch.randperm(d // 2, generator=g)
+    X = torch.cat([x, -x[:, order]], 1).to(dev)
+    W = torch.cat([w, w[order]]).to(dev).repeat(L, 1)
+    magnitude = X.double().abs() @ W[0].double().abs()
+    assert float((X.double() @ W[0].double()).abs().max()) < 1e-9  # of the order of its own roundings
+    full = lib().xfc_topk_workspace_bytes(B, L, K)
+    nbytes = groups * B * K * 8 + (B + 3) // 4 * 16 + B * (4096 + 12 * K) + 16 if groups else full
+    assert not groups or (-(-L // 256) >= 8 * groups and 3 * nbytes < full)
+    v, i = _run(X, W, K, nbytes)
+    assert torch.equal(i, torch.arange(K, device=dev).expand(B, K))
+    assert bool((v.double().abs() <= 4 * 2.0 ** -23 * magnitude[:, None]).all()) and float(v.abs().max()) > 0
+
+
 def test_the_least_workspace_costs_label_groups_and_not_launches(dev):
     """16 rows x 700,001 x 768, K = 1 in 1,088 bytes: 18 times what it takes with 2.8 MB.  (Range after range of labels: 300 times.)"""
     B, L, d, K = 16, 700001, 768, 1
