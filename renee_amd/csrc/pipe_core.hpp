@@ -41,6 +41,9 @@ __device__ __attribute__((aligned(16))) const uint32_t g_zero16[4] = {0u, 0u, 0u
 // eight L2s (32 MB) still hold to be written back.  THROUGH: past the L2 to the Infinity Cache at once (agent scope): nothing is left
 // to write back, for outputs about as large as the L2s or smaller; more of them, or pieces of lines, pass the fabric faster when the L2
 // has gathered them.  PAST: as what will not be wanted again, past the Infinity Cache too, for outputs that it would not hold.
+// THROUGH is inline asm, in which the compiler does not see a store: what it stores may come out of an addition, a conversion, a
+// load or a copy out of the accumulation registers, but not straight from an MFMA, behind which the compiler would put no wait states
+// (tests/test_host.py looks the built kernels over).
 enum StoreHow { CACHED = 0, PAST = 1, THROUGH = 2 };
 template <int HOW, class T>
 __device__ __forceinline__ void store(T* p, const T& v) {

@@ -420,3 +420,42 @@ def test_built_kernels_keep_the_distances_that_the_compiler_does_not_see_in_inli
                 products += 1
                 clear(n, 2, vectors(operands.partition(",")[2]), vectors)
     assert len(kernels) > 50 and accesses > 10000 and products > 4000 and joins > 1000
+
+
+def test_stores_in_inline_asm_take_no_result_straight_from_an_mfma():
+    """A store must stand some 20 wait states behind an MFMA that writes what it stores; the compiler keeps that distance for its own
+    stores but does not see those in inline asm (renee_amd/csrc/pipe_core.hpp: what is written through the L2, with an s_nop behind).
+    Whatever way leads to such a store, the last instruction that wrote what it stores is no MFMA.  The distance between an MFMA and
+    an instruction of another kind that reads its result is kept by the compiler, or by settle() where the MFMA is inline asm too."""
+
+    def vectors(operands):
+        out = set()
+        for kind, lo, hi in re.findall(r"\b([va])\[(\d+):(\d+)\]", operands):
+            out |= {(kind, n) for n in range(int(lo), int(hi) + 1)}
+        return out | {(kind, int(n)) for kind, n in re.findall(r"\b([va])(\d+)\b", operands)}
+
+    stores = 0
+    for kernel, code in _built_code().items():
+        place = {at: n for n, (at, *_) in enumerate(code)}
+        before = [[n - 1] if n and code[n - 1][1] not in ("s_branch", "s_endpgm", "s_setpc_b64") else [] for n in range(len(code))]
+        for n, (_, op, _, to) in enumerate(code):
+            if to is not None:
+                before[place[to]].append(n)
+        # not of memory: a load's first operand is what it writes too, an LDS write or a store writes no register
+        writes = [vectors(operands.split(",")[0]) if not re.match(r"(s_|ds_write|(global|flat|scratch|buffer)_(store|atomic|load_lds))", op) else set()
+                  for _, op, operands, _ in code]
+        for n, (_, op, operands, _) in enumerate(code):
+            if not (op.startswith("global_store") and "sc1" in operands and n + 1 < len(code) and code[n + 1][1:3] == ("s_nop", "1")):
+                continue
+            stores += 1
+            todo, seen = [(m, frozenset(vectors(operands.split(",")[1]))) for m in before[n]], set()
+            while todo:
+                m, wanted = todo.pop()
+                if (m, wanted) in seen:
+                    continue
+                seen.add((m, wanted))
+                assert not (code[m][1].startswith("v_mfma") and wanted & writes[m]), (kernel, code[n], code[m])
+                left = wanted - writes[m]
+                if left:
+                    todo += [(k, left) for k in before[m]]
+    assert stores > 100
