@@ -18,6 +18,7 @@
 #include "back_wide.hpp"
 #include "pipe_core.hpp"
 #include "small_step.hpp"
+#include "tile_plan.hpp"
 #include "topk.hpp"
 #include "topk_lists.hpp"
 #include "wide_core.hpp"
@@ -47,6 +48,9 @@ static_assert(FwdWide::LDS_BYTES <= 160 * 1024, "LDS budget");
 // The same loop on 128 labels x 128 rows, two workgroups to a CU (see fwd_plan).
 using FwdWide128 = WideCore<128, 128, 2, 2, true>;
 static_assert(2 * FwdWide128::LDS_BYTES <= 160 * 1024, "two to a CU");
+template <class C, FwdTile T>
+constexpr bool planned = C::BM == fwd_tile_labels(T) && C::BN == fwd_tile_rows(T) && C::BK == FWD_STAGE;
+static_assert(planned<FwdWide, FWD_WIDE> && planned<FwdWide128, FWD_WIDE128>, "tile_plan.hpp");
 // Batches of up to 128 and 64 rows (the reference's B = 32 plumbing case, --accum micro-batches, the last partial batch
 // of an epoch), where a 256-row tile would spend most of its MFMAs on padding: W streams from HBM, eight waves, three
 // ring slots.
@@ -60,7 +64,8 @@ struct FwdLds {
   static_assert(C::FN % 2 == 0, "staging read-back walks 64-label pieces");
   static_assert(BYTES <= 160 * 1024, "LDS budget");
 };
-static_assert(FwdCore::BN == FwdWide::BM && FwdCore64::BN == FwdWide::BM, "one label tile width");
+static_assert(FwdCore::BN == fwd_tile_labels(FWD_128) && FwdCore::BM == fwd_tile_rows(FWD_128) && FwdCore64::BN == fwd_tile_labels(FWD_64) &&
+              FwdCore64::BM == fwd_tile_rows(FWD_64), "tile_plan.hpp");
 
 constexpr int LOGIT_BLOCK = 32;
 // max of two packed halves each, and of three; an operand that is no number wins, so that a block with one can be told.
@@ -95,7 +100,7 @@ struct FwdArgs {
   half_t* out; int64_t ldo;         // M x n_store, row-major
   int M, N, K, n_store;             // columns N <= c < n_store are written as zero
   float alpha, beta;
-  double* loss_part;                // LOSS: one partial sum per workgroup
+  double* loss_part; int loss_have; // LOSS: one partial sum per workgroup, the first loss_have added to what is there
   half_t* bmax; int64_t ldb;        // BMAX: [M][ldb] the largest stored value of every LOGIT_BLOCK columns
   int tiles_m, tiles_n, n_ids;      // n_ids = tiles_m * round_up(tiles_n, 8)
   bool through;                     // out is stored through the L2 (see launch_fwd)
@@ -232,7 +237,7 @@ __global__ void __launch_bounds__(C::NT, 160 * 1024 / C::LDS_BYTES) fwd_wide_ker
     if (threadIdx.x == 0) {
       double t = 0.0;
       for (int i = 0; i < C::NW; ++i) t += red[i];
-      a.loss_part[w] = t;
+      a.loss_part[w] = w < a.loss_have ? a.loss_part[w] + t : t;
     }
   }
 }
@@ -1308,8 +1313,6 @@ using namespace xfc;
 
 namespace {
 
-inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
-inline int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 int check_launch() {
@@ -1385,60 +1388,20 @@ void* static_scratch_ptr() {
 
 // Scratch of the forward pass with the loss: a double per forward workgroup and a float per label pair.
 constexpr size_t LOSS_PART_BYTES = 4096;
-constexpr int MAX_FWD_GRID = LOSS_PART_BYTES / sizeof(double) - 8;  // 504, with room to align; a multiple of 8
 size_t fwd_ws_bytes(int64_t nnz) { return LOSS_PART_BYTES + (size_t)round_up((nnz > 0 ? nnz : 1) * 4, 256); }
 
 // Row-tile height for a batch of M rows (see FwdWide / FwdCore / FwdCore64).
 inline int row_tile(int64_t M) { return M <= 64 ? 64 : M <= 128 ? 128 : 256; }
 
-// Workgroups of a persistent pass over tiles: one resident per CU (the number of tile ids is a multiple of 8).
-inline int64_t fwd_grid(int64_t ids, int per_cu = 1) {
-  const int64_t all = per_cu * round_up(num_cus(), 8), grid = all < MAX_FWD_GRID ? all : MAX_FWD_GRID;
-  return grid < ids ? grid : ids;
-}
-
-// Which tile the forward pass takes: the labels [0, first) go by `tile`, those after them, if any, by FWD_WIDE128.
-enum FwdTile { FWD_64, FWD_128, FWD_WIDE, FWD_WIDE128 };
-struct FwdPlan {
-  FwdTile tile;
-  int64_t first;
+// Where the forward pass leaves the loss's partial sums, and how many: the workspace need not be aligned.
+struct LossPart {
+  double* at;
+  int64_t places;
 };
-inline int64_t fwd_ids(FwdTile t, int64_t M, int64_t n) {
-  const int64_t rows = t == FWD_64 ? 64 : t == FWD_WIDE ? 256 : 128, labels = t == FWD_WIDE128 ? 128 : 256;
-  return ceil_div(M, rows) * round_up(ceil_div(n, labels), 8);
-}
-// Large tiles move the fewest bytes through the fetch path, small ones fill the chip with few labels, leave no last round nearly
-// empty, and two of them on a CU work at each other's epilogues.  Time in rounds of the large tile, of 256 tiles on as many CUs: a round is
-// 8.6 us at 64 dims, 16.5 at 384, 26 at 768, 32 at 1024, 256 small tiles 0.31 of it (with the loss, whose epilogue is the longer,
-// 0.28); on the 128-row tile of the eight-wave loop a round is 14.5 to 22 us at 768 dims, and 256 small tiles 0.58 of it.  Measured
-// (fwd_grad without pairs, large and small, us): 200 rows x 8,001 labels x 768 dims 27.7 and 10.9, x 30,001 30.7 and 19.7, x
-// 60,001 34.6 and 35.7, x 131,073 84 and 73, 256 x 131,072 63 and 81, 512 x 60,001 57 and 70, x 20,001 x 256 21.1 and 13.5, 300 x
-// 131,073 x 384 80 and 61, 1024 x 131,072 x 768 219 and 262; 100 rows x 4,097 x 768 14.2 and 10.3, x 60,001 20.7 and 22.8, x 80,001 39.2 and
-// 34.3, x 250,001 85 and 96.  Where whole rounds of large tiles leave few labels over, those go by small tiles in a launch of their
-// own, 7.5 us and more: whole steps of 512 rows x 131,073 labels x 768 dims 379 -> 370 us, 256 rows 281 -> 273, 512 x 100,001 299 -> 290, with
-// the loss 512 x 131,073 414 -> 396.  Whole steps of few labels: 200 x 8,001 62.8 -> 45.4, 300 x 16,001 79 -> 68; top-100 of 200 x 20,001
-// 40.4 -> 29.3.
-FwdPlan fwd_plan(int64_t M, int64_t n, int64_t d, bool loss) {
-  if (M <= 64) return {FWD_64, n};
-  const int64_t cus = num_cus();
-  auto rounds = [&](FwdTile t, int64_t labels) { return (double)ceil_div(fwd_ids(t, M, labels), cus); };
-  if (M <= 128) return {0.58 * rounds(FWD_WIDE128, n) < rounds(FWD_128, n) ? FWD_WIDE128 : FWD_128, n};
-  const double small = loss ? 0.28 : 0.31, launch = 7.5 / (7.0 + 1.58 * (double)ceil_div(d, FwdWide::BK));
-  const double large = rounds(FWD_WIDE, n);
-  FwdPlan best = {FWD_WIDE, n};
-  double least = large;
-  if (small * rounds(FWD_WIDE128, n) < least) best = {FWD_WIDE128, n}, least = small * rounds(FWD_WIDE128, n);
-  // whole rounds, in label tiles that the 8 XCDs divide
-  const int64_t first = ((int64_t)large - 1) * cus / ceil_div(M, FwdWide::BN) / 8 * 8 * FwdWide::BM;
-  if (first > 0 && first < n && large - 1.0 + launch + small * rounds(FWD_WIDE128, n - first) < least) best = {FWD_WIDE, first};
-  return best;
-}
-// Workgroups of the pass, each with a partial sum of the loss.
-int64_t fwd_grid(const FwdPlan& p, int64_t M) { return fwd_grid(fwd_ids(p.tile, M, p.first), p.tile == FWD_WIDE128 ? 2 : 1); }
-int64_t fwd_rest_grid(const FwdPlan& p, int64_t M, int64_t n) {
-  if (p.first >= n) return 0;
-  const int64_t ids = fwd_ids(FWD_WIDE128, M, n - p.first), left = MAX_FWD_GRID - fwd_grid(p, M), grid = fwd_grid(ids, 2);
-  return grid < left ? grid : left;
+constexpr LossPart NO_LOSS = {nullptr, ANY_GRID};
+LossPart loss_part_of(void* ws) {
+  const uintptr_t from = (reinterpret_cast<uintptr_t>(ws) + 7) & ~(uintptr_t)7;
+  return {reinterpret_cast<double*>(from), (int64_t)(reinterpret_cast<uintptr_t>(ws) + LOSS_PART_BYTES - from) / 64 * 8};
 }
 
 template <class C>
@@ -1466,18 +1429,18 @@ int launch_fwd_c(int mode, const FwdArgs& a, dim3 g, hipStream_t st) {
 }
 
 int launch_fwd(const FwdPlan& p, int mode, const half_t* X, int64_t ldx, const half_t* W, int64_t ldw, half_t* out, int64_t ldo, int M,
-               int N, int K, int n_store, float alpha, float beta, hipStream_t st, double* loss_part = nullptr,
+               int N, int K, int n_store, float alpha, float beta, hipStream_t st, LossPart loss = NO_LOSS,
                half_t* bmax = nullptr, int64_t ldb = 0) {
   FwdArgs a;
   a.X = X; a.ldx = ldx; a.W = W; a.ldw = ldw; a.out = out; a.ldo = ldo;
   a.M = M; a.N = p.first < N ? (int)p.first : N; a.K = K; a.n_store = (int)p.first; a.alpha = alpha; a.beta = beta;
-  a.loss_part = loss_part;
+  a.loss_part = loss.at; a.loss_have = 0;
   a.bmax = bmax; a.ldb = ldb;
   // Few logits are written through: with whole steps of 40 rows x 30,001 labels x 64 dims 23.0 -> 22.3 us, 256 x 20,001 x 256 43.2 -> 42.3, 50 x
   // 10,001 x 1024 41.4 -> 39.3, but (the wide loop's pieces are half lines) 512 x 20,001 x 768 97.2 -> 98.9, 100 x 60,001 109.9 -> 110.7.
   a.through = (int64_t)M * n_store * 2 <= (int64_t)(p.tile == FWD_WIDE128 ? 10 : 8) << 20;
   auto tiles = [&](FwdTile t, int64_t n) {
-    a.tiles_n = ceil_div(n, t == FWD_WIDE128 ? FwdWide128::BM : FwdWide::BM);
+    a.tiles_n = ceil_div(n, fwd_tile_labels(t));
     const int64_t ids = fwd_ids(t, M, n);
     a.tiles_m = (int)(ids / round_up(a.tiles_n, 8));
     a.n_ids = (int)ids;
@@ -1485,7 +1448,7 @@ int launch_fwd(const FwdPlan& p, int mode, const half_t* X, int64_t ldx, const h
   };
   if (M <= 0 || n_store <= 0) return XFC_OK;
   if (!tiles(p.tile, p.first)) return XFC_ERR_INVALID;
-  const int64_t grid = fwd_grid(p, M), rest = fwd_rest_grid(p, M, n_store);
+  const int64_t grid = fwd_grid(p, M, num_cus(), loss.places), rest = fwd_rest_grid(p, M, n_store, num_cus(), loss.places);
   const dim3 g((unsigned)grid);
   int rc;
   switch (p.tile) {
@@ -1500,7 +1463,7 @@ int launch_fwd(const FwdPlan& p, int mode, const half_t* X, int64_t ldx, const h
   a.out += p.first;
   a.N = N - (int)p.first;
   a.n_store = n_store - (int)p.first;
-  if (loss_part) a.loss_part += grid;
+  a.loss_have = (int)grid;
   if (bmax) a.bmax += p.first / LOGIT_BLOCK;
   tiles(FWD_WIDE128, a.n_store);
   return launch_fwd_wide<FwdWide128>(mode, a, dim3((unsigned)rest), st);
@@ -2017,7 +1980,7 @@ int xfc_gemm(const void* in1, int64_t in1_rows, int64_t in1_cols, int64_t in1_s0
     const bool fast = out_s1 == 1 && out_s0 % 8 == 0 && aligned16(out) && in1_s0 % 8 == 0 && in2_s1 % 8 == 0 &&
                       K % 8 == 0 && aligned16(in1) && aligned16(in2) && K > 0;
     if (fast)
-      return launch_fwd(fwd_plan(M, N, K, false), FWD_SIGMOID, (const half_t*)in1, in1_s0, (const half_t*)in2, in2_s1, (half_t*)out,
+      return launch_fwd(fwd_plan(M, N, K, false, num_cus()), FWD_SIGMOID, (const half_t*)in1, in1_s0, (const half_t*)in2, in2_s1, (half_t*)out,
                         out_s0, (int)M, (int)N, (int)K, (int)N, alpha, beta, st);
     return launch_generic(in1, in1_s0, in1_s1, in2, in2_s0, in2_s1, out, out_s0, out_s1, (int)M, (int)N, (int)K, alpha,
                           beta, 1, 1, st);
@@ -2058,7 +2021,7 @@ int xfc_logits(const void* X, int64_t ldx, const void* W, int64_t ldw, void* out
   if (ldx % 8 || ldw % 8 || ldo % 8 || d % 8 || !aligned16(X) || !aligned16(W) || !aligned16(out))
     return XFC_ERR_ALIGN;
   if (ldo < L) return XFC_ERR_SHAPE;
-  return launch_fwd(fwd_plan(B, L, d, false), FWD_LINEAR, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)out, ldo, (int)B,
+  return launch_fwd(fwd_plan(B, L, d, false, num_cus()), FWD_LINEAR, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)out, ldo, (int)B,
                     (int)L, (int)d, (int)L, 1.0f, 0.0f, reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -2112,12 +2075,12 @@ static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw,
   if (!ws || ws_bytes < fwd_ws_bytes(nnz)) return XFC_ERR_WORKSPACE;
   bool taken;
   if (int rc0 = small_grad(X, ldx, W, ldw, rowptr, colidx, pos_x, pos_y, nnz, G, ldg, B, L, d, loss, st, &taken); taken) return rc0;
-  double* loss_part = loss ? reinterpret_cast<double*>((reinterpret_cast<uintptr_t>(ws) + 7) & ~(uintptr_t)7) : nullptr;
+  const LossPart loss_part = loss ? loss_part_of(ws) : NO_LOSS;
   float* loss_pos = loss ? reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(ws) + LOSS_PART_BYTES) : nullptr;
   // label columns L .. round_up(L, 8) are written as zero so that G can be read in 16-byte
   // pieces along the label axis by the dX and dW kernels (ldg is a multiple of 8, so they exist)
   const int64_t n_store = round_up(L, 8);
-  const FwdPlan plan = fwd_plan(B, n_store, d, loss != nullptr);
+  const FwdPlan plan = fwd_plan(B, n_store, d, loss != nullptr, num_cus());
   int rc = launch_fwd(plan, FWD_SIGMOID, (const half_t*)X, ldx, (const half_t*)W, ldw, (half_t*)G, ldg, (int)B, (int)L, (int)d,
                       (int)n_store, 1.0f, 0.0f, st, loss_part);
   if (rc) return rc;
@@ -2133,8 +2096,9 @@ static int fwd_grad_impl(const void* X, int64_t ldx, const void* W, int64_t ldw,
     if ((rc = check_launch())) return rc;
   }
   if (loss) {
-    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(1024), 0, st, (const double*)loss_part,
-                       (int)(fwd_grid(plan, B) + fwd_rest_grid(plan, B, n_store)), (const float*)loss_pos, nnz, loss);
+    const int64_t first = fwd_grid(plan, B, num_cus(), loss_part.places), rest = fwd_rest_grid(plan, B, n_store, num_cus(), loss_part.places);
+    hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(1024), 0, st, (const double*)loss_part.at, (int)(first > rest ? first : rest),
+                       (const float*)loss_pos, nnz, loss);
     return check_launch();
   }
   return XFC_OK;
@@ -2580,8 +2544,8 @@ static int topk_impl(const void* X, int64_t ldx, const void* W, int64_t ldw, int
     }
     for (int64_t r0 = 0; r0 < B; r0 += block) {
       const int64_t rows = B - r0 < block ? B - r0 : block;
-      int rc = launch_fwd(fwd_plan(rows, L, d, false), FWD_LINEAR, (const half_t*)X + r0 * ldx, ldx, (const half_t*)W, ldw,
-                          (half_t*)workspace, ldl, (int)rows, (int)L, (int)d, (int)L, 1.0f, 0.0f, st, nullptr, bmax, ldb);
+      int rc = launch_fwd(fwd_plan(rows, L, d, false, num_cus()), FWD_LINEAR, (const half_t*)X + r0 * ldx, ldx, (const half_t*)W, ldw,
+                          (half_t*)workspace, ldl, (int)rows, (int)L, (int)d, (int)L, 1.0f, 0.0f, st, NO_LOSS, bmax, ldb);
       if (rc) return rc;
       // sample every stride-th 16 KB block first when that still holds 16 K elements and points at about a
       // thousand candidates at most (half the sort buffer)
@@ -2622,7 +2586,7 @@ static int topk_impl(const void* X, int64_t ldx, const void* W, int64_t ldw, int
       a.n_ids = (int)ids;
       auto launch = [&](auto core) {
         using C = typename decltype(core)::type;
-        return launch_k<score_wide_kernel<C>>(dim3((unsigned)fwd_grid(ids)), dim3(C::NT), C::LDS_BYTES, st, a);
+        return launch_k<score_wide_kernel<C>>(dim3((unsigned)persistent_grid(ids, 1, num_cus())), dim3(C::NT), C::LDS_BYTES, st, a);
       };
       rc = row_tile(B) <= 128 ? launch(std::type_identity<ScoreWide128>{}) : launch(std::type_identity<ScoreWide>{});
     }
