@@ -1,4 +1,5 @@
-"""Which tiles the forward pass and dW take (renee_amd/csrc/tile_plan.hpp, where the launches take it from), on 256 CUs."""
+"""Which tiles the forward pass and dW take and how dW's outputs are stored (renee_amd/csrc/tile_plan.hpp, where the launches take it from), on
+256 CUs unless said otherwise; tests that run on the GPU take from here what their sizes lead to."""
 import pytest
 from test_back_wide_order import _compiled
 
@@ -7,34 +8,52 @@ TEXT = r'''
 #include "tile_plan.hpp"
 int main() {
   using namespace xfc;
-  long long M, n, d, loss;
-  while (scanf("%lld %lld %lld %lld", &M, &n, &d, &loss) == 4) {
-    const long long most = loss ? 512 : ANY_GRID;  // 4096 bytes of doubles
-    const FwdPlan p = fwd_plan(M, n, d, loss != 0, 256);
-    printf("%d %lld %lld %lld %lld %lld\n", (int)p.tile, (long long)p.first, (long long)fwd_ids(p.tile, M, p.first), (long long)fwd_grid(p, M, 256, most),
-           (long long)(p.first < n ? fwd_ids(FWD_WIDE128, M, n - p.first) : 0), (long long)fwd_rest_grid(p, M, n, 256, most));
+  long long what, cus, M, n, d, more;
+  while (scanf("%lld %lld %lld %lld %lld %lld", &what, &cus, &M, &n, &d, &more) == 6) {
+    if (what == 0) {
+      const long long most = more ? 512 : ANY_GRID;  // 4096 bytes of doubles
+      const FwdPlan p = fwd_plan(M, n, d, more != 0, cus);
+      printf("%d %lld %lld %lld %lld %lld\n", (int)p.tile, (long long)p.first, (long long)fwd_ids(p.tile, M, p.first), (long long)fwd_grid(p, M, cus, most),
+             (long long)(p.first < n ? fwd_ids(FWD_WIDE128, M, n - p.first) : 0), (long long)fwd_rest_grid(p, M, n, cus, most));
+    } else {
+      const DwPlan p = dw_plan((DwMode)more, n, d, M, cus);
+      printf("%d %d\n", (int)p.small, (int)p.how);
+    }
   }
 }
 '''
 TILES = ("64", "128", "wide", "wide128")
+OUT, UPDATE, MASTER = 0, 1, 2
+CACHED, PAST, THROUGH = 0, 1, 2
 
 
-@pytest.fixture(scope="module")
-def forward(tmp_path_factory):
-    """(rows, labels, dims, with the loss) -> tile, labels it takes, tiles, workgroups; tiles and workgroups of the labels after them."""
-    def plans(sizes):
-        lines = _compiled(tmp_path_factory, TEXT, [int(v) for s in sizes for v in s])
+class Plans:
+    def __init__(self, tmp_path_factory):
+        self.tmp = tmp_path_factory
+
+    def forward(self, sizes, cus=256):
+        """(rows, labels, dims, with the loss) -> tile, labels it takes, tiles, workgroups; tiles and workgroups of the labels after them."""
+        lines = _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (0, cus, *s)])
         return [(TILES[int(line.split()[0])], *map(int, line.split()[1:])) for line in lines]
-    return plans
+
+    def dw(self, sizes, cus=256):
+        """(rows, labels, dims, mode) -> whether by small tiles, how what is written is stored."""
+        lines = _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (1, cus, *s)])
+        return [(line.split()[0] == "1", int(line.split()[1])) for line in lines]
 
 
-def test_every_place_that_the_plan_prices_is_taken(forward):
+@pytest.fixture(scope="session")
+def plans(tmp_path_factory):
+    return Plans(tmp_path_factory)
+
+
+def test_every_place_that_the_plan_prices_is_taken(plans):
     """The plan counts two small tiles to a CU, one of any other: so many workgroups must run, with the loss and without, and for the
     labels that whole rounds of large tiles leave over."""
     sizes = [(M, n, d, loss) for M in (1, 64, 65, 100, 128, 129, 200, 256, 300, 512, 700, 1024) for d in (64, 384, 768, 1024) for loss in (0, 1)
              for n in (8, 1000, 8192, 16384, 32768, 31752, 60008, 72008, 80008, 100008, 131080, 196616, 320008, 655368, 2812288)]
     small = rest = 0
-    for size, (tile, first, ids, grid, rest_ids, rest_grid) in zip(sizes, forward(sizes)):
+    for size, (tile, first, ids, grid, rest_ids, rest_grid) in zip(sizes, plans.forward(sizes)):
         places = 512 if tile == "wide128" else 256
         assert grid == min(ids, places) and ids % 8 == 0 and 0 < first <= size[1], size
         assert rest_grid == min(rest_ids, 512) and (rest_ids == 0) == (first == size[1]), size
