@@ -23,6 +23,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "tile_plan.hpp"
+
 namespace xfc {
 
 typedef _Float16 half_t;
@@ -37,14 +39,9 @@ typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
 __device__ __attribute__((aligned(16))) const uint32_t g_zero16[4] = {0u, 0u, 0u, 0u};
 
-// How an output is stored.  CACHED: it stays in the L2 until something pushes it out or the kernel ends, which waits for what its
-// eight L2s (32 MB) still hold to be written back.  THROUGH: past the L2 to the Infinity Cache at once (agent scope): nothing is left
-// to write back, for outputs about as large as the L2s or smaller; more of them, or pieces of lines, pass the fabric faster when the L2
-// has gathered them.  PAST: as what will not be wanted again, past the Infinity Cache too, for outputs that it would not hold.
-// THROUGH is inline asm, in which the compiler does not see a store: what it stores may come out of an addition, a conversion, a
-// load or a copy out of the accumulation registers, but not straight from an MFMA, behind which the compiler would put no wait states
-// (tests/test_host.py looks the built kernels over).
-enum StoreHow { CACHED = 0, PAST = 1, THROUGH = 2 };
+// A store as StoreHow says.  THROUGH is inline asm, in which the compiler does not see a store: what it stores may come out of an
+// addition, a conversion, a load or a copy out of the accumulation registers, but not straight from an MFMA, behind which the compiler would
+// put no wait states (tests/test_host.py looks the built kernels over).
 template <int HOW, class T>
 __device__ __forceinline__ void store(T* p, const T& v) {
   static_assert(HOW != THROUGH || sizeof(T) == 16 || sizeof(T) == 8 || sizeof(T) == 4, "piece");

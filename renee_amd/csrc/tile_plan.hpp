@@ -9,6 +9,12 @@ namespace xfc {
 inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 inline int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 
+// How an output is stored.  CACHED: it stays in the L2 until something pushes it out or the kernel ends, which waits for what its
+// eight L2s (32 MB) still hold to be written back.  THROUGH: past the L2 to the Infinity Cache at once (agent scope): nothing is left
+// to write back, for outputs about as large as the L2s or smaller; more of them, or pieces of lines, pass the fabric faster when the L2
+// has gathered them.  PAST: as what will not be wanted again, past the Infinity Cache too, for outputs that it would not hold.
+enum StoreHow { CACHED = 0, PAST = 1, THROUGH = 2 };
+
 // ---------------------------------------------------------------------------------------------
 // forward pass
 // ---------------------------------------------------------------------------------------------
@@ -60,6 +66,62 @@ inline int64_t fwd_grid(const FwdPlan& p, int64_t M, int64_t cus, int64_t most) 
 }
 inline int64_t fwd_rest_grid(const FwdPlan& p, int64_t M, int64_t n, int64_t cus, int64_t most) {
   return p.first < n ? persistent_grid(fwd_ids(FWD_WIDE128, M, n - p.first), 2, cus, most) : 0;
+}
+
+// ---------------------------------------------------------------------------------------------
+// dW
+// ---------------------------------------------------------------------------------------------
+enum DwMode { DW_OUT = 0, DW_UPDATE = 1, DW_UPDATE_MASTER = 2 };  // MASTER: fp32 master weights and momentum, fp16 copy of W
+constexpr int DW_TILE = 256, DW_SMALL_TILE = 128;  // labels and dims
+struct DwPlan {
+  bool small;    // tiles of DW_SMALL_TILE
+  StoreHow how;  // what is written
+};
+// Large tiles move the fewest bytes through the fetch path and the L2s, small ones fill the chip with few labels, leave no last round
+// nearly empty, waste less of a width that is no multiple of 256, and two of them on a CU work at each other's epilogues.  Compared
+// by rounds of the large ones, four small tiles to one of them at a price: nothing while the update's traffic binds, up to a sixth
+// (of a gradient a quarter) at 1024 rows, 0.05 more for a state that no cache holds (fp32: from 160 Mi weights on); of a gradient a fifth for one that none does and
+// 256 rows or more, two fifths for a large one of whole large tiles, whose rows a small tile writes in pieces of 512 bytes.  Measured
+// (us, large and small).  Updates: 32 rows x 8,001 labels x 256 dims 10.9 and 5.7, 128 x 30,001 x 768 46 and 37, 600 x 4,097 x 768 22.3
+// and 11.8, 1024 x 20,001 x 1024 83 and 68, 384 x 700,001 x 384 583 and 537, 1024 x 1,000,001 x 128 728 and 636, but 512 x 655,363 x 768
+// 1000 and 1100, 1024 x 131,072 x 768 293 and 327.  Master weights: 300 x 20,001 x 1024 106 and 82, 512 x 131,072 x
+// 768 393 and 373, 512 x 700,001 x 384 1163 and 1064, whole steps of 512 x 450,001 x
+// 768 1943 and 1911, 128 x 450,001 1532 and 1556, 512 x 655,363 2581 and 2629 or 2828 and 2823, 1024 x 655,363 x 768 2262 and 2381.  Gradients: 128 x
+// 131,073 x 768 79.7 and 74.7, 300 x 8,001 x 768 13.2 and 10.0, 512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768 505 and 611, 136 x 1,096,208 x
+// 256 243 and 334, 248 x 234,640 x 1024 204 and 227, 712 x 80,256 x 512 86.8 and 90.7, 32 x 1,000,000 x 128 90 and 100, but 64 rows 97 and 92, 1024 x 20,000 x 1024 62 and 53, 256 x 400,000 x 384 156 and 147.
+inline bool dw_small_tiles(DwMode mode, int64_t labels, int64_t dims, int64_t rows, bool past, int64_t cus) {
+  auto rounds = [&](int64_t tile) {  // (a last one nearly empty leaves the others the more of the memory: half of it counts)
+    const double n = (double)(ceil_div(dims, tile) * round_up(ceil_div(labels, tile), 8)) / (double)cus;
+    return 0.5 * (n + ceil(n));
+  };
+  const double over = rows > 256 ? (double)((rows < 1024 ? rows : 1024) - 256) : 0.0;
+  double price = 1.0 + 0.0002 * over;
+  if (mode == DW_UPDATE && past) price += 0.05;
+  const int64_t Mi = (int64_t)1 << 20, weights = labels * dims;
+  if (mode == DW_OUT) {
+    if (past && dims % DW_TILE == 0 && weights > 120 * Mi) price = 1.4;
+    else if (past && rows >= 256) price = 1.2;
+    else if (past && rows <= 48 && dims > 64 && dims <= DW_SMALL_TILE) price = 2.2;  // (half of a large tile empty: what it multiplies is little)
+    else price += 0.0001 * over;
+  }
+  if (mode == DW_UPDATE_MASTER) price = 0.99 + (rows > 512 || weights > (rows <= 128 ? 160 : 380) * Mi ? 0.05 : 0.0);
+  return price * rounds(DW_SMALL_TILE) < 4.0 * rounds(DW_TILE);
+}
+// Non-temporal stores where what is written would push out of the caches what the next kernels read, from about their size on.  A
+// gradient: six-argument calls of 512 rows x 131,072 labels x 768 dims 384 -> 347 us, 128 rows 212 -> 178, 512 x 200,000 x 256 303
+// -> 261, x 80,000 x 768 258 -> 241, but x 32,768 118 -> 120.  Master weights: steps of 512 x 655,363 x 768 2868 -> 2813, 64 x
+// 200,001 717 -> 668, 256 x 131,072 x 256 201 -> 193, but 256 x 20,001 x 768 115 -> 123.  fp16 state: 1024 x 2,812,281 x 768 13.81 ->
+// 13.67 ms, x 700,001 3.48 -> 3.44, but 800 x 200,001 x 512 684 -> 688, 700 x 131,072 x 256 228 -> 235.  Not only back to back: the
+// calls of 512 rows x 131,072 each followed by a copy of 512 MiB 567 -> 522, by 0.6 ms of matrix products 1011 -> 978, waited for 409 -> 373.
+// Small ones are written through (see StoreHow).  Over three states in turn and over one (us): master weights 64 rows x 5,001
+// labels x 768 dims 49.7, 50.3 -> 45.3, 46.7, 300 x 10,001 94, 86 -> 93, 73, but 100 x 20,001 97.6, 83.9 -> 99.2, 81.2; fp16 state 600 x
+// 8,001 77.1, 77.4 -> 72.6, 73.8, 800 x 60,001 306, 305 -> 304, 301, but 1024 x 131,072 687 -> 694.  Gradients, six-argument calls of 128 x
+// 20,000 50.9 -> 47.9; by themselves, with G out of HBM, larger ones lose: 256 x 23,293 x 1024 32 -> 37, 512 x 27,823 x 1024 49 -> 61.
+inline DwPlan dw_plan(DwMode mode, int64_t labels, int64_t dims, int64_t rows, int64_t cus) {
+  const int64_t weights = labels * dims, Mi = (int64_t)1 << 20;
+  const bool through = weights <= (mode == DW_UPDATE ? 48 : mode == DW_UPDATE_MASTER ? 12 : 16) * Mi;
+  const bool past = weights > (mode == DW_UPDATE ? 140 : mode == DW_UPDATE_MASTER ? 28 : 40) * Mi;
+  return {dw_small_tiles(mode, labels, dims, rows, past, cus), past ? PAST : through ? THROUGH : CACHED};
 }
 
 }  // namespace xfc

@@ -982,15 +982,14 @@ __global__ void __launch_bounds__(32 * SG) dx_reduce_kernel(const float* __restr
 // ---------------------------------------------------------------------------------------------
 // dW = G^T . X; either written out (fp32, alpha/beta) or consumed by the momentum update
 // ---------------------------------------------------------------------------------------------
-enum DwMode { DW_OUT = 0, DW_UPDATE = 1, DW_UPDATE_MASTER = 2 };  // MASTER: fp32 master weights and momentum, fp16 copy of W
-
 // 256 labels x 256 dims x 64 batch rows per stage, eight waves of 64 labels x 128 dims, one workgroup per CU.
 // (A 128 x 256 x 32 tile with four waves and two workgroups per CU, meant to overlap one workgroup's update with
 // the other's GEMM, measured 7-11 % slower at every batch size: its stages move half again as much through LDS
 // and the fetch path per flop, and the update's streaming is bound by HBM either way.)
 using DwCore = PipeCore<256, 256, 64, 4, 2, 2, false, false, false, false, false, 4>;
-// 128 labels x 128 dims, eight waves of 32 x 64, two workgroups to a CU: see launch_dw.
+// 128 labels x 128 dims, eight waves of 32 x 64, two workgroups to a CU: see dw_plan.
 using DwCore128 = PipeCore<128, 128, 64, 4, 2, 2, false, false, false, false, false, 4>;
+static_assert(DwCore::BM == DW_TILE && DwCore::BN == DW_TILE && DwCore128::BM == DW_SMALL_TILE && DwCore128::BN == DW_SMALL_TILE, "tile_plan.hpp");
 constexpr int DW_STAGE_FLOATS = 8 * 64;  // per wave: 8 label rows x 64 dims
 template <class C>
 struct DwLds {
@@ -1017,7 +1016,7 @@ struct DwArgs {
 
 // Persistent, as many workgroups as the CUs hold: workgroup w takes tile ids w, w + gridDim.x, ...; the dim tiles of
 // one label tile have neighbouring ids on one XCD, so its slice of G is fetched from HBM once.
-// HOW what is written is stored: see launch_dw.
+// HOW what is written is stored: see dw_plan.
 template <class C, int MODE, int HOW>
 __global__ void __launch_bounds__(C::NT, C::NW * DwLds<C>::PER_CU / 4) dw_kernel(DwArgs a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
@@ -1544,38 +1543,8 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
   return check_launch();
 }
 
-// Large tiles move the fewest bytes through the fetch path and the L2s, small ones fill the chip with few labels, leave no last round
-// nearly empty, waste less of a width that is no multiple of 256, and two of them on a CU work at each other's epilogues.  Compared
-// by rounds of the large ones, four small tiles to one of them at a price: nothing while the update's traffic binds, up to a sixth
-// (of a gradient a quarter) at 1024 rows, 0.05 more for a state that no cache holds (fp32: from 160 Mi weights on); of a gradient a fifth for one that none does and
-// 256 rows or more, two fifths for a large one of whole large tiles, whose rows a small tile writes in pieces of 512 bytes.  Measured
-// (us, large and small).  Updates: 32 rows x 8,001 labels x 256 dims 10.9 and 5.7, 128 x 30,001 x 768 46 and 37, 600 x 4,097 x 768 22.3
-// and 11.8, 1024 x 20,001 x 1024 83 and 68, 384 x 700,001 x 384 583 and 537, 1024 x 1,000,001 x 128 728 and 636, but 512 x 655,363 x 768
-// 1000 and 1100, 1024 x 131,072 x 768 293 and 327.  Master weights: 300 x 20,001 x 1024 106 and 82, 512 x 131,072 x
-// 768 393 and 373, 512 x 700,001 x 384 1163 and 1064, whole steps of 512 x 450,001 x
-// 768 1943 and 1911, 128 x 450,001 1532 and 1556, 512 x 655,363 2581 and 2629 or 2828 and 2823, 1024 x 655,363 x 768 2262 and 2381.  Gradients: 128 x
-// 131,073 x 768 79.7 and 74.7, 300 x 8,001 x 768 13.2 and 10.0, 512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768 505 and 611, 136 x 1,096,208 x
-// 256 243 and 334, 248 x 234,640 x 1024 204 and 227, 712 x 80,256 x 512 86.8 and 90.7, 32 x 1,000,000 x 128 90 and 100, but 64 rows 97 and 92, 1024 x 20,000 x 1024 62 and 53, 256 x 400,000 x 384 156 and 147.
-bool dw_small_tiles(int mode, int64_t labels, int64_t dims, int64_t rows, bool past) {
-  auto rounds = [&](int64_t tile) {  // (a last one nearly empty leaves the others the more of the memory: half of it counts)
-    const double n = (double)(ceil_div(dims, tile) * round_up(ceil_div(labels, tile), 8)), cus = num_cus();
-    return 0.5 * (n / cus + ceil(n / cus));
-  };
-  const double over = rows > 256 ? (double)((rows < 1024 ? rows : 1024) - 256) : 0.0;
-  double price = 1.0 + 0.0002 * over;
-  if (mode == DW_UPDATE && past) price += 0.05;
-  const int64_t Mi = (int64_t)1 << 20, weights = labels * dims;
-  if (mode == DW_OUT) {
-    if (past && dims % DwCore::BN == 0 && weights > 120 * Mi) price = 1.4;
-    else if (past && rows >= 256) price = 1.2;
-    else if (past && rows <= 48 && dims > 64 && dims <= DwCore128::BN) price = 2.2;  // (half of a large tile empty: what it multiplies is little)
-    else price += 0.0001 * over;
-  }
-  if (mode == DW_UPDATE_MASTER) price = 0.99 + (rows > 512 || weights > (rows <= 128 ? 160 : 380) * Mi ? 0.05 : 0.0);
-  return price * rounds(DwCore128::BM) < 4.0 * rounds(DwCore::BM);
-}
 template <class C>
-int launch_dw_tiles(int mode, DwArgs a, bool past, bool through, hipStream_t st) {
+int launch_dw_tiles(DwMode mode, DwArgs a, StoreHow how, hipStream_t st) {
   a.tiles_m = ceil_div(a.M, C::BM);
   a.tiles_n = ceil_div(a.N, C::BN);
   const int64_t ids = (int64_t)a.tiles_n * round_up(a.tiles_m, 8);
@@ -1588,30 +1557,17 @@ int launch_dw_tiles(int mode, DwArgs a, bool past, bool through, hipStream_t st)
   constexpr int LDS = DwLds<C>::BYTES;
   auto launch = [&](auto mode_tag) {
     constexpr int MODE = decltype(mode_tag)::value;
-    if (past) return launch_k<dw_kernel<C, MODE, PAST>>(g, b, LDS, st, a);
-    if (through) return launch_k<dw_kernel<C, MODE, THROUGH>>(g, b, LDS, st, a);
+    if (how == PAST) return launch_k<dw_kernel<C, MODE, PAST>>(g, b, LDS, st, a);
+    if (how == THROUGH) return launch_k<dw_kernel<C, MODE, THROUGH>>(g, b, LDS, st, a);
     return launch_k<dw_kernel<C, MODE, CACHED>>(g, b, LDS, st, a);
   };
   if (mode == DW_UPDATE) return launch(std::integral_constant<int, DW_UPDATE>{});
   if (mode == DW_UPDATE_MASTER) return launch(std::integral_constant<int, DW_UPDATE_MASTER>{});
   return launch(std::integral_constant<int, DW_OUT>{});
 }
-int launch_dw(int mode, const DwArgs& a, hipStream_t st) {
-  // Non-temporal stores where what is written would push out of the caches what the next kernels read, from about their size on.  A
-  // gradient: six-argument calls of 512 rows x 131,072 labels x 768 dims 384 -> 347 us, 128 rows 212 -> 178, 512 x 200,000 x 256 303
-  // -> 261, x 80,000 x 768 258 -> 241, but x 32,768 118 -> 120.  Master weights: steps of 512 x 655,363 x 768 2868 -> 2813, 64 x
-  // 200,001 717 -> 668, 256 x 131,072 x 256 201 -> 193, but 256 x 20,001 x 768 115 -> 123.  fp16 state: 1024 x 2,812,281 x 768 13.81 ->
-  // 13.67 ms, x 700,001 3.48 -> 3.44, but 800 x 200,001 x 512 684 -> 688, 700 x 131,072 x 256 228 -> 235.  Not only back to back: the
-  // calls of 512 rows x 131,072 each followed by a copy of 512 MiB 567 -> 522, by 0.6 ms of matrix products 1011 -> 978, waited for 409 -> 373.
-  const int64_t weights = (int64_t)a.M * a.N, Mi = (int64_t)1 << 20;
-  // Small ones are written through (see StoreHow).  Over three states in turn and over one (us): master weights 64 rows x 5,001
-  // labels x 768 dims 49.7, 50.3 -> 45.3, 46.7, 300 x 10,001 94, 86 -> 93, 73, but 100 x 20,001 97.6, 83.9 -> 99.2, 81.2; fp16 state 600 x
-  // 8,001 77.1, 77.4 -> 72.6, 73.8, 800 x 60,001 306, 305 -> 304, 301, but 1024 x 131,072 687 -> 694.  Gradients, six-argument calls of 128 x
-  // 20,000 50.9 -> 47.9; by themselves, with G out of HBM, larger ones lose: 256 x 23,293 x 1024 32 -> 37, 512 x 27,823 x 1024 49 -> 61.
-  const bool through = weights <= (mode == DW_UPDATE ? 48 : mode == DW_UPDATE_MASTER ? 12 : 16) * Mi;
-  const bool past = weights > (mode == DW_UPDATE ? 140 : mode == DW_UPDATE_MASTER ? 28 : 40) * Mi;
-  return dw_small_tiles(mode, a.M, a.N, a.K, past) ? launch_dw_tiles<DwCore128>(mode, a, past, through, st)
-                                                   : launch_dw_tiles<DwCore>(mode, a, past, through, st);
+int launch_dw(DwMode mode, const DwArgs& a, hipStream_t st) {
+  const DwPlan p = dw_plan(mode, a.M, a.N, a.K, num_cus());
+  return p.small ? launch_dw_tiles<DwCore128>(mode, a, p.how, st) : launch_dw_tiles<DwCore>(mode, a, p.how, st);
 }
 
 // The one-pass step of small batches (small_step.hpp).  Fn::operator()<S>() is called with the kernel for d dims and B
