@@ -237,7 +237,8 @@ __global__ void __launch_bounds__(C::NT, 160 * 1024 / C::LDS_BYTES) fwd_wide_ker
     if (threadIdx.x == 0) {
       double t = 0.0;
       for (int i = 0; i < C::NW; ++i) t += red[i];
-      a.loss_part[w] = w < a.loss_have ? a.loss_part[w] + t : t;
+      // (only small tiles come after others; asked of large ones too, their kernel keeps 13 more scalars in vector lanes)
+      a.loss_part[w] = C::FM == 4 && w < a.loss_have ? a.loss_part[w] + t : t;
     }
   }
 }
