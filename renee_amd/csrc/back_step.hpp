@@ -35,7 +35,7 @@
 
 namespace xfc {
 
-constexpr int BACK_MAX_ROWS = 256, BACK_TILE = 64, BACK_DIMS = 128, BACK_AHEAD = 2;
+constexpr int BACK_MAX_ROWS = 256, BACK_TILE = 64, BACK_AHEAD = 2;
 enum BackMode { BACK_UPDATE = 0, BACK_OUT = 1, BACK_ADD = 2 };  // ADD: out = G^T.X + beta * out, else without the addend
 
 struct BackArgs {

@@ -124,4 +124,32 @@ inline DwPlan dw_plan(DwMode mode, int64_t labels, int64_t dims, int64_t rows, i
   return {dw_small_tiles(mode, labels, dims, rows, past, cus), past ? PAST : through ? THROUGH : CACHED};
 }
 
+// ---------------------------------------------------------------------------------------------
+// both gradients of a batch of up to 256 rows
+// ---------------------------------------------------------------------------------------------
+constexpr int BACK_DIMS = 128;  // of a slice of the joint pass
+
+// Whether dX and a gradient that is written out take two passes instead of the joint one (back_step.hpp).  Whole micro-batches, time by
+// the joint pass over that by two:
+//   Up to 48 rows of up to 64 dims, which leave half of the joint pass's slice empty: 5 rows 0.9 at 46 Mi weights and 1.12 to 1.16 above, 9 rows
+//   1.13 to 1.17, 33 rows 1.13 and at 100 Mi 1.05.  A gradient that is added to from 8 Mi on, 1.04 to 1.18, but 33 and 48 rows 0.93 to 1.03 from 52 Mi on.
+//   33 to 64 rows of 256 to 383 dims, or 512, up to 110 Mi weights: 256 dims 1.02 to 1.09 from 26 Mi on, 320 dims 1.06 to 1.14, 512 dims 0.87 to 1.05
+//   up to 56 Mi and 33 and 48 rows 1.09 at 100.  Of 33 to 128 rows of 384 to 512 up to 52 Mi only: 0.86 to 1.11 there, 0.87 to 1.05 above.
+//   129 rows and more on long axes where the slices do not come out even with the CUs (768 dims, six of them on 240 CUs: 192 rows x 1,500,001
+//   1.69 against 1.58 ms, 256 rows 1.98 against 1.77; 1024 dims, all CUs: 192 x 700,001 1.00 against 1.04).
+// The last two for a gradient that is only written, which leaves the joint pass little to save, the second reading of G; of one that is
+// added to it takes 0.7 to 0.9 from 46 Mi on.  Elsewhere it is the faster, or the same: up to 32 rows of 256, 512, 768 or 1024 dims x 46 Mi and
+// more 0.83 to 0.96, 33 to 64 rows of 768 or 1024 dims 0.83 to 1.0.  (65 to 128 rows of less than 5 Mi up to 1.2, 2 to 5 us.)
+inline bool gradients_apart(int64_t B, int64_t L, int64_t d, bool adds, int64_t cus) {
+  const int64_t weights = L * d, Mi = (int64_t)1 << 20;
+  if (d <= 64 && B <= 48) return adds ? weights > 8 * Mi && (B <= 32 || weights <= 48 * Mi) : weights > 48 * Mi;
+  if (adds || B <= 32) return false;
+  if (B <= 128) {
+    const int64_t most = B <= 64 && (d < 384 || d == 512) ? 110 : B <= 64 || d >= 384 ? 52 : 0;
+    return d >= 256 && d <= 512 && weights > 20 * Mi && weights <= most * Mi;
+  }
+  const bool even = (cus / 8) % ceil_div(d, BACK_DIMS) == 0;
+  return d % 256 == 0 && !even && weights > 400 * Mi;
+}
+
 }  // namespace xfc

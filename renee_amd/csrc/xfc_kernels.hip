@@ -1627,7 +1627,7 @@ size_t small_step_ws_bytes(int64_t B, int64_t L, int64_t d) {
 // dX and dW (or the update) of a batch of up to 256 rows in one pass over the labels (back_step.hpp).  Fn::operator()<S>() is
 // called with the kernel's sizes for B rows; false if there is none: more rows do not fit the LDS beside two images of their G.
 // (Above 64
-// rows it is the faster one at every size measured; see xfc_dx_dw for the others.)
+// rows it is the faster one at every size measured; see gradients_apart for the others.)
 template <int MODE, class Fn>
 bool back_step_for(int64_t B, Fn&& fn) {
   if (B < 1 || B > BACK_MAX_ROWS) return false;
@@ -2224,22 +2224,8 @@ int xfc_dx_dw_update(const void* G, int64_t ldg, const void* X, int64_t ldx, voi
 int xfc_dx_dw(const void* G, int64_t ldg, const void* X, int64_t ldx, const void* W, int64_t ldw, float* grad, int64_t ld_grad,
               float* dX, int64_t lddx, int64_t B, int64_t L, int64_t d, float beta, float scale, void* workspace,
               size_t workspace_bytes, void* stream) {
-  // Up to 64 rows the two passes read a gradient that no cache holds a little faster (16 rows x 700,001 x 768: 1,043 against 1,089
-  // us; x 320,001 x 768: 497 against 493; x 60,007: 86 to 91 against 97), unless the width leaves their tiles of 256 dims partly
-  // empty (x 700,001 x 384: 609 against 529).  A gradient that is only written leaves the one pass with little to save, the
-  // second reading of G: on long axes it is the slower from 129 rows on where its slices do not come out even with the CUs (768
-  // dims, six of them on 240: 192 rows x 1,500,001 1.58 against 1.69 ms, 256 rows 1.77 against 1.98; 1024 dims, all CUs: 192 x
-  // 700,001 1.04 against 1.00).
-  // 33 to 128 rows of 256 to 512 dims have a stretch of middle sizes, whose gradient and weights the Infinity Cache holds between
-  // two passes, where these write a first gradient the faster (whole steps, joint pass over two: 33 to 64 rows 1.07 to 1.09 x
-  // 384 dims x 131,072 labels, 1.05 x 512 x 60,007, 1.04 x 256 x 131,072; 100 rows 1.03 to 1.05 x 512, 0.97 to 1.01 x 384).
-  // Adding to a gradient has none: two passes 7 to 15 % the slower x 40,007 x 384 and 512, the same up to 131,072.
-  const bool sizes = dims_ok(B) && dims_ok(L) && dims_ok(d) && d > 0;
-  const int64_t weights = sizes ? L * d : 0, Mi = (int64_t)1 << 20;
-  const bool whole = sizes && d % 256 == 0, even = sizes && (num_cus() / 8) % ceil_div(d, BACK_DIMS) == 0;
-  const bool middle = beta == 0.f && B > 32 && B <= (d < 384 ? 64 : 128) && d >= 256 && d <= 512 && weights > 20 * Mi && weights <= 52 * Mi;
-  const bool slow = middle || (whole && ((B <= 64 && weights > 32 * Mi) || (beta == 0.f && B > 128 && !even && weights > 400 * Mi)));
-  if (!slow && back_ok(G, ldg, X, ldx, W, ldw, dX, B, L, d) && grad && ld_grad % 4 == 0 && aligned16(grad)) {
+  const bool apart = dims_ok(B) && dims_ok(L) && dims_ok(d) && d > 0 && gradients_apart(B, L, d, beta != 0.f, num_cus());
+  if (!apart && back_ok(G, ldg, X, ldx, W, ldw, dX, B, L, d) && grad && ld_grad % 4 == 0 && aligned16(grad)) {
     BackArgs a = back_args(G, ldg, X, ldx, W, ldw, B, L, d);
     a.out = grad; a.ldo = ld_grad; a.beta = beta;
     bool taken;

@@ -1,4 +1,4 @@
-"""Which tiles the forward pass and dW take and how dW's outputs are stored (renee_amd/csrc/tile_plan.hpp, where the launches take it from), on
+"""Which tiles the forward pass and dW take, how dW's outputs are stored, and when two gradients take two passes (renee_amd/csrc/tile_plan.hpp, where the launches take it from), on
 256 CUs unless said otherwise; tests that run on the GPU take from here what their sizes lead to."""
 import pytest
 from test_back_wide_order import _compiled
@@ -15,6 +15,8 @@ int main() {
       const FwdPlan p = fwd_plan(M, n, d, more != 0, cus);
       printf("%d %lld %lld %lld %lld %lld\n", (int)p.tile, (long long)p.first, (long long)fwd_ids(p.tile, M, p.first), (long long)fwd_grid(p, M, cus, most),
              (long long)(p.first < n ? fwd_ids(FWD_WIDE128, M, n - p.first) : 0), (long long)fwd_rest_grid(p, M, n, cus, most));
+    } else if (what == 2) {
+      printf("%d\n", (int)gradients_apart(M, n, d, more != 0, cus));
     } else {
       const DwPlan p = dw_plan((DwMode)more, n, d, M, cus);
       printf("%d %d\n", (int)p.small, (int)p.how);
@@ -41,6 +43,10 @@ class Plans:
         lines = _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (1, cus, *s)])
         return [(line.split()[0] == "1", int(line.split()[1])) for line in lines]
 
+    def gradients_apart(self, sizes, cus=256):
+        """(rows, labels, dims, whether the gradient is added to) -> whether the two gradients take two passes."""
+        return [line == "1" for line in _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (2, cus, *s)])]
+
 
 @pytest.fixture(scope="session")
 def plans(tmp_path_factory):
@@ -60,3 +66,14 @@ def test_every_place_that_the_plan_prices_is_taken(plans):
         small += tile == "wide128" and ids >= 512
         rest += rest_ids > 256
     assert small > 50 and rest > 5
+
+
+def test_gradients_take_the_pass_that_measured_faster(plans):
+    """Sizes where one of the two ways took at least a twentieth longer than the other."""
+    joint = [(9, 81921, 512, 0), (16, 163841, 256, 0), (33, 61441, 1024, 0), (64, 122881, 1024, 0), (5, 62805, 768, 0), (64, 62805, 768, 0),
+             (33, 81921, 768, 1), (64, 163841, 768, 1), (9, 1720321, 256, 1), (64, 245761, 256, 1), (48, 114689, 512, 1), (100, 131072, 384, 1),
+             (64, 1638401, 64, 1), (48, 1638401, 64, 1), (9, 262145, 64, 0), (5, 753665, 64, 0), (100, 1638401, 64, 0)]
+    apart = [(9, 917505, 64, 0), (33, 1638401, 64, 0), (9, 294913, 64, 1), (33, 655361, 64, 1), (33, 131073, 256, 0), (64, 229377, 256, 0),
+             (48, 183501, 320, 0), (48, 204801, 512, 0)]
+    assert plans.gradients_apart(joint) == [False] * len(joint)
+    assert plans.gradients_apart(apart) == [True] * len(apart)
