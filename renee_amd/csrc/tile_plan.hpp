@@ -86,9 +86,12 @@ struct DwPlan {
 // and 11.8, 1024 x 20,001 x 1024 83 and 68, 384 x 700,001 x 384 583 and 537, 1024 x 1,000,001 x 128 728 and 636, but 512 x 655,363 x 768
 // 1000 and 1100, 1024 x 131,072 x 768 293 and 327.  Master weights: 300 x 20,001 x 1024 106 and 82, 512 x 131,072 x
 // 768 393 and 373, 512 x 700,001 x 384 1163 and 1064, whole steps of 512 x 450,001 x
-// 768 1943 and 1911, 128 x 450,001 1532 and 1556, 512 x 655,363 2581 and 2629 or 2828 and 2823, 1024 x 655,363 x 768 2262 and 2381.  Gradients: 128 x
+// 768 1943 and 1911, 128 x 450,001 1532 and 1556, 512 x 655,363 2581 and 2629 or 2828 and 2823, 1024 x 655,363 x 768 2262 and 2381.  Of up to 64 rows x 256
+// dims, where the memory alone binds and a large tile writes its labels in one piece: whole steps x 450,561, small over large, 1.04 to 1.07, x 614,401 1.00 to 1.03, x
+// 286,721 0.98 to 0.99 (other widths 0.98 to 1.03, from 200 rows on 0.96 to 0.98).  Gradients: 128 x
 // 131,073 x 768 79.7 and 74.7, 300 x 8,001 x 768 13.2 and 10.0, 512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768 505 and 611, 136 x 1,096,208 x
-// 256 243 and 334, 248 x 234,640 x 1024 204 and 227, 712 x 80,256 x 512 86.8 and 90.7, 32 x 1,000,000 x 128 90 and 100, but 64 rows 97 and 92, 1024 x 20,000 x 1024 62 and 53, 256 x 400,000 x 384 156 and 147.
+// 256 243 and 334, 248 x 234,640 x 1024 204 and 227, 712 x 80,256 x 512 86.8 and 90.7, 32 x 1,000,000 x 128 90 and 100, 64 rows 97 and 92, but all three
+// calls of 64 rows 1.02 to 1.06 from 900,000 labels on and 0.98 x 370,000 to 570,000, of 128 rows x 110 Mi weights x 256, 512, 1024 1.05, 1.04, 1.04; 1024 x 20,000 x 1024 62 and 53, 256 x 400,000 x 384 156 and 147.
 inline bool dw_small_tiles(DwMode mode, int64_t labels, int64_t dims, int64_t rows, bool past, int64_t cus) {
   auto rounds = [&](int64_t tile) {  // (a last one nearly empty leaves the others the more of the memory: half of it counts)
     const double n = (double)(ceil_div(dims, tile) * round_up(ceil_div(labels, tile), 8)) / (double)cus;
@@ -99,12 +102,16 @@ inline bool dw_small_tiles(DwMode mode, int64_t labels, int64_t dims, int64_t ro
   if (mode == DW_UPDATE && past) price += 0.05;
   const int64_t Mi = (int64_t)1 << 20, weights = labels * dims;
   if (mode == DW_OUT) {
-    if (past && dims % DW_TILE == 0 && weights > 120 * Mi) price = 1.4;
+    if (past && dims % DW_TILE == 0 && weights > (rows < 128 ? 120 : 100) * Mi) price = 1.4;
     else if (past && rows >= 256) price = 1.2;
-    else if (past && rows <= 48 && dims > 64 && dims <= DW_SMALL_TILE) price = 2.2;  // (half of a large tile empty: what it multiplies is little)
+    else if (past && rows <= 64 && dims > 64 && dims <= DW_SMALL_TILE) price = 2.2;  // (half of a large tile empty: what it multiplies is little)
     else price += 0.0001 * over;
   }
-  if (mode == DW_UPDATE_MASTER) price = 0.99 + (rows > 512 || weights > (rows <= 128 ? 160 : 380) * Mi ? 0.05 : 0.0);
+  if (mode == DW_UPDATE_MASTER) {
+    price = 0.99;
+    if (rows > 512 || weights > (rows <= 128 ? 160 : 380) * Mi) price = 1.04;
+    else if (past && rows <= 64 && dims == DW_TILE) price = 1.03;
+  }
   return price * rounds(DW_SMALL_TILE) < 4.0 * rounds(DW_TILE);
 }
 // Non-temporal stores where what is written would push out of the caches what the next kernels read, from about their size on.  A

@@ -77,3 +77,14 @@ def test_gradients_take_the_pass_that_measured_faster(plans):
              (48, 183501, 320, 0), (48, 204801, 512, 0)]
     assert plans.gradients_apart(joint) == [False] * len(joint)
     assert plans.gradients_apart(apart) == [True] * len(apart)
+
+
+def test_dw_takes_the_tiles_that_measured_faster(plans):
+    """Sizes where one of the two tiles took at least a thirtieth longer than the other, whole calls."""
+    large = [(16, 450561, 256, MASTER), (35, 451991, 256, MASTER), (64, 450561, 256, MASTER), (16, 386599, 256, MASTER), (9, 614401, 256, MASTER),
+             (64, 1638401, 128, OUT), (40, 1228801, 128, OUT), (128, 450561, 256, OUT), (128, 225281, 512, OUT), (128, 112641, 1024, OUT),
+             (256, 655363, 768, OUT), (512, 131072, 768, OUT)]
+    small = [(16, 1000000, 128, MASTER), (200, 450561, 256, MASTER), (48, 286721, 256, MASTER), (35, 184321, 384, MASTER), (128, 131073, 768, OUT),
+             (600, 4097, 768, UPDATE), (384, 700001, 384, UPDATE), (300, 20001, 1024, MASTER), (128, 409601, 128, OUT)]
+    assert [p[0] for p in plans.dw(large)] == [False] * len(large)
+    assert [p[0] for p in plans.dw(small)] == [True] * len(small)
