@@ -14,6 +14,11 @@ inline int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 // to write back, for outputs about as large as the L2s or smaller; more of them, or pieces of lines, pass the fabric faster when the L2
 // has gathered them.  PAST: as what will not be wanted again, past the Infinity Cache too, for outputs that it would not hold.
 enum StoreHow { CACHED = 0, PAST = 1, THROUGH = 2 };
+// The last two want rows that are whole lines of 128 bytes: a line that two stores, of two labels or of two workgroups, make up is fetched
+// and written twice where the L2 may not gather it: 1.1 to 1.6 times the time (see dw_plan and back_how).
+inline bool whole_lines(const void* p, int64_t ld, int64_t row, int64_t element) {
+  return (reinterpret_cast<uintptr_t>(p) | (uintptr_t)(ld * element) | (uintptr_t)(row * element)) % 128 == 0;
+}
 
 // ---------------------------------------------------------------------------------------------
 // forward pass
@@ -92,7 +97,7 @@ struct DwPlan {
 // 131,073 x 768 79.7 and 74.7, 300 x 8,001 x 768 13.2 and 10.0, 512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768 505 and 611, 136 x 1,096,208 x
 // 256 243 and 334, 248 x 234,640 x 1024 204 and 227, 712 x 80,256 x 512 86.8 and 90.7, 32 x 1,000,000 x 128 90 and 100, 64 rows 97 and 92, but all three
 // calls of 64 rows 1.02 to 1.06 from 900,000 labels on and 0.98 x 370,000 to 570,000, of 128 rows x 110 Mi weights x 256, 512, 1024 1.05, 1.04, 1.04; 1024 x 20,000 x 1024 62 and 53, 256 x 400,000 x 384 156 and 147.
-inline bool dw_small_tiles(DwMode mode, int64_t labels, int64_t dims, int64_t rows, bool past, int64_t cus) {
+inline bool dw_small_tiles(DwMode mode, int64_t labels, int64_t dims, int64_t rows, bool past, bool lines, int64_t cus) {
   auto rounds = [&](int64_t tile) {  // (a last one nearly empty leaves the others the more of the memory: half of it counts)
     const double n = (double)(ceil_div(dims, tile) * round_up(ceil_div(labels, tile), 8)) / (double)cus;
     return 0.5 * (n + ceil(n));
@@ -112,6 +117,7 @@ inline bool dw_small_tiles(DwMode mode, int64_t labels, int64_t dims, int64_t ro
     if (rows > 512 || weights > (rows <= 128 ? 160 : 380) * Mi) price = 1.04;
     else if (past && rows <= 64 && dims == DW_TILE) price = 1.03;
   }
+  if (!lines && dims > DW_SMALL_TILE && dims < DW_TILE && weights > 24 * Mi && price < 1.1) price = 1.1;
   return price * rounds(DW_SMALL_TILE) < 4.0 * rounds(DW_TILE);
 }
 // Non-temporal stores where what is written would push out of the caches what the next kernels read, from about their size on.  A
@@ -124,17 +130,47 @@ inline bool dw_small_tiles(DwMode mode, int64_t labels, int64_t dims, int64_t ro
 // labels x 768 dims 49.7, 50.3 -> 45.3, 46.7, 300 x 10,001 94, 86 -> 93, 73, but 100 x 20,001 97.6, 83.9 -> 99.2, 81.2; fp16 state 600 x
 // 8,001 77.1, 77.4 -> 72.6, 73.8, 800 x 60,001 306, 305 -> 304, 301, but 1024 x 131,072 687 -> 694.  Gradients, six-argument calls of 128 x
 // 20,000 50.9 -> 47.9; by themselves, with G out of HBM, larger ones lose: 256 x 23,293 x 1024 32 -> 37, 512 x 27,823 x 1024 49 -> 61.
-inline DwPlan dw_plan(DwMode mode, int64_t labels, int64_t dims, int64_t rows, int64_t cus) {
+// Rows that are not whole lines are stored as usual, all but small ones, and those of 129 to 255 dims and more than 24 Mi weights by large tiles, whose workgroups share
+// no line of a label.  Whole calls, by the rules of whole lines and as usual (us): updates of 16 rows x 36 Mi weights of 136 dims 177 and 134, of 776 148 and
+// 110, of 1000 136 and 113, x 150 Mi of 136 703 and 511, of 776 624 and 501, 128 rows x 150 Mi of 200 772 and 580; master weights 16 x 36 Mi of 776 248 and
+// 220, 128 x 150 Mi of 200 1323 and 1072; gradients of 16 x 150 Mi of 776 404 and 294, 128 x 150 Mi of 200 510 and 394, but 6 to 12 Mi 0.94 to 0.97.
+inline DwPlan dw_plan(DwMode mode, int64_t labels, int64_t dims, int64_t rows, bool lines, int64_t cus) {
   const int64_t weights = labels * dims, Mi = (int64_t)1 << 20;
-  const bool through = weights <= (mode == DW_UPDATE ? 48 : mode == DW_UPDATE_MASTER ? 12 : 16) * Mi;
+  const bool through = weights <= (mode == DW_OUT ? 16 : mode == DW_UPDATE ? (lines ? 48 : 3) : lines ? 12 : 0) * Mi;
   const bool past = weights > (mode == DW_UPDATE ? 140 : mode == DW_UPDATE_MASTER ? 28 : 40) * Mi;
-  return {dw_small_tiles(mode, labels, dims, rows, past, cus), past ? PAST : through ? THROUGH : CACHED};
+  return {dw_small_tiles(mode, labels, dims, rows, past, lines, cus), past && lines ? PAST : through ? THROUGH : CACHED};
 }
 
 // ---------------------------------------------------------------------------------------------
 // both gradients of a batch of up to 256 rows
 // ---------------------------------------------------------------------------------------------
 constexpr int BACK_DIMS = 128;  // of a slice of the joint pass
+
+// How the joint pass stores what it writes, weights and momentum or a gradient.
+// PAST, the loads of these arrays with the same hint, from where they push out of the Infinity Cache (256 MB) what the forward pass left there of G and the
+// weights.  Whole steps with the hint over without, 9 to 256 rows x 64 to 1024 dims, means at some MiB of weights and momentum:
+//                                              80     120     150     180     210     240     320     480
+//   a state by itself, back to back          1.10    1.08    1.07    1.05    1.02    1.00    0.99    0.95
+//   three states in turn                     1.02    0.96    0.94    0.94    0.94    0.94    0.92    0.91
+//   with 0.6 ms of matrix products between   1.08    1.05    1.00    1.00    1.00    1.00    0.98
+//   with a copy of 256 MiB between                   0.97    0.97    0.97    0.97    0.96
+// (The products' operands are 96 MB, and their columns 110, 150, 180, 200, 220, 245 and 300.)  By itself a state of few rows loses the most, 9 to 64 rows x 150 MiB
+// 1.1 to 1.17, 224 and 256 rows x 180 0.96 to 1.08: what it stores through the caches is written back by whoever runs next, which is nobody there.  A
+// training step has the encoder's between, so the line is where the last three have come even.  A gradient: two micro-batches of 128 x 50,001 x 384 (110
+// MiB with W) without and with 167 and 169, by themselves 158 and 161, with products 793 and 794, of 100 x 90,001 x 384 (198) 270, 260, 907 and 269, 263, 904.
+// THROUGH for small updates.  Whole steps, over three states in turn and over one (us): 64 rows x 4,097 labels x 768 dims 25.2 -> 24.0, 100 x 10,001 40.5,
+// 40.7 -> 39.1, 38.8, 200 x 20,001 66.5, 60.7 -> 65.7, 59.6; but 100 x 40,001 88.4, 80.1 -> 90.4, 77.8.  (Of a gradient it makes no difference: 200 x 5,001 to
+// 256 x 40,001 x 384.)
+// Where rows are not whole lines, as a rule neither.  PAST over CACHED, a state by itself, three, and with the copy between: 9 rows x 150 MiB of 136 dims 1.66, 1.14,
+// 1.14, of 200 1.66, 1.32, 1.34, of 776 1.51, 1.15, 1.16, 256 rows x 245 MiB of 776 1.22, 1.17, 1.15, 48 x 245 of 56 1.10, 1.05, 1.06 (of 24 and 40 dims 0.97 to
+// 1.04); a gradient that is added to 1.0 to 1.29, one that is written 1.05 to 1.4 of 9 rows or 150 Mi weights, but 0.87 to 1.04 of 64 to 256 rows x 70 Mi.
+// THROUGH over CACHED 64 rows x 62 MiB of 72 dims 1.24, of 200 1.29, of 776 1.10, 256 x 30 MiB 1.05 to 1.07, but 0.93 to 0.97 of 6 MiB.
+inline StoreHow back_how(bool update, bool adds, int64_t B, int64_t L, int64_t d, bool lines) {
+  const int64_t weights = L * d, Mi = (int64_t)1 << 20;
+  if (weights * (update ? 4 : 6) > (update ? 144 : 224) * Mi)
+    return lines || (!update && !adds && B >= 64 && weights <= 100 * Mi) ? PAST : CACHED;
+  return update && weights * 4 <= (lines ? 64 : 8) * Mi ? THROUGH : CACHED;
+}
 
 // Whether dX and a gradient that is written out take two passes instead of the joint one (back_step.hpp).  Whole micro-batches, time by
 // the joint pass over that by two:

@@ -1567,7 +1567,10 @@ int launch_dw_tiles(DwMode mode, DwArgs a, StoreHow how, hipStream_t st) {
   return launch(std::integral_constant<int, DW_OUT>{});
 }
 int launch_dw(DwMode mode, const DwArgs& a, hipStream_t st) {
-  const DwPlan p = dw_plan(mode, a.M, a.N, a.K, num_cus());
+  const bool lines = mode == DW_OUT      ? whole_lines(a.out, a.ldo, a.N, 4)
+                     : mode == DW_UPDATE ? whole_lines(a.Wt, a.ldw, a.N, 2) && whole_lines(a.Mo, a.ldm, a.N, 2)
+                                         : whole_lines(a.W32, a.ldw32, a.N, 4) && whole_lines(a.M32, a.ldm32, a.N, 4);
+  const DwPlan p = dw_plan(mode, a.M, a.N, a.K, lines, num_cus());
   return p.small ? launch_dw_tiles<DwCore128>(mode, a, p.how, st) : launch_dw_tiles<DwCore>(mode, a, p.how, st);
 }
 
@@ -1695,28 +1698,16 @@ int launch_back(BackArgs a, float* dX, int64_t lddx, float scale, void* ws, size
   a.slices = ceil_div(a.d, BACK_DIMS);
   a.tiles = ceil_div(a.L, BACK_TILE);
   a.part = reinterpret_cast<float*>(ws);
-  // Non-temporal loads and stores of the arrays that are written, from where these push out of the Infinity Cache (256 MB) what the
-  // forward pass left there of G and the weights.  Whole steps with the hint from 224 MiB of weights and momentum on and with it
-  // as here, over three states in turn, over one, and over one with 0.6 ms of matrix products before each (us): 256 rows x 60,001 labels x
-  // 768 dims 148, 133, 796 -> 133, 132, 789; 100 x 70,001 x 768 142, 132, 763 -> 132, 131, 765; 200 x 120,001 x 384 146, 130, 783 -> 138,
-  // 137, 770; but 256 x 40,001 x 768 (117 MiB) 117, 99, 746 -> 107, 106, 740.  A gradient: two micro-batches of 128 x 50,001 x 384 (110
-  // MiB with W) 167, 158, 793 -> 169, 161, 794, of 100 x 90,001 x 384 (198) 270, 260, 907 -> 269, 263, 904.
-  // Not only back to back: steps of 256 x 131,072 x 768 each followed by a copy of 512 MiB 483 -> 451, by 0.6 ms of matrix products 890
-  // -> 868, waited for 277 -> 274; of 100 x 400,001 x 384 566 -> 543 and 956 -> 941, but waited for 346 -> 385: what is stored through
-  // the caches is written back by whoever runs next.  (Those are of the pass from the first labels on.)
-  const bool nt = (int64_t)a.L * a.d * (MODE == BACK_UPDATE ? 4 : 6) > (int64_t)(MODE == BACK_UPDATE ? 144 : 224) << 20;
-  // Small updates are written through.  Whole steps, over three states in turn and over one (us): 64 rows x 4,097 labels x 768 dims
-  // 25.2 -> 24.0, 100 x 10,001 40.5, 40.7 -> 39.1, 38.8, 200 x 20,001 66.5, 60.7 -> 65.7, 59.6; but 100 x 40,001 88.4, 80.1 -> 90.4, 77.8.  (Of
-  // a gradient it makes no difference: 200 x 5,001 to 256 x 40,001 x 384.)
-  const bool small = (int64_t)a.L * a.d * 4 <= (int64_t)64 << 20;
+  const bool lines = MODE == BACK_UPDATE ? whole_lines(a.W, a.ldw, a.d, 2) && whole_lines(a.Mo, a.ldm, a.d, 2) : whole_lines(a.out, a.ldo, a.d, 4);
+  const StoreHow how = back_how(MODE == BACK_UPDATE, MODE == BACK_ADD, a.B, a.L, a.d, lines);
   int rc = XFC_OK;
   *taken = back_step_for<MODE>(a.B, [&](auto s) {
     using S = decltype(s);
     const dim3 g((unsigned)(a.slices * a.ranges)), b(S::NT);
     constexpr int SMALL = MODE == BACK_UPDATE ? THROUGH : CACHED;
-    rc = nt      ? launch_k<back_step_kernel<S, MODE, PAST>>(g, b, S::LDS_BYTES, st, a)
-         : small ? launch_k<back_step_kernel<S, MODE, SMALL>>(g, b, S::LDS_BYTES, st, a)
-                 : launch_k<back_step_kernel<S, MODE, CACHED>>(g, b, S::LDS_BYTES, st, a);
+    rc = how == PAST      ? launch_k<back_step_kernel<S, MODE, PAST>>(g, b, S::LDS_BYTES, st, a)
+         : how == THROUGH ? launch_k<back_step_kernel<S, MODE, SMALL>>(g, b, S::LDS_BYTES, st, a)
+                          : launch_k<back_step_kernel<S, MODE, CACHED>>(g, b, S::LDS_BYTES, st, a);
     if (rc) return;
     launch_dx_reduce(a.part, dX, lddx, a.B, a.d, a.ranges * a.parts, scale, 0.0f, st);
     rc = check_launch();

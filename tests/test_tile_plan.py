@@ -8,8 +8,8 @@ TEXT = r'''
 #include "tile_plan.hpp"
 int main() {
   using namespace xfc;
-  long long what, cus, M, n, d, more;
-  while (scanf("%lld %lld %lld %lld %lld %lld", &what, &cus, &M, &n, &d, &more) == 6) {
+  long long what, cus, M, n, d, more, lines;
+  while (scanf("%lld %lld %lld %lld %lld %lld %lld", &what, &cus, &M, &n, &d, &more, &lines) == 7) {
     if (what == 0) {
       const long long most = more ? 512 : ANY_GRID;  // 4096 bytes of doubles
       const FwdPlan p = fwd_plan(M, n, d, more != 0, cus);
@@ -17,15 +17,18 @@ int main() {
              (long long)(p.first < n ? fwd_ids(FWD_WIDE128, M, n - p.first) : 0), (long long)fwd_rest_grid(p, M, n, cus, most));
     } else if (what == 2) {
       printf("%d\n", (int)gradients_apart(M, n, d, more != 0, cus));
+    } else if (what == 3) {
+      printf("%d\n", (int)back_how(more == 1, more == 2, M, n, d, lines != 0));
     } else {
-      const DwPlan p = dw_plan((DwMode)more, n, d, M, cus);
+      const DwPlan p = dw_plan((DwMode)more, n, d, M, lines != 0, cus);
       printf("%d %d\n", (int)p.small, (int)p.how);
     }
   }
 }
 '''
 TILES = ("64", "128", "wide", "wide128")
-OUT, UPDATE, MASTER = 0, 1, 2
+OUT, UPDATE, MASTER = 0, 1, 2  # of dW
+ADD = 2  # of the joint pass, beside OUT and UPDATE
 CACHED, PAST, THROUGH = 0, 1, 2
 
 
@@ -35,17 +38,21 @@ class Plans:
 
     def forward(self, sizes, cus=256):
         """(rows, labels, dims, with the loss) -> tile, labels it takes, tiles, workgroups; tiles and workgroups of the labels after them."""
-        lines = _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (0, cus, *s)])
+        lines = _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (0, cus, *s, 0)])
         return [(TILES[int(line.split()[0])], *map(int, line.split()[1:])) for line in lines]
 
-    def dw(self, sizes, cus=256):
-        """(rows, labels, dims, mode) -> whether by small tiles, how what is written is stored."""
-        lines = _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (1, cus, *s)])
+    def dw(self, sizes, cus=256, whole=True):
+        """(rows, labels, dims, mode) -> whether by small tiles, how what is written is stored; `whole`: its rows are whole lines."""
+        lines = _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (1, cus, *s, whole)])
         return [(line.split()[0] == "1", int(line.split()[1])) for line in lines]
 
     def gradients_apart(self, sizes, cus=256):
         """(rows, labels, dims, whether the gradient is added to) -> whether the two gradients take two passes."""
-        return [line == "1" for line in _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (2, cus, *s)])]
+        return [line == "1" for line in _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (2, cus, *s, 0)])]
+
+    def back(self, sizes, whole=True):
+        """(rows, labels, dims, mode: UPDATE, OUT, or ADD) -> how the joint pass stores weights and momentum, or the gradient."""
+        return [int(line) for line in _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (3, 256, *s, whole)])]
 
 
 @pytest.fixture(scope="session")
@@ -88,3 +95,19 @@ def test_dw_takes_the_tiles_that_measured_faster(plans):
              (600, 4097, 768, UPDATE), (384, 700001, 384, UPDATE), (300, 20001, 1024, MASTER), (128, 409601, 128, OUT)]
     assert [p[0] for p in plans.dw(large)] == [False] * len(large)
     assert [p[0] for p in plans.dw(small)] == [True] * len(small)
+
+
+def test_rows_that_are_not_whole_lines_are_stored_as_usual(plans):
+    """Stored past the L2 they took 1.1 to 1.6 times as long; those of 129 to 255 dims go by tiles that share no line."""
+    sizes = [(B, mi * (1 << 20) // d, d, mode) for B in (1, 16, 128, 600) for mi in (20, 50, 200) for d in (72, 136, 200, 776, 1000) for mode in (OUT, UPDATE, MASTER)]
+    assert {how for _, how in plans.dw(sizes, whole=False)} == {CACHED}
+    assert {how for _, how in plans.dw(sizes)} == {CACHED, PAST, THROUGH}
+    joint = [(B, mi * (1 << 20) // d, d, mode) for B in (1, 16, 128, 256) for mi in (4, 15, 30, 120) for d in (72, 136, 200, 776) for mode in (OUT, UPDATE, ADD)]
+    assert set(plans.back(joint, whole=False)) == {CACHED}
+    assert set(plans.back(joint)) == {CACHED, PAST, THROUGH}
+    large = [(16, 80 * (1 << 20) // d, d, mode) for d in (136, 200, 248) for mode in (OUT, UPDATE, MASTER)]
+    assert {small for small, _ in plans.dw(large, whole=False)} == {False}
+    ours = [(100, 20001, 768, UPDATE), (100, 40001, 768, UPDATE), (100, 80001, 768, UPDATE), (100, 40001, 768, OUT), (100, 80001, 768, ADD)]
+    assert plans.back(ours) == [THROUGH, CACHED, PAST, CACHED, PAST]
+    small = [(100, 2001, 776, UPDATE), (100, 90001, 776, OUT), (9, 90001, 776, OUT), (100, 90001, 776, ADD), (100, 200001, 776, OUT)]
+    assert plans.back(small, whole=False) == [THROUGH, PAST, CACHED, CACHED, CACHED]
