@@ -1,5 +1,6 @@
-// Which tiles the forward pass and dW take, on how many workgroups, and how dW's outputs are stored, as arithmetic on sizes and the number of
-// CUs: the launches take it from here, and tests/test_tile_plan.py goes through it on the host.  Plain C++, nothing of the GPU.
+// Which tiles the forward pass and dW take, on how many workgroups, how dW and the joint pass of up to 256 rows store what they write, and when two
+// gradients take two passes, as arithmetic on sizes, alignment and the number of CUs: the launches take it from here, and tests/test_tile_plan.py goes
+// through it on the host.  Plain C++, nothing of the GPU.
 #pragma once
 #include <math.h>
 #include <stdint.h>
@@ -82,21 +83,22 @@ struct DwPlan {
   bool small;    // tiles of DW_SMALL_TILE
   StoreHow how;  // what is written
 };
-// Large tiles move the fewest bytes through the fetch path and the L2s, small ones fill the chip with few labels, leave no last round
-// nearly empty, waste less of a width that is no multiple of 256, and two of them on a CU work at each other's epilogues.  Compared
-// by rounds of the large ones, four small tiles to one of them at a price: nothing while the update's traffic binds, up to a sixth
-// (of a gradient a quarter) at 1024 rows, 0.05 more for a state that no cache holds (fp32: from 160 Mi weights on); of a gradient a fifth for one that none does and
-// 256 rows or more, two fifths for a large one of whole large tiles, whose rows a small tile writes in pieces of 512 bytes.  Measured
-// (us, large and small).  Updates: 32 rows x 8,001 labels x 256 dims 10.9 and 5.7, 128 x 30,001 x 768 46 and 37, 600 x 4,097 x 768 22.3
-// and 11.8, 1024 x 20,001 x 1024 83 and 68, 384 x 700,001 x 384 583 and 537, 1024 x 1,000,001 x 128 728 and 636, but 512 x 655,363 x 768
-// 1000 and 1100, 1024 x 131,072 x 768 293 and 327.  Master weights: 300 x 20,001 x 1024 106 and 82, 512 x 131,072 x
-// 768 393 and 373, 512 x 700,001 x 384 1163 and 1064, whole steps of 512 x 450,001 x
-// 768 1943 and 1911, 128 x 450,001 1532 and 1556, 512 x 655,363 2581 and 2629 or 2828 and 2823, 1024 x 655,363 x 768 2262 and 2381.  Of up to 64 rows x 256
-// dims, where the memory alone binds and a large tile writes its labels in one piece: whole steps x 450,561, small over large, 1.04 to 1.07, x 614,401 1.00 to 1.03, x
-// 286,721 0.98 to 0.99 (other widths 0.98 to 1.03, from 200 rows on 0.96 to 0.98).  Gradients: 128 x
-// 131,073 x 768 79.7 and 74.7, 300 x 8,001 x 768 13.2 and 10.0, 512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768 505 and 611, 136 x 1,096,208 x
-// 256 243 and 334, 248 x 234,640 x 1024 204 and 227, 712 x 80,256 x 512 86.8 and 90.7, 32 x 1,000,000 x 128 90 and 100, 64 rows 97 and 92, but all three
-// calls of 64 rows 1.02 to 1.06 from 900,000 labels on and 0.98 x 370,000 to 570,000, of 128 rows x 110 Mi weights x 256, 512, 1024 1.05, 1.04, 1.04; 1024 x 20,000 x 1024 62 and 53, 256 x 400,000 x 384 156 and 147.
+// Large tiles move the fewest bytes through the fetch path and the L2s; small ones fill the chip with few labels, leave no last round nearly empty, waste less of a
+// width that is no multiple of 256, and two of them on a CU work at each other's epilogues.  Compared by rounds of the large ones, four small tiles to one of
+// them at a price (in brackets, large and small in us, by themselves unless they are calls):
+//   Updates: none while the update's traffic binds, up to a sixth at 1024 rows, whose operands do [32 rows x 8,001 labels x 256 dims 10.9 and 5.7, 128 x 30,001 x
+//   768 46 and 37, 600 x 4,097 x 768 22.3 and 11.8, 1024 x 20,001 x 1024 83 and 68, but 1024 x 131,072 x 768 293 and 327], 0.05 more for a state that no cache
+//   holds [384 x 700,001 x 384 583 and 537, 1024 x 1,000,001 x 128 728 and 636, but 512 x 655,363 x 768 1000 and 1100].
+//   Master weights, 18 bytes each, bind at any rows: none, 0.05 for the most rows and weights [300 x 20,001 x 1024 106 and 82, 512 x 131,072 x 768 393 and 373, 512 x
+//   700,001 x 384 1163 and 1064, steps of 512 x 450,001 x 768 1943 and 1911, 128 x 450,001 1532 and 1556, 512 x 655,363 2581 and 2629 or 2828 and 2823, 1024 x
+//   655,363 2262 and 2381].  Of up to 64 rows x 256 dims a large tile writes its labels in one piece [steps, small over large, x 450,561 1.04 to 1.07, x 614,401
+//   1.00 to 1.03, x 286,721 0.98 to 0.99; other widths 0.98 to 1.03, from 200 rows on 0.96 to 0.98].
+//   Gradients that the caches hold: up to a quarter at 1024 rows [300 x 8,001 x 768 13.2 and 10.0, 1024 x 20,000 x 1024 62 and 53].  Others go straight to HBM, in
+//   pieces of a tile's width by label, 512 bytes of a small one and 1 KB of a large one: a fifth from 256 rows on
+//   [256 x 400,000 x 384 156 and 147, 712 x 80,256 x 512 86.8 and 90.7], two fifths where large ones are whole [512 x 131,072 x 768 121 and 129, 256 x 655,363 x 768
+//   505 and 611, 136 x 1,096,208 x 256 243 and 334, 248 x 234,640 x 1024 204 and 227, but 128 x 131,073 x 768 79.7 and 74.7; calls of 128 rows x 110 Mi weights x
+//   256, 512, 1024, small over large, 1.05, 1.04, 1.04].  Of up to 64 rows x 65 to 128 dims both write the same pieces, and large ones in longer runs of them [32 x
+//   1,000,000 x 128 90 and 100; 64 rows 97 and 92, but calls, small over large, 1.02 to 1.06 from 900,000 labels on and 0.98 x 370,000 to 570,000].
 inline bool dw_small_tiles(DwMode mode, int64_t labels, int64_t dims, int64_t rows, bool past, bool lines, int64_t cus) {
   auto rounds = [&](int64_t tile) {  // (a last one nearly empty leaves the others the more of the memory: half of it counts)
     const double n = (double)(ceil_div(dims, tile) * round_up(ceil_div(labels, tile), 8)) / (double)cus;

@@ -984,9 +984,9 @@ __global__ void __launch_bounds__(32 * SG) dx_reduce_kernel(const float* __restr
 // dW = G^T . X; either written out (fp32, alpha/beta) or consumed by the momentum update
 // ---------------------------------------------------------------------------------------------
 // 256 labels x 256 dims x 64 batch rows per stage, eight waves of 64 labels x 128 dims, one workgroup per CU.
-// (A 128 x 256 x 32 tile with four waves and two workgroups per CU, meant to overlap one workgroup's update with
-// the other's GEMM, measured 7-11 % slower at every batch size: its stages move half again as much through LDS
-// and the fetch path per flop, and the update's streaming is bound by HBM either way.)
+// (A 128 x 256 x 32 tile with four waves and two workgroups per CU measured 7-11 % slower at every batch size tried: its stages are half as
+// deep, and move half again as much through LDS and the fetch path per flop.  DwCore128 keeps the depth of 64 rows and eight waves; per flop it
+// moves twice what DwCore does, and is taken where that is not what binds.)
 using DwCore = PipeCore<256, 256, 64, 4, 2, 2, false, false, false, false, false, 4>;
 // 128 labels x 128 dims, eight waves of 32 x 64, two workgroups to a CU: see dw_plan.
 using DwCore128 = PipeCore<128, 128, 64, 4, 2, 2, false, false, false, false, false, 4>;
