@@ -1,4 +1,4 @@
-// Which tiles the forward pass and dW take, on how many workgroups, how dW and the joint pass of up to 256 rows store what they write, and when two
+// Which tiles the forward pass and dW take, on how many workgroups, how dX, dW and the joint pass of up to 256 rows store what they write, and when two
 // gradients take two passes, as arithmetic on sizes, alignment and the number of CUs: the launches take it from here, and tests/test_tile_plan.py goes
 // through it on the host.  Plain C++, nothing of the GPU.
 #pragma once
@@ -16,7 +16,7 @@ inline int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
 // has gathered them.  PAST: as what will not be wanted again, past the Infinity Cache too, for outputs that it would not hold.
 enum StoreHow { CACHED = 0, PAST = 1, THROUGH = 2 };
 // The last two want rows that are whole lines of 128 bytes: a line that two stores, of two labels or of two workgroups, make up is fetched
-// and written twice where the L2 may not gather it: 1.1 to 1.6 times the time (see dw_plan and back_how).
+// and written twice where the L2 may not gather it: 1.1 to 1.6 times the time (see dw_plan, dx_how and back_how).
 inline bool whole_lines(const void* p, int64_t ld, int64_t row, int64_t element) {
   return (reinterpret_cast<uintptr_t>(p) | (uintptr_t)(ld * element) | (uintptr_t)(row * element)) % 128 == 0;
 }
@@ -141,6 +141,19 @@ inline DwPlan dw_plan(DwMode mode, int64_t labels, int64_t dims, int64_t rows, b
   const bool through = weights <= (mode == DW_OUT ? 16 : mode == DW_UPDATE ? (lines ? 48 : 3) : lines ? 12 : 0) * Mi;
   const bool past = weights > (mode == DW_UPDATE ? 140 : mode == DW_UPDATE_MASTER ? 28 : 40) * Mi;
   return {dw_small_tiles(mode, labels, dims, rows, past, lines, cus), past && lines ? PAST : through ? THROUGH : CACHED};
+}
+
+// ---------------------------------------------------------------------------------------------
+// dX
+// ---------------------------------------------------------------------------------------------
+// How dX's partial sums are stored.  Those that the L2s hold much of through them: six-argument calls of 512 rows x 20,000 labels x 768 dims 92.5 -> 90.0
+// us, steps of 600 x 8,001 77.0 -> 75.4, x 20,001 115.4 -> 113.7, but 512 x 60,000 192.6 -> 194.2, 1024 x 60,001 x 256 179 -> 184, and longer axes, whose pass is not
+// waited for as long, too (dX by itself: 100 x 119,605 x 384 35.2 -> 37.2, 899 x 106,385 x 768 162 -> 167).  Not where rows that are not whole lines go by tiles
+// of 256 rows, whose waves share the lines about dim 128: dX by itself through and as usual, 200 rows x 1,001 labels x 200 dims 15.4 and 12.0, 512 x 20,001 x
+// 328 30.0 and 26.2, 1024 x 4,001 x 776 31.5 and 29.1; up to 128 dims or rows through 0.94 to 0.95 of as usual, whatever the width.
+inline StoreHow dx_how(int64_t rows, int64_t dims, int64_t labels, int64_t bytes, bool lines) {
+  const bool apart = lines || rows <= 128 || dims <= 128;
+  return apart && bytes <= (int64_t)48 << 20 && labels <= 40000 ? THROUGH : CACHED;
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -1527,9 +1527,6 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
   if (grid <= 0 || M <= 0 || N <= 0) return XFC_OK;
   const dim3 g((unsigned)grid);
   int rc;
-  // Partial sums that the L2s hold much of are written through: six-argument calls of 512 rows x 20,000 labels x 768 dims 92.5 -> 90.0
-  // us, steps of 600 x 8,001 77.0 -> 75.4, x 20,001 115.4 -> 113.7, but 512 x 60,000 192.6 -> 194.2, 1024 x 60,001 x 256 179 -> 184,
-  // and longer axes, whose pass is not waited for as long, too (dX by itself: 100 x 119,605 x 384 35.2 -> 37.2, 899 x 106,385 x 768 162 -> 167).
   auto launch = [&](auto how) {
     constexpr int HOW = decltype(how)::value;
     switch (row_tile(M)) {
@@ -1538,7 +1535,8 @@ int launch_dx(const half_t* G, int64_t ldg, const half_t* W, int64_t ldw, float*
       default: return launch_k<dx_wide_kernel<HOW>>(g, dim3(DxWide::NT), DxWide::LDS_BYTES, st, a);
     }
   };
-  rc = need <= (size_t)48 << 20 && K <= 40000 ? launch(std::integral_constant<int, THROUGH>{}) : launch(std::integral_constant<int, CACHED>{});
+  const bool through = dx_how(M, N, K, (int64_t)need, whole_lines(a.part, N, N, 4)) == THROUGH;
+  rc = through ? launch(std::integral_constant<int, THROUGH>{}) : launch(std::integral_constant<int, CACHED>{});
   if (rc) return rc;
   launch_dx_reduce(a.part, out, ldo, M, N, a.splits, alpha, beta, st);
   return check_launch();

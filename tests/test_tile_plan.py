@@ -17,6 +17,8 @@ int main() {
              (long long)(p.first < n ? fwd_ids(FWD_WIDE128, M, n - p.first) : 0), (long long)fwd_rest_grid(p, M, n, cus, most));
     } else if (what == 2) {
       printf("%d\n", (int)gradients_apart(M, n, d, more != 0, cus));
+    } else if (what == 4) {
+      printf("%d\n", (int)dx_how(M, d, n, more, lines != 0));
     } else if (what == 3) {
       printf("%d\n", (int)back_how(more == 1, more == 2, M, n, d, lines != 0));
     } else {
@@ -53,6 +55,10 @@ class Plans:
     def back(self, sizes, whole=True):
         """(rows, labels, dims, mode: UPDATE, OUT, or ADD) -> how the joint pass stores weights and momentum, or the gradient."""
         return [int(line) for line in _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (3, 256, *s, whole)])]
+
+    def dx(self, sizes, whole=True):
+        """(rows, labels, dims, bytes of partial sums) -> how these are stored."""
+        return [int(line) for line in _compiled(self.tmp, TEXT, [int(v) for s in sizes for v in (4, 256, *s, whole)])]
 
 
 @pytest.fixture(scope="session")
@@ -111,3 +117,11 @@ def test_rows_that_are_not_whole_lines_are_stored_as_usual(plans):
     assert plans.back(ours) == [THROUGH, CACHED, PAST, CACHED, PAST]
     small = [(100, 2001, 776, UPDATE), (100, 90001, 776, OUT), (9, 90001, 776, OUT), (100, 90001, 776, ADD), (100, 200001, 776, OUT)]
     assert plans.back(small, whole=False) == [THROUGH, PAST, CACHED, CACHED, CACHED]
+
+
+def test_partial_sums_of_shared_lines_are_stored_as_usual(plans):
+    """Tiles of 256 rows x 256 dims, two waves to a row: 1.05 to 1.36 times as long through the L2s from 129 rows and dims on."""
+    sizes = [(B, L, d, 1 << 20) for B in (129, 200, 512, 1024) for L in (1001, 20001) for d in (136, 200, 328, 776, 1000)]
+    assert set(plans.dx(sizes, whole=False)) == {CACHED} and set(plans.dx(sizes)) == {THROUGH}
+    assert set(plans.dx([(128, 1001, 776, 1 << 20), (512, 1001, 72, 1 << 20)], whole=False)) == {THROUGH}
+    assert set(plans.dx([(128, 40001, 768, 1 << 20), (512, 1001, 768, 49 << 20)])) == {CACHED}
